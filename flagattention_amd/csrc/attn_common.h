@@ -98,18 +98,24 @@ int launch_fast(const AttnArgs& a, int head_dim, int v_dtype, bool causal, hipSt
 // workgroups share the keys of one (batch, head, q-block), 1 when the launch fills the chip anyway.
 // apply_key_split turns the arguments of the unsplit launch into those of the split one (partial results in
 // `workspace`, key_split_workspace_bytes large); launch_split_combine writes what the unsplit launch would have.
-int plan_key_split(int64_t batch, int64_t heads_q, int64_t qo_len, int64_t kv_len, bool causal);
+int plan_key_split(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal);
 int64_t key_split_workspace_bytes(int nsplit, int64_t batch, int64_t heads_q, int64_t qo_len, int64_t head_dim);
 void apply_key_split(AttnArgs& a, int nsplit, int64_t batch, int head_dim, void* workspace);
 int launch_split_combine(const AttnArgs& split, const AttnArgs& whole, int head_dim, int64_t batch, hipStream_t stream);
 
-// The same kernel under a bool mask tensor or an additive fp16 / bf16 one, where fast_serves_mask() says so (a.mask
+// The kernel for few query rows (attn_decode.hip): no mask tensor, qo_len rows of each query head that shares a K/V
+// head, kDecodeRows of them at most; any kv_len, causal with any qo_len.  Splits its keys like the pipelined kernel.
+constexpr int kDecodeRows = 64;
+bool decode_serves(int64_t heads_q, int64_t heads_kv, int64_t qo_len);
+int launch_decode(const AttnArgs& a, int64_t batch, int head_dim, int v_dtype, bool int8, hipStream_t stream);
+
+// The pipelined kernel under a bool mask tensor or an additive fp16 / bf16 one, where fast_serves_mask() says so (a.mask
 // set; esz: bytes per mask entry).
 bool fast_serves_mask(const AttnArgs& a, int esz);
 int launch_fast_masked(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
 int launch_fast_additive(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
 
-// The same kernel on 16-bit Q and K (dense attention); causal with any qo_len / kv_len.
+// The pipelined kernel on 16-bit Q and K (dense attention); causal with any qo_len / kv_len.
 int launch_flash(const AttnArgs& a, int head_dim, int dtype, bool causal, hipStream_t stream);
 
 }  // namespace attn

@@ -471,7 +471,7 @@ namespace {
 // The calls the pipelined kernel serves without a mask tensor are the ones whose keys can be split.
 int attn_key_splits(const sage_attn_params& p) {
     if (p.mask_kind != SAGE_MASK_NONE || (p.causal && p.qo_len > p.kv_len)) return 1;
-    return attn::plan_key_split(p.batch, p.heads_q, p.qo_len, p.kv_len, p.causal != 0);
+    return attn::plan_key_split(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0);
 }
 }  // namespace
 
@@ -526,15 +526,20 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
     else if (p.causal) mode = MODE_CAUSAL;
     const bool fast = p.mask_kind == SAGE_MASK_NONE && (!p.causal || p.qo_len <= p.kv_len);
     if (fast) {
+        const bool decode = attn::decode_serves(p.heads_q, p.heads_kv, p.qo_len);
+        auto launch = [&](const AttnArgs& x) {
+            return decode ? attn::launch_decode(x, p.batch, (int)p.head_dim, p.v_dtype, true, stream)
+                          : attn::launch_fast(x, (int)p.head_dim, p.v_dtype, p.causal != 0, stream);
+        };
         const int nsplit = workspace ? attn_key_splits(p) : 1;
         if (nsplit > 1 && workspace_bytes >= attn::key_split_workspace_bytes(nsplit, p.batch, p.heads_q, p.qo_len, p.head_dim)) {
             if (total * nsplit > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_attn_fwd: problem too large for 32-bit tile indices");
             AttnArgs s = a;
             attn::apply_key_split(s, nsplit, p.batch, (int)p.head_dim, workspace);
-            if (int rc = attn::launch_fast(s, (int)p.head_dim, p.v_dtype, p.causal != 0, stream)) return rc;
+            if (int rc = launch(s)) return rc;
             return attn::launch_split_combine(s, a, (int)p.head_dim, p.batch, stream);
         }
-        return attn::launch_fast(a, (int)p.head_dim, p.v_dtype, p.causal != 0, stream);
+        return launch(a);
     }
     a.mask_additive = additive;
     if ((is_bool && attn::fast_serves_mask(a, 1)) || (additive && attn::fast_serves_mask(a, dtype_bytes(a.mask_dt))))

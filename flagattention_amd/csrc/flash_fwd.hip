@@ -37,7 +37,7 @@ int launch_flash(const AttnArgs& a, int head_dim, int dtype, bool causal, hipStr
 }  // namespace attn
 
 static int flash_key_splits(const sage_flash_params& p) {
-    return attn::plan_key_split(p.batch, p.heads_q, p.qo_len, p.kv_len, p.causal != 0);
+    return attn::plan_key_split(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0);
 }
 
 int64_t flash_split_workspace_bytes(const sage_flash_params& p) {
@@ -67,15 +67,20 @@ int launch_flash_attn(const sage_flash_params& p, void* workspace, int64_t works
         return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd: k/v sequence stride out of range for 32-bit tile offsets");
     a.total_wg = (int)total;
     a.nsplit = 1; a.split_steps = a.nk;
+    const bool decode = decode_serves(p.heads_q, p.heads_kv, p.qo_len);
+    auto launch = [&](const AttnArgs& x) {
+        return decode ? launch_decode(x, p.batch, (int)p.head_dim, p.dtype, false, stream)
+                      : launch_flash(x, (int)p.head_dim, p.dtype, p.causal != 0, stream);
+    };
     const int nsplit = workspace ? flash_key_splits(p) : 1;
     if (nsplit > 1 && workspace_bytes >= key_split_workspace_bytes(nsplit, p.batch, p.heads_q, p.qo_len, p.head_dim)) {
         if (total * nsplit > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd: problem too large for 32-bit tile indices");
         AttnArgs s = a;
         apply_key_split(s, nsplit, p.batch, (int)p.head_dim, workspace);
-        if (int rc = launch_flash(s, (int)p.head_dim, p.dtype, p.causal != 0, stream)) return rc;
+        if (int rc = launch(s)) return rc;
         return launch_split_combine(s, a, (int)p.head_dim, p.batch, stream);
     }
-    return launch_flash(a, (int)p.head_dim, p.dtype, p.causal != 0, stream);
+    return launch(a);
 }
 
 }  // namespace sage

@@ -13,6 +13,7 @@ namespace {
 
 constexpr int kComputeUnits = 256;
 constexpr int kMaxSplits = 64;
+constexpr int kMaxDecodeSplits = 128;
 constexpr int kMinStepsPerSplit = 4;   // 256 keys: below that the prologue and epilogue of a workgroup dominate
 constexpr float kFixedSteps = 6.0f;    // what a workgroup spends outside its step loop, in steps
 
@@ -29,22 +30,27 @@ struct CombineArgs {
 
 constexpr int kCombineThreads = 256;
 
-// One thread per four channels of one row; the threads of a row read the same nsplit log-sum-exps.
-template <int D>
+// TPR threads per row, four channels each; SG groups of them share the runs of a row (group g takes runs g, g + SG, ...)
+// and meet through LDS.  SG = 1 where the rows alone fill the chip; with few rows (decoding) the runs of a row are read
+// side by side instead of one after the other.
+template <int D, int SG>
 __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineArgs a) {
-    constexpr int TPR = D / 4;  // threads per row
-    const int64_t row = (int64_t)blockIdx.x * (kCombineThreads / TPR) + threadIdx.x / TPR;
-    const int c = threadIdx.x % TPR;
-    if (row >= a.rows) return;
-    const float* pl = a.part_lse + row;
+    constexpr int TPR = D / 4;
+    constexpr int ROWS = kCombineThreads / (TPR * SG);  // rows per workgroup
+    __shared__ float sm_m[SG > 1 ? kCombineThreads : 1], sm_den[SG > 1 ? kCombineThreads : 1];
+    __shared__ v4f sm_acc[SG > 1 ? kCombineThreads : 1];
+    const int c = threadIdx.x % TPR, sg = (threadIdx.x / TPR) % SG;
+    const int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / (TPR * SG);
+    const bool ok = row < a.rows;
+    const float* pl = a.part_lse + (ok ? row : 0);
     float m = -INFINITY;
-    for (int s = 0; s < a.nsplit; s++) m = fmaxf(m, pl[(int64_t)s * a.rows]);
+    for (int s = sg; s < a.nsplit; s += SG) m = fmaxf(m, pl[(int64_t)s * a.rows]);
     v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
     float den = 0.0f;
     if (m > -INFINITY) {  // (a row that saw no key in any run: every partial is 0 and every lse_s -inf)
-        const float* po = a.part_o + row * D + 4 * c;
+        const float* po = a.part_o + (ok ? row : 0) * D + 4 * c;
 #pragma unroll 4
-        for (int s = 0; s < a.nsplit; s++) {
+        for (int s = sg; s < a.nsplit; s += SG) {
             const float w = __builtin_amdgcn_exp2f(pl[(int64_t)s * a.rows] - m);
             const v4f o = *reinterpret_cast<const v4f*>(po + (int64_t)s * a.rows * D);
             den += w;
@@ -52,6 +58,29 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineA
             for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(w, o[i], acc[i]);
         }
     }
+    if constexpr (SG > 1) {
+        sm_m[threadIdx.x] = m;
+        sm_den[threadIdx.x] = den;
+        sm_acc[threadIdx.x] = acc;
+        __syncthreads();
+        if (sg != 0) return;
+        const int t0 = threadIdx.x;
+#pragma unroll
+        for (int g = 1; g < SG; g++) m = fmaxf(m, sm_m[t0 + g * TPR]);
+        acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        den = 0.0f;
+        if (m > -INFINITY) {
+#pragma unroll
+            for (int g = 0; g < SG; g++) {
+                const float w = __builtin_amdgcn_exp2f(sm_m[t0 + g * TPR] - m);
+                const v4f o = sm_acc[t0 + g * TPR];
+                den = __builtin_fmaf(w, sm_den[t0 + g * TPR], den);
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(w, o[i], acc[i]);
+            }
+        }
+    }
+    if (!ok) return;
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;
     float r[4];
 #pragma unroll
@@ -73,7 +102,35 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineA
 
 }  // namespace
 
-int plan_key_split(int64_t batch, int64_t heads_q, int64_t qo_len, int64_t kv_len, bool causal) {
+// One row tile always: B1 H8/8 M1 N8192 19 us against 24 us on the 256-row tiles of the pipelined kernel, B4 H32/32 M1 N4096
+// 46 against 57 us (bf16, head_dim 128, dense).  Two row tiles (one wave per SIMD) where they hold several heads that
+// would otherwise walk over K and V one by one: B8 H32/4 M8 N8192 36 against 185 us.  A head that fills them alone
+// gains nothing (SageAttention B16 H32/32 M64 N1024: 54 against 52 us).
+bool decode_serves(int64_t heads_q, int64_t heads_kv, int64_t qo_len) {
+    const int64_t groups = heads_q / heads_kv, rows = groups * qo_len;
+    return rows <= 32 || (groups > 1 && rows <= kDecodeRows);
+}
+
+// Runs of the keys of one (batch, K/V head) for attn_decode_kernel: enough workgroups that every CU holds two (one
+// of those with two row tiles), which keeps the HBM busy; a run has at least one 32-key tile for each of its four waves.
+static int plan_decode_split(int64_t items, int64_t rows, int64_t nk) {
+    const int64_t slots = rows <= 32 ? 2 * kComputeUnits : kComputeUnits;
+    const int64_t smax = nk / 2 < kMaxDecodeSplits ? nk / 2 : kMaxDecodeSplits;
+    float best = 0.0f;
+    int best_s = 1;
+    for (int64_t s = 1; s <= smax; s++) {
+        const int64_t steps = (nk + s - 1) / s;
+        if ((nk + steps - 1) / steps != s) continue;  // (a run without a key)
+        const int64_t rounds = (items * s + slots - 1) / slots, tiles = (steps + 1) / 2;
+        const float cost = (float)rounds * ((float)tiles + 2.0f) + (s > 1 ? 0.5f + 0.01f * (float)s : 0.0f);
+        if (s == 1 || cost < 0.97f * best) { best = cost; best_s = (int)s; }
+    }
+    return best_s;
+}
+
+int plan_key_split(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal) {
+    if (decode_serves(heads_q, heads_kv, qo_len))
+        return plan_decode_split(batch * heads_kv, heads_q / heads_kv * qo_len, (kv_len + BN - 1) / BN);
     const int64_t nq2 = (qo_len + kFastRows - 1) / kFastRows;
     const int64_t per_head = causal ? (nq2 + 1) / 2 : nq2;  // under the causal flag a workgroup takes two q-blocks
     const int64_t base = batch * heads_q * per_head;
@@ -122,12 +179,19 @@ int launch_split_combine(const AttnArgs& split, const AttnArgs& whole, int head_
     c.rows = batch * whole.Hq * whole.M;
     c.Hq = whole.Hq; c.M = whole.M; c.nsplit = split.nsplit; c.out_dt = whole.out_dt;
     c.lse_mul = whole.lse_mul;
-    const int rows_per_wg = kCombineThreads / (head_dim / 4);
+    // eight groups per row while rows alone would leave compute units idle
+    const int sg = c.rows * (head_dim / 4) < kComputeUnits * kCombineThreads && c.nsplit >= 8 ? 8 : 1;
+    const int rows_per_wg = kCombineThreads / (head_dim / 4 * sg);
     const int64_t wgs = (c.rows + rows_per_wg - 1) / rows_per_wg;
     if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "split combine: too many rows for one launch");
     dim3 grid((unsigned)wgs), block(kCombineThreads);
-    if (head_dim == 128) hipLaunchKernelGGL((split_combine_kernel<128>), grid, block, 0, stream, c);
-    else hipLaunchKernelGGL((split_combine_kernel<64>), grid, block, 0, stream, c);
+    if (head_dim == 128) {
+        if (sg == 8) hipLaunchKernelGGL((split_combine_kernel<128, 8>), grid, block, 0, stream, c);
+        else hipLaunchKernelGGL((split_combine_kernel<128, 1>), grid, block, 0, stream, c);
+    } else {
+        if (sg == 8) hipLaunchKernelGGL((split_combine_kernel<64, 8>), grid, block, 0, stream, c);
+        else hipLaunchKernelGGL((split_combine_kernel<64, 1>), grid, block, 0, stream, c);
+    }
     return check_launch("split_combine_kernel");
 }
 

@@ -112,8 +112,9 @@ int sage_attn_fwd(const sage_attn_params* p, void* stream);
  * batch * heads_q * ceil(qo_len / 256) is well below the 256 compute units and no mask tensor is given, the keys
  * of every (batch, head, 256-query block) are cut into runs of whole 64-key steps, one workgroup each; the runs
  * write normalized fp32 partial outputs and their base-2 log-sum-exps to the workspace and a second kernel
- * combines them (out = sum_s 2^(lse_s - lse) o_s, lse = log2 sum_s 2^lse_s).  The reference's SageAttention
- * launch has no such split (attn_qk_int8_per_block.py:176-190 is one grid over q-blocks); its dense forward does
+ * combines them (out = sum_s 2^(lse_s - lse) o_s, lse = log2 sum_s 2^lse_s).  Calls with few query rows per K/V
+ * head (decoding: heads_q / heads_kv * qo_len of at most 32, or of at most 64 for grouped heads) cut the keys of a
+ * (batch, K/V head) in the same way, for the kernel that packs those rows.  The reference's SageAttention launch has no such split (attn_qk_int8_per_block.py:176-190 is one grid over q-blocks); its dense forward does
  * (see sage_flash_attn_fwd_ws).  Results agree with sage_attn_fwd to fp32 rounding of the combination.
  *   sage_attn_fwd_workspace_bytes  bytes the split of this call would use; 0 = the call would not split;
  *                                  -1 = invalid params (sage_hip_last_error says why)
