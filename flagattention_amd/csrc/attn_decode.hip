@@ -6,8 +6,8 @@
 // (row r = head r / qo_len of the group, query r % qo_len), where the kernel of attn_fast_kernel.h spends a 256-row
 // tile, and a walk over K and V of its own, on every query head.
 //
-// * A workgroup is four waves, and a wave walks over 32-key tiles of its own (tile w, w + 4, ... of the workgroup's
-//   keys) with no barrier: S^T = K.Q^T and O^T += V^T.P^T on the 32x32 matrix instructions, so a lane owns one query
+// * A workgroup is eight waves (four with two row tiles), and a wave walks over 32-key tiles of its own (tile w, w + 8,
+//   ... of the workgroup's keys) with no barrier: S^T = K.Q^T and O^T += V^T.P^T on the 32x32 matrix instructions, so a lane owns one query
 //   row.  Matrix and vector work of a tile is a small part of the time its 12-16 KB take to arrive.
 // * K rows are loaded straight into the A operand; V goes through registers into the wave's own slice of LDS, from
 //   where ds_read_b64_tr_b16 returns the transposed operand (chunks XOR-swizzled as in attn_fast_kernel.h).  The
@@ -16,8 +16,8 @@
 //   Measured (bf16, head_dim 128, with the combine launch; before: the 256-row tiles of the pipelined kernel): dense
 //   B8 H32/8 M1 N8192 197 -> 46 us = 5.8 TB/s of K and V (a 1 GiB copy moves 5.2 TB/s here), SageAttention on the same
 //   shape 144 -> 37 us = 5.4 TB/s, dense B64 H32/8 M1 N1024 229 -> 42 us = 6.4 TB/s.
-// * The keys of a (batch, K/V head) are cut into runs (plan_decode_split) so that every CU holds two workgroups; the
-//   four waves of a workgroup are combined through LDS, the runs by split_combine_kernel.
+// * The keys of a (batch, K/V head) are cut into runs (plan_decode_split) so that every CU holds eight waves; the
+//   waves of a workgroup are combined through LDS, the runs by split_combine_kernel.
 #include "attn_common.h"
 
 namespace sage {
@@ -28,16 +28,17 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
 
-constexpr int kDecodeWaves = 4;
-constexpr int kDecodeThreads = 64 * kDecodeWaves;
 constexpr int kTileKeys = 32;
 
 template <int D>
 __device__ __forceinline__ int v_swizzle(int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); }
 
 // RT: 32-row tiles of query rows (groups * qo_len <= 32 * RT)
-template <int D, typename VT, int QB, int RT>
-__global__ __launch_bounds__(kDecodeThreads, RT == 1 ? 2 : 1) void attn_decode_kernel(AttnArgs a) {
+// kDecodeWaves: eight (one workgroup per CU), or four: with one row tile where the items alone fill the chip (two
+// workgroups per CU, finer rounds: B11 H32/32 M1 N700 D128 26 us against 32 us), and with two row tiles, which leave
+// registers for one wave per SIMD only.
+template <int D, typename VT, int QB, int RT, int kDecodeWaves>
+__global__ __launch_bounds__(64 * kDecodeWaves, RT == 1 ? 8 / kDecodeWaves : 1) void attn_decode_kernel(AttnArgs a) {
     using PVT = PV<VT>;
     using vec16 = typename PVT::vec;
     constexpr bool INT8 = QB == 1;
@@ -69,45 +70,41 @@ __global__ __launch_bounds__(kDecodeThreads, RT == 1 ? 2 : 1) void attn_decode_k
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
         const int r = 32 * rt + l32;
-        const bool ok = r < rows;
+        const bool ok = r < rows;  // (rows past the last one multiply a copy of the group's first: nothing of theirs is stored)
         const int g = ok ? r / a.M : 0, mi = ok ? r - g * a.M : 0, h = hk * a.groups + g;
         const int8_t* qp = a.q + ((int64_t)b * a.qs_b + (int64_t)h * a.qs_h + (int64_t)mi * a.qs_n) * QB + 16 * half;
 #pragma unroll
-        for (int t = 0; t < KSTEPS; t++) qf[rt][t] = ok ? *reinterpret_cast<const v4i*>(qp + 32 * t) : v4i{0, 0, 0, 0};
+        for (int t = 0; t < KSTEPS; t++) qf[rt][t] = *reinterpret_cast<const v4i*>(qp + 32 * t);
         lim[rt] = ok && a.causal ? min(mi + a.N - a.M, a.N - 1) : a.N - 1;
         qs[rt] = INT8 ? a.q_scale[((int64_t)b * a.Hq + h) * a.nq + mi / BM] : a.qk_scale;
     }
     // keys below this one are visible to every row of the workgroup
     const int all_see = a.causal ? min(a.N - a.M + 1, a.N) : a.N;
-    const float* ksp = INT8 ? a.k_scale + ((int64_t)b * a.Hkv + hk) * a.nk : nullptr;
+    // (constant address space: scalar loads, which the waits for K and V do not count)
+    typedef __attribute__((address_space(4))) const float* const_f32_ptr;
+    const const_f32_ptr ksp = (const_f32_ptr)(uintptr_t)(INT8 ? a.k_scale + ((int64_t)b * a.Hkv + hk) * a.nk : nullptr);
 
     const unsigned char* kg = reinterpret_cast<const unsigned char*>(a.k) + ((int64_t)b * a.ks_b + (int64_t)hk * a.ks_h) * QB;
     const unsigned char* vg = static_cast<const unsigned char*>(a.v) + ((int64_t)b * a.vs_b + (int64_t)hk * a.vs_h) * 2;
     const int64_t krow = a.ks_n * QB, vrow = a.vs_n * 2;  // bytes from one key to the next
-    const unsigned koff = (unsigned)(l32 * (int)krow + 16 * half);
     const int vr0 = lane / VCPR, vchunk = lane % VCPR;    // V load e of a lane: row vr0 + e * 64 / VCPR, this chunk
-    const unsigned voff = (unsigned)(vr0 * (int)vrow + 16 * vchunk);
     unsigned char* vlds = smem + wave * V_TILE;
 
     v4i kf[KSTEPS], vr[VLOADS];
-    // (tiles that reach past the last key re-read its row: finite values under hidden scores)
+    // Rows past the last key re-read it (finite values under hidden scores).  The loads of a tile are unconditional and
+    // without branches, so that the waits for older loads leave them in flight.
     auto load_k = [&](int key0) {
-        const bool whole = key0 + kTileKeys <= a.N;
-        const unsigned char* p = kg + (int64_t)key0 * krow + (whole ? koff : (unsigned)(min(l32, a.N - 1 - key0) * (int)krow + 16 * half));
+        const unsigned char* p = kg + (int64_t)key0 * krow;
+        const unsigned off = (unsigned)(min(l32, a.N - 1 - key0) * (int)krow + 16 * half);
 #pragma unroll
-        for (int t = 0; t < KSTEPS; t++) kf[t] = *reinterpret_cast<const v4i*>(p + 32 * t);
+        for (int t = 0; t < KSTEPS; t++) kf[t] = *reinterpret_cast<const v4i*>(p + off + 32 * t);
     };
     auto load_v = [&](int key0) {
         const unsigned char* p = vg + (int64_t)key0 * vrow;
-        if (key0 + kTileKeys <= a.N) {
+        const int last = a.N - 1 - key0;
 #pragma unroll
-            for (int e = 0; e < VLOADS; e++) vr[e] = *reinterpret_cast<const v4i*>(p + (int64_t)(e * (64 / VCPR)) * vrow + voff);
-        } else {
-            const int last = a.N - 1 - key0;
-#pragma unroll
-            for (int e = 0; e < VLOADS; e++)
-                vr[e] = *reinterpret_cast<const v4i*>(p + (unsigned)(min(vr0 + e * (64 / VCPR), last) * (int)vrow + 16 * vchunk));
-        }
+        for (int e = 0; e < VLOADS; e++)
+            vr[e] = *reinterpret_cast<const v4i*>(p + (unsigned)(min(vr0 + e * (64 / VCPR), last) * (int)vrow + 16 * vchunk));
     };
     int vtr[DT];  // LDS offsets of the transposed fragment reads (see attn_fast_kernel.h)
     {
@@ -136,6 +133,7 @@ __global__ __launch_bounds__(kDecodeThreads, RT == 1 ? 2 : 1) void attn_decode_k
     }
     for (; key0 < kend; key0 += kTileKeys * kDecodeWaves) {
         const int next = key0 + kTileKeys * kDecodeWaves;
+        const int fetch = next < kend ? next : key0;  // (behind the last tile: the same lines once more)
         // ---- S^T = K.Q^T; the K registers are requested anew right behind it
         v16i s[RT];
 #pragma unroll
@@ -149,7 +147,7 @@ __global__ __launch_bounds__(kDecodeThreads, RT == 1 ? 2 : 1) void attn_decode_k
                                                                 __builtin_bit_cast(v16f, s[rt])));
             }
         }
-        if (next < kend) load_k(next);
+        load_k(fetch);
         __builtin_amdgcn_sched_barrier(0);
         // ---- V tile -> LDS (the wave's own slice: a wave's LDS instructions run in order, no barrier)
 #pragma unroll
@@ -157,7 +155,7 @@ __global__ __launch_bounds__(kDecodeThreads, RT == 1 ? 2 : 1) void attn_decode_k
             const int row = vr0 + e * (64 / VCPR);
             *reinterpret_cast<v4i*>(vlds + row * V_RS + 16 * (vchunk ^ v_swizzle<D>(row))) = vr[e];
         }
-        if (next < kend) load_v(next);
+        load_v(fetch);
         __builtin_amdgcn_sched_barrier(0);
         // ---- online softmax: register i of this lane is key key0 + 8 (i / 4) + 4 half + i % 4 of its row
         const float ks = INT8 ? ksp[key0 / BN] : 1.0f;
@@ -209,7 +207,7 @@ __global__ __launch_bounds__(kDecodeThreads, RT == 1 ? 2 : 1) void attn_decode_k
             }
     }
 
-    // ---- the four waves of the workgroup -> one normalized result and its log-sum-exp
+    // ---- the waves of the workgroup -> one normalized result and its log-sum-exp
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
         const float l_tot = l_i[rt] + __shfl_xor(l_i[rt], 32);
@@ -244,8 +242,8 @@ __global__ __launch_bounds__(kDecodeThreads, RT == 1 ? 2 : 1) void attn_decode_k
                 *reinterpret_cast<v4f*>(slice + (wave * 32 + l32) * SL_RS + 8 * g + 4 * half) =
                     v4f{o[rt][dt][4 * g] * f, o[rt][dt][4 * g + 1] * f, o[rt][dt][4 * g + 2] * f, o[rt][dt][4 * g + 3] * f};
             __syncthreads();
-            const int orow = 32 * rt + tid / 8, c = 4 * (tid % 8);  // 256 threads: 32 rows x 8 groups of four channels
-            if (orow < rows) {
+            const int orow = 32 * rt + tid / 8, c = 4 * (tid % 8);  // 32 rows x 8 groups of four channels
+            if (tid < 256 && orow < rows) {
                 v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int w = 0; w < kDecodeWaves; w++) {
@@ -274,9 +272,10 @@ template <int D, typename VT, int QB>
 int launch_rt(const AttnArgs& a, int64_t batch, hipStream_t stream) {
     const int64_t wgs = batch * a.Hkv * a.nsplit;
     if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "attention over few query rows: too many workgroups for one launch");
-    dim3 grid((unsigned)wgs), block(kDecodeThreads);
-    if (a.groups * a.M <= 32) hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 1>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 2>), grid, block, 0, stream, a);
+    dim3 grid((unsigned)wgs);
+    if (a.groups * a.M > 32) hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 2, 4>), grid, dim3(256), 0, stream, a);
+    else if (a.nsplit == 1 && wgs > 256) hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 1, 4>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 1, 8>), grid, dim3(512), 0, stream, a);
     return check_launch("attn_decode_kernel");
 }
 

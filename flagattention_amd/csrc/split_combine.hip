@@ -13,7 +13,6 @@ namespace {
 
 constexpr int kComputeUnits = 256;
 constexpr int kMaxSplits = 64;
-constexpr int kMaxDecodeSplits = 128;
 constexpr int kMinStepsPerSplit = 4;   // 256 keys: below that the prologue and epilogue of a workgroup dominate
 constexpr float kFixedSteps = 6.0f;    // what a workgroup spends outside its step loop, in steps
 
@@ -111,17 +110,19 @@ bool decode_serves(int64_t heads_q, int64_t heads_kv, int64_t qo_len) {
     return rows <= 32 || (groups > 1 && rows <= kDecodeRows);
 }
 
-// Runs of the keys of one (batch, K/V head) for attn_decode_kernel: enough workgroups that every CU holds two (one
-// of those with two row tiles), which keeps the HBM busy; a run has at least one 32-key tile for each of its four waves.
+// Runs of the keys of one (batch, K/V head) for attn_decode_kernel: a workgroup for every CU, whose eight waves keep
+// the HBM busy; at least one 32-key tile per wave.
 static int plan_decode_split(int64_t items, int64_t rows, int64_t nk) {
-    const int64_t slots = rows <= 32 ? 2 * kComputeUnits : kComputeUnits;
-    const int64_t smax = nk / 2 < kMaxDecodeSplits ? nk / 2 : kMaxDecodeSplits;
+    const int64_t smax = nk / kMinStepsPerSplit < kMaxSplits ? nk / kMinStepsPerSplit : kMaxSplits;
     float best = 0.0f;
     int best_s = 1;
     for (int64_t s = 1; s <= smax; s++) {
         const int64_t steps = (nk + s - 1) / s;
         if ((nk + steps - 1) / steps != s) continue;  // (a run without a key)
-        const int64_t rounds = (items * s + slots - 1) / slots, tiles = (steps + 1) / 2;
+        // (unsplit with more items than CUs: four-wave workgroups, two per CU; two row tiles: four waves, one per CU)
+        const bool pairs = s == 1 && rows <= 32 && items > kComputeUnits;
+        const int64_t slots = pairs ? 2 * kComputeUnits : kComputeUnits, waves = pairs || rows > 32 ? 4 : 8;
+        const int64_t rounds = (items * s + slots - 1) / slots, tiles = (2 * steps + waves - 1) / waves;  // tiles per wave
         const float cost = (float)rounds * ((float)tiles + 2.0f) + (s > 1 ? 0.5f + 0.01f * (float)s : 0.0f);
         if (s == 1 || cost < 0.97f * best) { best = cost; best_s = (int)s; }
     }
