@@ -71,6 +71,8 @@ EXPORTS = (
     "sage_flash_attn_fwd_workspace_bytes",
     "sage_flash_attn_fwd_ws",
     "sage_flash_total_attention",
+    "sage_flash_total_attention_workspace_bytes",
+    "sage_flash_total_attention_ws",
     "sage_flash_attn_fwd_dropout",
     "sage_flash_dropout_mask",
     "sage_k_mean",
@@ -117,6 +119,11 @@ def load():
     lib.sage_flash_attn_fwd_ws.restype = ctypes.c_int
     lib.sage_flash_total_attention.argtypes = [ctypes.POINTER(FlashParams), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
     lib.sage_flash_total_attention.restype = ctypes.c_int
+    lib.sage_flash_total_attention_workspace_bytes.argtypes = [ctypes.POINTER(FlashParams)]
+    lib.sage_flash_total_attention_workspace_bytes.restype = c_i64
+    lib.sage_flash_total_attention_ws.argtypes = [ctypes.POINTER(FlashParams), ctypes.c_void_p, ctypes.c_void_p,
+                                                  ctypes.c_void_p, c_i64, ctypes.c_void_p]
+    lib.sage_flash_total_attention_ws.restype = ctypes.c_int
     lib.sage_flash_attn_fwd_dropout.argtypes = [ctypes.POINTER(FlashParams), ctypes.c_float, ctypes.c_uint64,
                                                 ctypes.c_uint64, ctypes.c_void_p]
     lib.sage_flash_attn_fwd_dropout.restype = ctypes.c_int

@@ -1,5 +1,7 @@
 // Types shared by the attention kernels of libsage_attention_hip.so (gfx950).
 #pragma once
+#include <utility>
+
 #include "common.h"
 
 namespace sage {
@@ -11,6 +13,13 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+// compile-time loops: f(IC<0>{}), f(IC<1>{}), ...
+template <int I> struct IC { static constexpr int value = I; };
+template <typename Fn, int... Is>
+__device__ __forceinline__ void sfor_impl(Fn&& f, std::integer_sequence<int, Is...>) { (f(IC<Is>{}), ...); }
+template <int N, typename Fn>
+__device__ __forceinline__ void sfor(Fn&& f) { sfor_impl(f, std::make_integer_sequence<int, N>{}); }
 
 constexpr int kThreads = 256;
 constexpr int BM = 128;  // query rows per workgroup (= Q quantization block)

@@ -32,8 +32,6 @@
 // * Under the causal flag a workgroup takes two q-blocks of its head (the longest remaining and the
 //   shortest), so that all workgroups of a launch run the same number of steps.
 #pragma once
-#include <utility>
-
 #include "attn_common.h"
 
 namespace sage {
@@ -44,13 +42,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
-
-// compile-time loops: f(IC<0>{}), f(IC<1>{}), ...
-template <int I> struct IC { static constexpr int value = I; };
-template <typename Fn, int... Is>
-__device__ __forceinline__ void sfor_impl(Fn&& f, std::integer_sequence<int, Is...>) { (f(IC<Is>{}), ...); }
-template <int N, typename Fn>
-__device__ __forceinline__ void sfor(Fn&& f) { sfor_impl(f, std::make_integer_sequence<int, N>{}); }
 
 constexpr int kBiasBits = 0x4B400000;  // 12582912.0f = 1.5 * 2^23
 constexpr float kBias = 12582912.0f;

@@ -214,12 +214,28 @@ extern "C" int sage_flash_dropout_mask(uint8_t* mask, int64_t batch, int64_t hea
     return launch_dropout_mask(mask, batch * heads_q * qo_len * kv_len, dropout_p, seed, offset, (hipStream_t)stream);
 }
 
-extern "C" int sage_flash_total_attention(const sage_flash_params* p, const float* log_normalizer, float* total_attention,
-                                          void* stream) {
+static int total_attention(const sage_flash_params* p, const float* log_normalizer, float* total, void* workspace,
+                           int64_t workspace_bytes, void* stream) {
     if (int rc = check_flash_params(p, false)) return rc;
-    if (!log_normalizer || !total_attention)
+    if (!log_normalizer || !total)
         return fail(SAGE_E_INVALID, "sage_flash_total_attention: null log_normalizer or total_attention");
-    return launch_flash_total_attention(*p, log_normalizer, total_attention, (hipStream_t)stream);
+    return launch_flash_total_attention(*p, log_normalizer, total, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+extern "C" int sage_flash_total_attention(const sage_flash_params* p, const float* log_normalizer, float* total_attention_out,
+                                          void* stream) {
+    return total_attention(p, log_normalizer, total_attention_out, nullptr, 0, stream);
+}
+
+extern "C" int64_t sage_flash_total_attention_workspace_bytes(const sage_flash_params* p) {
+    if (check_flash_params(p, false)) return -1;
+    return total_workspace_bytes(*p);
+}
+
+extern "C" int sage_flash_total_attention_ws(const sage_flash_params* p, const float* log_normalizer, float* total_attention_out,
+                                             void* workspace, int64_t workspace_bytes, void* stream) {
+    if (int rc = check_workspace("sage_flash_total_attention_ws", workspace, workspace_bytes)) return rc;
+    return total_attention(p, log_normalizer, total_attention_out, workspace, workspace_bytes, stream);
 }
 
 static int check_flash_params(const sage_flash_params* p, bool forward) {

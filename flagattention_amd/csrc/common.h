@@ -31,7 +31,9 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
 int launch_flash_attn(const sage_flash_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 int64_t attn_split_workspace_bytes(const sage_attn_params& p);
 int64_t flash_split_workspace_bytes(const sage_flash_params& p);
-int launch_flash_total_attention(const sage_flash_params& p, const float* log_normalizer, float* total, hipStream_t stream);
+int launch_flash_total_attention(const sage_flash_params& p, const float* log_normalizer, float* total, void* workspace,
+                                 int64_t workspace_bytes, hipStream_t stream);
+int64_t total_workspace_bytes(const sage_flash_params& p);
 int launch_flash_dropout(const sage_flash_params& p, float dropout_p, uint64_t seed, uint64_t offset, hipStream_t stream);
 int launch_dropout_mask(uint8_t* mask, int64_t count, float dropout_p, uint64_t seed, uint64_t offset, hipStream_t stream);
 

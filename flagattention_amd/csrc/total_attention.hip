@@ -2,13 +2,23 @@
 // softmax(sm_scale * q.k^T)[m, n], recomputed from Q, K and the log normalizer the forward pass returned
 // (FlagAttention src/flag_attn/total.py:64-160 is the kernel it stands in for, flash.py:142-157 its call site).
 //
-// One wave owns 32 keys for the whole launch and walks over the queries 32 at a time:
-//   S^T[key, query] = K . Q^T   (v_mfma_f32_32x32x16_{bf16,f16}: A = the wave's K rows, kept in registers;
-//                                B = the query rows, each lane loading the 16-byte pieces of its own row)
+// A wave keeps 64 keys in registers for the whole launch and the workgroup's four waves (256 keys) walk over the queries
+// together, 32 at a time:
+//   S^T[key, query] = K . Q^T   (v_mfma_f32_32x32x16_{bf16,f16}: A = the wave's K rows, B = the query rows from LDS)
 //   p = exp2(S^T * sm_scale * log2(e) - L[query] * log2(e)),   zero where the causal mask hides the key.
-// A lane owns one query column of every tile and sixteen of the 32 keys, so the sum over queries is first kept
-// per lane (sixteen running sums) and folded across the 32 lanes of each half of the wave once, at the end.
-// No LDS, no barriers; the next tile's query pieces are requested before the current tile is multiplied.
+// A lane owns one query column of every tile and 32 of the 64 keys, so the sum over queries is first kept per lane (32
+// running sums) and folded across the 32 lanes of each half of the wave once, at the end.
+//
+// Bound by vector and matrix instructions (about 700 and 512 issue cycles per wave and tile at head_dim 128; full tiles
+// run at about 930 cycles each).  Query tiles go through LDS because four waves read each: every wave loading its own
+// (with only 32 keys per wave) asked the L1 for twice the bytes it delivers.  The tiles are loaded three ahead, straight
+// into LDS.  Workgroups are handed out longest first over all heads: with the key blocks of one head side by side, the
+// last heads' long blocks started late (B4 H32 M4096 N4096 D128 fp16 causal 425 us, longest first 280 us; without the
+// causal flag 523 us).  Where key blocks alone do not fill the chip the queries are cut into runs (total_runs), whose
+// sums go to a workspace and are added in order.  Before, with a wave per 32 keys loading queries into registers:
+// B1 H16 M4096 N4096 D128 causal 212 -> 41 us, B4 H32 M4096 N4096 1739 -> 275 us, B8 H16 M2048 N2048 D64 210 -> 50 us.
+// Issuing the matrix instructions of the next tile between the exponentials of the current one (two score sets, two
+// waves per SIMD) ran no faster than three waves in different phases.
 #include "attn_common.h"
 
 namespace sage {
@@ -20,111 +30,210 @@ struct TotalArgs {
     const void* q;
     const void* k;
     const float* log_normalizer;  // [B, Hq, M], natural log
-    float* total;                 // [B, Hq, N]
+    float* total;                 // [B, Hq, N]; of run r at total + r * run_stride
+    int64_t run_stride;
+    int32_t runs, run_tiles;      // runs of the queries, query tiles per run
+    int32_t BH;                   // batch * heads
     int64_t qs_b, qs_h, qs_n;
     int64_t ks_b, ks_h, ks_n;
     int32_t Hq, M, N, groups, causal;
     float qk_scale;  // sm_scale * log2(e)
 };
 
-constexpr int kTotalWaves = 4;  // 128 keys per workgroup
+constexpr int kTotalWaves = 4;
+constexpr int kTotalThreads = 64 * kTotalWaves;
+constexpr int kWaveKeys = 64;
+constexpr int kWgKeys = kWaveKeys * kTotalWaves;
+constexpr int kTileQ = 32;
+constexpr int kRing = 4;  // query tiles resident in LDS: the one in work and three on their way
 
 template <int D, typename VT>
-__global__ __launch_bounds__(64 * kTotalWaves) void total_attention_kernel(TotalArgs a) {
+__global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(TotalArgs a) {
     using PVT = PV<VT>;
     using vec16 = typename PVT::vec;
-    constexpr int KS = D / 16;  // matrix instructions per 32 x 32 tile
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int KS = D / 16;      // matrix instructions per 32 x 32 tile
+    constexpr int RS = 2 * D;       // bytes per query row
+    constexpr int CPR = RS / 16;    // 16-byte chunks per query row
+    constexpr int LOADS = kTileQ * CPR / kTotalThreads;  // 1 KB loads per wave and tile
+    __shared__ __attribute__((aligned(16))) unsigned char qtile[kRing][kTileQ * RS];
+    __shared__ float ltile[kRing][kTotalWaves][64];      // log normalizers of a tile's queries, a copy per wave
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, half = lane >> 5;
-    const int h = blockIdx.y, b = blockIdx.z;
-    const int n0 = (blockIdx.x * kTotalWaves + wave) * 32;
-    if (n0 >= a.N) return;  // (no barrier in this kernel)
-    const int hk = h / a.groups;
+    // Heads fastest, so that a head stays on one XCD and the workgroups with the most tiles come first: under the causal
+    // flag the last queries see every key and the first keys are seen by every query.
+    const int nkb = (a.N + kWgKeys - 1) / kWgKeys;
+    const int bh = blockIdx.x % a.BH, rest = blockIdx.x / a.BH;
+    const int kb = rest % nkb, run = a.runs - 1 - rest / nkb;
+    const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.groups;
+    const int n0 = kb * kWgKeys + wave * kWaveKeys;  // (may lie past the last key: such a wave multiplies copies of it)
     const int shift = a.N - a.M;
 
     // K rows of this wave: lane (key l32, half) holds elements 16 t + 8 half .. + 7 of its row for step t
-    vec16 kf[KS];
-    {
-        const int key = min(n0 + l32, a.N - 1);  // keys past the end re-read the last one; their sums are not stored
+    vec16 kf[2][KS];
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+        const int key = min(n0 + 32 * kt + l32, a.N - 1);  // keys past the end re-read the last one; their sums are not stored
         const VT* kp = static_cast<const VT*>(a.k) + (int64_t)b * a.ks_b + (int64_t)hk * a.ks_h + (int64_t)key * a.ks_n + 8 * half;
 #pragma unroll
-        for (int t = 0; t < KS; t++) kf[t] = *reinterpret_cast<const vec16*>(kp + 16 * t);
+        for (int t = 0; t < KS; t++) kf[kt][t] = *reinterpret_cast<const vec16*>(kp + 16 * t);
     }
-    const VT* qbase = static_cast<const VT*>(a.q) + (int64_t)b * a.qs_b + (int64_t)h * a.qs_h + 8 * half;
+    const VT* qbase = static_cast<const VT*>(a.q) + (int64_t)b * a.qs_b + (int64_t)h * a.qs_h;
     const float* lbase = a.log_normalizer + ((int64_t)b * a.Hq + h) * a.M;
 
-    // queries that can see any of this wave's keys: m + shift >= n0
-    int m_lo = 0;
-    if (a.causal) m_lo = (max(n0 - shift, 0) / 32) * 32;
-    float tot[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) tot[i] = 0.0f;
+    // the run's queries that can see any key of the workgroup: m + shift >= first key
+    int m_lo = run * a.run_tiles * kTileQ;
+    const int m_hi = min(m_lo + a.run_tiles * kTileQ, a.M);
+    if (a.causal) m_lo = max(m_lo, max(kb * kWgKeys - shift, 0) / kTileQ * kTileQ);
 
-    auto load_tile = [&](int m0, vec16 (&qf)[KS], float& lq) {
-        const int m = min(m0 + l32, a.M - 1);
-        const VT* qp = qbase + (int64_t)m * a.qs_n;
+    const int ntiles = max(m_hi - m_lo + kTileQ - 1, 0) / kTileQ;
+
+    // Query tile t of the run -> ring buffer t % 4, straight into LDS (16 bytes per lane; written in assembly because the
+    // compiler would wait for every outstanding load before each LDS read, tracked with s_waitcnt vmcnt below).  Chunk c
+    // of row r lies at chunk c ^ r of its LDS row (modulo the chunks of a row), so that the fragment reads, one chunk of
+    // 32 rows at a time, spread over all banks: the load fetches the chunk that belongs where a lane writes.
+    // m0 holds the LDS address of the load; nothing else in this kernel uses it.  Tiles past the last one load it again.
+    const unsigned lds_q = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&qtile[0][0];
+    const unsigned lds_l = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)&ltile[0][0][0];
+    unsigned qoff[LOADS];  // byte offsets of this lane's pieces of a tile (the host has checked that they fit)
+    auto set_offsets = [&](int last) {  // last: the tile's last row
 #pragma unroll
-        for (int t = 0; t < KS; t++) qf[t] = *reinterpret_cast<const vec16*>(qp + 16 * t);
-        lq = lbase[m] * 1.44269504088896340736f;
+        for (int e = 0; e < LOADS; e++) {
+            const int row = (64 / CPR) * (LOADS * wave + e) + lane / CPR;
+            qoff[e] = (unsigned)min(row, last) * (unsigned)(a.qs_n * 2) + 16 * ((lane % CPR) ^ (row & (CPR - 1)));
+        }
     };
-    vec16 qf[2][KS];
-    float lq[2];
-    if (m_lo < a.M) load_tile(m_lo, qf[0], lq[0]);
-    int buf = 0;
-    for (int m0 = m_lo; m0 < a.M; m0 += 32, buf ^= 1) {
-        if (m0 + 32 < a.M) {
-            if (buf == 0) load_tile(m0 + 32, qf[1], lq[1]);
-            else load_tile(m0 + 32, qf[0], lq[0]);
+    set_offsets(kTileQ - 1);
+    auto fetch = [&](int t) {
+        const int m0 = m_lo + kTileQ * min(t, ntiles - 1), buf = t & (kRing - 1);
+        if (m0 + kTileQ > a.M) set_offsets(a.M - 1 - m0);  // (every later tile is this one again)
+        const unsigned char* base = reinterpret_cast<const unsigned char*>(qbase + (int64_t)m0 * a.qs_n);
+#pragma unroll
+        for (int e = 0; e < LOADS; e++)
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                         :: "v"(qoff[e]), "s"(base), "s"(lds_q + (unsigned)(buf * kTileQ * RS + 1024 * (LOADS * wave + e))) : "memory");
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
+                     :: "v"((unsigned)(4 * min(l32, a.M - 1 - m0))), "s"(lbase + m0), "s"(lds_l + (unsigned)(256 * (kTotalWaves * buf + wave))) : "memory");
+    };
+    if (ntiles > 0) {
+        fetch(0);
+        fetch(1);
+        fetch(2);
+    }
+    // (waited for here: inside the loop the compiler's waits for them would also wait for the query tiles on their way)
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+        for (int t = 0; t < KS; t++) {
+            v4i bits = __builtin_bit_cast(v4i, kf[kt][t]);
+            asm volatile("" : "+v"(bits));
+            kf[kt][t] = __builtin_bit_cast(vec16, bits);
         }
-        v16f s;
+    float tot[2][16];
 #pragma unroll
-        for (int i = 0; i < 16; i++) s[i] = 0.0f;
-        if (buf == 0) {
+    for (int kt = 0; kt < 2; kt++)
 #pragma unroll
-            for (int t = 0; t < KS; t++) s = PVT::mfma(kf[t], qf[0][t], s);
-        } else {
+        for (int i = 0; i < 16; i++) tot[kt][i] = 0.0f;
+
+    for (int t = 0; t < ntiles; t++) {
+        // all but the two youngest tiles' loads of this wave have landed; past the barrier, those of all waves, and
+        // nobody reads the buffer of tile t - 1 any more
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * (LOADS + 1)));
+        __builtin_amdgcn_s_barrier();
+        fetch(t + 3);
+        const int mq = m_lo + kTileQ * t, buf = t & (kRing - 1);
+        if (a.causal && mq + kTileQ - 1 + shift < n0) continue;  // (the tile's last query sees no key of this wave)
+        // queries past the end, and queries that see no key (L = -inf), take L = +inf: every p of theirs is exp2(-inf) = 0
+        const float L = ltile[buf][wave][lane];
+        const float l2 = mq + l32 < a.M && L > -INFINITY ? L * 1.44269504088896340736f : INFINITY;
+        v16f s[2];
 #pragma unroll
-            for (int t = 0; t < KS; t++) s = PVT::mfma(kf[t], qf[1][t], s);
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) s[kt][i] = 0.0f;
+        const unsigned char* row = &qtile[buf][l32 * RS];
+#pragma unroll
+        for (int c = 0; c < KS; c++) {
+            const vec16 qf = *reinterpret_cast<const vec16*>(row + 16 * ((2 * c + half) ^ (l32 & (CPR - 1))));
+            s[0] = PVT::mfma(kf[0][c], qf, s[0]);
+            s[1] = PVT::mfma(kf[1][c], qf, s[1]);
         }
-        const float l2 = buf == 0 ? lq[0] : lq[1];
-        const int m = m0 + l32;
-        const bool row_ok = m < a.M;
+        if (a.causal && mq + shift < n0 + kWaveKeys - 1) {  // the tile's first query does not see the wave's last key
+            const int last = mq + l32 + shift - n0 - 4 * half;  // last key the query sees, from the lane's first one on
+#pragma unroll
+            for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)  // accumulator register i: key 32 kt + 8 (i / 4) + i % 4 from there
+                    s[kt][i] = 32 * kt + 8 * (i >> 2) + (i & 3) <= last ? s[kt][i] : -INFINITY;
+        }
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) tot[kt][i] += __builtin_amdgcn_exp2f(__builtin_fmaf(s[kt][i], a.qk_scale, -l2));
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // nothing of this workgroup is on its way into LDS when it ends
+    // Fold the 32 query columns of a key through LDS (the ring is free once every wave is here; 4 KB per wave): 32 keys at
+    // a time, entry (key, query) at column query ^ key of its row, so that neither the writes (a row at a time) nor the
+    // reads (a lane per key, both halves of the wave taking 16 columns each) meet in a bank.  Five rounds of lane
+    // exchanges per sum instead took as long as eight tiles.
+    __syncthreads();
+    float* out = a.total + ((int64_t)b * a.Hq + h) * a.N + run * a.run_stride;
+    float* fold = reinterpret_cast<float*>(&qtile[0][0]) + wave * 1024;
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
 #pragma unroll
         for (int i = 0; i < 16; i++) {
-            const int n = n0 + 8 * (i >> 2) + 4 * half + (i & 3);  // key of accumulator register i in this lane
-            const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.qk_scale, -l2));
-            const bool seen = row_ok && (!a.causal || n <= m + shift);
-            tot[i] += seen ? p : 0.0f;  // (a select, not a product: a query that sees no key has L = -inf, p = inf)
+            const int key = 8 * (i >> 2) + 4 * half + (i & 3);
+            fold[32 * key + (l32 ^ key)] = tot[kt][i];
         }
-    }
-    // fold the 32 query columns of each half
+        float x = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-        float x = tot[i];
-#pragma unroll
-        for (int off = 16; off > 0; off >>= 1) x += __shfl_xor(x, off);
-        tot[i] = x;
-    }
-    if (l32 == 0) {
-        float* out = a.total + ((int64_t)b * a.Hq + h) * a.N;
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int n = n0 + 8 * (i >> 2) + 4 * half + (i & 3);
-            if (n < a.N) out[n] = tot[i];
-        }
+        for (int c = 0; c < 16; c++) x += fold[32 * l32 + ((16 * half + c) ^ l32)];
+        x += __shfl_xor(x, 32);
+        const int n = n0 + 32 * kt + l32;
+        if (half == 0 && n < a.N) out[n] = x;
     }
 }
 
+// total[i] = sum of the runs' sums, in order
+__global__ __launch_bounds__(256) void total_runs_kernel(const float* part, float* total, int64_t count, int runs) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= count) return;
+    float x = 0.0f;
+#pragma unroll 8
+    for (int r = 0; r < runs; r++) x += part[(int64_t)r * count + i];
+    total[i] = x;
+}
+
+// Runs of the queries: four workgroups per CU (under the causal flag half of them have little or nothing to do), at
+// least eight query tiles each.  (B1 H16 M4096 N4096 causal with two / three / four / six per CU: 68 / 63 / 55 / 61 us.)
+int total_runs(int64_t B, int64_t H, int64_t M, int64_t N) {
+    const int64_t items = B * H * ((N + kWgKeys - 1) / kWgKeys), tiles = (M + kTileQ - 1) / kTileQ;
+    int64_t runs = (4 * 256 + items - 1) / items;
+    if (runs > tiles / 8) runs = tiles / 8;
+    if (runs > 64) runs = 64;
+    if (runs <= 1) return 1;
+    const int64_t per = (tiles + runs - 1) / runs;
+    return (int)((tiles + per - 1) / per);  // (no run without a query)
+}
+
 template <int D, typename VT>
-int launch_total(const TotalArgs& a, int64_t B, hipStream_t stream) {
-    dim3 grid((unsigned)((a.N + 32 * kTotalWaves - 1) / (32 * kTotalWaves)), (unsigned)a.Hq, (unsigned)B), block(64 * kTotalWaves);
+int launch_total(const TotalArgs& a, int64_t B, int runs, hipStream_t stream) {
+    const int64_t wgs = (int64_t)((a.N + kWgKeys - 1) / kWgKeys) * runs * B * a.Hq;
+    if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_total_attention: too many key blocks for one launch");
+    dim3 grid((unsigned)wgs), block(kTotalThreads);
     hipLaunchKernelGGL((total_attention_kernel<D, VT>), grid, block, 0, stream, a);
     return check_launch("total_attention_kernel");
 }
 
 }  // namespace
 
-int launch_flash_total_attention(const sage_flash_params& p, const float* log_normalizer, float* total, hipStream_t stream) {
+int64_t total_workspace_bytes(const sage_flash_params& p) {
+    const int runs = total_runs(p.batch, p.heads_q, p.qo_len, p.kv_len);
+    return runs > 1 ? (int64_t)runs * p.batch * p.heads_q * p.kv_len * (int64_t)sizeof(float) : 0;
+}
+
+int launch_flash_total_attention(const sage_flash_params& p, const float* log_normalizer, float* total, void* workspace,
+                                 int64_t workspace_bytes, hipStream_t stream) {
     TotalArgs a{};
     a.q = p.q.ptr; a.k = p.k.ptr; a.log_normalizer = log_normalizer; a.total = total;
     a.qs_b = p.q.stride_b; a.qs_h = p.q.stride_h; a.qs_n = p.q.stride_n;
@@ -132,10 +241,28 @@ int launch_flash_total_attention(const sage_flash_params& p, const float* log_no
     a.Hq = (int)p.heads_q; a.M = (int)p.qo_len; a.N = (int)p.kv_len; a.groups = (int)(p.heads_q / p.heads_kv);
     a.causal = p.causal ? 1 : 0;
     a.qk_scale = p.sm_scale * 1.44269504089f;
-    if (p.heads_q > 65535 || p.batch > 65535) return fail(SAGE_E_UNSUPPORTED, "sage_flash_total_attention: more than 65535 heads or batches");
+    if (p.q.stride_n < 0 || p.q.stride_n >= (1LL << 25))
+        return fail(SAGE_E_UNSUPPORTED, "sage_flash_total_attention: q sequence stride out of range for 32-bit tile offsets");
+    int runs = workspace ? total_runs(p.batch, p.heads_q, p.qo_len, p.kv_len) : 1;
+    if (runs > 1 && workspace_bytes < total_workspace_bytes(p)) runs = 1;
+    a.runs = runs;
+    a.BH = (int)(p.batch * p.heads_q);
+    a.run_tiles = (int)(((p.qo_len + kTileQ - 1) / kTileQ + runs - 1) / runs);
+    const int64_t count = p.batch * p.heads_q * p.kv_len;
+    if (runs > 1) {
+        a.total = static_cast<float*>(workspace);
+        a.run_stride = count;
+    }
+    int rc;
     if (p.head_dim == 128)
-        return p.dtype == SAGE_BF16 ? launch_total<128, __bf16>(a, p.batch, stream) : launch_total<128, _Float16>(a, p.batch, stream);
-    return p.dtype == SAGE_BF16 ? launch_total<64, __bf16>(a, p.batch, stream) : launch_total<64, _Float16>(a, p.batch, stream);
+        rc = p.dtype == SAGE_BF16 ? launch_total<128, __bf16>(a, p.batch, runs, stream) : launch_total<128, _Float16>(a, p.batch, runs, stream);
+    else
+        rc = p.dtype == SAGE_BF16 ? launch_total<64, __bf16>(a, p.batch, runs, stream) : launch_total<64, _Float16>(a, p.batch, runs, stream);
+    if (rc || runs == 1) return rc;
+    const int64_t wgs = (count + 255) / 256;
+    if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_total_attention: too many keys for one launch");
+    hipLaunchKernelGGL(total_runs_kernel, dim3((unsigned)wgs), dim3(256), 0, stream, (const float*)workspace, total, count, runs);
+    return check_launch("total_runs_kernel");
 }
 
 }  // namespace sage

@@ -101,6 +101,8 @@ def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
         # zero channels change neither Q K^T nor the first D columns of P V; sm_scale was fixed above from the true D
         q, k, v = (torch.nn.functional.pad(t, (0, 64 - D)) for t in (q, k, v))
     q, k, v = _rows16(q), _rows16(k), _rows16(v)
+    if return_total_attention and q.stride(2) >= 1 << 25:
+        q = q.contiguous()  # (that kernel reaches the 32 rows of a query tile with 32-bit byte offsets)
     o = torch.empty_like(q)  # (the reference allocates the same way, flash.py:84-90)
     if not rows_aligned(o):
         o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
@@ -134,8 +136,12 @@ def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
         tot = None
         if return_total_attention:
             tot = torch.empty((B, H, N), dtype=torch.float32, device=q.device)
-            _lib.check(lib.sage_flash_total_attention(p, L.data_ptr(), tot.data_ptr(), current_stream_ptr(q.device)),
-                       "sage_flash_total_attention")
+            tot_bytes = lib.sage_flash_total_attention_workspace_bytes(p)
+            if tot_bytes < 0:
+                _lib.check(-1, "sage_flash_total_attention_workspace_bytes")
+            tot_ws = torch.empty(tot_bytes, dtype=torch.uint8, device=q.device) if tot_bytes else None
+            _lib.check(lib.sage_flash_total_attention_ws(p, L.data_ptr(), tot.data_ptr(), tot_ws.data_ptr() if tot_bytes else None,
+                                                         tot_bytes, current_stream_ptr(q.device)), "sage_flash_total_attention_ws")
     if D < 64:
         o = o[..., :D].contiguous()
     if return_log_normalizer or return_total_attention or return_seed_offset:

@@ -239,6 +239,14 @@ int sage_flash_dropout_mask(uint8_t* mask, int64_t batch, int64_t heads_q, int64
 int sage_flash_total_attention(const sage_flash_params* p, const float* log_normalizer, float* total_attention,
                                void* stream);
 
+/*
+ * The same call with a workspace (rules of sage_attn_fwd_ws): where the key blocks alone would leave compute units idle
+ * the queries are cut into runs, whose sums meet in the workspace and are added in order by a second kernel.
+ */
+int64_t sage_flash_total_attention_workspace_bytes(const sage_flash_params* p);
+int sage_flash_total_attention_ws(const sage_flash_params* p, const float* log_normalizer, float* total_attention,
+                                  void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Message describing the last non-zero status returned on this thread ("" if none). */
 const char* sage_hip_last_error(void);
 
