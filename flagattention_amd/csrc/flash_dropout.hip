@@ -8,10 +8,19 @@
 // (x read as int32).  The row sums of the softmax are taken BEFORE the mask, the output is scaled by
 // 1 / (1 - dropout_p) at the end (flash.py:470-477, :499-502).
 //
-// Six rounds of 32 x 32 -> 64 bit products per score cost an order of magnitude more than the softmax itself, so
-// this kernel is a plain one, not the software-pipelined kernel of attn_fast_kernel.h: a wave owns 32 queries,
-// walks over the keys 32 at a time, S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16 with K rows loaded
-// straight into the A operand and V staged through LDS (two barriers per tile).
+// Six rounds of 32 x 32 -> 64 bit products per score cost more vector instructions than the softmax, so this kernel is
+// bound by the vector issue port and is built for it (rates measured with four waves per SIMD, in cycles at 2.4 GHz: integer
+// products 5.5, three-input XOR 4.8, exponential 9, FMA and XOR 3; with two waves per SIMD everything takes 5.7 or more):
+// * the generator is unrolled by hand (philox6_from_product): 4 full products, 3 high and 1 low half and one 64-bit addition per
+//   score instead of 12 full products; what depends on the row only is computed once per row;
+// * the keep decision is an integer threshold and a sign, applied to two 16-bit P at a time (no compare, no select);
+// * the rest is kept small: K and V tiles of 32 keys go straight into LDS for the four waves of a workgroup (32 queries
+//   each, S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16, V^T by ds_read_b64_tr_b16), one barrier per tile, loads
+//   one tile ahead (a tile takes microseconds), registers for four (head_dim 128: two) waves per SIMD;
+// * workgroups are handed out longest first over all heads.
+// B4 H16 M2048 N2048 D64 fp16 causal 403 -> 164 us, without the causal flag 404 -> 279 us; B2 H32 M4096 N4096 D128 3475 -> 1220
+// us, causal 3445 -> 626 us (before: the generator rolled out by the compiler, V^T gathered from LDS entry by entry,
+// short rows first).  At head_dim 128 three waves per SIMD need 18 spilled registers and run 6 % slower than two.
 #include "attn_common.h"
 
 namespace sage {
@@ -53,6 +62,9 @@ struct DropArgs {
     float* log_normalizer;  // [B, Hq, M] natural log, or null
     int64_t qs_b, qs_h, qs_n, ks_b, ks_h, ks_n, vs_b, vs_h, vs_n, os_b, os_h, os_n;
     int32_t Hq, M, N, groups, causal, out_dt;
+    int32_t BH, nmb;   // batch * heads, 128-query blocks
+    int32_t snake;     // blocks of one round over the CUs, 0: plain order
+    int32_t keep_from; // smallest folded output word that is kept
     float qk_scale;    // sm_scale * log2(e)
     float dropout_p, keep_scale;  // keep_scale = 1 / (1 - dropout_p)
     uint32_t seed_lo, seed_hi;
@@ -60,21 +72,79 @@ struct DropArgs {
 };
 
 constexpr int kDropWaves = 4;  // 128 queries per workgroup
+constexpr int kDropThreads = 64 * kDropWaves;
 constexpr int kDropKeys = 32;  // keys per tile
 
-template <int D, typename VT>
-__global__ __launch_bounds__(64 * kDropWaves) void flash_dropout_fwd_kernel(DropArgs a) {
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
+
+// Philox-4x32 of six rounds for consecutive counters whose high word does not change: what six rounds of
+//   (c0, c1, c2, c3) <- (hi(B c2) ^ c1 ^ k0, lo(B c2), hi(A c0) ^ c3 ^ k1, lo(A c0))
+// from (low, high, 0, 0) leave to be computed per low word for the first output word.
+struct PhiloxRow {
+    uint32_t hi_word;  // the counters' high word
+    uint32_t x2, x3;   // key words mixed with the product of round two, which depends on the high word only
+};
+
+constexpr uint32_t kPhiloxA = 0xD2511F53u, kPhiloxB = 0xCD9E8D57u, kPhiloxKeyA = 0x9E3779B9u, kPhiloxKeyB = 0xBB67AE85u;
+
+__device__ __forceinline__ PhiloxRow philox_row(uint32_t hi_word, uint32_t k0, uint32_t k1) {
+    const uint64_t u = (uint64_t)kPhiloxA * (hi_word ^ k0);
+    return {hi_word, (uint32_t)(u >> 32) ^ (k1 + kPhiloxKeyB), (uint32_t)u ^ (k1 + 2 * kPhiloxKeyB)};
+}
+
+// first: A * low word, all 64 bits
+__device__ __forceinline__ uint32_t philox6_from_product(uint64_t first, const PhiloxRow& r, uint32_t k0, uint32_t k1) {
+    auto hi = [](uint64_t x) { return (uint32_t)(x >> 32); };
+    const uint64_t b1 = (uint64_t)kPhiloxB * (hi(first) ^ k1);
+    const uint64_t a2 = (uint64_t)kPhiloxA * (hi(b1) ^ (k0 + kPhiloxKeyA));
+    const uint64_t b2 = (uint64_t)kPhiloxB * ((uint32_t)first ^ r.x2);
+    const uint64_t a3 = (uint64_t)kPhiloxA * (hi(b2) ^ (uint32_t)b1 ^ (k0 + 2 * kPhiloxKeyA));
+    const uint32_t c2 = hi(a2) ^ r.x3;
+    const uint32_t c0 = __umulhi(kPhiloxB, c2) ^ (uint32_t)b2 ^ (k0 + 3 * kPhiloxKeyA);
+    const uint32_t d2 = hi(a3) ^ (uint32_t)a2 ^ (k1 + 3 * kPhiloxKeyB);
+    const uint32_t e2 = __umulhi(kPhiloxA, c0) ^ (uint32_t)a3 ^ (k1 + 4 * kPhiloxKeyB);
+    return __umulhi(kPhiloxB, e2) ^ (kPhiloxB * d2) ^ (k0 + 5 * kPhiloxKeyA);
+}
+
+// negative iff the element with this output word is dropped: the word folds to [0, 2^31) and is kept from keep_from on
+__device__ __forceinline__ int32_t drop_sign(uint32_t word, int32_t keep_from) {
+    const int32_t x = (int32_t)word;
+    return (int32_t)((uint32_t)(x ^ (x >> 31)) - (uint32_t)keep_from);
+}
+
+template <int D> __device__ __forceinline__ int drop_v_swizzle(int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); }
+
+// KG: groups of four waves that share the queries of a workgroup and take its key tiles in turn (drop_groups)
+constexpr int drop_waves_per_simd(int head_dim) { return head_dim == 128 ? 2 : 4; }
+
+template <int D, typename VT, int KG>
+__global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D) / KG) void flash_dropout_fwd_kernel(DropArgs a) {
     using PVT = PV<VT>;
     using vec16 = typename PVT::vec;
     constexpr int KS = D / 16;      // matrix instructions of one 32 x 32 score tile
     constexpr int DT = D / 32;      // 32-channel tiles of the output
-    constexpr int V_RS = D + 2;     // LDS row stride in elements: rows four apart fall into different banks
-    __shared__ VT vtile[kDropKeys * V_RS];
+    constexpr int RS = 2 * D;       // bytes per K / V row
+    constexpr int CPR = RS / 16;    // 16-byte chunks per row
+    constexpr int TILE = kDropKeys * RS;
+    constexpr int LOADS = TILE / 1024 / kDropWaves;  // 1 KB loads per wave of a K (of a V) tile
+    __shared__ __attribute__((aligned(16))) unsigned char smem[KG][2][2][TILE];  // [group][buffer][K, V]
+    __shared__ float row_m[KG > 1 ? KG * 32 * kDropWaves : 1], row_l[KG > 1 ? KG * 32 * kDropWaves : 1];
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_all % kDropWaves, group = wave_all / kDropWaves;
     const int l32 = lane & 31, half = lane >> 5;
-    const int h = blockIdx.y, b = blockIdx.z, hk = h / a.groups;
-    const int m0 = blockIdx.x * (32 * kDropWaves);
+    // heads fastest (a head stays on one XCD); under the causal flag the last queries, which see the most keys, first
+    // (snake: all workgroups are resident at once, so every second round of 256, one per CU, goes in the reverse order of
+    // blocks and a CU holds long and short ones: B4 H16 M2048 N2048 D64 causal 177 -> 166 us)
+    const int bh = blockIdx.x % a.BH;
+    int rank = blockIdx.x / a.BH;
+    if (a.snake > 0 && (rank / a.snake) % 2 == 1 && (rank / a.snake + 1) * a.snake <= a.nmb)
+        rank = (rank / a.snake) * a.snake + a.snake - 1 - rank % a.snake;
+    const int mb = a.nmb - 1 - rank;
+    const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.groups;
+    const int m0 = mb * (32 * kDropWaves);
     const int my_m = m0 + 32 * wave + l32;
     const bool row_ok = my_m < a.M;
     const int shift = a.N - a.M;
@@ -87,95 +157,213 @@ __global__ __launch_bounds__(64 * kDropWaves) void flash_dropout_fwd_kernel(Drop
 #pragma unroll
         for (int t = 0; t < KS; t++) qf[t] = *reinterpret_cast<const vec16*>(qp + 16 * t);
     }
-    const VT* kbase = static_cast<const VT*>(a.k) + (int64_t)b * a.ks_b + (int64_t)hk * a.ks_h + 8 * half;
+    // (waited for here: inside the loop the compiler's waits for them would also wait for the tile on its way)
+#pragma unroll
+    for (int t = 0; t < KS; t++) {
+        v4i bits = __builtin_bit_cast(v4i, qf[t]);
+        asm volatile("" : "+v"(bits));
+        qf[t] = __builtin_bit_cast(vec16, bits);
+    }
+    const VT* kbase = static_cast<const VT*>(a.k) + (int64_t)b * a.ks_b + (int64_t)hk * a.ks_h;
     const VT* vbase = static_cast<const VT*>(a.v) + (int64_t)b * a.vs_b + (int64_t)hk * a.vs_h;
-    // offset of element (b, h, my_m, 0) in the random stream
-    const uint64_t rng_row = a.offset + (((uint64_t)b * a.Hq + h) * (uint64_t)a.M + (uint64_t)my_m) * (uint64_t)a.N;
 
-    // keys that any row of the workgroup can see
-    int n_end = a.N;
-    if (a.causal) n_end = max(min(a.N, min(m0 + 32 * kDropWaves, a.M) + shift), 0);
-    const int my_lim = a.causal ? min(my_m + shift, a.N - 1) : a.N - 1;  // last key this lane's query sees
+    // keys that any row of the workgroup / of this wave can see
+    int n_end = a.N, wave_end = a.N;
+    if (a.causal) {
+        n_end = max(min(a.N, min(m0 + 32 * kDropWaves, a.M) + shift), 0);
+        wave_end = min(m0 + 32 * wave + 32, a.M) + shift;
+    }
+    const int my_lim = a.causal ? min(my_m + shift, a.N - 1) : a.N - 1;              // last key this lane's query sees
+    const int first_lim = a.causal ? min(m0 + 32 * wave + shift, a.N - 1) : a.N - 1;  // ... the wave's first query
+    const int ntiles = (n_end + kDropKeys - 1) / kDropKeys;
+
+    // Tile t of K and V -> one of the group's two buffers, straight into LDS (written in assembly, as in attn_fast_kernel.h: the compiler would
+    // wait for every outstanding load before each LDS read; m0 holds the LDS address and nothing else here uses it).  Chunk
+    // c of row r lies at chunk c ^ (r mod chunks) for K and at c ^ drop_v_swizzle(r) for V: the load fetches the chunk
+    // that belongs where a lane writes, the fragment reads spread over all banks.  Rows past the end re-read the last one.
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&smem[group][0][0][0];
+    unsigned koff[LOADS], voff[LOADS];
+    auto set_offsets = [&](int last) {  // last: the tile's last row
+#pragma unroll
+        for (int e = 0; e < LOADS; e++) {
+            const int row = (64 / CPR) * (LOADS * wave + e) + lane / CPR;
+            koff[e] = (unsigned)min(row, last) * (unsigned)(a.ks_n * 2) + 16 * ((lane % CPR) ^ (row & (CPR - 1)));
+            voff[e] = (unsigned)min(row, last) * (unsigned)(a.vs_n * 2) + 16 * ((lane % CPR) ^ drop_v_swizzle<D>(row));
+        }
+    };
+    set_offsets(kDropKeys - 1);
+    auto fetch = [&](int t, int buf) {
+        const int n0 = kDropKeys * t;
+        if (n0 + kDropKeys > a.N) set_offsets(a.N - 1 - n0);  // (the last tile)
+        const VT* kt = kbase + (int64_t)n0 * a.ks_n;
+        const VT* vt = vbase + (int64_t)n0 * a.vs_n;
+        const unsigned dst = lds0 + (unsigned)(buf * 2 * TILE + 1024 * LOADS * wave);
+#pragma unroll
+        for (int e = 0; e < LOADS; e++) {
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(koff[e]), "s"(kt), "s"(dst + 1024 * e) : "memory");
+            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff[e]), "s"(vt), "s"(dst + TILE + 1024 * e) : "memory");
+        }
+    };
+    int vtr[DT];  // LDS offsets of the transposed fragment reads (see attn_fast_kernel.h)
+    {
+        const int s4 = (lane >> 2) & 3, a4 = lane & 3, g1 = (lane >> 4) & 1;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+            vtr[dt] = (4 * half + s4) * RS + 16 * ((4 * dt + 2 * g1 + (a4 >> 1)) ^ drop_v_swizzle<D>(s4)) + 8 * (a4 & 1);
+    }
+
+    // offset of element (b, h, my_m, 4 half) in the random stream: this lane's first key of a tile, from the tile's start on
+    const uint64_t rng_row = a.offset + (((uint64_t)b * a.Hq + h) * (uint64_t)a.M + (uint64_t)my_m) * (uint64_t)a.N + 4 * half;
+    PhiloxRow prow = philox_row((uint32_t)(rng_row >> 32), a.seed_lo, a.seed_hi);
 
     v16f acc[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[dt][i] = 0.0f;
-    float m_i = -INFINITY, l_i = 0.0f;  // running maximum (base-2 units) and this half's part of the row sum
+    float m_i = -INFINITY, l_i = 0.0f;  // running maximum (unscaled scores) and this half's part of the row sum
 
-    for (int n0 = 0; n0 < n_end; n0 += kDropKeys) {
-        // K rows as the A operand: lane (key l32, half); rows past the end re-read the last one (their scores are hidden)
-        vec16 kf[KS];
-        {
-            const VT* kp = kbase + (int64_t)min(n0 + l32, a.N - 1) * a.ks_n;
-#pragma unroll
-            for (int t = 0; t < KS; t++) kf[t] = *reinterpret_cast<const vec16*>(kp + 16 * t);
-        }
-        // V tile -> LDS, 16 bytes per thread and round
-        __syncthreads();  // the previous tile has been read
-#pragma unroll
-        for (int c = threadIdx.x; c < kDropKeys * D / 8; c += 64 * kDropWaves) {
-            const int row = c / (D / 8), piece = c % (D / 8);
-            const vec16 x = *reinterpret_cast<const vec16*>(vbase + (int64_t)min(n0 + row, a.N - 1) * a.vs_n + 8 * piece);
-            // (rows are 4-byte aligned only: V_RS is not a multiple of 8 elements)
-            typedef uint32_t __attribute__((may_alias)) word;
-            word w[4];
-            __builtin_memcpy(w, &x, 16);
-            word* dst = reinterpret_cast<word*>(&vtile[row * V_RS + 8 * piece]);
-#pragma unroll
-            for (int j = 0; j < 4; j++) dst[j] = w[j];
-        }
-        __syncthreads();
+    if (group < ntiles) fetch(group, 0);
+    const int rounds = (ntiles + KG - 1) / KG;
+    for (int r = 0; r < rounds; r++) {
+        // vmcnt(0): this round's tiles have landed, for all waves past the barrier; the last round's have been read
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __builtin_amdgcn_s_barrier();
+        const int t = r * KG + group;
+        if (t + KG < ntiles) fetch(t + KG, (r + 1) & 1);
+        const int n0 = kDropKeys * t;
+        if (t >= ntiles || (a.causal && n0 >= wave_end)) continue;  // (no query of this wave sees a key of the tile)
+        const unsigned char* ktile = smem[group][r & 1][0];
+        const unsigned char* vtile = smem[group][r & 1][1];
 
         v16f s;
 #pragma unroll
         for (int i = 0; i < 16; i++) s[i] = 0.0f;
+        int krow = l32 * RS + 16 * (half ^ (l32 & (CPR - 1)));
+        asm volatile("" : "+v"(krow));  // (the addresses of the fragments, krow ^ 32 c, are not kept from tile to tile)
 #pragma unroll
-        for (int t = 0; t < KS; t++) s = PVT::mfma(kf[t], qf[t], s);
+        for (int c = 0; c < KS; c++) s = PVT::mfma(*reinterpret_cast<const vec16*>(ktile + (krow ^ (32 * c))), qf[c], s);
 
         // accumulator i of this lane: key n0 + 8 (i / 4) + 4 half + i % 4 of query my_m
+        if (n0 + kDropKeys - 1 > first_lim) {
+            const int last = my_lim - n0 - 4 * half;
+#pragma unroll
+            for (int i = 0; i < 16; i++) s[i] = 8 * (i >> 2) + (i & 3) <= last ? s[i] : -INFINITY;
+        }
         float tile_max = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int n = n0 + 8 * (i >> 2) + 4 * half + (i & 3);
-            s[i] = n <= my_lim ? s[i] * a.qk_scale : -INFINITY;
-            tile_max = fmaxf(tile_max, s[i]);
-        }
+        for (int i = 0; i < 16; i++) tile_max = fmaxf(tile_max, s[i]);
         tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
         const float m_new = fmaxf(m_i, tile_max);
-        // (a query that has seen no key yet keeps m = -inf: every p below is then 0 and alpha is 1)
-        const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-        const float alpha = m_i == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_i - m_use);
-        float psum = 0.0f;
+        // (a query that has seen no key yet keeps m = -inf: every p below is then 0)
+        const float m_use = m_new == -INFINITY ? 0.0f : m_new * a.qk_scale;
+        if (__builtin_amdgcn_ballot_w64(m_new > m_i) != 0) {
+            const float alpha = m_i == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m_i, a.qk_scale, -m_use));
+            l_i *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc[dt][i] *= alpha;
+            m_i = m_new;
+        }
+        // ---- P, its row sum (which does not see the dropout mask), and the mask
+        const uint64_t first = rng_row + (uint64_t)n0;
+        const uint32_t lo = (uint32_t)first;
+        // (the low words of the tile run over 28 consecutive values; once per 2^32 draws they wrap inside one)
+        const bool wraps = __builtin_amdgcn_ballot_w64(lo + 27u < lo) != 0;
+        if ((uint32_t)(first >> 32) != prow.hi_word) prow = philox_row((uint32_t)(first >> 32), a.seed_lo, a.seed_hi);
         vec16 pf[2];
+        float psum = 0.0f;
+        uint32_t pbits[8];
+        // two scores and the signs of their words (bit 31 set: dropped) -> two 16-bit P
+        auto put = [&](int i, int32_t sign0, int32_t sign1) {
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.qk_scale, -m_use));  // hidden keys: exp2(-inf) = 0
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], a.qk_scale, -m_use));
+            psum += p0;
+            psum += p1;
+            typedef VT vt2 __attribute__((ext_vector_type(2)));
+            // bytes of the mask: the sign of the first word twice, that of the second twice (v_perm_b32 replicates bit 31)
+            const uint32_t dropped = __builtin_amdgcn_perm((uint32_t)sign1, (uint32_t)sign0, 0x0b0b0909u);
+            pbits[i / 2] = __builtin_bit_cast(uint32_t, vt2{(VT)p0, (VT)p1}) & ~dropped;
+        };
+        if (!wraps) {
+            const uint64_t product = (uint64_t)kPhiloxA * lo;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int n = n0 + 8 * (i >> 2) + 4 * half + (i & 3);
-            float p = __builtin_amdgcn_exp2f(s[i] - m_use);  // hidden keys: exp2(-inf) = 0
-            psum += p;                                        // the row sum does not see the dropout mask
-            if (!dropout_keeps(rng_row + (uint64_t)n, a.seed_lo, a.seed_hi, a.dropout_p)) p = 0.0f;
-            pf[i >> 3][i & 7] = (VT)p;
-        }
-        l_i = l_i * alpha + psum;
-        m_i = m_new;
+            for (int i = 0; i < 16; i += 2) {
+                int32_t sign[2];
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) acc[dt][i] *= alpha;
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                // V^T as the A operand, in the key order of pf[t]: element j is key 16 t + 8 (j / 4) + 4 half + j % 4
-                vec16 vf;
-#pragma unroll
-                for (int j = 0; j < 8; j++)
-                    vf[j] = vtile[(16 * t + 8 * (j >> 2) + 4 * half + (j & 3)) * V_RS + 32 * dt + l32];
-                acc[dt] = PVT::mfma(vf, pf[t], acc[dt]);
+                for (int e = 0; e < 2; e++) {
+                    const int k = 8 * ((i + e) >> 2) + ((i + e) & 3);
+                    sign[e] = drop_sign(philox6_from_product(product + (uint64_t)kPhiloxA * k, prow, a.seed_lo, a.seed_hi), a.keep_from);
+                }
+                put(i, sign[0], sign[1]);
+                __builtin_amdgcn_sched_barrier(0);  // (two scores at a time: all sixteen side by side would not fit the registers)
             }
+        } else {  // every counter with a high word of its own
+            uint32_t dropped = 0;
+#pragma unroll 1
+            for (int i = 0; i < 16; i++)
+                dropped |= (dropout_keeps(first + (uint64_t)(8 * (i >> 2) + (i & 3)), a.seed_lo, a.seed_hi, a.dropout_p) ? 0u : 1u) << i;
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) put(i, (int32_t)(dropped << (31 - i)), (int32_t)(dropped << (30 - i)));
         }
+        l_i += psum;
+#pragma unroll
+        for (int c = 0; c < 2; c++) pf[c] = __builtin_bit_cast(vec16, v4i{(int)pbits[4 * c], (int)pbits[4 * c + 1], (int)pbits[4 * c + 2], (int)pbits[4 * c + 3]});
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int dt = 0; dt < DT; dt++) {
+                const unsigned char* p0 = vtile + vtr[dt] + 16 * c * RS;
+                const s16x4 v_lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)p0);
+                const s16x4 v_hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(p0 + 8 * RS));
+                acc[dt] = PVT::mfma(__builtin_bit_cast(vec16, __builtin_shufflevector(v_lo, v_hi, 0, 1, 2, 3, 4, 5, 6, 7)), pf[c], acc[dt]);
+            }
     }
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // nothing of this workgroup is on its way into LDS when it ends
 
-    const float l_tot = l_i + __shfl_xor(l_i, 32);
+    float l_tot = l_i + __shfl_xor(l_i, 32);
+    if constexpr (KG > 1) {  // the groups' shares of a row -> group 0
+        static_assert(sizeof(float) * 32 * kDropWaves * D <= sizeof(smem), "one group's accumulators fit the tile buffers");
+        const int slot = 32 * wave + l32;
+        if (half == 0) {
+            row_m[group * 32 * kDropWaves + slot] = m_i;
+            row_l[group * 32 * kDropWaves + slot] = l_tot;
+        }
+        __syncthreads();
+        float m = -INFINITY, l = 0.0f;
+#pragma unroll
+        for (int g = 0; g < KG; g++) m = fmaxf(m, row_m[g * 32 * kDropWaves + slot]);
+        const float base = m == -INFINITY ? 0.0f : m * a.qk_scale;
+#pragma unroll
+        for (int g = 0; g < KG; g++)
+            l += row_l[g * 32 * kDropWaves + slot] * __builtin_amdgcn_exp2f(__builtin_fmaf(row_m[g * 32 * kDropWaves + slot], a.qk_scale, -base));
+        const float mine = __builtin_amdgcn_exp2f(__builtin_fmaf(m_i, a.qk_scale, -base));
+        float* park = reinterpret_cast<float*>(&smem[0][0][0][0]) + wave * 32 * D + lane;  // entry e of a lane: 64 e further on
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[dt][i] *= mine;
+        for (int g = 1; g < KG; g++) {
+            if (group == g) {
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) park[64 * (16 * dt + i)] = acc[dt][i];
+            }
+            __syncthreads();
+            if (group == 0) {
+#pragma unroll
+                for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                    for (int i = 0; i < 16; i++) acc[dt][i] += park[64 * (16 * dt + i)];
+            }
+            __syncthreads();
+        }
+        if (group != 0) return;
+        m_i = m;
+        l_tot = l;
+    }
     const float inv = l_tot > 0.0f ? a.keep_scale / l_tot : 0.0f;  // l = 0: a query that saw no key: zero row
     if (!row_ok) return;
     // accumulator i of tile dt: channel 32 dt + 8 (i / 4) + 4 half + i % 4 of query my_m
@@ -200,7 +388,7 @@ __global__ __launch_bounds__(64 * kDropWaves) void flash_dropout_fwd_kernel(Drop
         }
     if (a.log_normalizer && half == 0)
         a.log_normalizer[((int64_t)b * a.Hq + h) * a.M + my_m] =
-            l_tot > 0.0f ? (__builtin_log2f(l_tot) + m_i) * 0.693147180559945309f : -INFINITY;
+            l_tot > 0.0f ? (__builtin_log2f(l_tot) + m_i * a.qk_scale) * 0.693147180559945309f : -INFINITY;
 }
 
 __global__ void dropout_mask_kernel(uint8_t* mask, int64_t count, uint64_t offset, uint32_t seed_lo, uint32_t seed_hi,
@@ -209,10 +397,26 @@ __global__ void dropout_mask_kernel(uint8_t* mask, int64_t count, uint64_t offse
     if (i < count) mask[i] = dropout_keeps(offset + (uint64_t)i, seed_lo, seed_hi, dropout_p) ? 1 : 0;
 }
 
+// Groups of waves per workgroup: as many as the SIMDs hold waves for, where there are fewer workgroups than that takes (a
+// SIMD with one wave issues a vector instruction every 5.7 cycles, with four waves every 3).
+int drop_groups(int64_t wgs, int head_dim) {
+    int groups = 1;
+    while (groups < drop_waves_per_simd(head_dim) && wgs * groups * 2 <= 256 * drop_waves_per_simd(head_dim)) groups *= 2;
+    return groups;
+}
+
 template <int D, typename VT>
-int launch_drop(const DropArgs& a, int64_t B, hipStream_t stream) {
-    dim3 grid((unsigned)((a.M + 32 * kDropWaves - 1) / (32 * kDropWaves)), (unsigned)a.Hq, (unsigned)B), block(64 * kDropWaves);
-    hipLaunchKernelGGL((flash_dropout_fwd_kernel<D, VT>), grid, block, 0, stream, a);
+int launch_drop(DropArgs a, int64_t B, hipStream_t stream) {
+    const int64_t wgs = B * a.Hq * a.nmb;
+    if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd_dropout: too many query blocks for one launch");
+    const int groups = drop_groups(wgs, D);
+    if (a.causal && wgs * groups <= 256 * drop_waves_per_simd(D) && a.BH < 256) a.snake = 256 / a.BH;
+    dim3 grid((unsigned)wgs);
+    if constexpr (D == 64) {
+        if (groups == 4) hipLaunchKernelGGL((flash_dropout_fwd_kernel<D, VT, 4>), grid, dim3(4 * kDropThreads), 0, stream, a);
+    }
+    if (groups == 2) hipLaunchKernelGGL((flash_dropout_fwd_kernel<D, VT, 2>), grid, dim3(2 * kDropThreads), 0, stream, a);
+    else if (groups == 1) hipLaunchKernelGGL((flash_dropout_fwd_kernel<D, VT, 1>), grid, dim3(kDropThreads), 0, stream, a);
     return check_launch("flash_dropout_fwd_kernel");
 }
 
@@ -232,8 +436,20 @@ int launch_flash_dropout(const sage_flash_params& p, float dropout_p, uint64_t s
     a.keep_scale = 1.0f / (1.0f - dropout_p);
     a.seed_lo = (uint32_t)seed; a.seed_hi = (uint32_t)(seed >> 32);
     a.offset = offset;
-    if (p.heads_q > 65535 || p.batch > 65535)
-        return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd_dropout: more than 65535 heads or batches");
+    // the threshold on the folded word, from the comparison it stands for: (float)word * 4.6566127342e-10f > dropout_p
+    {
+        int64_t lo = 0, hi = 1LL << 31;  // hi: none is kept (drop_sign is then negative for every word)
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) / 2;
+            if ((float)(int32_t)mid * 4.6566127342e-10f > dropout_p) hi = mid;
+            else lo = mid + 1;
+        }
+        a.keep_from = (int32_t)(uint32_t)lo;
+    }
+    a.BH = (int)(p.batch * p.heads_q);
+    a.nmb = (a.M + 32 * kDropWaves - 1) / (32 * kDropWaves);
+    if (p.k.stride_n < 0 || p.v.stride_n < 0 || p.k.stride_n >= (1LL << 25) || p.v.stride_n >= (1LL << 25))
+        return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd_dropout: k/v sequence stride out of range for 32-bit tile offsets");
     if (p.head_dim == 128)
         return p.dtype == SAGE_BF16 ? launch_drop<128, __bf16>(a, p.batch, stream) : launch_drop<128, _Float16>(a, p.batch, stream);
     return p.dtype == SAGE_BF16 ? launch_drop<64, __bf16>(a, p.batch, stream) : launch_drop<64, _Float16>(a, p.batch, stream);

@@ -103,6 +103,8 @@ def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
     q, k, v = _rows16(q), _rows16(k), _rows16(v)
     if return_total_attention and q.stride(2) >= 1 << 25:
         q = q.contiguous()  # (that kernel reaches the 32 rows of a query tile with 32-bit byte offsets)
+    if is_dropout and max(k.stride(2), v.stride(2)) >= 1 << 25:
+        k, v = k.contiguous(), v.contiguous()  # (the same holds for the key tiles of the dropout kernel)
     o = torch.empty_like(q)  # (the reference allocates the same way, flash.py:84-90)
     if not rows_aligned(o):
         o = torch.empty(q.shape, dtype=q.dtype, device=q.device)

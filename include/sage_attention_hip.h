@@ -219,7 +219,7 @@ int sage_flash_attn_fwd_ws(const sage_flash_params* p, void* workspace, int64_t 
  * the seed, first output word -> fp32 in [0, 1)); the softmax row sums and the log normalizer do not see the mask,
  * the output is scaled by 1 / (1 - dropout_p).  seed and offset are the caller's (the reference takes them from
  * torch's CUDA generator, dropout.py:17-28).  dropout_p in (0, 1); batch * heads_q * qo_len * kv_len < 2^31.
- * A plain kernel, an order of magnitude slower than sage_flash_attn_fwd: the generator dominates.
+ * A kernel of its own, several times slower than sage_flash_attn_fwd: the generator dominates.
  *
  * sage_flash_dropout_mask writes the same mask on its own (src/flag_attn/testing/dropout.py:19-39):
  *   mask   [batch, heads_q, qo_len, kv_len] bytes, contiguous, 1 = kept

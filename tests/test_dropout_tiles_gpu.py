@@ -1,0 +1,40 @@
+"""The dropout forward kernel where its own choices change: one, two or four groups of waves per workgroup (by the number of
+128-query blocks), tile edges (32 keys, 128 queries), a random stream whose low counter word wraps inside the call, drop
+probabilities at the ends of the range.  Rule of the other dropout tests: at most twice the deviation of the 16-bit form."""
+import pytest
+import torch
+
+from oracle import flash_oracle as FO
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("p,offset", [(0.3, 0), (1e-6, 2 ** 32 - 4096), (0.9, 2 ** 32 - 70000)])
+@pytest.mark.parametrize("B,H,Hk,M,N,D,causal", [
+    (1, 2, 1, 1, 33, 64, False), (1, 2, 2, 129, 31, 64, True), (2, 3, 3, 127, 128, 128, True),   # four / two groups
+    (6, 16, 8, 600, 70, 64, True),     # 480 blocks: two groups
+    (6, 16, 16, 800, 65, 64, True),    # 672 blocks: one
+    (3, 16, 16, 700, 97, 128, True),   # 288 blocks at head_dim 128: one
+    (1, 16, 16, 130, 300, 128, False),
+])
+def test_dropout_forward_tiles(B, H, Hk, M, N, D, causal, p, offset, gpu_device):
+    import flag_attn
+
+    dtype = torch.bfloat16 if (M + D) % 2 else torch.float16
+    g = torch.Generator().manual_seed(41)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(dtype) for h, n in ((H, M), (Hk, N), (Hk, N)))
+    dq, dk, dv = (t.to(gpu_device) for t in (q, k, v))
+    gen = torch.cuda.default_generators[gpu_device.index or 0]
+    gen.manual_seed(99)
+    gen.set_offset(offset)
+    o, L, _, seed, off = flag_attn.flash_attention(dq, dk, dv, causal, dropout_p=p,
+                                                   return_log_normalizer=True, return_seed_offset=True)
+    assert (seed, off) == (99, offset)
+    mask = flag_attn.testing.recompute_mask(B, H, M, N, p, seed, off, gpu_device).cpu()
+    o_ref, L_ref = FO.attention(q, k, v, causal, dropout_p=p, dropout_mask=mask, return_log_normalizer=True, upcast=True)
+    yard = FO.max_diff(FO.attention(q, k, v, causal, dropout_p=p, dropout_mask=mask, upcast=False), o_ref)
+    got = FO.max_diff(o.cpu(), o_ref)
+    assert got <= 2 * yard + 1e-5, (got, yard)
+    inf = torch.isinf(L_ref)
+    assert torch.equal(torch.isinf(L.cpu()), inf)
+    torch.testing.assert_close(L.cpu()[~inf], L_ref[~inf], atol=2e-3, rtol=2e-4)
