@@ -44,6 +44,10 @@ struct QuantArgs {
     // the per-row shift K smoothing takes out of every logit of row n.  km is then NOT subtracted from x.
     float* dot;
     int32_t dot_groups;
+    // Optional (K blocks of the K-smoothing entry point, short sequences): km is not there yet; every block adds the chunk
+    // partials of its head in order (k_mean_final_kernel's arithmetic), the head's first block writes km as well.
+    const float* part;   // [B * H, nblk, D]
+    void* km_write;      // [B * H, D], km_dt
     int32_t small_offsets;  // every byte offset inside one block of x and of out fits 31 bits (host-checked)
 };
 
@@ -125,11 +129,24 @@ __device__ __forceinline__ uint2 quantize8(const float (&v)[8], float scale, flo
     return make_uint2(pack4(q[0], q[1], q[2], q[3]), pack4(q[4], q[5], q[6], q[7]));
 }
 
+// max of the wave's non-negative values, in every lane: lane permutations inside the vector instructions (row_shr 1, 2, 4, 8,
+// then lane 15 of a row to the next row, lane 31 to the upper half), where __shfl_xor takes a trip through LDS per step
+__device__ __forceinline__ float wave_max_nonneg(float x) {
+#define SAGE_DPP_MAX(ctrl) x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), ctrl, 0xf, 0xf, false)))
+    SAGE_DPP_MAX(0x111);
+    SAGE_DPP_MAX(0x112);
+    SAGE_DPP_MAX(0x114);
+    SAGE_DPP_MAX(0x118);
+    SAGE_DPP_MAX(0x142);
+    SAGE_DPP_MAX(0x143);
+#undef SAGE_DPP_MAX
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
+}
+
 // max |x| of the workgroup (every thread gets it)
 template <int THREADS>
 __device__ __forceinline__ float block_amax(float amax, float* wave_max) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+    amax = wave_max_nonneg(amax);
     const int tid = threadIdx.x;
     if ((tid & 63) == 0) wave_max[tid >> 6] = amax;
     __syncthreads();
@@ -139,10 +156,37 @@ __device__ __forceinline__ float block_amax(float amax, float* wave_max) {
     return amax;
 }
 
+// The K mean of one head from its chunk partials: added in chunk order from 0.0f, one IEEE divide by the number of rows, one
+// rounding; a thread per channel.  km: the rounded means as fp32; out: where they are stored in their own type, or null.
+__device__ __forceinline__ void mean_from_partials(const float* part, int nchunk, int D, int rows, int out_dt, float* km, void* out, int64_t out_off) {
+    for (int d = threadIdx.x; d < D; d += blockDim.x) {
+        const float* p = part + d;
+        float tot = 0.0f;
+        int c = 0;
+        for (; c + 16 <= nchunk; c += 16) {  // loads issued together, additions kept in chunk order
+            float v[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = p[(int64_t)(c + i) * D];
+#pragma unroll
+            for (int i = 0; i < 16; i++) tot = tot + v[i];
+        }
+        for (; c < nchunk; c++) tot = tot + p[(int64_t)c * D];
+        const float mean = round_to(tot / (float)rows, out_dt);
+        km[d] = mean;
+        if (out) {
+            if (out_dt == SAGE_F32) static_cast<float*>(out)[out_off + d] = mean;
+            else if (out_dt == SAGE_BF16) static_cast<__bf16*>(out)[out_off + d] = (__bf16)mean;
+            else static_cast<_Float16*>(out)[out_off + d] = (_Float16)mean;
+        }
+    }
+}
+
 // One workgroup = one quantization block of `blk` rows; UNITS 8-element groups per thread.
 // wave_max: THREADS / 64 floats of LDS.
+constexpr int kMaxFusedMeanDim = 256;  // head_dim up to which a block adds its head's chunk partials on its own
+
 template <int DT, int UNITS, int THREADS>
-__device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* wave_max) {
+__device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* wave_max, float* km_lds = nullptr) {
     const int tid = threadIdx.x;
     const int ib = bid % a.nblk;
     const int h = (bid / a.nblk) % a.H;
@@ -159,6 +203,14 @@ __device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* 
     // group is loaded once.
     const bool fixed_c8 = a.ks_n == 0 && a.d8_shift >= 0 && a.D8 <= THREADS;
     float m_fixed[8];
+    const bool own_mean = km_lds != nullptr && a.part != nullptr;
+    if (own_mean) {
+        mean_from_partials(a.part + ((int64_t)b * a.H + h) * a.nblk * (a.D8 * 8), a.nblk, a.D8 * 8, a.L, a.km_dt, km_lds,
+                           ib == 0 ? a.km_write : nullptr, ((int64_t)b * a.H + h) * (a.D8 * 8));
+        __syncthreads();
+#pragma unroll
+        for (int e = 0; e < 8; e++) m_fixed[e] = km_lds[(tid & (a.D8 - 1)) * 8 + e];
+    }
     if (a.km && fixed_c8) load8_rt(a.km, a.km_dt, k_base + (tid & (a.D8 - 1)) * 8, m_fixed);
 
     constexpr int ESZ = DT == SAGE_F32 ? 4 : 2;
@@ -167,6 +219,7 @@ __device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* 
     //      a uniform base plus one 32-bit per-thread offset, nothing is masked and nothing is clamped.
     const bool whole = a.d8_shift >= 0 && a.D8 <= THREADS && total_units == UNITS * THREADS && (ib + 1) * a.blk <= a.L &&
                        (!a.km || fixed_c8) && a.small_offsets;
+    const bool subtract = a.km || own_mean;
     if (whole) {
         const int row0 = tid >> a.d8_shift, c8 = tid & (a.D8 - 1);
         const int rpp = THREADS >> a.d8_shift;  // rows per pass of the threads
@@ -202,7 +255,7 @@ __device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* 
                 for (int e = 0; e < 8; e++) d = d + v[j][e] * m_fixed[e];
                 for (int off = 1; off < a.D8; off <<= 1) d = d + __shfl_xor(d, off);
                 if (c8 == 0) a.dot[((int64_t)b * a.H + h) * a.L + ib * a.blk + row0 + j * rpp] = d;
-            } else if (a.km) {
+            } else if (subtract) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) v[j][e] = round_to(v[j][e] - m_fixed[e], a.diff_dt);
             }
@@ -274,9 +327,9 @@ __device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* 
         } else {
             unpack8(raw16[j], DT, v[j]);
         }
-        if (a.km) {
+        if (subtract) {
             float m[8];
-            if (fixed_c8) {
+            if (fixed_c8 || own_mean) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) m[e] = m_fixed[e];
             } else {
@@ -342,12 +395,58 @@ __global__ __launch_bounds__(THREADS) void quant_per_block_int8_kernel(QuantArgs
     quant_block<DT, UNITS, THREADS>(a, blockIdx.x, wave_max);
 }
 
+// The same for K blocks that take the mean from its chunk partials (a.part).
+template <int DT, int UNITS, int THREADS>
+__global__ __launch_bounds__(THREADS) void quant_own_mean_kernel(QuantArgs a) {
+    __shared__ float wave_max[THREADS / 64];
+    __shared__ float km_lds[kMaxFusedMeanDim];
+    quant_block<DT, UNITS, THREADS>(a, blockIdx.x, wave_max, km_lds);
+}
+
+// K and Q blocks in one grid, for calls so small that a second launch costs more than the better shape of workgroup for the Q
+// blocks (kBothBlocks): GPU time B1 H2 N256 D64 fp16 6.5 -> 3.6 us, B1 H32 N1024 D128 bf16 8.9 -> 6.8 us.
+constexpr int64_t kBothBlocks = 1024;
+template <int DT, int KU, int QU>
+__global__ __launch_bounds__(kThreads) void quant_both_kernel(QuantArgs kq, QuantArgs qq, int k_blocks) {
+    __shared__ float wave_max[kThreads / 64];
+    if ((int)blockIdx.x < k_blocks) quant_block<DT, KU, kThreads>(kq, blockIdx.x, wave_max);
+    else quant_block<DT, QU, kThreads>(qq, blockIdx.x - k_blocks, wave_max);
+}
+
+template <int DT>
+int launch_both_dt(const QuantArgs& kq, const QuantArgs& qq, int64_t k_blocks, int64_t q_blocks, hipStream_t stream) {
+    dim3 grid((unsigned)(k_blocks + q_blocks));
+    if (kq.blk * kq.D8 <= 2 * kThreads && qq.blk * qq.D8 <= 4 * kThreads)
+        hipLaunchKernelGGL((quant_both_kernel<DT, 2, 4>), grid, dim3(kThreads), 0, stream, kq, qq, (int)k_blocks);
+    else
+        hipLaunchKernelGGL((quant_both_kernel<DT, 4, 8>), grid, dim3(kThreads), 0, stream, kq, qq, (int)k_blocks);
+    return check_launch("quant_both_kernel");
+}
+
+bool both_fit(const QuantArgs& kq, const QuantArgs& qq, int64_t k_blocks, int64_t q_blocks) {
+    return k_blocks > 0 && q_blocks > 0 && k_blocks + q_blocks <= kBothBlocks && !kq.part && kq.blk * kq.D8 <= 4 * kThreads &&
+           qq.blk * qq.D8 <= 8 * kThreads;
+}
+
+int launch_both(const QuantArgs& kq, const QuantArgs& qq, int in_dtype, int64_t k_blocks, int64_t q_blocks, hipStream_t stream) {
+    switch (in_dtype) {
+        case SAGE_F16: return launch_both_dt<SAGE_F16>(kq, qq, k_blocks, q_blocks, stream);
+        case SAGE_BF16: return launch_both_dt<SAGE_BF16>(kq, qq, k_blocks, q_blocks, stream);
+        default: return launch_both_dt<SAGE_F32>(kq, qq, k_blocks, q_blocks, stream);
+    }
+}
+
 template <int DT>
 int launch_one(const QuantArgs& a, int64_t nblocks, hipStream_t stream) {
     // four 16-byte loads in flight per thread wherever the block is large enough, and a register
     // footprint that keeps eight waves per SIMD resident
     const int total_units = a.blk * a.D8;
     dim3 grid((unsigned)nblocks);
+    if (a.part) {
+        if (total_units <= 512) hipLaunchKernelGGL((quant_own_mean_kernel<DT, 2, 256>), grid, dim3(256), 0, stream, a);
+        else hipLaunchKernelGGL((quant_own_mean_kernel<DT, 4, 256>), grid, dim3(256), 0, stream, a);
+        return check_launch("quant_own_mean_kernel");
+    }
     if (total_units <= 256) hipLaunchKernelGGL((quant_per_block_int8_kernel<DT, 1, 256>), grid, dim3(256), 0, stream, a);
     else if (total_units <= 512) hipLaunchKernelGGL((quant_per_block_int8_kernel<DT, 2, 256>), grid, dim3(256), 0, stream, a);
     else if (total_units <= 1024) hipLaunchKernelGGL((quant_per_block_int8_kernel<DT, 4, 256>), grid, dim3(256), 0, stream, a);
@@ -483,6 +582,121 @@ __global__ __launch_bounds__(kStage1Threads) void smooth_stage1_kernel(QuantArgs
         k_mean_partial_item<DT, kMeanW>(ka, (int64_t)(i / period) * kStage1Threads + threadIdx.x);
     } else {
         quant_block<DT, UNITS, kStage1Threads>(qa, i - before, wave_max);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// K smoothing of short sequences in one launch: a workgroup holds all of one head's K in registers (K is read once), so mean,
+// difference and quantization need no other workgroup; the Q blocks share the grid.  The arithmetic is that of the
+// kernels above: 64-row chunks added row by row (from LDS, two channels per thread), chunk partials added in order.
+// Bound by latency (one burst of loads, four barriers).  GPU time with the Q blocks, three launches
+// before: B1 H2 N256 D64 fp16 9.5 -> 6.0 us, B2 H8 N250 D128 bf16 14.7 -> 7.9 us, B16 H32 N256 D128 34.9 -> 26.9 us.  With eight
+// units per thread (512 keys at head_dim 128) B16 H32 takes 61 us against 53 us for the separate launches: not used.
+// UNITS groups of eight elements per thread: kv_len rounded up to 64 rows times head_dim / 8 <= UNITS * THREADS.
+// ---------------------------------------------------------------------------------------------
+constexpr int kHeadPass = 4;  // units per thread that are in LDS at a time
+template <int DT, int THREADS, int UNITS>
+__global__ __launch_bounds__(THREADS) void smooth_head_kernel(QuantArgs kq, QuantArgs qq, void* km_out, int nheads) {
+    constexpr int kMaxBlocksTimesD8 = UNITS * THREADS / 64;  // 64-row blocks x D8
+    __shared__ __attribute__((aligned(16))) uint4 rows[kHeadPass * THREADS];
+    __shared__ float part[UNITS * THREADS / 8];              // [chunk][D]
+    __shared__ float km[128];
+    __shared__ float amax_s[kMaxBlocksTimesD8], scale_s[kMaxBlocksTimesD8], rcp_s[kMaxBlocksTimesD8];
+    if ((int)blockIdx.x >= nheads) {  // a Q block
+        const int bid = blockIdx.x - nheads;
+        if (qq.blk * qq.D8 == 2048) quant_block<DT, (2048 + THREADS - 1) / THREADS, THREADS>(qq, bid, amax_s);
+        else quant_block<DT, (1024 + THREADS - 1) / THREADS, THREADS>(qq, bid, amax_s);
+        return;
+    }
+    const int tid = threadIdx.x, h = blockIdx.x % kq.H, b = blockIdx.x / kq.H;
+    const int D8 = kq.D8, D = 8 * D8, N = kq.L, nblk = kq.nblk;
+    const int row0 = tid >> kq.d8_shift, c8 = tid & (D8 - 1), rpp = THREADS >> kq.d8_shift;  // unit j: row row0 + j * rpp
+    const uint16_t* src = static_cast<const uint16_t*>(kq.x) + (int64_t)b * kq.xs_b + (int64_t)h * kq.xs_h + 8 * c8;
+    uint4 raw[UNITS];
+#pragma unroll
+    for (int j = 0; j < UNITS; j++) raw[j] = *reinterpret_cast<const uint4*>(src + (int64_t)min(row0 + j * rpp, N - 1) * kq.xs_n);
+    // ---- chunk partials
+#pragma unroll
+    for (int pass = 0; pass < UNITS / kHeadPass; pass++) {
+        if (pass > 0) __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kHeadPass; j++) rows[THREADS * j + tid] = raw[kHeadPass * pass + j];  // [row][channel group]
+        __syncthreads();
+        const int first_row = kHeadPass * pass * rpp, chunks = kHeadPass * rpp / 64;
+        const uint32_t* words = reinterpret_cast<const uint32_t*>(rows);
+        for (int item = tid; item < chunks * (D / 2); item += THREADS) {
+            const int cp = item & (D / 2 - 1), chunk = item >> (kq.d8_shift + 2);
+            const int n = min(64, N - (first_row + 64 * chunk));
+            float s0 = 0.0f, s1 = 0.0f;
+            const uint32_t* p = words + (64 * chunk) * (D / 2) + cp;
+            auto add = [&](uint32_t w) {
+                if (DT == SAGE_BF16) {
+                    s0 = s0 + __builtin_bit_cast(float, w << 16);
+                    s1 = s1 + __builtin_bit_cast(float, w & 0xffff0000u);
+                } else {
+                    s0 = s0 + (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xffffu));
+                    s1 = s1 + (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
+                }
+            };
+            int r = 0;
+            for (; r + 16 <= n; r += 16) {
+                uint32_t w[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) w[i] = p[(r + i) * (D / 2)];
+#pragma unroll
+                for (int i = 0; i < 16; i++) add(w[i]);
+            }
+            for (; r < n; r++) add(p[r * (D / 2)]);
+            float* dst = part + (first_row / 64 + chunk) * D + 2 * cp;
+            dst[0] = s0;
+            dst[1] = s1;
+        }
+    }
+    __syncthreads();
+    mean_from_partials(part, nblk, D, N, DT, km, km_out, ((int64_t)b * kq.H + h) * D);
+    __syncthreads();
+    // ---- |k - km| per 64-row block: a wave's rows of one unit lie in one block, D8 waves per block and unit
+    float m[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) m[e] = km[8 * c8 + e];
+    auto diff8 = [&](int j, float (&v)[8]) {
+        unpack8(raw[j], DT, v);
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = round_to(v[e] - m[e], DT);
+    };
+#pragma unroll
+    for (int j = 0; j < UNITS; j++) {
+        float v[8], amax = 0.0f;
+        diff8(j, v);
+#pragma unroll
+        for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
+        if (row0 + j * rpp >= N) amax = 0.0f;
+        amax = wave_max_nonneg(amax);
+        // 64 / D8 rows per wave and unit: block * D8 + wave of the block == first row / (64 / D8)
+        if ((tid & 63) == 0) amax_s[(row0 + j * rpp) >> (6 - kq.d8_shift)] = amax;
+    }
+    __syncthreads();
+    for (int blk = tid; blk < nblk; blk += THREADS) {
+        float amax = 0.0f;
+        for (int w = 0; w < D8; w++) amax = fmaxf(amax, amax_s[blk * D8 + w]);
+        const float scale = amax / 127.0f;
+        kq.scale[((int64_t)b * kq.H + h) * nblk + blk] = scale;
+        scale_s[blk] = scale;
+        rcp_s[blk] = 1.0f / scale;
+    }
+    __syncthreads();
+    int8_t* out = kq.out + (int64_t)b * kq.os_b + (int64_t)h * kq.os_h + 8 * c8;
+#pragma unroll
+    for (int j = 0; j < UNITS; j++) {
+        const int row = row0 + j * rpp;
+        if (row >= N) continue;
+        float v[8];
+        diff8(j, v);
+        const float scale = scale_s[row >> 6];
+        const uint32_t sbits = __builtin_bit_cast(uint32_t, scale);
+        const bool fast_div = scale >= 0x1p-60f && scale <= 0x1p60f && (sbits & 0x7fffffu) != 0x7fffffu;
+        const uint2 packed = scale > 0.0f ? quantize8(v, scale, rcp_s[row >> 6], fast_div) : make_uint2(0u, 0u);
+        *reinterpret_cast<uint2*>(out + (int64_t)row * kq.os_n) = packed;
     }
 }
 
@@ -626,6 +840,23 @@ int launch_stage1(const QuantArgs& qa, const KMeanArgs& ka, int64_t q_blocks, hi
     return check_launch("smooth_stage1_kernel");
 }
 
+// One launch for a K that fits the registers of a workgroup per head (and the Q blocks, unless they need the mean first).
+template <int DT>
+int launch_head(const QuantArgs& kq, const QuantArgs* qq, void* km_out, int64_t heads, int64_t q_blocks, hipStream_t stream) {
+    const int64_t units = (int64_t)kq.nblk * 64 * kq.D8;
+    const QuantArgs q = qq ? *qq : QuantArgs{};
+    dim3 grid((unsigned)(heads + q_blocks));
+    if (units <= 1024) hipLaunchKernelGGL((smooth_head_kernel<DT, 256, 4>), grid, dim3(256), 0, stream, kq, q, km_out, (int)heads);
+    else if (units <= 2048) hipLaunchKernelGGL((smooth_head_kernel<DT, 512, 4>), grid, dim3(512), 0, stream, kq, q, km_out, (int)heads);
+    else hipLaunchKernelGGL((smooth_head_kernel<DT, 1024, 4>), grid, dim3(1024), 0, stream, kq, q, km_out, (int)heads);
+    return check_launch("smooth_head_kernel");
+}
+
+// Is a head's K small enough for smooth_head_kernel?  (256 keys at head_dim 128, 512 at 64.)
+bool head_fits(const QuantArgs& kq, int in_dtype) {
+    return in_dtype != SAGE_F32 && kq.blk == 64 && kq.d8_shift >= 0 && kq.D8 <= 16 && (int64_t)kq.nblk * 64 * kq.D8 <= 4096;
+}
+
 int launch_k_mean_partial(const KMeanArgs& a, int k_dtype, hipStream_t stream) {
     const int64_t g1 = (a.total_items + kThreads - 1) / kThreads;
     dim3 block(kThreads);
@@ -640,6 +871,13 @@ int launch_k_mean_partial(const KMeanArgs& a, int k_dtype, hipStream_t stream) {
 }  // namespace
 
 int launch_quant(const sage_quant_params& p, hipStream_t stream) {
+    if (p.k.ptr && p.kv_len > 0 && p.q.ptr && p.qo_len > 0) {
+        QuantArgs kq, qq;
+        if (int rc = k_args(p, true, kq)) return rc;
+        if (int rc = q_args(p, qq)) return rc;
+        const int64_t k_blocks = p.batch * p.heads_kv * kq.nblk, q_blocks = p.batch * p.heads_q * qq.nblk;
+        if (both_fit(kq, qq, k_blocks, q_blocks)) return launch_both(kq, qq, p.in_dtype, k_blocks, q_blocks, stream);
+    }
     // K first: a caller that has just taken the K mean finds K still in the memory-side cache.
     if (p.k.ptr && p.kv_len > 0) {
         QuantArgs a;
@@ -662,9 +900,15 @@ int launch_kmean(const sage_tensor& k, int k_dtype, void* km_out, int out_dtype,
     return launch_k_mean_final(a, B * H * D, stream);
 }
 
-// K mean -> k - km -> quantization of K, and quantization of Q, in three launches:
+// Sequences of up to this many 64-row chunks, in calls of up to this many K blocks, have the partials of the K mean added by
+// every K block instead of by a launch of its own: GPU time B1 H32 N1024 D128 16.6 -> 14.0 us, B8 H16 N1024 D64 23.2 -> 20.4
+// us; longer ones (B2 H32 N2048 33.3 -> 32.8 us) and larger calls (B16 H32 N512, 4096 blocks: 53.2 -> 54.7 us) gain nothing.
+constexpr int kOwnMeanChunks = 16, kOwnMeanBlocks = 2048;
+
+// K mean -> k - km -> quantization of K, and quantization of Q.  Short sequences: smooth_head_kernel, one launch.  Others:
 //   1. Q blocks and the chunk partials of the K mean, side by side in one grid;
-//   2. the mean per channel (chunk partials added in order, one division, one rounding to K's dtype);
+//   2. the mean per channel (chunk partials added in order, one division, one rounding to K's dtype), up to kOwnMeanChunks
+//      chunks inside 3;
 //   3. K blocks, subtracting the mean just written.
 // With q_dot_km the Q blocks need the mean as well and move behind it: partials, mean, K blocks, Q blocks.
 int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_km, void* workspace, hipStream_t stream) {
@@ -682,20 +926,35 @@ int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_k
     }
     const int64_t q_blocks = have_q ? p.batch * p.heads_q * qq.nblk : 0;
     bool fused = false;
-    if (have_q && !q_dot_km) {
-        int rc;
-        switch (p.in_dtype) {
-            case SAGE_F16: rc = launch_stage1<SAGE_F16>(qq, ka, q_blocks, stream, fused); break;
-            case SAGE_BF16: rc = launch_stage1<SAGE_BF16>(qq, ka, q_blocks, stream, fused); break;
-            default: rc = launch_stage1<SAGE_F32>(qq, ka, q_blocks, stream, fused); break;
-        }
+    if (head_fits(kq, p.in_dtype)) {
+        const int q_units = have_q ? qq.blk * qq.D8 : 0;
+        fused = have_q && !q_dot_km && (q_units == 1024 || q_units == 2048);
+        if (B * H + (fused ? q_blocks : 0) > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_per_block_int8_smooth_k: too many blocks");
+        kq.km = nullptr;
+        const int rc = p.in_dtype == SAGE_F16 ? launch_head<SAGE_F16>(kq, fused ? &qq : nullptr, km_out, B * H, fused ? q_blocks : 0, stream)
+                                              : launch_head<SAGE_BF16>(kq, fused ? &qq : nullptr, km_out, B * H, fused ? q_blocks : 0, stream);
         if (rc) return rc;
+    } else {
+        if (have_q && !q_dot_km) {
+            int rc;
+            switch (p.in_dtype) {
+                case SAGE_F16: rc = launch_stage1<SAGE_F16>(qq, ka, q_blocks, stream, fused); break;
+                case SAGE_BF16: rc = launch_stage1<SAGE_BF16>(qq, ka, q_blocks, stream, fused); break;
+                default: rc = launch_stage1<SAGE_F32>(qq, ka, q_blocks, stream, fused); break;
+            }
+            if (rc) return rc;
+        }
+        if (!fused) {
+            if (int rc = launch_k_mean_partial(ka, p.in_dtype, stream)) return rc;
+        }
+        if (kq.blk == 64 && kq.d8_shift >= 0 && D <= kMaxFusedMeanDim && kq.blk * kq.D8 <= 1024 && kq.nblk <= kOwnMeanChunks &&
+            B * H * kq.nblk <= kOwnMeanBlocks) {
+            kq.km = nullptr; kq.part = ka.part; kq.km_write = km_out;  // every block adds the chunk partials itself
+        } else {
+            if (int rc = launch_k_mean_final(ka, B * H * D, stream)) return rc;
+        }
+        if (int rc = launch_tensor(kq, p.in_dtype, B * H * kq.nblk, stream)) return rc;
     }
-    if (!fused) {
-        if (int rc = launch_k_mean_partial(ka, p.in_dtype, stream)) return rc;
-    }
-    if (int rc = launch_k_mean_final(ka, B * H * D, stream)) return rc;
-    if (int rc = launch_tensor(kq, p.in_dtype, B * H * kq.nblk, stream)) return rc;
     if (have_q && !fused) {
         if (q_dot_km) {
             qq.km = km_out; qq.ks_b = H * D; qq.ks_h = D; qq.ks_n = 0; qq.km_dt = p.in_dtype; qq.diff_dt = p.in_dtype;

@@ -1,0 +1,61 @@
+"""The quantizer's fused launches at their edges, bit for bit against the oracle: one workgroup per head (up to 256 keys at
+head_dim 128, 512 at 64), K blocks that add the chunk partials of the mean themselves (up to 16 chunks), K and Q blocks in one
+grid, and the sizes just beyond each."""
+import pytest
+import torch
+
+from oracle import c_oracle as C
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(got, want):
+    for g, w, name in zip(got, want, ("q_int8", "q_scale", "k_int8", "k_scale")):
+        g = g.cpu()
+        assert g.shape == w.shape and g.dtype == w.dtype
+        assert torch.equal(g.view(torch.int32) if g.dtype == torch.float32 else g, w.view(torch.int32) if w.dtype == torch.float32 else w), name
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d,n", [(64, 1), (64, 63), (64, 64), (64, 65), (64, 128), (64, 129), (64, 256), (64, 300), (64, 512), (64, 513),
+                                 (128, 1), (128, 64), (128, 65), (128, 128), (128, 191), (128, 256), (128, 257), (128, 1024),
+                                 (128, 1025), (32, 700), (32, 1100), (16, 90), (256, 200)])
+def test_smoothing_launch_forms(d, n, dtype, gpu_device):
+    from flag_attn import sage_attention as sa
+    from flagattention_amd.sage_attention.quant import per_block_int8_smooth_k
+
+    g = torch.Generator().manual_seed(n + d)
+    b, hq, hkv, m = 2, 4, 2, max(1, n - 37)
+    for layout in ("HND", "NHD"):
+        q = torch.randn(b, hq, m, d, generator=g).to(dtype)
+        k = (torch.randn(b, hkv, n, d, generator=g) + 3.0 * torch.randn(1, hkv, 1, d, generator=g)).to(dtype)
+        k[0, 0, : min(n, 64)] = 0  # a block of zeros (before the mean is taken off)
+        if layout == "NHD":
+            q, k = q.transpose(1, 2).contiguous(), k.transpose(1, 2).contiguous()
+        km = C.k_mean_fixed_order(k, layout)
+        want = C.per_block_int8(q, k, km=km, tensor_layout=layout)
+        dq, dk = q.to(gpu_device), k.to(gpu_device)
+        _check(sa.per_block_int8(dq, dk, tensor_layout=layout, smooth_k=True), want)
+        *got, km_got, dot = per_block_int8_smooth_k(dq, dk, tensor_layout=layout, with_q_dot_km=True)
+        _check(got, want)
+        assert torch.equal(km_got.cpu().view(torch.int16), km.view(torch.int16))
+        assert torch.equal(sa.k_mean(dk, layout).cpu().view(torch.int16), km.view(torch.int16))
+        qh, kmh = (q, km) if layout == "HND" else (q.transpose(1, 2), km.transpose(1, 2))
+        ref = (qh.double() * kmh.double().repeat_interleave(hq // hkv, dim=1)).sum(-1)
+        # fp32 sums of d products: each addition rounds once, d roundings of the running sum's magnitude
+        bound = d * 2.0 ** -24 * (qh.double().abs() * kmh.double().abs().repeat_interleave(hq // hkv, dim=1)).sum(-1)
+        assert bool(((dot.cpu().double() - ref).abs() <= bound + 1e-12).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("b,hq,hkv,m,n,d", [(1, 2, 2, 1, 1, 64), (2, 4, 2, 200, 77, 128), (1, 3, 1, 129, 1000, 64),
+                                            (4, 32, 8, 2048, 4032, 64), (4, 32, 8, 2048, 4160, 64), (1, 2, 1, 90, 130, 256)])
+def test_k_and_q_in_one_grid(b, hq, hkv, m, n, d, dtype, gpu_device):
+    from flag_attn import sage_attention as sa
+
+    g = torch.Generator().manual_seed(3)
+    q, k = torch.randn(b, hq, m, d, generator=g).to(dtype), torch.randn(b, hkv, n, d, generator=g).to(dtype)
+    km = k.float().mean(2, keepdim=True).to(dtype)
+    for mean in (None, km):
+        got = sa.per_block_int8(q.to(gpu_device), k.to(gpu_device), km=None if mean is None else mean.to(gpu_device))
+        _check(got, C.per_block_int8(q, k, km=mean))
