@@ -144,6 +144,23 @@ def load():
     return lib
 
 
+_host_module = None
+
+
+def host():
+    """The native host side of calls whose shape has been seen before (csrc/host.cpp), or raises: it is built with the
+    library."""
+    global _host_module
+    if _host_module is None:
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise ImportError("flagattention_amd/_host.so is missing or does not load: build it with "
+                              f"`make -C flagattention_amd/csrc` ({e})") from e
+        _host_module = module
+    return _host_module
+
+
 def check(status: int, what: str):
     if status != 0:
         msg = load().sage_hip_last_error().decode("utf-8", "replace")

@@ -69,6 +69,15 @@ def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
     ``[B, H, N]`` (the attention every key receives, summed over the queries) in fp32, ``seed`` / ``offset`` of the
     dropout mask (``return_seed_offset`` with ``dropout_p > 0``); None where not asked for.
     """
+    need_L = bool(return_log_normalizer or return_total_attention)
+    call = None
+    if dropout_p == 0 and not return_total_attention:
+        call = (q, k, v, causal, sm_scale, need_L)
+        out = (_lib._host_module or _lib.host()).flash(*call)  # a call shape seen before: (o, log normalizer), or a status
+        if out is not None:
+            if type(out) is int:
+                _lib.check(out, "sage_flash_attn_fwd")
+            return (out[0], out[1], None, None, None) if return_log_normalizer or return_seed_offset else out[0]
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise ValueError("q, k, v must be (batch, heads, sequence, head_dim) tensors")
     Dq, Dk, Dv = q.shape[-1], k.shape[-1], v.shape[-1]
@@ -107,8 +116,7 @@ def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
         k, v = k.contiguous(), v.contiguous()  # (the same holds for the key tiles of the dropout kernel)
     o = torch.empty_like(q)  # (the reference allocates the same way, flash.py:84-90)
     if not rows_aligned(o):
-        o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    need_L = return_log_normalizer or return_total_attention
+        o, call = torch.empty(q.shape, dtype=q.dtype, device=q.device), None
     L = torch.empty((B, H, M), dtype=torch.float32, device=q.device) if need_L else None
 
     p = _lib.FlashParams()
@@ -123,6 +131,8 @@ def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
     with torch.cuda.device(q.device):
         # (the reference decides on its split over the keys at the same point, flash.py:73-75)
         ws_bytes = 0 if is_dropout else lib.sage_flash_attn_fwd_workspace_bytes(p)
+        if call is not None and ws_bytes >= 0 and q is call[0] and k is call[1] and v is call[2]:  # (nothing was copied)
+            _lib.host().put_flash(*call, bytes(p), ws_bytes)
         if is_dropout:
             seed, offset = philox_seed_offset(B * H * M * N, q.device)  # (flash.py:67-69)
             _lib.check(lib.sage_flash_attn_fwd_dropout(p, float(dropout_p), seed & (2 ** 64 - 1), offset,

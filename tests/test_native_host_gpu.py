@@ -1,0 +1,91 @@
+"""Calls whose shape has been seen before take the native host side (csrc/host.cpp): the same results as the first call of
+that shape, bit for bit, and everything its key does not cover goes back to the Python checks."""
+import threading
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _qkv(seed, dev, b=1, h=4, hkv=2, m=77, n=130, d=64, dtype=torch.float16):
+    g = torch.Generator().manual_seed(seed)
+    return tuple(torch.randn(b, x, s, d, generator=g).to(dtype).to(dev) for x, s in ((h, m), (hkv, n), (hkv, n)))
+
+
+def _calls(sa, flag_attn, q, k, v, mask):
+    q8, qs, k8, ks = sa.per_block_int8(q, k, smooth_k=True)
+    plain = sa.per_block_int8(q, k)
+    km = sa.per_block_int8(q, k, km=k.mean(dim=2, keepdim=True))
+    out = [q8, qs, k8, ks, *plain, *km]
+    for kw in ({}, {"return_lse": True, "output_dtype": torch.float32}, {"attn_mask": mask}, {"causal": True}):
+        out += list(sa.sage_attention(q8, k8, v, qs, ks, **kw))
+    out += [flag_attn.flash_attention(q, k, v), *flag_attn.flash_attention(q, k, v, True, return_log_normalizer=True)[:2]]
+    out += list(sa.sageattn(q, k, v, return_lse=True))
+    return out
+
+
+def test_repeated_shapes_give_the_first_call_s_results(gpu_device):
+    import flag_attn
+    from flag_attn import sage_attention as sa
+    from flagattention_amd import _lib
+
+    mask = torch.rand(1, 1, 77, 128, generator=torch.Generator().manual_seed(1)).to(gpu_device) > 0.3
+    a, b = _qkv(1, gpu_device, n=128), _qkv(2, gpu_device, n=128)
+    first_a = [t.clone() for t in _calls(sa, flag_attn, *a, mask)]
+    assert _lib.host().flash(*a, False, None, False) is not None  # (the shape is known now)
+    second_b = [t.clone() for t in _calls(sa, flag_attn, *b, mask)]
+    again_a = _calls(sa, flag_attn, *a, mask)
+    assert all(x.shape == y.shape and x.stride() == y.stride() and torch.equal(x, y) for x, y in zip(first_a, again_a))
+    # other inputs of the same shape, in threads of their own (each with a plan table of its own) and on their own streams
+    results = {}
+
+    def work(name, args):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            for _ in range(3):
+                results[name] = _calls(sa, flag_attn, *args, mask)
+        s.synchronize()
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(name, args)) for name, args in (("a", a), ("b", b))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert all(torch.equal(x, y) for x, y in zip(results["a"], first_a)) and all(torch.equal(x, y) for x, y in zip(results["b"], second_b))
+
+
+def test_what_the_key_does_not_cover_is_checked_again(gpu_device):
+    import flag_attn
+    from flag_attn import sage_attention as sa
+    from flagattention_amd import _lib
+
+    q, k, v = _qkv(3, gpu_device)
+    want = flag_attn.flash_attention(q, k, v)
+    host = _lib.host()
+    assert host.flash(q, k, v, False, None, False) is not None
+    with pytest.raises(NotImplementedError, match="forward only"):
+        flag_attn.flash_attention(q.clone().requires_grad_(), k, v)
+    # the same shape and strides, but rows that are not 16-byte aligned: the library refuses them, as on a first call
+    shifted = torch.empty(q.numel() + 8, dtype=q.dtype, device=gpu_device)[1:1 + q.numel()].view(q.shape).copy_(q)
+    assert shifted.stride() == q.stride() and host.flash(shifted, k, v, False, None, False) is None
+    with pytest.raises(_lib.SageHipError, match="aligned"):
+        flag_attn.flash_attention(shifted, k, v)
+    assert torch.equal(flag_attn.flash_attention(q, k, v), want)
+    assert host.flash(q, k[:, :, :100], v[:, :, :100], False, None, False) is None
+    assert host.flash(q.cpu(), k, v, False, None, False) is None
+    with pytest.raises(RuntimeError):
+        flag_attn.flash_attention(q.cpu(), k, v)
+    q8, qs, k8, ks = sa.per_block_int8(q, k)
+    o, _ = sa.sage_attention(q8, k8, v, qs, ks)
+    with pytest.raises(ValueError, match="q_scale"):
+        sa.sage_attention(q8, k8, v, qs[..., :0], ks)
+    with pytest.raises(ValueError, match="maxnreg"):
+        sa.sage_attention(q8, k8, v, qs, ks, maxnreg=0)
+    with pytest.raises(ValueError, match="layout"):
+        sa.sage_attention(q8, k8, v, qs, ks, "HDN")
+    # a mask of a known shape whose contents change, and one of the same shape that has to be staged first
+    mask = torch.ones(1, 1, 77, 144, dtype=torch.bool, device=gpu_device)[..., :130]
+    for _ in range(2):
+        assert torch.equal(sa.sage_attention(q8, k8, v, qs, ks, attn_mask=mask)[0], sa.sage_attention(q8, k8, v, qs, ks, attn_mask=mask.clone())[0])
