@@ -61,9 +61,61 @@ struct AttnArgs {
     // out + s * out_split_stride / lse + s * lse_split_stride, which a second kernel combines.  Unsplit: 1, nk, 0, 0.
     int32_t nsplit, split_steps;
     int64_t out_split_stride, lse_split_stride;
+    int32_t longest_first;  // (causal, pipelined kernel) a workgroup per q-block, those with the most steps first over all heads; 0: pairs
+    // Cut of the whole launch into cut_wgs equal shares of its steps (0: a workgroup per q-block, or pair of them): see
+    // CutLine.  Items cut in two or more leave normalized fp32 outputs in part_o and base-2 log-sum-exps in part_lse.
+    int32_t cut_wgs, cut_total;  // workgroups; steps of the whole launch
+    float* part_o;     // [2 * cut_wgs slots][256 rows x D, in the order of the accumulator registers]
+    float* part_lse;   // [2 * cut_wgs][256]
     float lse_mul;     // factor on the base-2 log-sum-exp on its way out (1: as is; ln 2: natural log)
     float qk_scale;    // 16-bit Q and K only: sm_scale * log2(e), the one scale of every score (q/k point at 16-bit data)
 };
+
+// The steps of a launch as one line, which is cut into equal shares: head after head, within a head its items
+// (q-blocks of 256 rows), within an item its 64-key steps.  Under the causal flag the items of a head lie in pairs of a
+// long and a short one (nq - 1 - j, then j), whose lengths add up to the same: where a share is a pair's length over a
+// whole number, every pair ends at a cut.  `dead` leading items see no key (qo_len > kv_len): one step each (all of it
+// hidden), at the end of the head.
+struct CutLine {
+    int nq, nk, dead, c, first_pair, pair, head;  // live item i (counted from `dead`): 4 (i + 1) + c steps, the last one nk
+    bool causal;
+    __host__ __device__ CutLine(int M, int N, bool causal_) : nq((M + kFastRows - 1) / kFastRows), nk((N + BN - 1) / BN), causal(causal_) {
+        dead = 0; c = 0; first_pair = nk; pair = nk; head = nq * nk;
+        if (!causal) return;
+        const int shift = N - M;
+        c = shift >= 0 ? (shift + BN - 1) / BN : -((-shift) / BN);  // floor((shift + 63) / 64)
+        dead = c < 0 ? (-c) / 4 : 0;
+        if (dead >= nq) dead = nq - 1;
+        c += 4 * dead;
+        const int live = nq - dead;
+        first_pair = nk + (live > 1 ? 4 + c : 0);
+        pair = 4 * (live + 1) + 2 * c;
+        const int pairs = live / 2;  // whole ones; an odd count leaves the middle item alone
+        head = (pairs > 0 ? first_pair + (pairs - 1) * pair : 0) + (live & 1 ? len(dead + live / 2) : 0) + dead;
+    }
+    __host__ __device__ int len(int iq) const {  // steps of item iq
+        if (!causal) return nk;
+        return iq < dead ? 1 : iq == nq - 1 ? nk : 4 * (iq - dead + 1) + c;
+    }
+    __host__ __device__ int start(int iq) const {  // of item iq, within its head
+        if (!causal) return iq * nk;
+        if (iq < dead) return head - dead + iq;
+        const int live = nq - dead, i = iq - dead, mirror = live - 1 - i, p = i < mirror ? i : mirror;
+        return (p == 0 ? 0 : first_pair + (p - 1) * pair) + (i < mirror ? len(dead + mirror) : 0);
+    }
+    __host__ __device__ int item(int r) const {  // the item that holds position r of a head
+        if (!causal) return r / nk;
+        if (r >= head - dead) return r - (head - dead);
+        const int live = nq - dead, p = r < first_pair ? 0 : 1 + (r - first_pair) / pair;
+        const int longer = nq - 1 - p;
+        return r - (p == 0 ? 0 : first_pair + (p - 1) * pair) < len(longer) || 2 * p == live - 1 ? longer : dead + p;
+    }
+};
+// first step of share w of W (total steps < 2^23, W <= 256), and the share that holds step pos
+__host__ __device__ inline int cut_begin(int w, int W, int total) { return (int)((unsigned)w * (unsigned)total / (unsigned)W); }
+__host__ __device__ inline int cut_owner(int pos, int W, int total) {
+    return (int)((((unsigned)pos + 1u) * (unsigned)W - 1u) / (unsigned)total);
+}
 
 template <typename VT> struct PV;
 template <> struct PV<__bf16> {
@@ -103,12 +155,17 @@ template <> struct PV<_Float16> {
 // head_dim 64 / 128, V dtype fp16 / bf16.
 int launch_fast(const AttnArgs& a, int head_dim, int v_dtype, bool causal, hipStream_t stream);
 
-// Key split for launches that would leave most compute units idle (split_combine.hip).  plan_key_split: how many
-// workgroups share the keys of one (batch, head, q-block), 1 when the launch fills the chip anyway.
-// apply_key_split turns the arguments of the unsplit launch into those of the split one (partial results in
-// `workspace`, key_split_workspace_bytes large); launch_split_combine writes what the unsplit launch would have.
-int plan_key_split(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal);
-int64_t key_split_workspace_bytes(int nsplit, int64_t batch, int64_t heads_q, int64_t qo_len, int64_t head_dim);
+// How a launch is laid out (split_combine.hip).  Whole: a workgroup per item (256 queries of a head), or under the causal
+// flag per pair of a short and a long one; longest_first: per item under the causal flag too, the longest first.  With a
+// workspace, where that leaves compute units idle: nsplit > 1 workgroups share the keys of each item (pair), or cut_wgs > 0
+// workgroups take equal shares of all steps of the launch.  apply_* turn the arguments of the whole launch into those of
+// the other (partial results in `workspace`, plan_workspace_bytes large); launch_*_combine then write what the whole launch would have.
+struct LaunchPlan { int nsplit, cut_wgs; bool longest_first; };
+LaunchPlan plan_launch(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal,
+                       bool with_workspace);
+int64_t plan_workspace_bytes(const LaunchPlan& plan, int64_t batch, int64_t heads_q, int64_t qo_len, int64_t head_dim);
+void apply_cut(AttnArgs& a, int cut_wgs, int64_t batch, int head_dim, void* workspace);
+int launch_cut_combine(const AttnArgs& a, int head_dim, hipStream_t stream);
 void apply_key_split(AttnArgs& a, int nsplit, int64_t batch, int head_dim, void* workspace);
 int launch_split_combine(const AttnArgs& split, const AttnArgs& whole, int head_dim, int64_t batch, hipStream_t stream);
 

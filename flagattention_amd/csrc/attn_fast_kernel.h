@@ -30,7 +30,8 @@
 //   sums are needed anyway, so the common step pays nothing for the check but a compare.
 // * 16-bit outputs are transposed through LDS and written as whole rows.
 // * Under the causal flag a workgroup takes two q-blocks of its head (the longest remaining and the
-//   shortest), so that all workgroups of a launch run the same number of steps.
+//   shortest), so that all workgroups of a launch run the same number of steps; launches that leave
+//   compute units idle that way take one q-block each, longest first, or are cut into equal shares (CUT).
 #pragma once
 #include "attn_common.h"
 
@@ -133,8 +134,12 @@ template <> __device__ __forceinline__ float mask_entry<_Float16>(unsigned word,
     return (float)__builtin_bit_cast(_Float16, (unsigned short)(hi ? (word >> 16) : (word & 0xffffu)));
 }
 
-template <int D, typename VT, bool CAUSAL, int QB, typename MT = void>
-__global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast_kernel(AttnArgs a, int nq2) {
+// CUT: a workgroup takes share blockIdx of the launch's steps (CutLine) instead of whole q-blocks: the end of one item,
+// whole ones, the beginning of another.  Without a mask tensor.  The step loop is that of the whole launch (B2 H32/8 N4096
+// causal, where no item is cut: 214 us against 210 us for pairs); a piece costs about five steps, a partial result 2.5.
+template <int D, typename VT, bool CAUSAL, int QB, typename MT = void, bool CUT = false>
+__global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast_kernel(AttnArgs args, int nq2) {
+    const AttnArgs& a = args;
     using F = FT<D, QB>;
     constexpr bool INT8 = QB == 1;
     constexpr bool MASK = MaskT<MT>::ON;         // a mask tensor is staged
@@ -161,25 +166,56 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     // (1.35x the K/V bytes from memory at 8192 keys).
     int wg = blockIdx.x;
     if ((a.total_wg & 7) == 0) wg = (wg & 7) * (a.total_wg >> 3) + (wg >> 3);
-    const bool paired = CAUSAL && a.causal;
+    const bool paired = CAUSAL && !CUT && a.causal && !a.longest_first;
     const int per_head = paired ? (nq2 + 1) / 2 : nq2;  // workgroups per (batch, head)
     // The keys of one (batch, head, q-block) may be split over `nsplit` workgroups (never under a mask tensor).  A
     // workgroup then sees the problem that starts at its first key: kv_len, the number of tiles and the causal
     // limits below all count from there, and its steps end where the next workgroup's begin.
-    const int nsplit = MASK ? 1 : a.nsplit;
+    const int nsplit = MASK || CUT ? 1 : a.nsplit;
     const int split = wg % nsplit;
-    wg /= nsplit;
-    const int step0 = split * a.split_steps;  // first step of this workgroup's share of the keys
-    const int kv_len = a.N - step0 * BN, nk = a.nk - step0;
+    const int item0 = wg / nsplit;
     // heads that alternate within a q-block: measured to pay only under a mask with the causal mask folded in
     // (-7 %; +1..3 % for other shared masks, whose launches keep a head's q-blocks together for its K/V)
     const int ht = MASK && a.mask_causal ? a.head_tile : 1;
-    const int jq = (wg / ht) % per_head;
-    const int h = (wg / (ht * per_head)) % (a.Hq / ht) * ht + wg % ht;
-    const int b = wg / (per_head * a.Hq);
+    int jq = (item0 / ht) % per_head;
+    int h0 = (item0 / (ht * per_head)) % (a.Hq / ht) * ht + item0 % ht;
+    int b0 = item0 / (per_head * a.Hq);
+    if (CAUSAL && !CUT && !MASK && a.longest_first) {  // the heads of an XCD take turns, q-block after q-block from the last one
+        const int heads = a.total_wg / nq2, xcds = heads & 7 ? 1 : 8;
+        const int i = blockIdx.x / xcds, own = heads / xcds, bh = blockIdx.x % xcds * own + i % own;
+        jq = nq2 - 1 - i / own;
+        h0 = bh % a.Hq;
+        b0 = bh / a.Hq;
+    }
+    int pos = 0, pos_end = 0;  // (CUT) this workgroup's steps on the line
+    if constexpr (CUT) {
+        pos = cut_begin(wg, a.cut_wgs, a.cut_total);
+        pos_end = cut_begin(wg + 1, a.cut_wgs, a.cut_total);
+    }
+  for (int pass = 0; CUT ? pos < pos_end : pass < 2; pass++) {
+    if (pass == 1 && !CUT && (!paired || nq2 - 1 - jq == jq)) break;  // one q-block only, or the middle one of an odd count
+    // (CUT: the arguments are read again from the kernel argument segment for each piece, behind an opaque pointer: kept
+    // across the pieces they cost scalar registers the step loop cannot spare, 40 spilled)
+    typedef __attribute__((address_space(4))) const void* const_ptr;
+    const_ptr args_again = (const_ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    if constexpr (CUT) asm volatile("" : "+s"(args_again));
+    const AttnArgs& a = CUT ? *(const AttnArgs*)args_again : args;
+    int b = b0, h = h0, step0 = split * a.split_steps, cut_steps = 0;  // step0: first step of this workgroup's share of the keys
+    int iq = (paired && pass == 1) || (MASK && a.mask_causal) ? nq2 - 1 - jq : jq;  // (a mask with the causal mask folded in: no pairs, the q-blocks with the most tiles are handed out first)
+    bool partial = false;  // (CUT) the item has steps in other workgroups too
+    if constexpr (CUT) {
+        const CutLine line(a.M, a.N, CAUSAL && a.causal);
+        const int head = pos / line.head, r = pos - head * line.head;
+        iq = line.item(r);
+        step0 = r - line.start(iq);
+        cut_steps = min(line.len(iq) - step0, pos_end - pos);
+        partial = cut_steps != line.len(iq);
+        h = head % a.Hq;
+        b = head / a.Hq;
+        pos += cut_steps;
+    }
     const int hk = h / a.groups;
-  for (int pass = 0; pass < 2; pass++) {
-    if (pass == 1 && (!paired || nq2 - 1 - jq == jq)) break;  // one q-block only, or the middle one of an odd count
+    const int kv_len = a.N - step0 * BN, nk = a.nk - step0;
     // Everything a pass needs is derived again from the thread index, made opaque here: values the compiler
     // would otherwise keep across the two passes cost registers the step loop cannot spare.
     int tid = threadIdx.x;
@@ -188,8 +224,6 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     const int lane = tid & 63;
     const int l32 = lane & 31;
     const int half = lane >> 5;
-    // (a mask with the causal mask folded in: no pairs, the q-blocks with the most tiles are handed out first)
-    const int iq = (paired && pass == 1) || (MASK && a.mask_causal) ? nq2 - 1 - jq : jq;
     const int m0 = iq * kFastRows;
     const int my_m = m0 + 32 * wave + l32;
     const bool row_ok = my_m < a.M;
@@ -200,8 +234,8 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     const int lim = !CAUSAL ? 0 : a.causal ? min(my_m + shift, kv_len - 1) : kv_len - 1;                  // this lane's row
     const int wlim = !CAUSAL ? 0 : a.causal ? min(m0 + 32 * wave + shift, kv_len - 1) : kv_len - 1;      // first row of the wave
 
-    int nsteps = min(a.split_steps, nk);
-    if (CAUSAL && (a.causal || (MASK && a.mask_causal))) {  // (a mask with the causal mask folded in: same bound)
+    int nsteps = CUT ? cut_steps : min(a.split_steps, nk);
+    if (CAUSAL && !CUT && (a.causal || (MASK && a.mask_causal))) {  // (a mask with the causal mask folded in: same bound)
         const int last_row = min(m0 + kFastRows, a.M) - 1;
         nsteps = max(min(nsteps, (last_row + shift + BN) / BN), 0);  // 0: no row of the workgroup sees a key (qo_len > kv_len)
     }
@@ -955,7 +989,20 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     const float l_tot = kWholeRowSums ? l_i : half ? (l_o + l_i) : (l_i + l_o);
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;  // l = 0: a row that saw no key; its output is 0, its lse -inf
     const int64_t obase_wave = (int64_t)b * a.os_b + (int64_t)h * a.os_h + (int64_t)(m0 + 32 * wave) * a.os_n + split * a.out_split_stride;
-    if (a.out_dt != SAGE_F32) {
+    bool to_part = false;
+    if constexpr (CUT) to_part = partial;
+    if (to_part) {
+        // slot 2 w: the item whose steps share w begins with; 2 w + 1: the one it ends with.  Registers as they lie,
+        // 1 KB per wave instruction.
+        const int64_t slot = 2 * wg + (pass > 0);
+        v4f* outp = reinterpret_cast<v4f*>(a.part_o) + (slot * kFastWaves + wave) * (8 * D) + lane;
+#pragma unroll
+        for (int dt = 0; dt < F::DTILES; dt++)
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+                outp[64 * (4 * dt + g)] = v4f{o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv};
+        if (half == 0) a.part_lse[slot * kFastRows + 32 * wave + l32] = __builtin_log2f(l_tot) + m_i;
+    } else if (a.out_dt != SAGE_F32) {
         // 16-bit outputs: a lane holds its row in 8-byte pieces, which stored directly would scatter 32
         // partial lines per instruction.  Each wave transposes its 32 rows through its own slice of LDS
         // and writes whole rows, 16 bytes per lane.
@@ -998,10 +1045,13 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                 *reinterpret_cast<v4f*>(outp + d) = v4f{o[dt][4 * g] * inv, o[dt][4 * g + 1] * inv, o[dt][4 * g + 2] * inv, o[dt][4 * g + 3] * inv};
             }
     }
-    if (row_ok) {
+    if (row_ok && !to_part) {
         if (a.lse && half == 0) a.lse[((int64_t)b * a.Hq + h) * a.M + my_m + split * a.lse_split_stride] = (__builtin_log2f(l_tot) + m_i) * a.lse_mul;
     }
-    __syncthreads();  // the output staging in LDS has been read: the next q-block may fill the tile buffers
+    // The output staging in LDS has been read: the next q-block may fill the tile buffers.  (Not __syncthreads, which
+    // would wait for the output to arrive in memory as well.)
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
   }
 }
 

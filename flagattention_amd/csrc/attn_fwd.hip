@@ -467,16 +467,10 @@ int launch_mode(const AttnArgs& a, int mode, hipStream_t stream) {
 
 }  // namespace
 
-namespace {
-// The calls the pipelined kernel serves without a mask tensor are the ones whose keys can be split.
-int attn_key_splits(const sage_attn_params& p) {
-    if (p.mask_kind != SAGE_MASK_NONE || (p.causal && p.qo_len > p.kv_len)) return 1;
-    return attn::plan_key_split(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0);
-}
-}  // namespace
-
 int64_t attn_split_workspace_bytes(const sage_attn_params& p) {
-    return attn::key_split_workspace_bytes(attn_key_splits(p), p.batch, p.heads_q, p.qo_len, p.head_dim);
+    if (p.mask_kind != SAGE_MASK_NONE || (p.causal && p.qo_len > p.kv_len)) return 0;  // (not a launch that can be split)
+    const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, true);
+    return attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim);
 }
 
 int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
@@ -531,15 +525,23 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
             return decode ? attn::launch_decode(x, p.batch, (int)p.head_dim, p.v_dtype, true, stream)
                           : attn::launch_fast(x, (int)p.head_dim, p.v_dtype, p.causal != 0, stream);
         };
-        const int nsplit = workspace ? attn_key_splits(p) : 1;
-        if (nsplit > 1 && workspace_bytes >= attn::key_split_workspace_bytes(nsplit, p.batch, p.heads_q, p.qo_len, p.head_dim)) {
-            if (total * nsplit > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_attn_fwd: problem too large for 32-bit tile indices");
-            AttnArgs s = a;
-            attn::apply_key_split(s, nsplit, p.batch, (int)p.head_dim, workspace);
+        attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, workspace != nullptr);
+        if (attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim) > workspace_bytes)  // (the whole launch then)
+            plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, false);
+        AttnArgs s = a;
+        if (plan.cut_wgs > 0) {
+            attn::apply_cut(s, plan.cut_wgs, p.batch, (int)p.head_dim, workspace);
+            if (int rc = launch(s)) return rc;
+            return attn::launch_cut_combine(s, (int)p.head_dim, stream);
+        }
+        if (plan.nsplit > 1) {
+            if (total * plan.nsplit > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_attn_fwd: problem too large for 32-bit tile indices");
+            attn::apply_key_split(s, plan.nsplit, p.batch, (int)p.head_dim, workspace);
             if (int rc = launch(s)) return rc;
             return attn::launch_split_combine(s, a, (int)p.head_dim, p.batch, stream);
         }
-        return launch(a);
+        s.longest_first = plan.longest_first;
+        return launch(s);
     }
     a.mask_additive = additive;
     if ((is_bool && attn::fast_serves_mask(a, 1)) || (additive && attn::fast_serves_mask(a, dtype_bytes(a.mask_dt))))

@@ -13,10 +13,15 @@ template <int D, typename VT>
 int launch_causal(const AttnArgs& a, bool causal, hipStream_t stream) {
     AttnArgs b = a;
     const int nq2 = (a.M + kFastRows - 1) / kFastRows;
-    const int per_head = a.causal ? (nq2 + 1) / 2 : nq2;  // under the causal flag a workgroup takes two q-blocks
+    const int per_head = a.causal && !a.longest_first ? (nq2 + 1) / 2 : nq2;  // under the causal flag a workgroup takes two q-blocks
     b.total_wg = (int)((int64_t)a.total_wg / a.nq * per_head) * a.nsplit;
     dim3 grid((unsigned)b.total_wg), block(kFastThreads);
-    if (causal) hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1>), grid, block, 0, stream, b, nq2);
+    if (a.cut_wgs) {
+        b.total_wg = a.cut_wgs;
+        grid.x = (unsigned)a.cut_wgs;
+        if (causal) hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1, void, true>), grid, block, 0, stream, b, nq2);
+        else hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, false, 1, void, true>), grid, block, 0, stream, b, nq2);
+    } else if (causal) hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1>), grid, block, 0, stream, b, nq2);
     else hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, false, 1>), grid, block, 0, stream, b, nq2);
     return check_launch("sage_attn_fwd_fast_kernel");
 }

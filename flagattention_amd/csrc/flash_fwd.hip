@@ -15,10 +15,15 @@ template <int D, typename VT>
 int launch_dense(const AttnArgs& a, bool hides_keys, hipStream_t stream) {
     const int nq2 = (a.M + kFastRows - 1) / kFastRows;
     AttnArgs b = a;
-    const int per_head = a.causal ? (nq2 + 1) / 2 : nq2;  // under the causal flag a workgroup takes two q-blocks
+    const int per_head = a.causal && !a.longest_first ? (nq2 + 1) / 2 : nq2;  // under the causal flag a workgroup takes two q-blocks
     b.total_wg = (int)((int64_t)a.total_wg / nq2 * per_head) * a.nsplit;
     dim3 grid((unsigned)b.total_wg), block(kFastThreads);
-    if (hides_keys) hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 2>), grid, block, 0, stream, b, nq2);
+    if (a.cut_wgs) {
+        b.total_wg = a.cut_wgs;
+        grid.x = (unsigned)a.cut_wgs;
+        if (hides_keys) hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 2, void, true>), grid, block, 0, stream, b, nq2);
+        else hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, false, 2, void, true>), grid, block, 0, stream, b, nq2);
+    } else if (hides_keys) hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 2>), grid, block, 0, stream, b, nq2);
     else hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, false, 2>), grid, block, 0, stream, b, nq2);
     return check_launch("sage_attn_fwd_fast_kernel (16-bit Q, K)");
 }
@@ -36,12 +41,9 @@ int launch_flash(const AttnArgs& a, int head_dim, int dtype, bool causal, hipStr
 
 }  // namespace attn
 
-static int flash_key_splits(const sage_flash_params& p) {
-    return attn::plan_key_split(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0);
-}
-
 int64_t flash_split_workspace_bytes(const sage_flash_params& p) {
-    return attn::key_split_workspace_bytes(flash_key_splits(p), p.batch, p.heads_q, p.qo_len, p.head_dim);
+    const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, true);
+    return attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim);
 }
 
 int launch_flash_attn(const sage_flash_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
@@ -72,15 +74,23 @@ int launch_flash_attn(const sage_flash_params& p, void* workspace, int64_t works
         return decode ? launch_decode(x, p.batch, (int)p.head_dim, p.dtype, false, stream)
                       : launch_flash(x, (int)p.head_dim, p.dtype, p.causal != 0, stream);
     };
-    const int nsplit = workspace ? flash_key_splits(p) : 1;
-    if (nsplit > 1 && workspace_bytes >= key_split_workspace_bytes(nsplit, p.batch, p.heads_q, p.qo_len, p.head_dim)) {
-        if (total * nsplit > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd: problem too large for 32-bit tile indices");
-        AttnArgs s = a;
-        apply_key_split(s, nsplit, p.batch, (int)p.head_dim, workspace);
+    LaunchPlan plan = plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, workspace != nullptr);
+    if (plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim) > workspace_bytes)  // (the whole launch then)
+        plan = plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, false);
+    AttnArgs s = a;
+    if (plan.cut_wgs > 0) {
+        apply_cut(s, plan.cut_wgs, p.batch, (int)p.head_dim, workspace);
+        if (int rc = launch(s)) return rc;
+        return launch_cut_combine(s, (int)p.head_dim, stream);
+    }
+    if (plan.nsplit > 1) {
+        if (total * plan.nsplit > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd: problem too large for 32-bit tile indices");
+        apply_key_split(s, plan.nsplit, p.batch, (int)p.head_dim, workspace);
         if (int rc = launch(s)) return rc;
         return launch_split_combine(s, a, (int)p.head_dim, p.batch, stream);
     }
-    return launch(a);
+    s.longest_first = plan.longest_first;
+    return launch(s);
 }
 
 }  // namespace sage

@@ -1,7 +1,8 @@
-// Key split of the pipelined attention kernel for gfx950: planning, and the kernel that combines the partial
-// results.  A launch with few (batch, head, q-block) items leaves most of the 256 compute units idle; the keys of
+// How launches of the pipelined attention kernel for gfx950 are laid out over the 256 compute units, and the kernels that
+// combine partial results.  Key split: a launch with few (batch, head, q-block) items leaves most CUs idle; the keys of
 // every item are then cut into `nsplit` runs of whole 64-key steps, one workgroup each, which write a normalized
-// fp32 partial output o_s and its base-2 log-sum-exp lse_s.  The combine kernel forms
+// fp32 partial output o_s and its base-2 log-sum-exp lse_s.  Cut launch: all steps of the launch form one line
+// (CutLine), of which every workgroup takes an equal share.  Either way the combine kernel forms
 //     lse = log2 sum_s 2^lse_s,      out = sum_s 2^(lse_s - lse) o_s
 // (FlagAttention src/flag_attn/flash.py:73-75, :106-141 is the dense forward's use of the same idea,
 // split_kv.py:250-278 its choice of the number of runs, :155-214 its combine kernel).
@@ -14,7 +15,8 @@ namespace {
 constexpr int kComputeUnits = 256;
 constexpr int kMaxSplits = 64;
 constexpr int kMinStepsPerSplit = 4;   // 256 keys: below that the prologue and epilogue of a workgroup dominate
-constexpr float kFixedSteps = 6.0f;    // what a workgroup spends outside its step loop, in steps
+constexpr int kFewItems = 16;          // up to here every piece of the work has a CU to itself: the longest run alone counts
+constexpr int kMinStepsPerShare = 8;   // of a cut launch: a share may hold two pieces
 
 struct CombineArgs {
     const float* part_o;    // [nsplit, rows, D]
@@ -28,6 +30,18 @@ struct CombineArgs {
 };
 
 constexpr int kCombineThreads = 256;
+
+__device__ __forceinline__ void store4(void* out, int out_dt, int64_t o, v4f r) {
+    if (out_dt == SAGE_BF16) {
+        typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<b4*>(static_cast<__bf16*>(out) + o) = b4{(__bf16)r[0], (__bf16)r[1], (__bf16)r[2], (__bf16)r[3]};
+    } else if (out_dt == SAGE_F16) {
+        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+        *reinterpret_cast<h4*>(static_cast<_Float16*>(out) + o) = h4{(_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3]};
+    } else {
+        *reinterpret_cast<v4f*>(static_cast<float*>(out) + o) = r;
+    }
+}
 
 // TPR threads per row, four channels each; SG groups of them share the runs of a row (group g takes runs g, g + SG, ...)
 // and meet through LDS.  SG = 1 where the rows alone fill the chip; with few rows (decoding) the runs of a row are read
@@ -81,22 +95,75 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineA
     }
     if (!ok) return;
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;
-    float r[4];
+    v4f r;
 #pragma unroll
     for (int i = 0; i < 4; i++) r[i] = acc[i] * inv;
     const int mi = (int)(row % a.M), h = (int)((row / a.M) % a.Hq);
     const int64_t b = row / ((int64_t)a.M * a.Hq);
     const int64_t o = b * a.os_b + (int64_t)h * a.os_h + (int64_t)mi * a.os_n + 4 * c;
-    if (a.out_dt == SAGE_BF16) {
-        typedef __bf16 b4 __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<b4*>(static_cast<__bf16*>(a.out) + o) = b4{(__bf16)r[0], (__bf16)r[1], (__bf16)r[2], (__bf16)r[3]};
-    } else if (a.out_dt == SAGE_F16) {
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<h4*>(static_cast<_Float16*>(a.out) + o) = h4{(_Float16)r[0], (_Float16)r[1], (_Float16)r[2], (_Float16)r[3]};
-    } else {
-        *reinterpret_cast<v4f*>(static_cast<float*>(a.out) + o) = v4f{r[0], r[1], r[2], r[3]};
-    }
+    store4(a.out, a.out_dt, o, r);
     if (a.lse && c == 0) a.lse[row] = (__builtin_log2f(den) + m) * a.lse_mul;  // den = 0: log2(0) + (-inf) = -inf
+}
+
+// One wave tile (32 rows) of one item of a cut launch: the parts lie in the order of the accumulator registers, so a
+// thread adds up four-channel pieces of one row; the sum is turned through LDS and written as whole rows.  Bound by the
+// bytes of the parts: 67 MB at head_dim 128 when every share leaves two, 11.5 us (5.8 TB/s).
+template <int D>
+__global__ __launch_bounds__(kCombineThreads) void cut_combine_kernel(AttnArgs a) {
+    constexpr int kPieces = 32 * D / 4 / kCombineThreads;  // per thread: 4 | 2
+    constexpr int RS = D + 4;                              // floats per row in LDS
+    __shared__ float rows[32 * RS];
+    // blockIdx: one of the cuts between two shares x tile.  The first cut inside an item takes care of the item.
+    const int tile = blockIdx.x % 8, cut = blockIdx.x / 8 + 1, pos = cut_begin(cut, a.cut_wgs, a.cut_total);
+    const CutLine line(a.M, a.N, a.causal);
+    const int bh = pos / line.head, iq = line.item(pos - bh * line.head);
+    const int begin = bh * line.head + line.start(iq), m0 = kFastRows * iq + 32 * tile;
+    const int first = cut_owner(begin, a.cut_wgs, a.cut_total);
+    if (begin == pos || first + 1 != cut || m0 >= a.M) return;
+    const int last = cut_owner(begin + line.len(iq) - 1, a.cut_wgs, a.cut_total);
+    const int t = threadIdx.x, lane = t & 63, row = t & 31;
+    auto slot = [&](int w) { return 2 * w + (w == first && begin != cut_begin(w, a.cut_wgs, a.cut_total)); };
+    float m = -INFINITY;
+    for (int w = first; w <= last; w++) m = fmaxf(m, a.part_lse[(int64_t)slot(w) * kFastRows + 32 * tile + row]);
+    v4f acc[kPieces];
+#pragma unroll
+    for (int e = 0; e < kPieces; e++) acc[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    float den = 0.0f;
+    if (m > -INFINITY) {  // (a row that saw no key)
+#pragma unroll 2
+        for (int w = first; w <= last; w++) {
+            const int64_t s = slot(w);
+            const float f = __builtin_amdgcn_exp2f(a.part_lse[s * kFastRows + 32 * tile + row] - m);
+            const v4f* po = reinterpret_cast<const v4f*>(a.part_o) + (s * 8 + tile) * (8 * D) + t;
+            den += f;
+#pragma unroll
+            for (int e = 0; e < kPieces; e++) {
+                const v4f o = po[kCombineThreads * e];
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[e][i] = __builtin_fmaf(f, o[i], acc[e][i]);
+            }
+        }
+    }
+    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+    const int b = bh / a.Hq, h = bh % a.Hq;
+    if (a.lse && t < 32 && m0 + row < a.M) a.lse[(int64_t)bh * a.M + m0 + row] = (__builtin_log2f(den) + m) * a.lse_mul;
+#pragma unroll
+    for (int e = 0; e < kPieces; e++) {
+        const int piece = t / 64 + 4 * e;  // 4 * (32-channel tile) + register group
+        v4f r;
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = acc[e][i] * inv;
+        *reinterpret_cast<v4f*>(rows + row * RS + 32 * (piece / 4) + 8 * (piece % 4) + 4 * (lane >> 5)) = r;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kPieces; e++) {
+        const int p = t + kCombineThreads * e, r = p / (D / 4), c = 4 * (p % (D / 4));
+        if (m0 + r >= a.M) continue;
+        const v4f x = *reinterpret_cast<const v4f*>(rows + r * RS + c);
+        const int64_t o = (int64_t)b * a.os_b + (int64_t)h * a.os_h + (int64_t)(m0 + r) * a.os_n + c;
+        store4(a.out, a.out_dt, o, x);
+    }
 }
 
 }  // namespace
@@ -129,32 +196,102 @@ static int plan_decode_split(int64_t items, int64_t rows, int64_t nk) {
     return best_s;
 }
 
-int plan_key_split(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal) {
-    if (decode_serves(heads_q, heads_kv, qo_len))
-        return plan_decode_split(batch * heads_kv, heads_q / heads_kv * qo_len, (kv_len + BN - 1) / BN);
-    const int64_t nq2 = (qo_len + kFastRows - 1) / kFastRows;
-    const int64_t per_head = causal ? (nq2 + 1) / 2 : nq2;  // under the causal flag a workgroup takes two q-blocks
-    const int64_t base = batch * heads_q * per_head;
+// Plans of the pipelined kernel, in steps.  Fitted to 38 shapes (1 to 96 heads, 512 to 16384 keys, both flags, both
+// head_dims, int8 and 16-bit Q and K) within 5 % for the cut launch and 10 % for the others: a workgroup spends kFixed on
+// the prologue and epilogue of each item or piece of one, a launch kLaunch, a second one kCombine, a piece that leaves a
+// partial result kPartial (132 KB stored, read again by the combine kernel).  A chip that is partly idle clocks higher
+// (head_dim 128: 79 us a workgroup at half the CUs, 100 us at all of them).
+constexpr float kFixed = 5.0f, kLaunch = 4.0f, kCombine = 3.0f, kPartial = 2.5f;
+constexpr float kCombineRows = 4.0f, kPartialRows = 4.0f;  // the key split stores its partial results row by row, in 16-byte pieces
+
+// Measured (us, pairs or key split -> plan taken; SageAttention / dense, bf16):
+//   longest first  B1 H32/8 N3001 causal 86 -> 78 / 99 -> 93, B1 H40 N4096 causal 189 -> 157 / 246 -> 192,
+//                  B2 H24 N3001 D64 causal 113 -> 84 / 120 -> 84; many heads per XCD lose the L2 (B16 H32 N2048 536 -> 599)
+//   cut            B1 H16 N4096 causal 108 -> 79 / 129 -> 91, B1 H12 N8192 D64 causal 206 -> 127 / 222 -> 131,
+//                  B1 H33 N4096 250 -> 215 / 303 -> 259, B1 H5 N14000 524 -> 372 / 709 -> 488;
+//                  short items lose (B6 H16 N1000 causal 46 -> 62)
+//   key split      B1 H30 M512 N4096 70 -> 44 / 76 -> 48; not B2 H16 N512 (25 against 14), B1 H20 N1024 (31 against 23)
+LaunchPlan plan_launch(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal,
+                       bool with_workspace) {
+    LaunchPlan plan{1, 0, false};
     const int64_t nk = (kv_len + BN - 1) / BN;
-    if (base * 5 >= kComputeUnits * 4 || nk < 2 * kMinStepsPerSplit) return 1;
-    // cost of a plan in steps: rounds of workgroups over the compute units x (steps of a run + fixed part)
-    const int smax = (int)(nk / kMinStepsPerSplit < kMaxSplits ? nk / kMinStepsPerSplit : kMaxSplits);
-    float best = 0.0f;
-    int best_s = 1;
-    for (int s = 1; s <= smax; s++) {
-        const int64_t steps = (nk + s - 1) / s;
-        const int64_t runs = (nk + steps - 1) / steps;  // runs that hold a key
-        if (runs != s) continue;
-        const int64_t rounds = (base * s + kComputeUnits - 1) / kComputeUnits;
-        const float cost = (float)rounds * ((float)steps + kFixedSteps) + (s > 1 ? 0.25f * (float)s : 0.0f);
-        if (s == 1 || cost < 0.95f * best) { best = cost; best_s = s; }
+    if (decode_serves(heads_q, heads_kv, qo_len)) {
+        if (with_workspace) plan.nsplit = plan_decode_split(batch * heads_kv, heads_q / heads_kv * qo_len, nk);
+        return plan;
     }
-    return best_s;
+    const int64_t nq = (qo_len + kFastRows - 1) / kFastRows, heads = batch * heads_q;
+    const int64_t per_head = causal ? (nq + 1) / 2 : nq;  // pairs under the causal flag
+    const int64_t base = heads * per_head;
+    // beyond eight rounds the hand-over between rounds hides what a plan could gain
+    if (heads <= 0 || base >= 8 * kComputeUnits || qo_len >= (1 << 22) || kv_len >= (1 << 22)) return plan;
+    const CutLine line((int)qo_len, (int)kv_len, causal);
+    const int64_t items = heads * line.nq, total = heads * line.head;
+    const float cus = (float)kComputeUnits;
+    auto busy = [&](float longest) {  // the chip's higher clock while CUs idle
+        const float util = (float)total / (cus * longest);
+        return util < 1.0f ? 0.7f + 0.3f * util : 1.0f;
+    };
+    // ---- whole items: as they come, or in pairs
+    const int shorter = causal && nq > 1 ? line.len((int)(nq / 2 - 1)) : 0;  // the most even pair is the longest
+    const int mirror = line.len((int)(nq - 1 - (nq > 1 ? nq / 2 - 1 : 0)));
+    const float pair = causal ? fmaxf((float)(shorter + mirror), (float)(line.len((int)nq - 1) + (nq > 1 ? line.len(0) : 0))) : (float)nk;
+    const float each = pair + kFixed * (causal && nq > 1 ? 2.0f : 1.0f);
+    const int64_t full = base / kComputeUnits, rest = base % kComputeUnits;
+    float best = kLaunch;
+    if (full == 0) best += each * busy(pair);
+    else best += each * ((float)full + (rest == 0 ? 0.0f : 0.66f + 0.34f * fmaxf(0.0f, (float)(2 * rest) / cus - 1.0f)));
+    // ---- one workgroup per item, longest first (causal): the bounds of any such order
+    if (causal && nq > 1) {
+        float lpt = fmaxf(((float)nk + kFixed) * busy((float)nk), ((float)total + kFixed * (float)items) / cus + 3.0f);
+        for (int64_t i = kComputeUnits, k = 2; i < items; i += kComputeUnits, k++)
+            lpt = fmaxf(lpt, (float)k * ((float)line.len((int)(line.nq - 1 - i / heads)) + kFixed));
+        lpt += kLaunch;
+        if (lpt < 0.95f * best) { best = lpt; plan.longest_first = true; }
+    }
+    // ---- the keys of every item (pair) split, where the chip would be less than 80 % busy
+    const int smax = !with_workspace || base * 5 >= kComputeUnits * 4 ? 1
+                     : (int)(nk / kMinStepsPerSplit < kMaxSplits ? nk / kMinStepsPerSplit : kMaxSplits);
+    const bool few = items <= kFewItems;
+    if (few) best = pair + 6.0f;
+    for (int s = 2; s <= smax; s++) {
+        const int64_t steps = (nk + s - 1) / s;
+        if ((nk + steps - 1) / steps != s) continue;  // (a run without a key)
+        const float rounds = (float)((base * s + kComputeUnits - 1) / kComputeUnits);
+        const float run = causal && nq > 1 ? (float)steps + fminf((float)steps, (float)shorter) + 2.0f * kFixed : (float)steps + kFixed;
+        const float cost = few ? (float)steps + 6.0f + 0.25f * (float)s
+                               : kLaunch + kCombineRows + rounds * run + kPartialRows * fminf(1.0f, (float)(base * s) / cus) + 0.25f * (float)s;
+        if (cost < 0.95f * best) { best = cost; plan.nsplit = s; plan.longest_first = false; }
+    }
+    if (few) return plan;
+    // ---- the launch cut into equal shares.  (Without the causal flag not where one round fills 80 % of the chip.)
+    const bool one_round = !causal && base * 5 >= kComputeUnits * 4 && base <= kComputeUnits;
+    if (with_workspace && !one_round && total < (1 << 23) && total >= 2 * kMinStepsPerShare) {
+        const int64_t wgs = total / kMinStepsPerShare < kComputeUnits ? total / kMinStepsPerShare : kComputeUnits;
+        const float cost = kLaunch + kCombine + (float)total / (float)wgs + kFixed * (1.0f + (float)items / (float)wgs) + 2.0f * kPartial +
+                           0.25f * (float)nk * (float)wgs / (float)total;  // (the parts of an item)
+        if (cost < 0.93f * best) plan = LaunchPlan{1, (int)wgs, false};
+    }
+    return plan;
 }
 
-int64_t key_split_workspace_bytes(int nsplit, int64_t batch, int64_t heads_q, int64_t qo_len, int64_t head_dim) {
-    if (nsplit <= 1) return 0;
-    return (int64_t)nsplit * batch * heads_q * qo_len * (head_dim + 1) * (int64_t)sizeof(float);
+int64_t plan_workspace_bytes(const LaunchPlan& plan, int64_t batch, int64_t heads_q, int64_t qo_len, int64_t head_dim) {
+    if (plan.cut_wgs > 0) return (int64_t)2 * plan.cut_wgs * kFastRows * (head_dim + 1) * (int64_t)sizeof(float);
+    if (plan.nsplit > 1) return (int64_t)plan.nsplit * batch * heads_q * qo_len * (head_dim + 1) * (int64_t)sizeof(float);
+    return 0;
+}
+
+void apply_cut(AttnArgs& a, int cut_wgs, int64_t batch, int head_dim, void* workspace) {
+    a.cut_wgs = cut_wgs;
+    a.cut_total = (int)(batch * a.Hq * CutLine(a.M, a.N, a.causal).head);
+    a.part_o = static_cast<float*>(workspace);
+    a.part_lse = a.part_o + (int64_t)2 * cut_wgs * kFastRows * head_dim;
+}
+
+int launch_cut_combine(const AttnArgs& a, int head_dim, hipStream_t stream) {
+    dim3 grid((unsigned)((a.cut_wgs - 1) * 8)), block(kCombineThreads);
+    if (head_dim == 128) hipLaunchKernelGGL((cut_combine_kernel<128>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((cut_combine_kernel<64>), grid, block, 0, stream, a);
+    return check_launch("cut_combine_kernel");
 }
 
 // Points `a` (a complete description of the unsplit launch) at the workspace and sets the split fields.

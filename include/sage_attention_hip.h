@@ -114,7 +114,9 @@ int sage_attn_fwd(const sage_attn_params* p, void* stream);
  * write normalized fp32 partial outputs and their base-2 log-sum-exps to the workspace and a second kernel
  * combines them (out = sum_s 2^(lse_s - lse) o_s, lse = log2 sum_s 2^lse_s).  Calls with few query rows per K/V
  * head (decoding: heads_q / heads_kv * qo_len of at most 32, or of at most 64 for grouped heads) cut the keys of a
- * (batch, K/V head) in the same way, for the kernel that packs those rows.  The reference's SageAttention launch has no such split (attn_qk_int8_per_block.py:176-190 is one grid over q-blocks); its dense forward does
+ * (batch, K/V head) in the same way, for the kernel that packs those rows.  Launches whose last round over the compute
+ * units, or whose causal q-blocks, leave many of them idle are cut into up to 256 equal shares of all their 64-key steps
+ * instead (at most two partial results of 256 rows per share, 68 MB at head_dim 128).  The reference's SageAttention launch has no such split (attn_qk_int8_per_block.py:176-190 is one grid over q-blocks); its dense forward does
  * (see sage_flash_attn_fwd_ws).  Results agree with sage_attn_fwd to fp32 rounding of the combination.
  *   sage_attn_fwd_workspace_bytes  bytes the split of this call would use; 0 = the call would not split;
  *                                  -1 = invalid params (sage_hip_last_error says why)
