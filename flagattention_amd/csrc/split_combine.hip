@@ -202,7 +202,7 @@ static int plan_decode_split(int64_t items, int64_t rows, int64_t nk) {
 // partial result kPartial (132 KB stored, read again by the combine kernel).  A chip that is partly idle clocks higher
 // (head_dim 128: 79 us a workgroup at half the CUs, 100 us at all of them).
 constexpr float kFixed = 5.0f, kLaunch = 4.0f, kCombine = 3.0f, kPartial = 2.5f;
-constexpr float kCombineRows = 4.0f, kPartialRows = 4.0f;  // the key split stores its partial results row by row, in 16-byte pieces
+constexpr float kCombineRows = 4.0f, kPartialRows = 4.0f;  // the key split stores its partial results row by row, in 16-byte pieces; per 256 rows of each CU
 
 // Measured (us, pairs or key split -> plan taken; SageAttention / dense, bf16):
 //   longest first  B1 H32/8 N3001 causal 86 -> 78 / 99 -> 93, B1 H40 N4096 causal 189 -> 157 / 246 -> 192,
@@ -259,7 +259,7 @@ LaunchPlan plan_launch(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t
         const float rounds = (float)((base * s + kComputeUnits - 1) / kComputeUnits);
         const float run = causal && nq > 1 ? (float)steps + fminf((float)steps, (float)shorter) + 2.0f * kFixed : (float)steps + kFixed;
         const float cost = few ? (float)steps + 6.0f + 0.25f * (float)s
-                               : kLaunch + kCombineRows + rounds * run + kPartialRows * fminf(1.0f, (float)(base * s) / cus) + 0.25f * (float)s;
+                               : kLaunch + kCombineRows + rounds * run + kPartialRows * (float)(s * heads * qo_len) / (cus * (float)kFastRows) + 0.25f * (float)s;
         if (cost < 0.95f * best) { best = cost; plan.nsplit = s; plan.longest_first = false; }
     }
     if (few) return plan;
