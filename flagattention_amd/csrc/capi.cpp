@@ -167,6 +167,12 @@ extern "C" int sage_attn_fwd_ws(const sage_attn_params* p, void* workspace, int6
     return launch_attn(*p, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+extern "C" int sage_lse_natural(float* lse, const float* shift, float shift_mul, int64_t n, void* stream) {
+    if (!lse || n < 0) return fail(SAGE_E_INVALID, "sage_lse_natural: null pointer or negative size");
+    if (n == 0) return SAGE_OK;
+    return attn::launch_lse_natural(lse, shift, shift_mul, n, (hipStream_t)stream);
+}
+
 static int check_flash_params(const sage_flash_params* p, bool forward);
 
 extern "C" int sage_flash_attn_fwd(const sage_flash_params* p, void* stream) {

@@ -35,6 +35,7 @@ int launch_flash_total_attention(const sage_flash_params& p, const float* log_no
                                  int64_t workspace_bytes, hipStream_t stream);
 int64_t total_workspace_bytes(const sage_flash_params& p);
 int launch_flash_dropout(const sage_flash_params& p, float dropout_p, uint64_t seed, uint64_t offset, hipStream_t stream);
+namespace attn { int launch_lse_natural(float* lse, const float* shift, float shift_mul, int64_t n, hipStream_t stream); }
 int launch_dropout_mask(uint8_t* mask, int64_t count, float dropout_p, uint64_t seed, uint64_t offset, hipStream_t stream);
 
 }  // namespace sage

@@ -166,7 +166,22 @@ __global__ __launch_bounds__(kCombineThreads) void cut_combine_kernel(AttnArgs a
     }
 }
 
+// lse = ln 2 * lse + shift_mul * shift, in place: 12 bytes per row, a launch of 2-3 us.
+__global__ __launch_bounds__(kCombineThreads) void lse_natural_kernel(float* lse, const float* shift, float shift_mul, int64_t n) {
+    const int64_t i = (int64_t)blockIdx.x * kCombineThreads + threadIdx.x;
+    if (i >= n) return;
+    const float x = lse[i] * 0.693147180559945309f;
+    lse[i] = shift ? __builtin_fmaf(shift[i], shift_mul, x) : x;
+}
+
 }  // namespace
+
+int launch_lse_natural(float* lse, const float* shift, float shift_mul, int64_t n, hipStream_t stream) {
+    const int64_t wgs = (n + kCombineThreads - 1) / kCombineThreads;
+    if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_lse_natural: too many rows for one launch");
+    hipLaunchKernelGGL(lse_natural_kernel, dim3((unsigned)wgs), dim3(kCombineThreads), 0, stream, lse, shift, shift_mul, n);
+    return check_launch("lse_natural_kernel");
+}
 
 // One row tile always: B1 H8/8 M1 N8192 19 us against 24 us on the 256-row tiles of the pipelined kernel, B4 H32/32 M1 N4096
 // 46 against 57 us (bf16, head_dim 128, dense).  Two row tiles (one wave per SIMD) where they hold several heads that

@@ -1,10 +1,8 @@
 """One-call SageAttention: K mean -> fused smoothing + quantization -> INT8 attention."""
 from __future__ import annotations
 
-import math
-
-import torch
-
+from .. import _lib
+from ._common import current_stream_ptr, device_guard
 from .attention import forward
 from .quant import per_block_int8, per_block_int8_smooth_k
 
@@ -32,7 +30,12 @@ def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smoot
                       return_lse=return_lse, causal=is_causal)
     if not return_lse:
         return o
-    lse = lse2 * math.log(2.0)
-    if q_dot_km is not None:
-        lse = torch.addcmul(lse, q_dot_km, torch.tensor(sm_scale, dtype=torch.float32, device=lse.device))
-    return o, lse
+    # one pass over the fresh lse (three torch calls with the scale copied to the device cost 14 us of GPU time and
+    # a host wait of 30 us at B1 H32 M3001)
+    if lse2.numel():
+        shift = None if q_dot_km is None else q_dot_km.contiguous()
+        with device_guard(lse2.device):
+            _lib.check(_lib.load().sage_lse_natural(lse2.data_ptr(), None if shift is None else shift.data_ptr(),
+                                                    float(sm_scale), lse2.numel(), current_stream_ptr(lse2.device)),
+                       "sage_lse_natural")
+    return o, lse2

@@ -128,6 +128,13 @@ int64_t sage_attn_fwd_workspace_bytes(const sage_attn_params* p);
 int sage_attn_fwd_ws(const sage_attn_params* p, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
+ * Turns the base-2 log-sum-exps of the calls above into natural-log ones of the unsmoothed logits, in place:
+ * lse[i] = ln 2 * lse[i] + shift_mul * shift[i] for n contiguous values.  shift: what smoothing took off the logits of a
+ * row before scaling (q_dot_km of sage_per_block_int8_smooth_k, shift_mul = sm_scale), or NULL.
+ */
+int sage_lse_natural(float* lse, const float* shift, float shift_mul, int64_t n, void* stream);
+
+/*
  * Mean of K over the sequence axis in a fixed fp32 order, for callers that want the library
  * to produce the `km` argument of per_block_int8 (the reference leaves km to its caller,
  * quant_per_block.py:49,53-54, so this entry point has no reference counterpart).
