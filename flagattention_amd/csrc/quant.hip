@@ -902,8 +902,9 @@ int launch_kmean(const sage_tensor& k, int k_dtype, void* km_out, int out_dtype,
 
 // Sequences of up to this many 64-row chunks, in calls of up to this many K blocks, have the partials of the K mean added by
 // every K block instead of by a launch of its own: GPU time B1 H32 N1024 D128 16.6 -> 14.0 us, B8 H16 N1024 D64 23.2 -> 20.4
-// us; longer ones (B2 H32 N2048 33.3 -> 32.8 us) and larger calls (B16 H32 N512, 4096 blocks: 53.2 -> 54.7 us) gain nothing.
-constexpr int kOwnMeanChunks = 16, kOwnMeanBlocks = 2048;
+// us, B1 H32 N2000 D128 21.2 -> 20.0 us, B2 H16 N2048 D64 16.3 -> 15.0 us; longer ones (B1 H32/8 N3001 22.6 -> 22.7 us, B1 H16
+// N5000 fp32 32.7 -> 33.6 us) and larger calls (B16 H32 N512, 4096 blocks: 53.2 -> 54.7 us) gain nothing.
+constexpr int kOwnMeanChunks = 32, kOwnMeanBlocks = 2048;
 
 // K mean -> k - km -> quantization of K, and quantization of Q.  Short sequences: smooth_head_kernel, one launch.  Others:
 //   1. Q blocks and the chunk partials of the K mean, side by side in one grid;

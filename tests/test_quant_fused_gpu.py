@@ -19,7 +19,7 @@ def _check(got, want):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("d,n", [(64, 1), (64, 63), (64, 64), (64, 65), (64, 128), (64, 129), (64, 256), (64, 300), (64, 512), (64, 513),
                                  (128, 1), (128, 64), (128, 65), (128, 128), (128, 191), (128, 256), (128, 257), (128, 1024),
-                                 (128, 1025), (32, 700), (32, 1100), (16, 90), (256, 200)])
+                                 (128, 1025), (128, 2048), (64, 2049), (32, 700), (32, 1100), (16, 90), (256, 200)])
 def test_smoothing_launch_forms(d, n, dtype, gpu_device):
     from flag_attn import sage_attention as sa
     from flagattention_amd.sage_attention.quant import per_block_int8_smooth_k
