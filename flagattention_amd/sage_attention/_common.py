@@ -92,17 +92,8 @@ def plans() -> PlanCache:
     return cache
 
 
-_WORKSPACES = {}
-
-
-def split_workspace(device, stream: int, nbytes: int) -> torch.Tensor:
-    """A byte buffer of at least ``nbytes`` for the scratch data of a launch (partial results of a key split, chunk
-    partials of the K mean), kept per (device, stream): launches on one stream run in order, so they can share
-    it; different streams get buffers of their own.  16-byte aligned (torch allocations are)."""
-    key = (device.index, stream)
-    ws = _WORKSPACES.get(key)
-    if ws is None or ws.numel() < nbytes:
-        if len(_WORKSPACES) >= 16:
-            _WORKSPACES.clear()
-        ws = _WORKSPACES[key] = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-    return ws
+def split_workspace(device, nbytes: int) -> torch.Tensor:
+    """A byte buffer of ``nbytes`` for the scratch data of a launch (partial results of a key split, chunk partials of
+    the K mean).  Taken from torch's allocator on every call: a captured graph holds its address, so nothing may
+    outlive the call that a later one could free.  16-byte aligned (torch allocations are)."""
+    return torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)

@@ -300,7 +300,7 @@ def forward(q, k, v, q_scale, k_scale, tensor_layout="HND", attn_mask=None,
         p.lse = lse.data_ptr() if return_lse else None
         p.mask = None if m is None else m.data_ptr()
         if ws_bytes > 0:
-            ws = split_workspace(dev, stream, ws_bytes)
+            ws = split_workspace(dev, ws_bytes)
             _lib.check(lib.sage_attn_fwd_ws(p_ref, ws.data_ptr(), ws.numel(), stream), "sage_attn_fwd_ws")
         else:
             _lib.check(lib.sage_attn_fwd(p_ref, stream), "sage_attn_fwd")

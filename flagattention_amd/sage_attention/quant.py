@@ -47,7 +47,7 @@ def k_mean(k: torch.Tensor, tensor_layout: str = "HND") -> torch.Tensor:
     with device_guard(k.device):
         out = torch.empty((b, h, d), dtype=k.dtype, device=k.device)
         stream = current_stream_ptr(k.device)
-        ws = split_workspace(k.device, stream, max(4, lib.sage_k_mean_workspace_bytes(b, h, n, d)))
+        ws = split_workspace(k.device, lib.sage_k_mean_workspace_bytes(b, h, n, d))
         desc = tensor_desc(k, hnd)
         _lib.check(lib.sage_k_mean(ctypes.byref(desc), DTYPE_CODE[k.dtype], out.data_ptr(), DTYPE_CODE[k.dtype],
                                    b, h, n, d, ws.data_ptr(), stream), "sage_k_mean")
@@ -172,7 +172,7 @@ def _quantize(q, k, km, BLKQ, BLKK, sm_scale, tensor_layout, smooth, want_dot):
         p.q_scale, p.k_scale = q_scale.data_ptr(), k_scale.data_ptr()
         if fused:
             km_flat = torch.empty((b, h_kv, head_dim), dtype=k.dtype, device=dev)
-            ws = split_workspace(dev, stream, max(ws_bytes, 4))
+            ws = split_workspace(dev, ws_bytes)
             sp.km_out, sp.workspace = km_flat.data_ptr(), ws.data_ptr()
             if want_dot:
                 dot = torch.empty((b, h_qo, qo_len), dtype=torch.float32, device=dev)

@@ -89,3 +89,47 @@ def test_what_the_key_does_not_cover_is_checked_again(gpu_device):
     mask = torch.ones(1, 1, 77, 144, dtype=torch.bool, device=gpu_device)[..., :130]
     for _ in range(2):
         assert torch.equal(sa.sage_attention(q8, k8, v, qs, ks, attn_mask=mask)[0], sa.sage_attention(q8, k8, v, qs, ks, attn_mask=mask.clone())[0])
+
+
+@pytest.mark.parametrize("first", [True, False])  # whether the captured call is the first of its shape (the Python side) or not
+def test_a_captured_graph_owns_its_scratch_memory(gpu_device, first):
+    """The partial results of a captured call lie in memory that no other tensor gets while the graph lives, also when later
+    calls on the capture stream need more of it; every replay gives the eager result and touches nothing else."""
+    import flag_attn
+    from flag_attn import sage_attention as sa
+    from flagattention_amd import _lib
+
+    n = 1030 if first else 1040
+    q, k, v = _qkv(5, gpu_device, m=40, n=n, d=128)
+    big = _qkv(6, gpu_device, h=16, hkv=16, m=256, n=4096, d=128)
+
+    def run():
+        q8, qs, k8, ks = sa.per_block_int8(q, k, smooth_k=True)
+        return [*sa.sage_attention(q8, k8, v, qs, ks, return_lse=True), flag_attn.flash_attention(q, k, v)]
+
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):  # scratch memory of the capture stream from before the capture
+        for other in (big if not first else _qkv(7, gpu_device, m=40, n=1100, d=128),):
+            sa.sageattn(*other)
+            flag_attn.flash_attention(*other)
+        if not first:
+            run()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        captured = run()
+    want = [t.clone() for t in run()]
+    assert _lib.host().flash(q, k, v, False, None, False) is not None
+    with torch.cuda.stream(side):
+        flag_attn.flash_attention(*_qkv(8, gpu_device, h=32, hkv=32, m=512, n=8192, d=128))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        kept = [torch.full((1 << s,), 7, dtype=torch.uint8, device=gpu_device) for s in (16, 18, 20, 20, 22, 24)]
+    for rep in range(3):
+        for t in captured:
+            t.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(captured, want)), f"replay {rep}"
+        assert all(bool((t == 7).all()) for t in kept), f"replay {rep} wrote to another tensor"
