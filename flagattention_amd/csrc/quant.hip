@@ -403,29 +403,47 @@ __global__ __launch_bounds__(THREADS) void quant_own_mean_kernel(QuantArgs a) {
     quant_block<DT, UNITS, THREADS>(a, blockIdx.x, wave_max, km_lds);
 }
 
-// K and Q blocks in one grid, for calls so small that a second launch costs more than the better shape of workgroup for the Q
-// blocks (kBothBlocks): GPU time B1 H2 N256 D64 fp16 6.5 -> 3.6 us, B1 H32 N1024 D128 bf16 8.9 -> 6.8 us.
+// K and Q blocks in one grid: what a second launch costs is saved, and no tail of the first is waited for.  Up to kBothBlocks
+// blocks any shape of block (GPU time B1 H2 N256 D64 fp16 6.5 -> 3.6 us, B1 H32 N1024 D128 bf16 8.9 -> 6.8 us); beyond that
+// the block shapes of wide_both, which fill every unit of the threads.
 constexpr int64_t kBothBlocks = 1024;
-template <int DT, int KU, int QU>
-__global__ __launch_bounds__(kThreads) void quant_both_kernel(QuantArgs kq, QuantArgs qq, int k_blocks) {
-    __shared__ float wave_max[kThreads / 64];
-    if ((int)blockIdx.x < k_blocks) quant_block<DT, KU, kThreads>(kq, blockIdx.x, wave_max);
-    else quant_block<DT, QU, kThreads>(qq, blockIdx.x - k_blocks, wave_max);
+
+template <int DT, int KU, int QU, int THREADS>
+__global__ __launch_bounds__(THREADS) void quant_both_kernel(QuantArgs kq, QuantArgs qq, int k_blocks) {
+    __shared__ float wave_max[THREADS / 64];
+    if ((int)blockIdx.x < k_blocks) quant_block<DT, KU, THREADS>(kq, blockIdx.x, wave_max);
+    else quant_block<DT, QU, THREADS>(qq, blockIdx.x - k_blocks, wave_max);
 }
 
 template <int DT>
 int launch_both_dt(const QuantArgs& kq, const QuantArgs& qq, int64_t k_blocks, int64_t q_blocks, hipStream_t stream) {
     dim3 grid((unsigned)(k_blocks + q_blocks));
     if (kq.blk * kq.D8 <= 2 * kThreads && qq.blk * qq.D8 <= 4 * kThreads)
-        hipLaunchKernelGGL((quant_both_kernel<DT, 2, 4>), grid, dim3(kThreads), 0, stream, kq, qq, (int)k_blocks);
+        hipLaunchKernelGGL((quant_both_kernel<DT, 2, 4, kThreads>), grid, dim3(kThreads), 0, stream, kq, qq, (int)k_blocks);
+    else if (k_blocks + q_blocks <= kBothBlocks)
+        hipLaunchKernelGGL((quant_both_kernel<DT, 4, 8, kThreads>), grid, dim3(kThreads), 0, stream, kq, qq, (int)k_blocks);
     else
-        hipLaunchKernelGGL((quant_both_kernel<DT, 4, 8>), grid, dim3(kThreads), 0, stream, kq, qq, (int)k_blocks);
+        hipLaunchKernelGGL((quant_both_kernel<DT, 2, 4, 2 * kThreads>), grid, dim3(2 * kThreads), 0, stream, kq, qq, (int)k_blocks);
     return check_launch("quant_both_kernel");
 }
 
+// 64-row K and 128-row Q blocks at head_dim 64, in workgroups as their own launches have, and at 128, where the K blocks get
+// workgroups of 512 instead of 256 threads: fewer of them fit a CU side by side, which costs more than the launch in larger
+// calls.  GPU time, two launches -> one (bf16; in brackets mean, K and Q with q . km, where Q follows the mean):
+//   D64   B1 H16 N3000 8.8 -> 6.7 us (21.5 -> 18.7), B8 H16 N2048 22.2 -> 19.3, B8 H16/2 N4096 22.8 -> 19.1 (36.5 -> 30.3),
+//         B8 H32/8 N8192, 24576 blocks, 91.6 -> 89.0 (129.4 -> 125.0); 49152 blocks 142 -> 143 (227 -> 228)
+//   D128  B1 H32/8 N3001 12.6 -> 10.3 (29.2 -> 26.2), B1 H32/8 N6000 20.2 -> 17.5 (35.7 -> 32.5), B1 H40 N4096, 3840 blocks,
+//         25.0 -> 24.1 (41.7 -> 41.9); B2 H32 N4096, 6144 blocks, 35.4 -> 35.7 (57.9 -> 59.6)
+bool wide_both(const QuantArgs& kq, const QuantArgs& qq, int64_t blocks) {
+    const int ku = kq.blk * kq.D8, qu = qq.blk * qq.D8;
+    if (kq.d8_shift < 0 || qq.d8_shift < 0 || qu != 2 * ku) return false;
+    return ku == 2 * kThreads ? blocks <= 32768 : ku == 4 * kThreads && blocks <= 4096;
+}
+
 bool both_fit(const QuantArgs& kq, const QuantArgs& qq, int64_t k_blocks, int64_t q_blocks) {
-    return k_blocks > 0 && q_blocks > 0 && k_blocks + q_blocks <= kBothBlocks && !kq.part && kq.blk * kq.D8 <= 4 * kThreads &&
-           qq.blk * qq.D8 <= 8 * kThreads;
+    const int64_t blocks = k_blocks + q_blocks;
+    return k_blocks > 0 && q_blocks > 0 && !kq.part && kq.blk * kq.D8 <= 4 * kThreads && qq.blk * qq.D8 <= 8 * kThreads &&
+           (blocks <= kBothBlocks || wide_both(kq, qq, blocks));
 }
 
 int launch_both(const QuantArgs& kq, const QuantArgs& qq, int in_dtype, int64_t k_blocks, int64_t q_blocks, hipStream_t stream) {
@@ -911,7 +929,8 @@ constexpr int kOwnMeanChunks = 32, kOwnMeanBlocks = 2048;
 //   2. the mean per channel (chunk partials added in order, one division, one rounding to K's dtype), up to kOwnMeanChunks
 //      chunks inside 3;
 //   3. K blocks, subtracting the mean just written.
-// With q_dot_km the Q blocks need the mean as well and move behind it: partials, mean, K blocks, Q blocks.
+// With q_dot_km the Q blocks need the mean as well and move behind it: partials, mean, K and Q blocks in one grid (which the
+// K blocks that add the partials themselves cannot share: their Q blocks follow).
 int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_km, void* workspace, hipStream_t stream) {
     const int64_t B = p.batch, H = p.heads_kv, N = p.kv_len, D = p.head_dim;
     KMeanArgs ka;
@@ -926,6 +945,10 @@ int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_k
         if (int rc = q_args(p, qq)) return rc;
     }
     const int64_t q_blocks = have_q ? p.batch * p.heads_q * qq.nblk : 0;
+    auto q_dot = [&] {  // the Q blocks read the mean that an earlier launch has written
+        qq.km = km_out; qq.ks_b = H * D; qq.ks_h = D; qq.ks_n = 0; qq.km_dt = p.in_dtype; qq.diff_dt = p.in_dtype;
+        qq.dot = q_dot_km; qq.dot_groups = (int)(p.heads_q / p.heads_kv);
+    };
     bool fused = false;
     if (head_fits(kq, p.in_dtype)) {
         const int q_units = have_q ? qq.blk * qq.D8 : 0;
@@ -954,13 +977,14 @@ int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_k
         } else {
             if (int rc = launch_k_mean_final(ka, B * H * D, stream)) return rc;
         }
+        if (have_q && q_dot_km) {
+            q_dot();
+            if (both_fit(kq, qq, B * H * kq.nblk, q_blocks)) return launch_both(kq, qq, p.in_dtype, B * H * kq.nblk, q_blocks, stream);
+        }
         if (int rc = launch_tensor(kq, p.in_dtype, B * H * kq.nblk, stream)) return rc;
     }
     if (have_q && !fused) {
-        if (q_dot_km) {
-            qq.km = km_out; qq.ks_b = H * D; qq.ks_h = D; qq.ks_n = 0; qq.km_dt = p.in_dtype; qq.diff_dt = p.in_dtype;
-            qq.dot = q_dot_km; qq.dot_groups = (int)(p.heads_q / p.heads_kv);
-        }
+        if (q_dot_km) q_dot();
         if (int rc = launch_tensor(qq, p.in_dtype, q_blocks, stream)) return rc;
     }
     return SAGE_OK;

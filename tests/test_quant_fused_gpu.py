@@ -49,7 +49,8 @@ def test_smoothing_launch_forms(d, n, dtype, gpu_device):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("b,hq,hkv,m,n,d", [(1, 2, 2, 1, 1, 64), (2, 4, 2, 200, 77, 128), (1, 3, 1, 129, 1000, 64),
-                                            (4, 32, 8, 2048, 4032, 64), (4, 32, 8, 2048, 4160, 64), (1, 2, 1, 90, 130, 256)])
+                                            (4, 32, 8, 2048, 4032, 64), (4, 32, 8, 2048, 4160, 64), (1, 2, 1, 90, 130, 256),
+                                            (2, 16, 16, 2000, 2049, 128), (1, 33, 11, 4095, 129, 128), (3, 8, 8, 65, 8191, 32)])
 def test_k_and_q_in_one_grid(b, hq, hkv, m, n, d, dtype, gpu_device):
     from flag_attn import sage_attention as sa
 
@@ -59,3 +60,25 @@ def test_k_and_q_in_one_grid(b, hq, hkv, m, n, d, dtype, gpu_device):
     for mean in (None, km):
         got = sa.per_block_int8(q.to(gpu_device), k.to(gpu_device), km=None if mean is None else mean.to(gpu_device))
         _check(got, C.per_block_int8(q, k, km=mean))
+
+
+@pytest.mark.parametrize("layout", ["HND", "NHD"])
+@pytest.mark.parametrize("b,hq,hkv,m,n,d", [(1, 16, 4, 2100, 2113, 128), (2, 32, 8, 2047, 2049, 128), (2, 32, 16, 2500, 4100, 64)])
+def test_k_and_q_in_one_grid_behind_the_mean(b, hq, hkv, m, n, d, layout, gpu_device):
+    """Q blocks that also give q . km, at up to 1024 blocks and beyond: the bits of the K and Q blocks on their own, and the
+    same dot products as for one head alone (which is in a smaller grid)."""
+    from flagattention_amd.sage_attention.quant import per_block_int8_smooth_k
+
+    g = torch.Generator().manual_seed(4)
+    q, k = torch.randn(b, hq, m, d, generator=g).bfloat16(), (torch.randn(b, hkv, n, d, generator=g) + 2.0).bfloat16()
+    if layout == "NHD":
+        q, k = q.transpose(1, 2).contiguous(), k.transpose(1, 2).contiguous()
+    km = C.k_mean_fixed_order(k, layout)
+    *got, km_got, dot = per_block_int8_smooth_k(q.to(gpu_device), k.to(gpu_device), tensor_layout=layout, with_q_dot_km=True)
+    _check(got, C.per_block_int8(q, k, km=km, tensor_layout=layout))
+    assert torch.equal(km_got.cpu().view(torch.int16), km.view(torch.int16))
+    if layout == "NHD":
+        q, k = q.transpose(1, 2), k.transpose(1, 2)
+    h = hq - 1
+    *_, one = per_block_int8_smooth_k(q[-1:, h:].contiguous().to(gpu_device), k[-1:, hkv - 1:].contiguous().to(gpu_device), with_q_dot_km=True)
+    assert torch.equal(dot[-1, h], one[0, 0])
