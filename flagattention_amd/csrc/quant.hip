@@ -929,8 +929,9 @@ constexpr int kOwnMeanChunks = 32, kOwnMeanBlocks = 2048;
 //   2. the mean per channel (chunk partials added in order, one division, one rounding to K's dtype), up to kOwnMeanChunks
 //      chunks inside 3;
 //   3. K blocks, subtracting the mean just written.
-// With q_dot_km the Q blocks need the mean as well and move behind it: partials, mean, K and Q blocks in one grid (which the
-// K blocks that add the partials themselves cannot share: their Q blocks follow).
+// With q_dot_km the Q blocks need the mean as well and move behind it: partials, mean, K and Q blocks in one grid (where
+// both_fit, also for few chunks: K blocks that add the partials themselves and the Q blocks behind them took B1 H32/8 N600
+// D128 19.2 us, this 17.1, B1 H8 N700 D64 17.5 -> 14.0, B4 H32/8 N1024 D128 25.4 -> 23.7, B2 H32 N2000 D128 35.4 -> 35.2).
 int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_km, void* workspace, hipStream_t stream) {
     const int64_t B = p.batch, H = p.heads_kv, N = p.kv_len, D = p.head_dim;
     KMeanArgs ka;
@@ -971,15 +972,16 @@ int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_k
         if (!fused) {
             if (int rc = launch_k_mean_partial(ka, p.in_dtype, stream)) return rc;
         }
-        if (kq.blk == 64 && kq.d8_shift >= 0 && D <= kMaxFusedMeanDim && kq.blk * kq.D8 <= 1024 && kq.nblk <= kOwnMeanChunks &&
+        const bool shared = have_q && q_dot_km && both_fit(kq, qq, B * H * kq.nblk, q_blocks);  // one grid with the Q blocks
+        if (!shared && kq.blk == 64 && kq.d8_shift >= 0 && D <= kMaxFusedMeanDim && kq.blk * kq.D8 <= 1024 && kq.nblk <= kOwnMeanChunks &&
             B * H * kq.nblk <= kOwnMeanBlocks) {
             kq.km = nullptr; kq.part = ka.part; kq.km_write = km_out;  // every block adds the chunk partials itself
         } else {
             if (int rc = launch_k_mean_final(ka, B * H * D, stream)) return rc;
         }
-        if (have_q && q_dot_km) {
+        if (shared) {
             q_dot();
-            if (both_fit(kq, qq, B * H * kq.nblk, q_blocks)) return launch_both(kq, qq, p.in_dtype, B * H * kq.nblk, q_blocks, stream);
+            return launch_both(kq, qq, p.in_dtype, B * H * kq.nblk, q_blocks, stream);
         }
         if (int rc = launch_tensor(kq, p.in_dtype, B * H * kq.nblk, stream)) return rc;
     }
