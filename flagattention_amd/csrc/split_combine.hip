@@ -31,6 +31,10 @@ struct CombineArgs {
 
 constexpr int kCombineThreads = 256;
 
+// Maximum of log-sum-exps.  NaN stays: it stands for NaN scores (a NaN or an infinity in Q or K), which make the whole row
+// NaN, where fmaxf would leave the -inf of a row that saw no key, or the other runs alone.
+__device__ __forceinline__ float max_or_nan(float m, float x) { return x > m || x != x ? x : m; }
+
 __device__ __forceinline__ void store4(void* out, int out_dt, int64_t o, v4f r) {
     if (out_dt == SAGE_BF16) {
         typedef __bf16 b4 __attribute__((ext_vector_type(4)));
@@ -57,10 +61,10 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineA
     const bool ok = row < a.rows;
     const float* pl = a.part_lse + (ok ? row : 0);
     float m = -INFINITY;
-    for (int s = sg; s < a.nsplit; s += SG) m = fmaxf(m, pl[(int64_t)s * a.rows]);
+    for (int s = sg; s < a.nsplit; s += SG) m = max_or_nan(m, pl[(int64_t)s * a.rows]);
     v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
     float den = 0.0f;
-    if (m > -INFINITY) {  // (a row that saw no key in any run: every partial is 0 and every lse_s -inf)
+    if (m != -INFINITY) {  // (a row that saw no key in any run: every partial is 0 and every lse_s -inf)
         const float* po = a.part_o + (ok ? row : 0) * D + 4 * c;
 #pragma unroll 4
         for (int s = sg; s < a.nsplit; s += SG) {
@@ -79,10 +83,10 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineA
         if (sg != 0) return;
         const int t0 = threadIdx.x;
 #pragma unroll
-        for (int g = 1; g < SG; g++) m = fmaxf(m, sm_m[t0 + g * TPR]);
+        for (int g = 1; g < SG; g++) m = max_or_nan(m, sm_m[t0 + g * TPR]);
         acc = v4f{0.0f, 0.0f, 0.0f, 0.0f};
         den = 0.0f;
-        if (m > -INFINITY) {
+        if (m != -INFINITY) {
 #pragma unroll
             for (int g = 0; g < SG; g++) {
                 const float w = __builtin_amdgcn_exp2f(sm_m[t0 + g * TPR] - m);
@@ -124,12 +128,12 @@ __global__ __launch_bounds__(kCombineThreads) void cut_combine_kernel(AttnArgs a
     const int t = threadIdx.x, lane = t & 63, row = t & 31;
     auto slot = [&](int w) { return 2 * w + (w == first && begin != cut_begin(w, a.cut_wgs, a.cut_total)); };
     float m = -INFINITY;
-    for (int w = first; w <= last; w++) m = fmaxf(m, a.part_lse[(int64_t)slot(w) * kFastRows + 32 * tile + row]);
+    for (int w = first; w <= last; w++) m = max_or_nan(m, a.part_lse[(int64_t)slot(w) * kFastRows + 32 * tile + row]);
     v4f acc[kPieces];
 #pragma unroll
     for (int e = 0; e < kPieces; e++) acc[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     float den = 0.0f;
-    if (m > -INFINITY) {  // (a row that saw no key)
+    if (m != -INFINITY) {  // (a row that saw no key)
 #pragma unroll 2
         for (int w = first; w <= last; w++) {
             const int64_t s = slot(w);

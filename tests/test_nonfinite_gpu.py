@@ -1,0 +1,125 @@
+"""A NaN or an infinity in Q or K makes the rows that see it NaN, output and log-sum-exp alike, whether a launch is whole or
+leaves partial results in a workspace that a second kernel combines."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# (batch, heads_q, heads_kv, M, N, D, causal)
+SHAPES = [
+    (8, 32, 8, 1, 8192, 128, False),    # few query rows, four runs of the keys
+    (1, 8, 8, 1, 8192, 64, False),      # ... many runs, which eight groups of threads per row share
+    (1, 32, 32, 1, 8192, 64, False),    # ... a run for each of the groups
+    (1, 8, 2, 5, 3000, 128, True),
+    (1, 4, 2, 300, 4096, 64, True),     # keys of a 256-row block split
+    (1, 2, 2, 20, 4096, 128, False),
+    (1, 9, 9, 3000, 3000, 128, True),   # launch cut into equal shares
+    (1, 33, 33, 2100, 2100, 64, False),
+]
+
+
+def _launch(lib, kind, p, workspace, device):
+    stream = torch.cuda.current_stream().cuda_stream
+    need = getattr(lib, f"sage_{kind}_workspace_bytes")(ctypes.byref(p))
+    assert need > 0, "this shape was meant to leave partial results"
+    if workspace:
+        ws = torch.empty(need, dtype=torch.uint8, device=device)
+        rc = getattr(lib, f"sage_{kind}_ws")(ctypes.byref(p), ws.data_ptr(), need, stream)
+    else:
+        rc = getattr(lib, f"sage_{kind}")(ctypes.byref(p), stream)
+    assert rc == 0, lib.sage_hip_last_error()
+    torch.cuda.synchronize()
+
+
+def _check(results, want, empty=None):
+    """``want`` [B, H, M]: the rows that are NaN in every channel and in the log-sum-exp; all others are finite, but for the
+    log-sum-exp of ``empty`` ones, whose scores are all -inf."""
+    for workspace, (o, lse) in enumerate(results):
+        infinite = want if empty is None else want | empty
+        for got, expected in ((torch.isnan(lse), want), (~torch.isfinite(lse), infinite), (torch.isnan(o).all(-1), want),
+                              (~torch.isfinite(o).all(-1), want)):
+            wrong = (got != expected).nonzero()
+            assert not len(wrong), (f"workspace {workspace}: {len(wrong)} rows", wrong[:4].tolist(), wrong[-4:].tolist())
+
+
+def _sees(m, n, key, causal, device):
+    """[M]: which queries see key ``key``."""
+    return torch.arange(m, device=device) + (n - m) >= key if causal else torch.ones(m, dtype=torch.bool, device=device)
+
+
+@pytest.mark.parametrize("where", ["query_nan", "query_inf", "key_nan"])
+@pytest.mark.parametrize("b,h,hkv,m,n,d,causal", SHAPES)
+def test_dense_rows(b, h, hkv, m, n, d, causal, where, gpu_device):
+    from flagattention_amd import _lib
+    from flagattention_amd.sage_attention._common import DTYPE_CODE, tensor_desc
+
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(b, x, y, d, generator=g).to(torch.bfloat16).to(gpu_device) for x, y in ((h, m), (hkv, n), (hkv, n)))
+    want = torch.zeros((b, h, m), dtype=torch.bool, device=gpu_device)
+    if where == "key_nan":
+        k[0, hkv - 1, 100, 7] = float("nan")
+        want[0, (hkv - 1) * (h // hkv):] = _sees(m, n, 100, causal, gpu_device)
+    else:
+        row = m // 2
+        q[0, 1, row, 5] = float("nan" if where == "query_nan" else "inf")
+        want[0, 1, row] = True
+    lib = _lib.load()
+    results = []
+    for workspace in (False, True):
+        o, lse = torch.empty_like(q), torch.empty((b, h, m), dtype=torch.float32, device=gpu_device)
+        p = _lib.FlashParams()
+        p.q, p.k, p.v, p.out = (tensor_desc(t, True) for t in (q, k, v, o))
+        p.log_normalizer = lse.data_ptr()
+        p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.head_dim, p.causal = b, h, hkv, m, n, d, causal
+        p.dtype = p.out_dtype = DTYPE_CODE[torch.bfloat16]
+        p.sm_scale = d ** -0.5
+        _launch(lib, "flash_attn_fwd", p, workspace, gpu_device)
+        results.append((o, lse))
+    _check(results, want)
+
+
+@pytest.mark.parametrize("where", ["query_scale", "key_scale"])
+@pytest.mark.parametrize("b,h,hkv,m,n,d,causal", SHAPES)
+def test_quantized_rows(b, h, hkv, m, n, d, causal, where, gpu_device):
+    """An infinite scale, as the quantizer gives a block that holds an infinity: scores of +inf or (product 0) NaN make their
+    rows NaN, a score of -inf is a key of weight 0."""
+    from flag_attn import sage_attention as sa
+    from flagattention_amd import _lib
+    from flagattention_amd.sage_attention._common import DTYPE_CODE, tensor_desc
+
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(b, x, y, d, generator=g).to(torch.bfloat16).to(gpu_device) for x, y in ((h, m), (hkv, n), (hkv, n)))
+    q8, qs, k8, ks = sa.per_block_int8(q, k)
+    want = torch.zeros((b, h, m), dtype=torch.bool, device=gpu_device)
+    keys = torch.arange(n, device=gpu_device)
+    sees = keys[None, :] <= torch.arange(m, device=gpu_device)[:, None] + (n - m) if causal else torch.ones((m, n), dtype=torch.bool, device=gpu_device)
+    rows = torch.ones(m, dtype=torch.bool, device=gpu_device)
+    if where == "key_scale":
+        heads = range((hkv - 1) * (h // hkv), h)
+        ks[0, hkv - 1, 1] = float("inf")  # keys 64 to 127
+        sees = sees & (keys >= 64) & (keys < 128)
+    else:
+        heads = [1]
+        qs[0, 1, 0] = float("inf")  # queries 0 to 127
+        rows[128:] = False
+    for head in heads:
+        dot = q8[0, head].float() @ k8[0, head // (h // hkv)].float().T
+        want[0, head] = rows & ((dot >= 0) & sees).any(1)
+    assert bool(want.any())
+    empty = torch.zeros_like(want)
+    if where == "query_scale":  # (the first queries under the causal flag see few keys)
+        empty[0, 1] = rows & ~want[0, 1]
+    lib = _lib.load()
+    results = []
+    for workspace in (False, True):
+        o, lse = torch.empty_like(q), torch.empty((b, h, m), dtype=torch.float32, device=gpu_device)
+        p = _lib.AttnParams()
+        p.q, p.k, p.v, p.out = (tensor_desc(t, True) for t in (q8, k8, v, o))
+        p.q_scale, p.k_scale, p.lse = qs.data_ptr(), ks.data_ptr(), lse.data_ptr()
+        p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.head_dim, p.causal = b, h, hkv, m, n, d, causal
+        p.v_dtype = p.out_dtype = DTYPE_CODE[torch.bfloat16]
+        _launch(lib, "attn_fwd", p, workspace, gpu_device)
+        results.append((o, lse))
+    _check(results, want, empty)
