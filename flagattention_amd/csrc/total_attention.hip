@@ -67,6 +67,7 @@ __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(Total
     const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.groups;
     const int n0 = kb * kWgKeys + wave * kWaveKeys;  // (may lie past the last key: such a wave multiplies copies of it)
     const int shift = a.N - a.M;
+    const int m_sees = a.causal ? max(-shift, 0) : 0;  // first query that sees a key
 
     // K rows of this wave: lane (key l32, half) holds elements 16 t + 8 half .. + 7 of its row for step t
     vec16 kf[2][KS];
@@ -142,9 +143,9 @@ __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(Total
         fetch(t + 3);
         const int mq = m_lo + kTileQ * t, buf = t & (kRing - 1);
         if (a.causal && mq + kTileQ - 1 + shift < n0) continue;  // (the tile's last query sees no key of this wave)
-        // queries past the end, and queries that see no key (L = -inf), take L = +inf: every p of theirs is exp2(-inf) = 0
+        // queries past the end, and queries that see no key, take L = +inf: every p of theirs is exp2(-inf) = 0
         const float L = ltile[buf][wave][lane];
-        const float l2 = mq + l32 < a.M && L > -INFINITY ? L * 1.44269504088896340736f : INFINITY;
+        float l2 = (unsigned)(mq + l32 - m_sees) < (unsigned)(a.M - m_sees) ? L * 1.44269504088896340736f : INFINITY;
         v16f s[2];
 #pragma unroll
         for (int kt = 0; kt < 2; kt++)
@@ -159,11 +160,15 @@ __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(Total
         }
         if (a.causal && mq + shift < n0 + kWaveKeys - 1) {  // the tile's first query does not see the wave's last key
             const int last = mq + l32 + shift - n0 - 4 * half;  // last key the query sees, from the lane's first one on
+            // A log normalizer of NaN (NaN scores) or -inf joins the scores of the keys the query sees: in the exponent it
+            // would make the hidden ones NaN as well.
+            const float odd = l2 > -INFINITY ? 0.0f : -l2;
+            l2 = l2 > -INFINITY ? l2 : 0.0f;
 #pragma unroll
             for (int kt = 0; kt < 2; kt++)
 #pragma unroll
                 for (int i = 0; i < 16; i++)  // accumulator register i: key 32 kt + 8 (i / 4) + i % 4 from there
-                    s[kt][i] = 32 * kt + 8 * (i >> 2) + (i & 3) <= last ? s[kt][i] : -INFINITY;
+                    s[kt][i] = 32 * kt + 8 * (i >> 2) + (i & 3) <= last ? s[kt][i] + odd : -INFINITY;
         }
 #pragma unroll
         for (int kt = 0; kt < 2; kt++)

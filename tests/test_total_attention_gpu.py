@@ -37,3 +37,49 @@ def test_total_attention_tile_edges(M, N, D, dtype, gpu_device):
         _lib.check(lib.sage_flash_total_attention(p, L.data_ptr(), one.data_ptr(), torch.cuda.current_stream().cuda_stream), "total")
         torch.cuda.synchronize()
         torch.testing.assert_close(one, tot, rtol=2 * M * 2.0 ** -24, atol=1e-6)
+
+
+@pytest.mark.parametrize("where", ["query_nan", "query_inf", "key_nan", "normalizer_nan"])
+@pytest.mark.parametrize("M,N,causal", [(600, 700, False), (600, 700, True), (700, 600, True), (33, 65, True), (2100, 2100, True)])
+def test_total_attention_keeps_nan(M, N, causal, where, gpu_device):
+    """A query whose log normalizer is NaN makes the sums of all keys it sees NaN, and no other: with runs of the queries and
+    without, also where the causal limit runs through a tile."""
+    import flag_attn
+    from flagattention_amd import _lib
+    from flagattention_amd.sage_attention._common import DTYPE_CODE, tensor_desc
+
+    B, H, D = 1, 2, 64
+    g = torch.Generator().manual_seed(6)
+    q, k, v = (torch.randn(B, H, n, D, generator=g).to(torch.bfloat16).to(gpu_device) for n in (M, N, N))
+    row = M // 2 + 5
+    if where == "key_nan":
+        k[0, 1, N // 3, 0] = float("nan")
+    elif where != "normalizer_nan":
+        q[0, 1, row, 0] = float(where[6:])
+    _, L, tot, *_ = flag_attn.flash_attention(q, k, v, causal, return_log_normalizer=True, return_total_attention=True)
+    if where == "normalizer_nan":
+        L[0, 1, row] = float("nan")
+    sees = torch.ones(M, N, dtype=torch.bool, device=gpu_device)
+    if causal:
+        sees = torch.arange(N, device=gpu_device)[None, :] <= torch.arange(M, device=gpu_device)[:, None] + (N - M)
+    bad = torch.zeros(M, dtype=torch.bool, device=gpu_device)
+    bad[row] = True
+    if where == "key_nan":
+        bad = sees[:, N // 3]
+    want = torch.zeros((B, H, N), dtype=torch.bool, device=gpu_device)
+    want[0, 1] = sees[bad].any(0)
+    assert torch.equal(torch.isnan(L)[0, 1], bad)
+    lib = _lib.load()
+    p = _lib.FlashParams()
+    p.q, p.k = tensor_desc(q, True), tensor_desc(k, True)
+    p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.head_dim = B, H, H, M, N, D
+    p.dtype, p.causal, p.sm_scale = DTYPE_CODE[torch.bfloat16], int(causal), D ** -0.5
+    one, runs = torch.empty_like(tot), torch.empty_like(tot)
+    stream = torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.sage_flash_total_attention(p, L.data_ptr(), one.data_ptr(), stream), "total")
+    need = lib.sage_flash_total_attention_workspace_bytes(p)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=gpu_device)
+    _lib.check(lib.sage_flash_total_attention_ws(p, L.data_ptr(), runs.data_ptr(), ws.data_ptr(), ws.numel(), stream), "total")
+    torch.cuda.synchronize()
+    for got in (one, runs) if where == "normalizer_nan" else (tot, one, runs):
+        assert torch.equal(torch.isnan(got), want) and bool(torch.isfinite(got[~want]).all())
