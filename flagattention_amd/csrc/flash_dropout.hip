@@ -364,7 +364,8 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D) / KG) voi
         m_i = m;
         l_tot = l;
     }
-    const float inv = l_tot > 0.0f ? a.keep_scale / l_tot : 0.0f;  // l = 0: a query that saw no key: zero row
+    // l = 0: a query that saw no key: zero row.  (NaN stays, also where every NaN element of the row was dropped.)
+    const float inv = l_tot != 0.0f ? a.keep_scale / l_tot : 0.0f;
     if (!row_ok) return;
     // accumulator i of tile dt: channel 32 dt + 8 (i / 4) + 4 half + i % 4 of query my_m
     const int64_t obase = (int64_t)b * a.os_b + (int64_t)h * a.os_h + (int64_t)my_m * a.os_n;
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D) / KG) voi
         }
     if (a.log_normalizer && half == 0)
         a.log_normalizer[((int64_t)b * a.Hq + h) * a.M + my_m] =
-            l_tot > 0.0f ? (__builtin_log2f(l_tot) + m_i * a.qk_scale) * 0.693147180559945309f : -INFINITY;
+            l_tot != 0.0f ? (__builtin_log2f(l_tot) + m_i * a.qk_scale) * 0.693147180559945309f : -INFINITY;
 }
 
 __global__ void dropout_mask_kernel(uint8_t* mask, int64_t count, uint64_t offset, uint32_t seed_lo, uint32_t seed_hi,

@@ -38,3 +38,23 @@ def test_dropout_forward_tiles(B, H, Hk, M, N, D, causal, p, offset, gpu_device)
     inf = torch.isinf(L_ref)
     assert torch.equal(torch.isinf(L.cpu()), inf)
     torch.testing.assert_close(L.cpu()[~inf], L_ref[~inf], atol=2e-3, rtol=2e-4)
+
+
+@pytest.mark.parametrize("B,H,M,N,D,causal", [(1, 2, 129, 200, 64, True), (6, 16, 600, 70, 64, False), (1, 2, 100, 97, 128, False), (3, 16, 700, 97, 128, True)])
+@pytest.mark.parametrize("p", [0.3, 0.999])
+def test_dropout_forward_keeps_nan(B, H, M, N, D, causal, p, gpu_device):
+    """The row sums do not see the dropout mask: a NaN score makes its row NaN, output and log normalizer, also where the
+    element is dropped."""
+    import flag_attn
+
+    g = torch.Generator().manual_seed(42)
+    q, k, v = (torch.randn(B, H, n, D, generator=g).to(torch.float16).to(gpu_device) for n in (M, N, N))
+    q[0, 1, M - 2, 3] = float("nan")
+    k[B - 1, 0, N // 2, 1] = float("nan")
+    o, L, *_ = flag_attn.flash_attention(q, k, v, causal, dropout_p=p, return_log_normalizer=True)
+    want = torch.zeros((B, H, M), dtype=torch.bool, device=gpu_device)
+    want[0, 1, M - 2] = True
+    want[B - 1, 0] = torch.arange(M, device=gpu_device) + (N - M) >= N // 2 if causal else True
+    sees = torch.arange(M, device=gpu_device) + (N - M) >= 0 if causal else torch.ones(M, dtype=torch.bool, device=gpu_device)
+    assert torch.equal(torch.isnan(L), want) and torch.equal(torch.isneginf(L), ~sees.expand(B, H, M))
+    assert torch.equal(torch.isnan(o).all(-1), want) and bool(torch.isfinite(o[~want]).all())
