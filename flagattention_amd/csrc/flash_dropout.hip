@@ -18,8 +18,8 @@
 //   each, S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16, V^T by ds_read_b64_tr_b16), one barrier per tile, loads
 //   one tile ahead (a tile takes microseconds), registers for four (head_dim 128: two) waves per SIMD;
 // * workgroups are handed out longest first over all heads.
-// B4 H16 M2048 N2048 D64 fp16 causal 403 -> 164 us, without the causal flag 404 -> 279 us; B2 H32 M4096 N4096 D128 3475 -> 1220
-// us, causal 3445 -> 626 us (before: the generator rolled out by the compiler, V^T gathered from LDS entry by entry,
+// B4 H16 M2048 N2048 D64 fp16 causal 397 -> 143 us, without the causal flag 404 -> 273 us; B2 H32 M4096 N4096 D128 3475 -> 1223
+// us, causal 3445 -> 629 us (before: the generator rolled out by the compiler, V^T gathered from LDS entry by entry,
 // short rows first).  At head_dim 128 three waves per SIMD need 18 spilled registers and run 6 % slower than two.
 #include "attn_common.h"
 
@@ -116,11 +116,14 @@ __device__ __forceinline__ int32_t drop_sign(uint32_t word, int32_t keep_from) {
 
 template <int D> __device__ __forceinline__ int drop_v_swizzle(int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); }
 
-// KG: groups of four waves that share the queries of a workgroup and take its key tiles in turn (drop_groups)
+// KG: groups of four waves that share the queries of a workgroup and take its key tiles in turn (drop_groups).  The second
+// launch bound is waves per SIMD, whatever KG is: with fewer asked for, two groups at head_dim 64 took 132 registers and one
+// workgroup filled a CU (B1 H32 M2048 N2048 D64 153 -> 140 us, causal 107 -> 80 us, B4 H16 M1024 N1024 83 -> 77 and 58 -> 45
+// us; where a lone workgroup of the longest blocks decides, B2 H16 M1500 causal, two spilled registers cost 59 -> 60 us).
 constexpr int drop_waves_per_simd(int head_dim) { return head_dim == 128 ? 2 : 4; }
 
 template <int D, typename VT, int KG>
-__global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D) / KG) void flash_dropout_fwd_kernel(DropArgs a) {
+__global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void flash_dropout_fwd_kernel(DropArgs a) {
     using PVT = PV<VT>;
     using vec16 = typename PVT::vec;
     constexpr int KS = D / 16;      // matrix instructions of one 32 x 32 score tile
@@ -140,8 +143,14 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D) / KG) voi
     // blocks and a CU holds long and short ones: B4 H16 M2048 N2048 D64 causal 177 -> 166 us)
     const int bh = blockIdx.x % a.BH;
     int rank = blockIdx.x / a.BH;
-    if (a.snake > 0 && (rank / a.snake) % 2 == 1 && (rank / a.snake + 1) * a.snake <= a.nmb)
+    if (a.snake > 0 && a.snake < a.nmb && a.nmb < 2 * a.snake) {
+        // a second round on some of the CUs only: these, the first ones, hold the shorter blocks of the first round (in plain
+        // order B2 H16 M1500 N1500 D64 causal, 384 blocks, takes 68 us instead of 60)
+        const int extra = a.nmb - a.snake;
+        rank = rank < extra ? a.snake - extra + rank : rank < a.snake ? rank - extra : a.nmb - 1 - (rank - a.snake);
+    } else if (a.snake > 0 && (rank / a.snake) % 2 == 1 && (rank / a.snake + 1) * a.snake <= a.nmb) {
         rank = (rank / a.snake) * a.snake + a.snake - 1 - rank % a.snake;
+    }
     const int mb = a.nmb - 1 - rank;
     const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.groups;
     const int m0 = mb * (32 * kDropWaves);

@@ -16,6 +16,7 @@ pytestmark = pytest.mark.gpu
     (6, 16, 16, 800, 65, 64, True),    # 672 blocks: one
     (3, 16, 16, 700, 97, 128, True),   # 288 blocks at head_dim 128: one
     (1, 16, 16, 130, 300, 128, False),
+    (1, 24, 8, 1700, 97, 64, True), (1, 20, 20, 1700, 40, 128, True),  # a second round of blocks on some of the CUs
 ])
 def test_dropout_forward_tiles(B, H, Hk, M, N, D, causal, p, offset, gpu_device):
     import flag_attn
