@@ -18,7 +18,7 @@ BLOCK_N = 64  # attn_qk_int8_per_block.py:132
 # Largest staging copy of a bool mask this wrapper makes.  A mask that needs a larger one (a per-head [B, H, M, N]
 # mask with unaligned rows at long sequences) is served by the general kernel as it is, without a copy.
 _STAGED_MASK_MAX_BYTES = 256 << 20
-_STAGED = {}  # device index -> (key, StagedBoolMask): the mask staged last on that device
+_STAGED = {}  # device index -> (key, staged mask, source mask, buffer[, causal mask]) of the mask staged last on that device
 
 
 def _bool_mask_is_direct(m: torch.Tensor, kv_len: int) -> bool:
@@ -51,32 +51,48 @@ def stage_bool_mask(mask, b, h, qo_len, kv_len, causal, device=None):
     the conjunction of the two is what the reference's mask path would be given).  Returns a ``StagedBoolMask``,
     or None when the copy would pass ``_STAGED_MASK_MAX_BYTES``.
 
-    ``forward`` stages on its own and keeps the last staged mask of a device (found again through the source
-    mask's storage address, version counter, shape and strides); a caller that reuses one mask over many calls
-    (all layers of a model) can stage it once here and pass the result as ``attn_mask``.  The copy is enqueued on
-    the current stream, like any torch operation: a call on another stream has to be ordered behind it by the
-    caller."""
+    ``forward`` stages on its own, on every call; a caller that reuses one mask over many calls (all layers of a
+    model) can stage it once here and pass the result as ``attn_mask``.  The copy is enqueued on the current
+    stream, like any torch operation: a call on another stream has to be ordered behind it by the caller."""
+    return _stage_bool(mask, b, h, qo_len, kv_len, causal, device)[0]
+
+
+def _stage_bool(mask, b, h, qo_len, kv_len, causal, device):
+    """(StagedBoolMask, the ``kv_len`` columns of its buffer, the causal mask or None), or Nones above the cap."""
     padded = (kv_len + 15) // 16 * 16
     if mask is None:
         bb, hh, mm = 1, 1, qo_len
     else:
         if mask.dtype != torch.bool:
             raise TypeError(f"stage_bool_mask takes a bool mask, got {mask.dtype}")
-        m4 = mask.reshape((1,) * (4 - mask.dim()) + tuple(mask.shape))
-        bb, hh, mm = m4.shape[0], m4.shape[1], (qo_len if causal else m4.shape[2])
+        bb, hh, mm = ((1,) * (4 - mask.dim()) + tuple(mask.shape))[:3]
+        mm = qo_len if causal else mm
         device = mask.device
     if bb * hh * mm * padded > _STAGED_MASK_MAX_BYTES:
-        return None
-    buf = torch.zeros((bb, hh, mm, padded), dtype=torch.bool, device=device)
-    live = buf[..., :kv_len]
+        return None, None, None
+    with torch.inference_mode(False):  # (the buffer may be filled again outside inference mode)
+        live = torch.zeros((bb, hh, mm, padded), dtype=torch.bool, device=device)[..., :kv_len]
+        seen = None
+        if causal:
+            rows = torch.arange(qo_len, device=device).unsqueeze(1) + (kv_len - qo_len)
+            seen = torch.arange(kv_len, device=device).unsqueeze(0) <= rows
     if mask is not None:
-        live.copy_(m4.expand(bb, hh, mm, kv_len))
+        _fill_staged(live, mask, seen)
+    elif causal:
+        live.copy_(seen)
     else:
         live.fill_(True)
-    if causal:
-        rows = torch.arange(qo_len, device=buf.device).unsqueeze(1) + (kv_len - qo_len)
-        live.logical_and_(torch.arange(kv_len, device=buf.device).unsqueeze(0) <= rows)
-    return StagedBoolMask(live.expand(b, h, qo_len, kv_len), b, h, qo_len, kv_len, causal)
+    return StagedBoolMask(live.expand(b, h, qo_len, kv_len), b, h, qo_len, kv_len, causal), live, seen
+
+
+def _fill_staged(live, mask, seen=None):
+    """Writes the mask's present contents, and ``seen`` where there is a causal mask, into a staging buffer.  One
+    operation: threads that stage the same mask on one stream write the same bytes."""
+    m4 = mask.detach().reshape((1,) * (4 - mask.dim()) + tuple(mask.shape))
+    if seen is None:
+        live.copy_(m4.expand(live.shape))
+    else:
+        torch.logical_and(m4, seen, out=live)
 
 
 def _additive_mask_is_direct(m: torch.Tensor, kv_len: int) -> bool:
@@ -88,48 +104,54 @@ def _additive_mask_is_direct(m: torch.Tensor, kv_len: int) -> bool:
 
 
 def _stage_additive_mask(mask, b, h, qo_len, kv_len):
-    """A copy of an fp16 / bf16 / fp32 additive mask with unit stride along the keys and rows padded (with zeros) to
-    a multiple of 16 bytes, broadcast dimensions kept; None when the copy would pass ``_STAGED_MASK_MAX_BYTES``."""
+    """(a copy of an fp16 / bf16 / fp32 additive mask with unit stride along the keys and rows padded (with zeros) to
+    a multiple of 16 bytes, broadcast dimensions kept; the ``kv_len`` columns of its buffer), or (None, None) when
+    the copy would pass ``_STAGED_MASK_MAX_BYTES``."""
     per16 = 16 // mask.element_size()
     padded = (kv_len + per16 - 1) // per16 * per16
-    m4 = mask.reshape((1,) * (4 - mask.dim()) + tuple(mask.shape))
-    bb, hh, mm = m4.shape[0], m4.shape[1], m4.shape[2]
+    bb, hh, mm = ((1,) * (4 - mask.dim()) + tuple(mask.shape))[:3]
     if bb * hh * mm * padded * mask.element_size() > _STAGED_MASK_MAX_BYTES:
-        return None
-    buf = torch.zeros((bb, hh, mm, padded), dtype=mask.dtype, device=mask.device)
-    live = buf[..., :kv_len]
-    live.copy_(m4.expand(bb, hh, mm, kv_len))
-    return live.expand(b, h, qo_len, kv_len)
+        return None, None
+    with torch.inference_mode(False):
+        live = torch.zeros((bb, hh, mm, padded), dtype=mask.dtype, device=mask.device)[..., :kv_len]
+    _fill_staged(live, mask)
+    return live.expand(b, h, qo_len, kv_len), live
+
+
+# The buffer of the mask staged last on a device is kept for the next call with that mask, its contents are not: they are
+# copied from the mask on every call (an in-place write may leave no trace in the tensor object: through ``.data``, by a
+# replayed graph, through a raw pointer).  What the kept buffer saves is the zero fill of the padding and the causal
+# mask.  The stream is part of the key: the copies and the launches that read the buffer are ordered on one stream.
+# Calls under stream capture neither use nor leave a buffer here (``forward`` decides): a graph owns what it addresses.
+def _mask_key(mask):
+    version = 0 if mask.is_inference() else mask._version  # (inference tensors have no version counter)
+    return mask.data_ptr(), version, tuple(mask.shape), mask.stride(), mask.dtype
 
 
 def _staged_additive_cached(mask, b, h, qo_len, kv_len, device, stream):
-    key = ("additive", mask.data_ptr(), mask._version, tuple(mask.shape), mask.stride(), mask.dtype, b, h, qo_len, kv_len,
-           stream)
+    key = ("additive", _mask_key(mask), b, h, qo_len, kv_len, stream)
     hit = _STAGED.get(device.index)
     if hit is not None and hit[0] == key:
+        _fill_staged(hit[3], mask)
         return hit[1]
-    staged = _stage_additive_mask(mask, b, h, qo_len, kv_len)
+    staged, live = _stage_additive_mask(mask, b, h, qo_len, kv_len)
     if staged is not None:
-        _STAGED[device.index] = (key, staged, mask)
+        _STAGED[device.index] = (key, staged, mask, live)
     return staged
 
 
 def _staged_cached(mask, b, h, qo_len, kv_len, causal, device, stream):
-    """``stage_bool_mask`` behind a one-entry cache per device: the same mask object contents (storage address,
-    version counter: every in-place write bumps it) under the same call shape is not staged again.  The stream is
-    part of the key: the copy was enqueued on the stream that was current then, and only launches on that stream
-    are ordered behind it."""
-    if mask is None:
-        key = (None, b, h, qo_len, kv_len, causal, stream)
-    else:
-        key = (mask.data_ptr(), mask._version, tuple(mask.shape), mask.stride(), b, h, qo_len, kv_len, causal, stream)
+    """``stage_bool_mask`` into a buffer that is kept between calls."""
+    key = (None if mask is None else _mask_key(mask), b, h, qo_len, kv_len, causal, stream)
     hit = _STAGED.get(device.index)
     if hit is not None and hit[0] == key:
+        if mask is not None:  # (the causal mask alone depends on the sizes only)
+            _fill_staged(hit[3], mask, hit[4])
         return hit[1]
-    staged = stage_bool_mask(mask, b, h, qo_len, kv_len, causal, device=device)
+    staged, live, seen = _stage_bool(mask, b, h, qo_len, kv_len, causal, device)
     if staged is not None:
         # (the source mask is kept alive with the entry: its address cannot be handed to another tensor meanwhile)
-        _STAGED[device.index] = (key, staged, mask)
+        _STAGED[device.index] = (key, staged, mask, live, seen)
     return staged
 
 
@@ -234,16 +256,22 @@ def forward(q, k, v, q_scale, k_scale, tensor_layout="HND", attn_mask=None,
         else:
             if attn_mask is not None:
                 require_gpu(attn_mask, "attn_mask")
+
+            def stage(mask):
+                if torch.cuda.is_current_stream_capturing():
+                    return stage_bool_mask(mask, b, h_qo, qo_len, kv_len, causal, device=dev)
+                return _staged_cached(mask, b, h_qo, qo_len, kv_len, causal, dev, stream)
+
             staged = None
             if attn_mask is not None and attn_mask.dtype == torch.bool:
                 # bool masks run on the pipelined kernel; one that it cannot stage as it is (rows that are not 16-byte
                 # aligned, kv_len not a multiple of 16, a causal flag on top) goes there through a padded copy
                 if causal or not _bool_mask_is_direct(attn_mask.expand(b, h_qo, qo_len, kv_len), kv_len):
-                    staged = _staged_cached(attn_mask, b, h_qo, qo_len, kv_len, causal, dev, stream)
+                    staged = stage(attn_mask)
             elif attn_mask is None and causal and qo_len > kv_len:
                 # rows that see no key follow the reference's mask arithmetic (-1e6, whole-tile skip), which the
                 # pipelined kernel implements for mask tensors: hand it the causal mask as one
-                staged = _staged_cached(None, b, h_qo, qo_len, kv_len, True, dev, stream)
+                staged = stage(None)
             if staged is not None:
                 m = staged.tensor
             elif attn_mask is not None:
@@ -260,7 +288,10 @@ def forward(q, k, v, q_scale, k_scale, tensor_layout="HND", attn_mask=None,
                     # additive masks run on the pipelined kernel (no causal flag on top); one whose rows it cannot load
                     # 16 bytes at a time goes there through a padded copy
                     if not causal and not _additive_mask_is_direct(m.expand(b, h_qo, qo_len, kv_len), kv_len):
-                        padded = _staged_additive_cached(m, b, h_qo, qo_len, kv_len, dev, stream)
+                        if torch.cuda.is_current_stream_capturing():
+                            padded, _ = _stage_additive_mask(m, b, h_qo, qo_len, kv_len)
+                        else:
+                            padded = _staged_additive_cached(m, b, h_qo, qo_len, kv_len, dev, stream)
                         if padded is not None:
                             m, mask_kind = padded, padded_kind
                 m = m.expand(b, h_qo, qo_len, kv_len)
