@@ -122,7 +122,9 @@ template <int D> __device__ __forceinline__ int drop_v_swizzle(int row) { return
 // us; where a lone workgroup of the longest blocks decides, B2 H16 M1500 causal, two spilled registers cost 59 -> 60 us).
 constexpr int drop_waves_per_simd(int head_dim) { return head_dim == 128 ? 2 : 4; }
 
-template <int D, typename VT, int KG>
+// WIDE: the rows of a K or V tile lie further apart than 32-bit byte offsets reach, or in descending order (64-bit
+// addresses per lane; one group of waves only).
+template <int D, typename VT, int KG, bool WIDE = false>
 __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void flash_dropout_fwd_kernel(DropArgs a) {
     using PVT = PV<VT>;
     using vec16 = typename PVT::vec;
@@ -203,14 +205,22 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
     set_offsets(kDropKeys - 1);
     auto fetch = [&](int t, int buf) {
         const int n0 = kDropKeys * t;
-        if (n0 + kDropKeys > a.N) set_offsets(a.N - 1 - n0);  // (the last tile)
+        if (!WIDE && n0 + kDropKeys > a.N) set_offsets(a.N - 1 - n0);  // (the last tile)
         const VT* kt = kbase + (int64_t)n0 * a.ks_n;
         const VT* vt = vbase + (int64_t)n0 * a.vs_n;
         const unsigned dst = lds0 + (unsigned)(buf * 2 * TILE + 1024 * LOADS * wave);
 #pragma unroll
         for (int e = 0; e < LOADS; e++) {
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(koff[e]), "s"(kt), "s"(dst + 1024 * e) : "memory");
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff[e]), "s"(vt), "s"(dst + TILE + 1024 * e) : "memory");
+            if constexpr (WIDE) {
+                const int row = (64 / CPR) * (LOADS * wave + e) + lane / CPR, r = min(row, a.N - 1 - n0);
+                const VT* ksrc = kt + (int64_t)r * a.ks_n + 8 * ((lane % CPR) ^ (row & (CPR - 1)));
+                const VT* vsrc = vt + (int64_t)r * a.vs_n + 8 * ((lane % CPR) ^ drop_v_swizzle<D>(row));
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(ksrc), "s"(dst + 1024 * e) : "memory");
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(vsrc), "s"(dst + TILE + 1024 * e) : "memory");
+            } else {
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(koff[e]), "s"(kt), "s"(dst + 1024 * e) : "memory");
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff[e]), "s"(vt), "s"(dst + TILE + 1024 * e) : "memory");
+            }
         }
     };
     int vtr[DT];  // LDS offsets of the transposed fragment reads (see attn_fast_kernel.h)
@@ -419,9 +429,15 @@ template <int D, typename VT>
 int launch_drop(DropArgs a, int64_t B, hipStream_t stream) {
     const int64_t wgs = B * a.Hq * a.nmb;
     if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd_dropout: too many query blocks for one launch");
-    const int groups = drop_groups(wgs, D);
+    auto far = [](int64_t stride) { return stride < 0 || stride >= (1LL << 25); };  // 31 rows of 2-byte elements pass 2^31 bytes
+    const bool wide = far(a.ks_n) || far(a.vs_n);
+    const int groups = wide ? 1 : drop_groups(wgs, D);
     if (a.causal && wgs * groups <= 256 * drop_waves_per_simd(D) && a.BH < 256) a.snake = 256 / a.BH;
     dim3 grid((unsigned)wgs);
+    if (wide) {
+        hipLaunchKernelGGL((flash_dropout_fwd_kernel<D, VT, 1, true>), grid, dim3(kDropThreads), 0, stream, a);
+        return check_launch("flash_dropout_fwd_kernel (wide rows)");
+    }
     if constexpr (D == 64) {
         if (groups == 4) hipLaunchKernelGGL((flash_dropout_fwd_kernel<D, VT, 4>), grid, dim3(4 * kDropThreads), 0, stream, a);
     }
@@ -458,8 +474,6 @@ int launch_flash_dropout(const sage_flash_params& p, float dropout_p, uint64_t s
     }
     a.BH = (int)(p.batch * p.heads_q);
     a.nmb = (a.M + 32 * kDropWaves - 1) / (32 * kDropWaves);
-    if (p.k.stride_n < 0 || p.v.stride_n < 0 || p.k.stride_n >= (1LL << 25) || p.v.stride_n >= (1LL << 25))
-        return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd_dropout: k/v sequence stride out of range for 32-bit tile offsets");
     if (p.head_dim == 128)
         return p.dtype == SAGE_BF16 ? launch_drop<128, __bf16>(a, p.batch, stream) : launch_drop<128, _Float16>(a, p.batch, stream);
     return p.dtype == SAGE_BF16 ? launch_drop<64, __bf16>(a, p.batch, stream) : launch_drop<64, _Float16>(a, p.batch, stream);

@@ -47,7 +47,9 @@ constexpr int kWgKeys = kWaveKeys * kTotalWaves;
 constexpr int kTileQ = 32;
 constexpr int kRing = 4;  // query tiles resident in LDS: the one in work and three on their way
 
-template <int D, typename VT>
+// WIDE: the rows of a query tile lie further apart than 32-bit byte offsets reach, or in descending order (64-bit addresses
+// per lane).
+template <int D, typename VT, bool WIDE>
 __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(TotalArgs a) {
     using PVT = PV<VT>;
     using vec16 = typename PVT::vec;
@@ -95,7 +97,7 @@ __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(Total
     // m0 holds the LDS address of the load; nothing else in this kernel uses it.  Tiles past the last one load it again.
     const unsigned lds_q = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&qtile[0][0];
     const unsigned lds_l = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float*)&ltile[0][0][0];
-    unsigned qoff[LOADS];  // byte offsets of this lane's pieces of a tile (the host has checked that they fit)
+    unsigned qoff[LOADS];  // byte offsets of this lane's pieces of a tile
     auto set_offsets = [&](int last) {  // last: the tile's last row
 #pragma unroll
         for (int e = 0; e < LOADS; e++) {
@@ -106,12 +108,19 @@ __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(Total
     set_offsets(kTileQ - 1);
     auto fetch = [&](int t) {
         const int m0 = m_lo + kTileQ * min(t, ntiles - 1), buf = t & (kRing - 1);
-        if (m0 + kTileQ > a.M) set_offsets(a.M - 1 - m0);  // (every later tile is this one again)
+        if (!WIDE && m0 + kTileQ > a.M) set_offsets(a.M - 1 - m0);  // (every later tile is this one again)
         const unsigned char* base = reinterpret_cast<const unsigned char*>(qbase + (int64_t)m0 * a.qs_n);
 #pragma unroll
-        for (int e = 0; e < LOADS; e++)
-            asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                         :: "v"(qoff[e]), "s"(base), "s"(lds_q + (unsigned)(buf * kTileQ * RS + 1024 * (LOADS * wave + e))) : "memory");
+        for (int e = 0; e < LOADS; e++) {
+            const unsigned dst = lds_q + (unsigned)(buf * kTileQ * RS + 1024 * (LOADS * wave + e));
+            if constexpr (WIDE) {
+                const int row = (64 / CPR) * (LOADS * wave + e) + lane / CPR;
+                const unsigned char* src = base + (int64_t)min(row, a.M - 1 - m0) * (a.qs_n * 2) + 16 * ((lane % CPR) ^ (row & (CPR - 1)));
+                asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(src), "s"(dst) : "memory");
+            } else {
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" :: "v"(qoff[e]), "s"(base), "s"(dst) : "memory");
+            }
+        }
         asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1"
                      :: "v"((unsigned)(4 * min(l32, a.M - 1 - m0))), "s"(lbase + m0), "s"(lds_l + (unsigned)(256 * (kTotalWaves * buf + wave))) : "memory");
     };
@@ -226,7 +235,9 @@ int launch_total(const TotalArgs& a, int64_t B, int runs, hipStream_t stream) {
     const int64_t wgs = (int64_t)((a.N + kWgKeys - 1) / kWgKeys) * runs * B * a.Hq;
     if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_total_attention: too many key blocks for one launch");
     dim3 grid((unsigned)wgs), block(kTotalThreads);
-    hipLaunchKernelGGL((total_attention_kernel<D, VT>), grid, block, 0, stream, a);
+    const bool wide = a.qs_n < 0 || a.qs_n >= (1LL << 25);  // 31 rows of 2-byte elements pass 2^31 bytes
+    if (wide) hipLaunchKernelGGL((total_attention_kernel<D, VT, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((total_attention_kernel<D, VT, false>), grid, block, 0, stream, a);
     return check_launch("total_attention_kernel");
 }
 
@@ -246,8 +257,6 @@ int launch_flash_total_attention(const sage_flash_params& p, const float* log_no
     a.Hq = (int)p.heads_q; a.M = (int)p.qo_len; a.N = (int)p.kv_len; a.groups = (int)(p.heads_q / p.heads_kv);
     a.causal = p.causal ? 1 : 0;
     a.qk_scale = p.sm_scale * 1.44269504089f;
-    if (p.q.stride_n < 0 || p.q.stride_n >= (1LL << 25))
-        return fail(SAGE_E_UNSUPPORTED, "sage_flash_total_attention: q sequence stride out of range for 32-bit tile offsets");
     int runs = workspace ? total_runs(p.batch, p.heads_q, p.qo_len, p.kv_len) : 1;
     if (runs > 1 && workspace_bytes < total_workspace_bytes(p)) runs = 1;
     a.runs = runs;

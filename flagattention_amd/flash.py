@@ -110,10 +110,6 @@ def attention(q, k, v, causal=False, sm_scale=None, dropout_p=0.0,
         # zero channels change neither Q K^T nor the first D columns of P V; sm_scale was fixed above from the true D
         q, k, v = (torch.nn.functional.pad(t, (0, 64 - D)) for t in (q, k, v))
     q, k, v = _rows16(q), _rows16(k), _rows16(v)
-    if return_total_attention and q.stride(2) >= 1 << 25:
-        q = q.contiguous()  # (that kernel reaches the 32 rows of a query tile with 32-bit byte offsets)
-    if is_dropout and max(k.stride(2), v.stride(2)) >= 1 << 25:
-        k, v = k.contiguous(), v.contiguous()  # (the same holds for the key tiles of the dropout kernel)
     o = torch.empty_like(q)  # (the reference allocates the same way, flash.py:84-90)
     if not rows_aligned(o):
         o, call = torch.empty(q.shape, dtype=q.dtype, device=q.device), None

@@ -16,8 +16,8 @@ def test_dropout_kernels_hold_the_waves_their_groups_are_chosen_by():
                           "-target-feature", "-Xclang", "-packed-fp32-ops", "-Rpass-analysis=kernel-resource-usage", "-c",
                           "--cuda-device-only", "-o", os.devnull, os.path.join(CSRC, "flash_dropout.hip")],
                          check=True, capture_output=True, text=True, timeout=600)
-    waves = re.findall(r"Function Name: \S*flash_dropout_fwd_kernelILi(\d+)E\S*Li(\d)EE.*?Occupancy \[waves/SIMD\]: (\d+)", run.stderr, re.S)
-    assert sorted((int(d), int(groups)) for d, groups, _ in waves) == [(64, 1), (64, 1), (64, 2), (64, 2), (64, 4), (64, 4),
-                                                                       (128, 1), (128, 1), (128, 2), (128, 2)]
-    for d, groups, n in waves:
-        assert int(n) >= (4 if d == "64" else 2), (d, groups, n)
+    waves = re.findall(r"Function Name: \S*flash_dropout_fwd_kernelILi(\d+)E\S*Li(\d)ELb([01])EE.*?Occupancy \[waves/SIMD\]: (\d+)", run.stderr, re.S)
+    assert {(int(d), int(groups), int(wide)) for d, groups, wide, _ in waves} == {
+        (64, 1, 0), (64, 2, 0), (64, 4, 0), (64, 1, 1), (128, 1, 0), (128, 2, 0), (128, 1, 1)}
+    for d, groups, wide, n in waves:
+        assert int(n) >= (4 if d == "64" else 2), (d, groups, wide, n)
