@@ -28,7 +28,7 @@
 
 namespace {
 
-constexpr size_t kMaxPlans = 64;
+constexpr size_t kMaxPlans = 64;  // of a thread
 
 // The key of a call: its integers as bytes.
 struct Key {
@@ -55,12 +55,26 @@ struct Plan {
     bool fused = false;      // (quantizer) sage_smooth_quant_params
 };
 
-// One table per thread: a parameter struct is written by one thread at a time.  Cleared when full.
-thread_local std::unordered_map<std::string, Plan> t_plans;
+// Tables of one thread: a parameter struct is written by one thread at a time.  A plan that is used lies in the young table;
+// when that is full it becomes the old one, whose plans go unless they are used before the next time.  So sizes that come
+// once (the keys of a growing cache) do not push out those that return.
+typedef std::unordered_map<std::string, Plan> Table;
+thread_local Table t_young, t_old;
+
+void make_room() {
+    if (t_young.size() < kMaxPlans / 2) return;
+    t_old.swap(t_young);
+    t_young.clear();
+}
 
 Plan* find(const Key& k) {
-    auto it = t_plans.find(k.bytes);
-    return it == t_plans.end() ? nullptr : &it->second;
+    auto it = t_young.find(k.bytes);
+    if (it != t_young.end()) return &it->second;
+    it = t_old.find(k.bytes);
+    if (it == t_old.end()) return nullptr;
+    auto node = t_old.extract(it);
+    make_room();
+    return &t_young.insert(std::move(node)).position->second;
 }
 
 // Scratch memory of one call: from the caching allocator, which gives it to the next call on this stream once the launches
@@ -132,8 +146,8 @@ PyObject* put(const Key& key, PyObject* params, PyObject* ws, bool fused) {
     plan.workspace = PyLong_AsLongLong(ws);
     if (PyErr_Occurred()) return nullptr;
     plan.fused = fused;
-    if (t_plans.size() >= kMaxPlans) t_plans.clear();
-    t_plans[key.bytes] = std::move(plan);
+    make_room();
+    t_young[key.bytes] = std::move(plan);
     return none();
 }
 

@@ -133,3 +133,20 @@ def test_a_captured_graph_owns_its_scratch_memory(gpu_device, first):
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(captured, want)), f"replay {rep}"
         assert all(bool((t == 7).all()) for t in kept), f"replay {rep} wrote to another tensor"
+
+
+def test_shapes_that_return_stay_known(gpu_device):
+    """A hundred shapes that come once each, as the keys of a growing cache do, do not push out the plan of a shape that is
+    used between them; plans that are not used go."""
+    import flag_attn
+    from flagattention_amd import _lib
+
+    host = _lib.host()
+    q, k, v = _qkv(9, gpu_device, m=1, n=400)
+    kept, first = (q, k[:, :, :290], v[:, :, :290]), (q, k[:, :, :300], v[:, :, :300])
+    flag_attn.flash_attention(*kept)
+    for n in range(300, 400):
+        flag_attn.flash_attention(q, k[:, :, :n], v[:, :, :n])
+        assert host.flash(*kept, False, None, False) is not None, n
+    assert host.flash(q, k[:, :, :399], v[:, :, :399], False, None, False) is not None
+    assert host.flash(*first, False, None, False) is None
