@@ -3,6 +3,9 @@ from __future__ import annotations
 
 import ctypes
 import os
+import warnings
+
+import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsage_attention_hip.so")
@@ -150,16 +153,36 @@ def load():
 _host_module = None
 
 
+class _PythonHost:
+    """Knows no call shape: every call takes the checks and the parameter structs of the Python side."""
+
+    @staticmethod
+    def quant(*call):
+        return None
+
+    attn = flash = put_quant = put_attn = put_flash = quant
+
+
 def host():
-    """The native host side of calls whose shape has been seen before (csrc/host.cpp), or raises: it is built with the
-    library."""
+    """The native host side of calls whose shape has been seen before (csrc/host.cpp).  It is built with the library and
+    raises where it was not.  A module that was built against another torch costs host time only: the Python side, which
+    needs nothing but the C library, then serves every call."""
     global _host_module
     if _host_module is None:
+        problem = None
         try:
             from . import _host as module
+            if module.torch_version != torch.__version__.split("+")[0]:
+                problem = f"was built against torch {module.torch_version}, this is {torch.__version__}"
         except ImportError as e:
-            raise ImportError("flagattention_amd/_host.so is missing or does not load: build it with "
-                              f"`make -C flagattention_amd/csrc` ({e})") from e
+            if not os.path.exists(os.path.join(_HERE, "_host.so")):
+                raise ImportError("flagattention_amd/_host.so is missing: build it with "
+                                  f"`make -C flagattention_amd/csrc` ({e})") from e
+            problem = f"does not load ({e})"
+        if problem is not None:
+            warnings.warn(f"flagattention_amd/_host.so {problem}: calls are prepared in Python, which takes about 10 us more "
+                          "each; build it again with `make -C flagattention_amd/csrc`", RuntimeWarning, stacklevel=3)
+            module = _PythonHost
         _host_module = module
     return _host_module
 

@@ -347,3 +347,32 @@ def test_torch_library_operators_have_shape_functions():
         assert tuple(lse.shape) == (2, 4, 300) and lse.dtype == torch.float32
         o, lse = ops.sage_attention_forward(q8, k8, k, qs, ks, "NHD")
         assert o.dtype == torch.float16 and tuple(lse.shape) == (0,) and lse.device.type == "cpu"
+
+
+def test_a_host_module_of_another_torch_leaves_the_python_side(monkeypatch):
+    """_host.so that does not load, or that another torch was built with: a warning, and every call goes to the Python side.
+    A missing one raises."""
+    import sys
+    import types
+
+    import flagattention_amd
+    from flagattention_amd import _lib
+
+    assert _lib.host().torch_version  # (the built one)
+    for module in (None, types.SimpleNamespace(torch_version="1.0.0")):
+        monkeypatch.setattr(_lib, "_host_module", None)
+        monkeypatch.delattr(flagattention_amd, "_host", raising=False)
+        monkeypatch.setitem(sys.modules, "flagattention_amd._host", module)
+        if module is not None:
+            monkeypatch.setattr(flagattention_amd, "_host", module, raising=False)
+        with pytest.warns(RuntimeWarning, match="prepared in Python"):
+            host = _lib.host()
+        assert _lib.host() is host  # (one warning)
+        assert host.quant(1, 2) is None and host.attn() is None and host.flash() is None
+        assert host.put_quant(1) is None and host.put_attn() is None and host.put_flash() is None
+    monkeypatch.setattr(_lib, "_host_module", None)
+    monkeypatch.delattr(flagattention_amd, "_host", raising=False)
+    monkeypatch.setitem(sys.modules, "flagattention_amd._host", None)
+    monkeypatch.setattr(_lib, "_HERE", "/nonexistent")
+    with pytest.raises(ImportError, match="missing"):
+        _lib.host()

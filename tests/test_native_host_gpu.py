@@ -150,3 +150,18 @@ def test_shapes_that_return_stay_known(gpu_device):
         assert host.flash(*kept, False, None, False) is not None, n
     assert host.flash(q, k[:, :, :399], v[:, :, :399], False, None, False) is not None
     assert host.flash(*first, False, None, False) is None
+
+
+def test_the_python_side_alone_gives_the_same_results(gpu_device, monkeypatch):
+    import flag_attn
+    from flag_attn import sage_attention as sa
+    from flagattention_amd import _lib
+
+    mask = torch.rand(1, 1, 77, 128, generator=torch.Generator().manual_seed(1)).to(gpu_device) > 0.3
+    q, k, v = _qkv(10, gpu_device, n=128)
+    for _ in range(2):
+        want = _calls(sa, flag_attn, q, k, v, mask)
+    monkeypatch.setattr(_lib, "_host_module", _lib._PythonHost)
+    for _ in range(2):
+        got = _calls(sa, flag_attn, q, k, v, mask)
+        assert all(x.shape == y.shape and x.stride() == y.stride() and torch.equal(x, y) for x, y in zip(want, got))
