@@ -306,14 +306,14 @@ def test_benchmark_rows_record_format(tmp_path, monkeypatch):
 
 @pytest.mark.skipif(not os.path.exists("/opt/rocm/bin/hipcc"), reason="needs hipcc")
 def test_only_the_lds_load_sequence_touches_m0(tmp_path):
-    """The pipelined attention kernel sets m0 in inline assembly, which the compiler cannot be told about.  Compile
-    its translation units to assembly and check that m0 appears nowhere else: only as the destination of the
-    s_mov_b32 that precedes each direct-to-LDS load."""
+    """The pipelined attention kernel, the dropout forward and the total attention set m0 in inline assembly, which the
+    compiler cannot be told about.  Compile their translation units to assembly and check that m0 appears nowhere else:
+    only as the destination of the s_mov_b32 that precedes each direct-to-LDS load."""
     import re
     import subprocess
 
     csrc = os.path.join(ROOT, "flagattention_amd", "csrc")
-    for unit in ("attn_fwd_fast.hip", "attn_fwd_fast_addmask.hip", "flash_fwd.hip"):
+    for unit in ("attn_fwd_fast.hip", "attn_fwd_fast_addmask.hip", "flash_fwd.hip", "flash_dropout.hip", "total_attention.hip"):
         out = tmp_path / (unit + ".s")
         subprocess.run(["/opt/rocm/bin/hipcc", "-O3", "-std=c++17", "--offload-arch=gfx950", "-ffp-contract=off", "-Xclang",
                         "-target-feature", "-Xclang", "-packed-fp32-ops", "-S", "--cuda-device-only", "-o", str(out),
@@ -322,8 +322,12 @@ def test_only_the_lds_load_sequence_touches_m0(tmp_path):
         assert mentions, "expected the direct-to-LDS load sequence in " + unit
         other = [ln for ln in mentions if not re.fullmatch(r"s_mov_b32 m0, s\d+", ln)]
         assert not other, other[:5]
-        loads = sum(1 for ln in out.read_text().splitlines() if ln.strip().startswith("global_load_lds_dwordx4"))
-        assert loads == len(mentions)
+        lines = [ln.split(";")[0].split() for ln in out.read_text().splitlines()]
+        lines = [ln for ln in lines if ln and not ln[0].startswith((".", "s_nop"))]
+        loads = [i for i, ln in enumerate(lines) if ln[0].startswith("global_load_lds_")]
+        assert len(loads) == len(mentions)
+        for i in loads:  # each load behind a write of its own
+            assert lines[i - 1][0] == "s_mov_b32" and lines[i - 1][1] == "m0,", lines[i - 2:i + 1]
 
 
 def test_torch_library_operators_have_shape_functions():

@@ -1,5 +1,5 @@
 """The quantizer's fused launches at their edges, bit for bit against the oracle: one workgroup per head (up to 256 keys at
-head_dim 128, 512 at 64), K blocks that add the chunk partials of the mean themselves (up to 16 chunks), K and Q blocks in one
+head_dim 128, 512 at 64), K blocks that add the chunk partials of the mean themselves (up to 32 chunks), K and Q blocks in one
 grid, and the sizes just beyond each."""
 import pytest
 import torch
