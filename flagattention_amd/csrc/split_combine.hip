@@ -111,7 +111,8 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineA
 
 // One wave tile (32 rows) of one item of a cut launch: the parts lie in the order of the accumulator registers, so a
 // thread adds up four-channel pieces of one row; the sum is turned through LDS and written as whole rows.  Bound by the
-// bytes of the parts: 67 MB at head_dim 128 when every share leaves two, 11.5 us (5.8 TB/s).
+// bytes of the parts: 67 MB at head_dim 128 when every share leaves two, 11.5 us (5.8 TB/s).  With fewer items to combine
+// (64 of them from 288 parts, 38 MB) a quarter of the workgroups have work, and it takes 11 to 13 us (about 3 TB/s).
 template <int D>
 __global__ __launch_bounds__(kCombineThreads) void cut_combine_kernel(AttnArgs a) {
     constexpr int kPieces = 32 * D / 4 / kCombineThreads;  // per thread: 4 | 2
