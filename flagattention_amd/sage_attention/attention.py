@@ -88,11 +88,12 @@ def _stage_bool(mask, b, h, qo_len, kv_len, causal, device):
 def _fill_staged(live, mask, seen=None):
     """Writes the mask's present contents, and ``seen`` where there is a causal mask, into a staging buffer.  One
     operation: threads that stage the same mask on one stream write the same bytes."""
-    m4 = mask.detach().reshape((1,) * (4 - mask.dim()) + tuple(mask.shape))
+    if mask.requires_grad:
+        mask = mask.detach()
     if seen is None:
-        live.copy_(m4.expand(live.shape))
+        live.copy_(mask)  # (broadcasts)
     else:
-        torch.logical_and(m4, seen, out=live)
+        torch.logical_and(mask if mask.dim() == 4 else mask.reshape((1,) * (4 - mask.dim()) + tuple(mask.shape)), seen, out=live)
 
 
 def _additive_mask_is_direct(m: torch.Tensor, kv_len: int) -> bool:
