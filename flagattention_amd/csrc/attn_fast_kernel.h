@@ -774,7 +774,8 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                         pf[tp][2 * w + 1] = (VT)__builtin_amdgcn_exp2f(as_f(b1) - m_i);
                         lsum = PVT::dot2_ones(pf[tp], w, lsum);
                     });
-                    lsum = __builtin_fmaf(past_end, __builtin_amdgcn_exp2f(kMaskedScore - m_i), lsum);
+                    // (a row that has seen hidden keys only keeps the reference point -1e30: 0 times the infinite term is NaN)
+                    if (past_end > 0.0f) lsum = __builtin_fmaf(past_end, __builtin_amdgcn_exp2f(kMaskedScore - m_i), lsum);
                 }
                 return;
             }

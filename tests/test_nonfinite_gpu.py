@@ -1,6 +1,7 @@
 """A NaN or an infinity in Q or K makes the rows that see it NaN, output and log-sum-exp alike, whether a launch is whole or
 leaves partial results in a workspace that a second kernel combines."""
 import ctypes
+import math
 
 import pytest
 import torch
@@ -123,3 +124,28 @@ def test_quantized_rows(b, h, hkv, m, n, d, causal, where, gpu_device):
         _launch(lib, "attn_fwd", p, workspace, gpu_device)
         results.append((o, lse))
     _check(results, want, empty)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("mask_dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_additive_mask_rows_that_meet_hidden_tiles_first(mask_dtype, d, gpu_device):
+    """A sliding window as an additive mask of the type's lowest value: the first tiles hide every key of a row while other
+    rows of its wave already see some."""
+    from flag_attn import sage_attention as sa
+    from oracle import sage_oracle as O
+
+    g = torch.Generator().manual_seed(5)
+    n = 768
+    q, k, v = (torch.randn(1, 2, n, d, generator=g).to(torch.bfloat16) for _ in range(3))
+    q8, qs, k8, ks = O.per_block_int8(q, k)
+    rows, cols = torch.arange(n).view(n, 1), torch.arange(n)
+    keep = ((cols <= rows) & (cols > rows - 100)).view(1, 1, n, n)
+    mask = torch.zeros(keep.shape, dtype=mask_dtype).masked_fill_(~keep, torch.finfo(mask_dtype).min)
+    o, lse = sa.sage_attention(*(t.to(gpu_device) for t in (q8, k8, v, qs, ks)), attn_mask=mask.to(gpu_device), return_lse=True)
+    # (float64: hidden scores lie beyond the exponent's range there too)
+    sc = qs.double().repeat_interleave(128, -1)[..., :n, None] * ks.double().repeat_interleave(64, -1)[..., None, :n]
+    s = (q8.double() @ k8.double().transpose(-1, -2)) * sc
+    s = s.masked_fill(~keep, float("-inf"))
+    want = torch.softmax(s * math.log(2.0), -1) @ v.double()
+    torch.testing.assert_close(o.double().cpu(), want, rtol=2e-2, atol=2e-2)
+    torch.testing.assert_close(lse.double().cpu(), torch.logsumexp(s * math.log(2.0), -1) / math.log(2.0), rtol=1e-4, atol=2e-3)
