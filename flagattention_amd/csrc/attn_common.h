@@ -25,6 +25,7 @@ constexpr int kThreads = 256;
 constexpr int BM = 128;  // query rows per workgroup (= Q quantization block)
 constexpr int BN = 64;   // keys per step (= K quantization block)
 constexpr int kFastRows = 256;  // query rows per workgroup of the pipelined kernel (attn_fast_kernel.h)
+constexpr int kScanRows = 16;  // mask rows per strip of mask_scan_kernel
 constexpr float kMasked = -1.0e6f;
 constexpr float kTau = 8.0f;  // log2 of the largest P tolerated before the running maximum is advanced
 
@@ -68,6 +69,13 @@ struct AttnArgs {
     float* part_o;     // [2 * cut_wgs slots][256 rows x D, in the order of the accumulator registers]
     float* part_lse;   // [2 * cut_wgs][256]
     float lse_mul;     // factor on the base-2 log-sum-exp on its way out (1: as is; ln 2: natural log)
+    // (mask tensors, pipelined kernel) what mask_scan_kernel found (null: every tile is visited): per strip of kScanRows mask
+    // rows and 64-key tile the largest entry, per strip the smallest of its rows' largest entries, per 64-key tile of V
+    // whether it holds an Inf or NaN.  scan_strips: strips of a mask batch.  visit_group: tiles per bit of the visit word.
+    const float* scan_top;  // [mask batches][scan_strips][nk]
+    const float* scan_low;  // [mask batches][scan_strips]
+    const unsigned* scan_v; // [B][Hkv][nk]
+    int32_t scan_strips, visit_group;
     float qk_scale;    // 16-bit Q and K only: sm_scale * log2(e), the one scale of every score (q/k point at 16-bit data)
 };
 
@@ -180,6 +188,11 @@ int launch_decode(const AttnArgs& a, int64_t batch, int head_dim, int v_dtype, b
 bool fast_serves_mask(const AttnArgs& a, int esz);
 int launch_fast_masked(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
 int launch_fast_additive(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
+
+// The scan of a mask that the heads share, ahead of the pipelined kernel (mask_scan.hip): bytes of workspace it takes (0: the
+// rule on sizes says no), and its launch, which fills the scan fields of `a`.
+int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch);
+int launch_mask_scan(AttnArgs& a, int64_t batch, int head_dim, int v_dtype, void* workspace, hipStream_t stream);
 
 // The pipelined kernel on 16-bit Q and K (dense attention); causal with any qo_len / kv_len.
 int launch_flash(const AttnArgs& a, int head_dim, int dtype, bool causal, hipStream_t stream);

@@ -166,7 +166,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     // (1.35x the K/V bytes from memory at 8192 keys).
     int wg = blockIdx.x;
     if ((a.total_wg & 7) == 0) wg = (wg & 7) * (a.total_wg >> 3) + (wg >> 3);
-    const bool paired = CAUSAL && !CUT && a.causal && !a.longest_first;
+    const bool paired = CAUSAL && !CUT && !MASK && a.causal && !a.longest_first;
     const int per_head = paired ? (nq2 + 1) / 2 : nq2;  // workgroups per (batch, head)
     // The keys of one (batch, head, q-block) may be split over `nsplit` workgroups (never under a mask tensor).  A
     // workgroup then sees the problem that starts at its first key: kv_len, the number of tiles and the causal
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     int jq = (item0 / ht) % per_head;
     int h0 = (item0 / (ht * per_head)) % (a.Hq / ht) * ht + item0 % ht;
     int b0 = item0 / (per_head * a.Hq);
-    if (CAUSAL && !CUT && !MASK && a.longest_first) {  // the heads of an XCD take turns, q-block after q-block from the last one
+    if (CAUSAL && !CUT && a.longest_first) {  // the heads of an XCD take turns, q-block after q-block from the last one
         const int heads = a.total_wg / nq2, xcds = heads & 7 ? 1 : 8;
         const int i = blockIdx.x / xcds, own = heads / xcds, bh = blockIdx.x % xcds * own + i % own;
         jq = nq2 - 1 - i / own;
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     if constexpr (CUT) asm volatile("" : "+s"(args_again));
     const AttnArgs& a = CUT ? *(const AttnArgs*)args_again : args;
     int b = b0, h = h0, step0 = split * a.split_steps, cut_steps = 0;  // step0: first step of this workgroup's share of the keys
-    int iq = (paired && pass == 1) || (MASK && a.mask_causal) ? nq2 - 1 - jq : jq;  // (a mask with the causal mask folded in: no pairs, the q-blocks with the most tiles are handed out first)
+    int iq = (paired && pass == 1) || (MASK && a.mask_causal && !a.longest_first) ? nq2 - 1 - jq : jq;  // (a mask with the causal mask folded in: no pairs, the q-blocks with the most tiles are handed out first)
     bool partial = false;  // (CUT) the item has steps in other workgroups too
     if constexpr (CUT) {
         const CutLine line(a.M, a.N, CAUSAL && a.causal);
@@ -415,6 +415,70 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         }
         return __builtin_amdgcn_ballot_w64(any != 0) != 0;
     };
+    // ---- (MASK) the tiles this workgroup visits.  Bit g of `visits` stands for tiles g * visit_group .. of the walk
+    //      over the keys (visit_group = 1 up to 4096 keys); clear where mask_scan_kernel found that a visit changes nothing:
+    //      an additive entry so far below the largest one of every row that its P is exactly 0 whatever the scores
+    //      (|q.k| <= 2^14 D and the scales bound them), a bool tile without a visible key (the reference skips it), and no
+    //      Inf or NaN in V (0 times those is NaN).  Comparisons with a NaN scale or entry are false: such a tile is visited.
+    unsigned long long visits = ~0ull;
+    int visit_group = 1, visit_g = 0, visit_rest = 0;  // tiles per bit; the bit of the youngest tile below, the tile within it
+    // (k_at / v_at below hide the tiles' addresses from the compiler: known as base + tile * bytes they end in vector registers,
+    // 180 of which the instances at head_dim 128 then spill)
+    int vt0 = 0, vt1 = 0, vt2 = 0, vt3 = 0;  // tiles of this step and the next three (the last one again past the end)
+    auto next_tile = [&](int t, bool more) {  // the tile visited after t, t itself if there are no more (no branch: this runs in the step loop)
+        const bool same = visit_rest + 1 < visit_group;
+        const int g = visit_g + 1 + __builtin_ctzll((visits >> visit_g) >> 1 | 1ull << 63);
+        const int next = same ? t + 1 : g * visit_group;
+        visit_rest = !more ? visit_rest : same ? visit_rest + 1 : 0;
+        visit_g = more && !same ? g : visit_g;
+        return more ? next : t;
+    };
+    if constexpr (MASK) {
+        visit_group = a.visit_group;
+        const int groups = (nsteps + visit_group - 1) / visit_group;
+        if (a.scan_top) {
+            const int mb = a.ms_b ? b : 0;
+            const int s0 = a.ms_m ? (kFastRows / kScanRows) * iq : 0, s1 = min(s0 + kFastRows / kScanRows, a.scan_strips);
+            const float* tops = a.scan_top + (int64_t)mb * a.scan_strips * a.nk;
+            float low = a.scan_low[(int64_t)mb * a.scan_strips + min(s0 + (lane & (kFastRows / kScanRows - 1)), s1 - 1)];
+#pragma unroll
+            for (int x = 1; x < kFastRows / kScanRows; x <<= 1) low = fminf(low, __shfl_xor(low, x));
+            const int64_t kv_row = ((int64_t)b * a.Hkv + hk) * a.nk;
+            float top = -INFINITY, ks_max = 0.0f;
+            bool odd = false;
+            for (int r = 0; r < visit_group; r++) {
+                const int t = min(lane * visit_group + r, a.nk - 1);
+                const float ks = a.k_scale[kv_row + t];
+                odd |= !(ks < 3.0e38f) || a.scan_v[kv_row + t] != 0;
+                ks_max = fmaxf(ks_max, ks);
+                float e[kFastRows / kScanRows];
+#pragma unroll
+                for (int x = 0; x < kFastRows / kScanRows; x++) e[x] = tops[(int64_t)min(s0 + x, s1 - 1) * a.nk + t];
+#pragma unroll
+                for (int x = 0; x < kFastRows / kScanRows; x++) top = fmaxf(top, e[x]);
+            }
+#pragma unroll
+            for (int x = 1; x < 64; x <<= 1) ks_max = fmaxf(ks_max, __shfl_xor(ks_max, x));
+            const float* qsp = a.q_scale + ((int64_t)b * a.Hq + h) * a.nq;
+            const float bound = MADD ? 2.0f * 16384.0f * D * ks_max : 0.0f;  // 2 max |q.k| over the Q scale
+            const float q0 = qsp[min((kFastRows / BM) * iq, a.nq - 1)], q1 = qsp[min((kFastRows / BM) * iq + 1, a.nq - 1)];
+            const bool skip = top < low - 150.0f - bound * q0 && top < low - 150.0f - bound * q1 && !odd;
+            visits = ~__builtin_amdgcn_ballot_w64(skip);
+            asm volatile("" : "+s"(visits));
+        }
+        if (groups < 64) visits &= (1ull << groups) - 1;
+        if (nsteps > 0) {
+            const bool last_group = (visits >> (groups - 1)) & 1;
+            nsteps = __builtin_popcountll(visits) * visit_group - (last_group ? groups * visit_group - nsteps : 0);
+        }
+        if (nsteps > 0) {
+            visit_g = __builtin_ctzll(visits);
+            vt0 = visit_g * visit_group;
+            vt1 = next_tile(vt0, nsteps > 1);
+            vt2 = next_tile(vt1, nsteps > 2);
+            vt3 = next_tile(vt2, nsteps > 3);
+        }
+    }
     // ---- fragment read offsets (undoing the swizzle)
     // K: lane (row l32, half) reads chunk half * K_RS/32 + t of its row for k-step t
     int kf_off[F::KSTEPS];
@@ -533,24 +597,30 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     const unsigned char* k_fetch = reinterpret_cast<const unsigned char*>(kg);
     const unsigned char* v_fetch = reinterpret_cast<const unsigned char*>(vg);
     int k_tile = 0, v_tile = 0;  // indices of the tiles behind k_fetch / v_fetch
+    auto k_at = [&](int t) { k_tile = t; k_fetch = reinterpret_cast<const unsigned char*>(kg) + t * k_tile_bytes; asm volatile("" : "+s"(k_fetch)); };  // (MASK)
+    auto v_at = [&](int t) { v_tile = t; v_fetch = reinterpret_cast<const unsigned char*>(vg) + t * v_tile_bytes; asm volatile("" : "+s"(v_fetch)); };
+    if constexpr (MASK) { k_at(vt0); v_at(vt0); }
     sfor<NDMA_KV>([&](auto ec) { dma_unit(ec, IC<1>{}, 0, k_fetch, k_tile, 0, v_fetch, v_tile); });
-    if (nsteps > 1) { k_fetch += k_tile_bytes; v_fetch += v_tile_bytes; k_tile++; v_tile++; }
+    if constexpr (MASK) { k_at(vt1); v_at(vt1); }
+    else if (nsteps > 1) { k_fetch += k_tile_bytes; v_fetch += v_tile_bytes; k_tile++; v_tile++; }
     sfor<NDMA_KV>([&](auto ec) { dma_unit(ec, IC<1>{}, 1, k_fetch, k_tile, 1, v_fetch, v_tile); });
-    if (nsteps > 2) { k_fetch += k_tile_bytes; v_fetch += v_tile_bytes; k_tile++; v_tile++; }
+    if constexpr (MASK) { k_at(vt2); v_at(vt2); }
+    else if (nsteps > 2) { k_fetch += k_tile_bytes; v_fetch += v_tile_bytes; k_tile++; v_tile++; }
     sfor<F::NK>([&](auto ec) { dma_unit(ec, IC<1>{}, 2, k_fetch, k_tile, 2, v_fetch, v_tile); });
     // from here on k_fetch / v_fetch point at the tiles fetched during step 0: K of step 3, V of step 2
-    if (nsteps > 3) { k_fetch += k_tile_bytes; k_tile++; }
-    dma_mask(0, 0);
-    if constexpr (kMaskSlots == 3) dma_mask(max(min(1, nsteps - 1), 0), 1);  // (nsteps = 0: a workgroup that sees no key; tile 0 exists all the same)
+    if constexpr (MASK) k_at(vt3);
+    else if (nsteps > 3) { k_fetch += k_tile_bytes; k_tile++; }
+    dma_mask(vt0, 0);  // (nsteps = 0: a workgroup that sees no key; tile 0 exists all the same)
+    if constexpr (kMaskSlots == 3) dma_mask(vt1, 1);
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the direct-to-LDS loads have landed
     __syncthreads();
     sbuf[0][0] = qk_tile(smem, 0);
     sbuf[0][1] = qk_tile(smem, 1);
-    sc = step_scale(0, true);
+    sc = step_scale(vt0, true);
     {   // the row maximum of the first tile is the reference point the row starts from
         float raw_max = -INFINITY;
-        const bool masked0 = CAUSAL && (BN - 1 > wlim);
-        sfor<8>([&](auto uc) { head_unit(IC<0>{}, uc, 0, masked0, raw_max); });
+        const bool masked0 = CAUSAL && (vt0 * BN + BN - 1 > wlim);
+        sfor<8>([&](auto uc) { head_unit(IC<0>{}, uc, vt0 * BN, masked0, raw_max); });
         // (a row that sees no key at all, qo_len > kv_len under the causal flag, keeps a finite reference
         // point: its exponentials are then exp2(-inf) = 0 and it ends with l = 0)
         m_i = fmaxf((row_pair_max(raw_max) - BIAS) * sc, -1.0e30f);
@@ -618,7 +688,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             const unsigned char* p0 = smem + vaddr[j % F::DTILES] + 16 * (j / F::DTILES) * F::V_RS;
             vfr[j] = tr_pair<VT>(p0, p0 + 8 * F::V_RS);
         };
-        const int n0 = step * BN;
+        const int n0 = (MASK ? vt0 : step) * BN, n0_next = (MASK ? vt1 : step + 1) * BN;  // first keys of this step and the next
         const bool live = step < nsteps;  // false only for the padding step after an odd number of steps
 
         // ===== VALU phase: exponentials of this step (scores in sbuf[P]) =====
@@ -645,9 +715,9 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         const int mslot_next = mslot == kMaskSlots - 1 ? 0 : mslot + 1;
         // (additive: the entries of step + 1, into the slot that step - 1 left; ahead of the K/V loads, because they
         // are the ones waited for first: at the end of the coming matrix phase)
-        if constexpr (MADD && !MF32) dma_mask(min(step + 1, nsteps - 1), mslot_next);
+        if constexpr (MADD && !MF32) dma_mask(vt1, mslot_next);
         sfor<NDMA_KV>([&](auto ec) { dma_unit(ec, IC<HIDES>{}, (step + 3) & 3, k_fetch, k_tile, (step + 2) & 3, v_fetch, v_tile); });
-        if constexpr (MASK && !MADD) dma_mask(min(step + 2, nsteps - 1), mslot_next == kMaskSlots - 1 ? 0 : mslot_next + 1);  // the mask bytes of step + 2
+        if constexpr (MASK && !MADD) dma_mask(vt2, mslot_next == kMaskSlots - 1 ? 0 : mslot_next + 1);  // the mask bytes of step + 2
         vec16 pf[4];
         float lsum = 0.0f;
         const float sc_e = sc;  // this step's scale (sc moves on to the next step below)
@@ -705,7 +775,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             lsum = PVT::dot2_ones(pf[3], 3, lsum);
         }
         // (fp32 mask entries: the last one of this step has been read; the one slot takes those of the next step)
-        if constexpr (MF32) dma_mask(min(step + 1, nsteps - 1), 0);
+        if constexpr (MF32) dma_mask(vt1, 0);
         // A lane's 32 P of a step sum to less than kSumLimit, or the step is redone: so no P overflows the
         // 16-bit type (nor does a sum or a product with V come near the fp32 range), and a row whose scores
         // rise keeps its reference point within log2(kSumLimit) of its maximum.  Wave-wide decision; rare
@@ -724,7 +794,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             if constexpr (MADD) {
                 // a ragged last tile always comes here: its keys past kv_len score -1e6 (the reference reads their
                 // mask entries as -1e6 and their K as zeros), which only this path accounts for
-                if (large != 0 || (ragged && step == nk - 1)) {
+                if (large != 0 || (ragged && live && vt0 == nk - 1)) {
                     float raw = -INFINITY;
                     float past_end = 0.0f;  // number of the lane's keys of this step that lie past kv_len
                     sfor<4>([&](auto tc) {
@@ -866,7 +936,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             }
         };
         if constexpr (kSumsEarly) large = __builtin_amdgcn_ballot_w64(!(lsum < kSumLimit));
-        sc = step_scale(min(step + 1, nsteps - 1), HIDES);
+        sc = step_scale(MASK ? vt1 : min(step + 1, nsteps - 1), HIDES);
         __builtin_amdgcn_sched_barrier(0);
         // The first K fragments of the coming MFMA phase are requested before the barrier (their tile
         // landed a step ago), so the phase does not open with an LDS round trip.
@@ -880,7 +950,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
 
         // ===== MFMA phase =====
         __builtin_amdgcn_s_setprio(1);
-        const bool masked_n = HIDES && (n0 + 2 * BN - 1 > wlim);
+        const bool masked_n = HIDES && (n0_next + BN - 1 > wlim);
         sfor<NSLOTS>([&](auto ic) {
             constexpr int i = decltype(ic)::value;
             if constexpr (i < QK_SLOTS) {
@@ -932,7 +1002,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                         constexpr int u = j * (8 / PV_SLOTS + (8 % PV_SLOTS != 0)) + decltype(rc)::value;
                         if constexpr (u < 8) {
                             float unused = 0.0f;
-                            if (masked_n) head_unit(IC<1 - P>{}, IC<u>{}, n0 + BN, true, unused);
+                            if (masked_n) head_unit(IC<1 - P>{}, IC<u>{}, n0_next, true, unused);
                         }
                     });
                 }
@@ -948,8 +1018,16 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         });
         l_i += lsum;
         mslot = mslot_next;
-        if (step + 4 < nsteps) { k_fetch += k_tile_bytes; k_tile++; }  // next iteration fetches K of step+4, V of step+3
-        if (step + 3 < nsteps) { v_fetch += v_tile_bytes; v_tile++; }
+        if constexpr (MASK) {
+            v_at(vt3);
+            vt0 = vt1;
+            vt1 = vt2;
+            vt2 = vt3;
+            k_at(vt3 = next_tile(vt3, step + 4 < nsteps));
+        } else {
+            if (step + 4 < nsteps) { k_fetch += k_tile_bytes; k_tile++; }  // next iteration fetches K of step+4, V of step+3
+            if (step + 3 < nsteps) { v_fetch += v_tile_bytes; v_tile++; }
+        }
         __builtin_amdgcn_s_setprio(0);
         // (additive mask: the entries of the next step, requested ahead of this step's K/V loads, have landed)
         if constexpr (MF32) __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -969,6 +1047,10 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     if (CAUSAL) {
         const int first_hidden_step = (__builtin_amdgcn_readfirstlane(wlim) + 1) / BN;  // tile that holds key wlim + 1 (may lie past the last step); wave-uniform
         hide_from = max(min(first_hidden_step - 1, ragged ? nk - 4 : nsteps), 0) & ~1;
+        if constexpr (MASK) {  // (no causal limit: only a ragged last tile hides keys, the last step if it is visited at all)
+            const int last_group = (nk - 1) / visit_group;
+            hide_from = ragged && last_group < 64 && (visits >> last_group) & 1 ? max(nsteps - 4, 0) & ~1 : nsteps + 1;
+        }
     }
     int step = 0;
     if (CAUSAL) {

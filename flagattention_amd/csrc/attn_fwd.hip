@@ -467,13 +467,14 @@ int launch_mode(const AttnArgs& a, int mode, hipStream_t stream) {
 
 }  // namespace
 
-int64_t attn_split_workspace_bytes(const sage_attn_params& p) {
-    if (p.mask_kind != SAGE_MASK_NONE || (p.causal && p.qo_len > p.kv_len)) return 0;  // (not a launch that can be split)
-    const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, true);
-    return attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim);
+namespace {
+
+bool mask_is_bool(const sage_attn_params& p) {
+    return p.mask_kind == SAGE_MASK_BOOL || p.mask_kind == SAGE_MASK_BOOL_PADDED || p.mask_kind == SAGE_MASK_BOOL_PADDED_CAUSAL;
 }
 
-int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+// the arguments of the whole launch
+AttnArgs attn_args(const sage_attn_params& p) {
     AttnArgs a{};
     a.q = (const int8_t*)p.q.ptr; a.k = (const int8_t*)p.k.ptr; a.v = p.v.ptr; a.out = p.out.ptr;
     a.q_scale = p.q_scale; a.k_scale = p.k_scale; a.lse = p.lse; a.mask = p.mask;
@@ -487,8 +488,7 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
     a.groups = (int)(p.heads_q / p.heads_kv);
     a.out_dt = p.out_dtype; a.causal = p.causal ? 1 : 0;
     a.lse_mul = 1.0f;
-    const bool is_bool = p.mask_kind == SAGE_MASK_BOOL || p.mask_kind == SAGE_MASK_BOOL_PADDED ||
-                         p.mask_kind == SAGE_MASK_BOOL_PADDED_CAUSAL;
+    const bool is_bool = mask_is_bool(p);
     a.mask_padded = p.mask_kind == SAGE_MASK_BOOL_PADDED || p.mask_kind == SAGE_MASK_BOOL_PADDED_CAUSAL ||
                     p.mask_kind == SAGE_MASK_F16_PADDED || p.mask_kind == SAGE_MASK_BF16_PADDED ||
                     p.mask_kind == SAGE_MASK_F32_PADDED;
@@ -503,6 +503,34 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
         a.mask_vec = ((uintptr_t)p.mask % align) == 0 && (p.mask_stride_b * esz) % align == 0 &&
                      (p.mask_stride_h * esz) % align == 0 && (p.mask_stride_m * esz) % align == 0;
     }
+    a.mask_additive = additive;
+    a.visit_group = (a.nk + 63) / 64;
+    a.nsplit = 1; a.split_steps = a.nk;
+    a.head_tile = 1;
+    if (p.mask_kind != SAGE_MASK_NONE && p.mask_stride_h == 0 && p.heads_q > 1)
+        a.head_tile = p.heads_q % 8 == 0 ? 8 : p.heads_q % 4 == 0 ? 4 : p.heads_q % 2 == 0 ? 2 : 1;
+    return a;
+}
+
+// a mask tensor that the pipelined kernel stages
+bool fast_masked(const sage_attn_params& p, const AttnArgs& a) {
+    return p.mask_kind != SAGE_MASK_NONE && attn::fast_serves_mask(a, a.mask_additive ? dtype_bytes(a.mask_dt) : 1);
+}
+
+}  // namespace
+
+int64_t attn_split_workspace_bytes(const sage_attn_params& p) {
+    if (p.mask_kind != SAGE_MASK_NONE) {
+        const AttnArgs a = attn_args(p);
+        return fast_masked(p, a) ? attn::mask_scan_bytes(a, p.batch) : 0;
+    }
+    if (p.causal && p.qo_len > p.kv_len) return 0;  // (not a launch that can be split)
+    const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, true);
+    return attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim);
+}
+
+int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+    AttnArgs a = attn_args(p);
     const int64_t total = p.batch * p.heads_q * a.nq;
     if (total > 0x7fffffffLL || p.qo_len > 0x7fffffffLL - BM || p.kv_len > 0x7fffffffLL - BN)
         return fail(SAGE_E_UNSUPPORTED, "sage_attn_fwd: problem too large for 32-bit tile indices");
@@ -510,13 +538,9 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
         (int64_t)BN * p.v.stride_n >= (1LL << 29))
         return fail(SAGE_E_UNSUPPORTED, "sage_attn_fwd: k/v sequence stride out of range for 32-bit tile offsets");
     a.total_wg = (int)total;
-    a.nsplit = 1; a.split_steps = a.nk;
-    a.head_tile = 1;
-    if (p.mask_kind != SAGE_MASK_NONE && p.mask_stride_h == 0 && p.heads_q > 1)
-        a.head_tile = p.heads_q % 8 == 0 ? 8 : p.heads_q % 4 == 0 ? 4 : p.heads_q % 2 == 0 ? 2 : 1;
     int mode = MODE_PLAIN;
-    if (is_bool) mode = MODE_MASK_BOOL;
-    else if (additive) mode = MODE_MASK_F32;
+    if (mask_is_bool(p)) mode = MODE_MASK_BOOL;
+    else if (a.mask_additive) mode = MODE_MASK_F32;
     else if (p.causal) mode = MODE_CAUSAL;
     const bool fast = p.mask_kind == SAGE_MASK_NONE && (!p.causal || p.qo_len <= p.kv_len);
     if (fast) {
@@ -543,9 +567,12 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
         s.longest_first = plan.longest_first;
         return launch(s);
     }
-    a.mask_additive = additive;
-    if ((is_bool && attn::fast_serves_mask(a, 1)) || (additive && attn::fast_serves_mask(a, dtype_bytes(a.mask_dt))))
+    if (fast_masked(p, a)) {
+        const int64_t scan = attn::mask_scan_bytes(a, p.batch);
+        if (scan > 0 && workspace && workspace_bytes >= scan)
+            if (int rc = attn::launch_mask_scan(a, p.batch, (int)p.head_dim, p.v_dtype, workspace, stream)) return rc;
         return attn::launch_fast_masked(a, (int)p.head_dim, p.v_dtype, stream);
+    }
     if (p.head_dim == 128) {
         return p.v_dtype == SAGE_BF16 ? launch_mode<128, __bf16>(a, mode, stream)
                                       : launch_mode<128, _Float16>(a, mode, stream);

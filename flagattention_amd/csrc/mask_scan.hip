@@ -1,0 +1,208 @@
+// Which 64-key tiles of a mask tensor the pipelined attention kernel has to visit (gfx950): one pass over a mask that the heads
+// share, and over V, ahead of the attention launch.
+//
+// FlagAttention src/flag_attn/sage_attention/attn_qk_int8_per_block.py:33-36 skips the 128 x 64 tiles of a bool mask without a
+// visible key; under an additive mask it computes every tile.  There a tile can be left out where it changes nothing: its largest
+// entry lies so far below the largest entry of every row that every P of the tile is exactly 0, whatever the scores (bounded by
+// the block scales, which the attention kernel looks at: `visits` in attn_fast_kernel.h).  Padding and causal masks in additive
+// form, the ones model code builds, leave out their hidden half that way; a row that sees no key at all makes its q-block visit
+// every tile.  A tile of V with an Inf or NaN is visited by all (0 times those is NaN).
+//
+// Bound by the bytes of the mask and of V.  A workgroup takes a strip of 16 mask rows, a thread 16 bytes of each of them at a time
+// (16 loads on their way), so that the scan of one [M, N] mask fills the chip; or one 64-key tile of V.
+// B4 H16 M1536 N1536 D128, [B, 1, M, N] bf16 mask (19 MB, V 25 MB) with causal and padding in one: attention 102 us -> scan 12
+// and attention 56; quantization and attention 117.5 -> 90.7 us.  B1 H32/8 M2560 N2560, bool: 150 -> 77 us; B2 H24 M3840 N3840
+// D64, fp32 entries (118 MB): 301 -> 200 us.
+#include <type_traits>
+
+#include "attn_common.h"
+
+namespace sage {
+namespace {
+
+using attn::AttnArgs;
+using attn::BN;
+using attn::kScanRows;
+
+constexpr int kScanThreads = 256;
+
+struct ScanArgs {
+    const unsigned char* mask;
+    const unsigned char* v;
+    float* top;
+    float* low;
+    unsigned* odd;
+    int64_t ms_b, ms_m;        // bytes
+    int64_t vs_b, vs_h, vs_n;  // bytes
+    int32_t M, N, nk, Hkv;
+    int32_t strips, mask_wgs;  // strips of a mask batch; workgroups that scan the mask (the others: V)
+    int32_t v_tiles;           // batch * Hkv * nk
+};
+
+// the largest of the first `live` entries of a 16-byte chunk; NaN counts as +inf (bool: 0 where a key is visible, else -inf)
+template <typename MT>
+__device__ __forceinline__ float chunk_max(uint4 w, int live) {
+    constexpr int E = 16 / sizeof(MT);
+    const unsigned word[4] = {w.x, w.y, w.z, w.w};
+    float m = -INFINITY;
+    if constexpr (sizeof(MT) == 1) {
+        unsigned any = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int bytes = live - 4 * i;
+            any |= bytes >= 4 ? word[i] : bytes <= 0 ? 0u : word[i] & ((1u << (8 * bytes)) - 1);
+        }
+        m = any ? 0.0f : -INFINITY;
+    } else {
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            float x;
+            if constexpr (sizeof(MT) == 4) x = __builtin_bit_cast(float, word[i]);
+            else {
+                const unsigned short bits = (unsigned short)(i & 1 ? word[i >> 1] >> 16 : word[i >> 1]);
+                x = (float)__builtin_bit_cast(MT, bits);
+            }
+            x = x == x ? x : INFINITY;
+            m = i < live ? fmaxf(m, x) : m;
+        }
+    }
+    return m;
+}
+
+template <typename MT>
+__device__ __forceinline__ void scan_strip(const ScanArgs& a, int wg) {
+    constexpr int E = 16 / sizeof(MT), LPT = BN / E;  // entries per chunk; chunks (lanes) per tile
+    __shared__ float row_top[kScanThreads / 64][kScanRows];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int mb = wg / a.strips, strip = wg % a.strips;
+    const unsigned char* base = a.mask + mb * a.ms_b;
+    float row[kScanRows];
+#pragma unroll
+    for (int r = 0; r < kScanRows; r++) row[r] = -INFINITY;
+    const int chunks = a.nk * LPT;
+    for (int c0 = 0; c0 < chunks; c0 += kScanThreads) {
+        const int c = c0 + tid, live = a.N - c * E;  // entries of the chunk that are keys
+        float t = -INFINITY;
+        if (live > 0) {
+            uint4 w[kScanRows];
+#pragma unroll
+            for (int r = 0; r < kScanRows; r++)  // (rows past the last one: that one again)
+                w[r] = *reinterpret_cast<const uint4*>(base + (int64_t)min(strip * kScanRows + r, a.M - 1) * a.ms_m + (int64_t)16 * c);
+#pragma unroll
+            for (int r = 0; r < kScanRows; r++) {
+                const float m = chunk_max<MT>(w[r], live);
+                row[r] = fmaxf(row[r], m);
+                t = fmaxf(t, m);
+            }
+        }
+#pragma unroll
+        for (int x = 1; x < LPT; x <<= 1) t = fmaxf(t, __shfl_xor(t, x));
+        const int tile = c / LPT;
+        if (c < chunks && c % LPT == 0) {
+            // (additive: the last tile of a kv_len that is not a multiple of 64 also holds keys that score -1e6)
+            if (sizeof(MT) > 1 && tile == a.nk - 1 && a.N % BN) t = fmaxf(t, attn::kMasked);
+            a.top[(int64_t)wg * a.nk + tile] = t;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kScanRows; r++) {
+#pragma unroll
+        for (int x = 1; x < 64; x <<= 1) row[r] = fmaxf(row[r], __shfl_xor(row[r], x));
+        if (lane == 0) row_top[wave][r] = row[r];
+    }
+    __syncthreads();
+    if (tid == 0) {
+        float low = INFINITY;
+        for (int r = 0; r < kScanRows; r++) {
+            float m = row_top[0][r];
+            for (int w = 1; w < kScanThreads / 64; w++) m = fmaxf(m, row_top[w][r]);
+            low = fminf(low, m);
+        }
+        a.low[wg] = sizeof(MT) == 1 ? 0.0f : low;  // (bool: a tile is visited if it holds a visible key)
+    }
+}
+
+// A wave takes a 64-key tile of V, every load of it on its way before the first is looked at.
+template <int D, typename VT>
+__device__ __forceinline__ void scan_v(const ScanArgs& a, int wg) {
+    constexpr int CPR = 2 * D / 16, LOADS = BN * CPR / 64;  // 16-byte chunks per row; of a tile per lane
+    constexpr unsigned exponent = std::is_same_v<VT, __bf16> ? 0x7f807f80u : 0x7c007c00u;  // all ones: Inf or NaN
+    const int i = wg * (kScanThreads / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= a.v_tiles) return;
+    const int t = i % a.nk, bh = i / a.nk, hk = bh % a.Hkv, b = bh / a.Hkv;
+    const unsigned char* base = a.v + b * a.vs_b + hk * a.vs_h + 16 * (lane % CPR);
+    uint4 w[LOADS];
+#pragma unroll
+    for (int x = 0; x < LOADS; x++)
+        w[x] = *reinterpret_cast<const uint4*>(base + (int64_t)min(BN * t + x * (64 / CPR) + lane / CPR, a.N - 1) * a.vs_n);
+    bool odd = false;
+#pragma unroll
+    for (int x = 0; x < LOADS; x++) {
+        const unsigned word[4] = {w[x].x, w[x].y, w[x].z, w[x].w};
+#pragma unroll
+        for (int y = 0; y < 4; y++) {
+            const unsigned e = word[y] & exponent;
+            odd |= (e & 0xffffu) == (exponent & 0xffffu) || (e >> 16) == (exponent >> 16);
+        }
+    }
+    const bool any = __builtin_amdgcn_ballot_w64(odd) != 0;
+    if (lane == 0) a.odd[i] = any ? 1u : 0u;
+}
+
+template <int D, typename VT, typename MT>
+__global__ __launch_bounds__(kScanThreads) void mask_scan_kernel(ScanArgs a) {
+    const int wg = blockIdx.x;
+    if (wg < a.mask_wgs) scan_strip<MT>(a, wg);
+    else scan_v<D, VT>(a, wg - a.mask_wgs);
+}
+
+int64_t mask_batches(const AttnArgs& a, int64_t batch) { return a.ms_b ? batch : 1; }
+int64_t scan_strips(const AttnArgs& a) { return a.ms_m ? (a.M + kScanRows - 1) / kScanRows : 1; }
+
+template <int D, typename VT>
+int launch_scan(const AttnArgs& a, const ScanArgs& s, int64_t wgs, hipStream_t stream) {
+    dim3 grid((unsigned)wgs), block(kScanThreads);
+    if (!a.mask_additive) hipLaunchKernelGGL((mask_scan_kernel<D, VT, uint8_t>), grid, block, 0, stream, s);
+    else if (a.mask_dt == SAGE_F32) hipLaunchKernelGGL((mask_scan_kernel<D, VT, float>), grid, block, 0, stream, s);
+    else if (a.mask_dt == SAGE_BF16) hipLaunchKernelGGL((mask_scan_kernel<D, VT, __bf16>), grid, block, 0, stream, s);
+    else hipLaunchKernelGGL((mask_scan_kernel<D, VT, _Float16>), grid, block, 0, stream, s);
+    return check_launch("mask_scan_kernel");
+}
+
+}  // namespace
+
+namespace attn {
+
+// Worth its launch where the heads share the mask (one read of it serves all of them; a mask per head is a position bias as a
+// rule, and read once either way) and enough steps can go.  Where every q-block has a compute unit of its own only the longest
+// one counts, which padding shortens and a causal mask does not: 20 tiles (B3 H16 M640 N640 D128 causal and padded, bool: 39 us
+// without, 43 with; B2 H8 M1286 fp16 62, 53); with more q-blocks 12 (B3 H32 M858 N858 D128 padded fp32: 99.8, 98.4).  V is read
+// once more, so the queries per K/V head have to be many as well.
+int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch) {
+    const int64_t q_blocks = batch * a.Hq * ((a.M + kFastRows - 1) / kFastRows);
+    if (a.ms_h != 0 || a.Hq < 2 || a.nk < (q_blocks > 256 ? 12 : 20) || (int64_t)a.groups * a.M < 512) return 0;
+    const int64_t mask_wgs = mask_batches(a, batch) * scan_strips(a), v_tiles = batch * a.Hkv * a.nk;
+    if (mask_wgs + v_tiles > 0x7fffffffLL) return 0;
+    const int64_t bytes = 4 * (mask_wgs * (a.nk + 1) + v_tiles);
+    return (bytes + 15) / 16 * 16;
+}
+
+int launch_mask_scan(AttnArgs& a, int64_t batch, int head_dim, int v_dtype, void* workspace, hipStream_t stream) {
+    const int64_t strips = scan_strips(a), mask_wgs = mask_batches(a, batch) * strips, v_tiles = batch * a.Hkv * a.nk;
+    ScanArgs s{};
+    s.mask = static_cast<const unsigned char*>(a.mask); s.v = static_cast<const unsigned char*>(a.v);
+    s.top = static_cast<float*>(workspace); s.low = s.top + mask_wgs * a.nk; s.odd = reinterpret_cast<unsigned*>(s.low + mask_wgs);
+    const int64_t esz = a.mask_additive ? dtype_bytes(a.mask_dt) : 1;
+    s.ms_b = a.ms_b * esz; s.ms_m = a.ms_m * esz;
+    s.vs_b = 2 * a.vs_b; s.vs_h = 2 * a.vs_h; s.vs_n = 2 * a.vs_n;
+    s.M = a.M; s.N = a.N; s.nk = a.nk; s.Hkv = a.Hkv; s.strips = (int)strips; s.mask_wgs = (int)mask_wgs; s.v_tiles = (int)v_tiles;
+    const int64_t v_wgs = (v_tiles + kScanThreads / 64 - 1) / (kScanThreads / 64);
+    a.scan_top = s.top; a.scan_low = s.low; a.scan_v = s.odd; a.scan_strips = s.strips;
+    a.longest_first = a.ms_m != 0;
+    if (head_dim == 128)
+        return v_dtype == SAGE_BF16 ? launch_scan<128, __bf16>(a, s, mask_wgs + v_wgs, stream) : launch_scan<128, _Float16>(a, s, mask_wgs + v_wgs, stream);
+    return v_dtype == SAGE_BF16 ? launch_scan<64, __bf16>(a, s, mask_wgs + v_wgs, stream) : launch_scan<64, _Float16>(a, s, mask_wgs + v_wgs, stream);
+}
+
+}  // namespace attn
+}  // namespace sage

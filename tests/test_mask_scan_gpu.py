@@ -1,0 +1,199 @@
+"""Tiles left out under a mask tensor that the heads share (csrc/mask_scan.hip): the launch with the scan (workspace given) against
+the one that visits every tile (no workspace), and against the oracle's arithmetic through the latter's own tests."""
+import ctypes
+
+import pytest
+import torch
+
+from flagattention_amd import _lib
+from flagattention_amd.sage_attention import attention as A
+from flagattention_amd.sage_attention._common import tensor_desc
+
+gpu = pytest.mark.gpu
+KIND = {torch.bool: _lib.MASK_BOOL, torch.float16: _lib.MASK_F16, torch.bfloat16: _lib.MASK_BF16, torch.float32: _lib.MASK_F32}
+
+
+def _params(q8, qs, k8, ks, v, mask, o, lse, kind, hnd):
+    p = _lib.AttnParams()
+    p.q, p.k, p.v, p.out = (tensor_desc(t, hnd) for t in (q8, k8, v, o))
+    if hnd:
+        (b, h, m, d), (_, hkv, n, _) = q8.shape, k8.shape
+    else:
+        (b, m, h, d), (_, n, hkv, _) = q8.shape, k8.shape
+    p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.head_dim = b, h, hkv, m, n, d
+    code = {torch.float16: _lib.SAGE_F16, torch.bfloat16: _lib.SAGE_BF16, torch.float32: _lib.SAGE_F32}
+    p.v_dtype, p.out_dtype, p.mask_kind = code[v.dtype], code[o.dtype], kind
+    p.q_scale, p.k_scale, p.lse = qs.data_ptr(), ks.data_ptr(), lse.data_ptr()
+    mask = mask.expand(b, h, m, n)
+    p.mask = mask.data_ptr()
+    p.mask_stride_b, p.mask_stride_h, p.mask_stride_m, p.mask_stride_n = mask.stride()
+    return p
+
+
+def _inputs(b, h, hkv, m, n, d, dt, hnd, scale=1.0):
+    g = torch.Generator().manual_seed(3 * n + m)
+    dev = "cuda:0"
+
+    def t(heads, length):
+        return torch.randint(-127, 128, (b, heads, length, d) if hnd else (b, length, heads, d), generator=g, dtype=torch.int8).to(dev)
+
+    q8, k8 = t(h, m), t(hkv, n)
+    qs = (torch.rand(b, h, -(-m // 128), generator=g) * 2e-3 * scale + 1e-4).to(dev)
+    ks = (torch.rand(b, hkv, -(-n // 64), generator=g) * 2e-2 + 1e-3).to(dev)
+    v = torch.randn(k8.shape, generator=g).to(dt).to(dev)
+    return q8, qs, k8, ks, v
+
+
+def _mask(kind, dt, b, m, n):
+    """Masks shared by the heads, and how many of 256 x 64 tiles a scan may leave out at least (share of all)."""
+    dev = "cuda:0"
+    g = torch.Generator().manual_seed(n)
+    cols, rows = torch.arange(n), torch.arange(m).view(m, 1) + (n - m)
+    lengths = torch.tensor([n // 2 + 3 + 70 * i for i in range(b)]).view(b, 1, 1, 1)
+    if kind == "padding":
+        keep = (cols < lengths).expand(b, 1, 1, n)
+    elif kind == "causal_padding":
+        keep = (cols < lengths) & (cols <= rows)
+    elif kind == "left":  # left padding under the causal mask: the first rows see no key
+        keep = (cols >= n - lengths) & (cols <= rows)
+    elif kind == "window":
+        keep = ((cols <= rows) & (cols > rows - 100)).view(1, 1, m, n)
+    elif kind == "holes":  # any pattern, some 64-key columns of tiles hidden
+        keep = (torch.rand(b, 1, m, n, generator=g) < 0.3) & ((cols // 64) % 3 != 1)
+    elif kind == "none":
+        keep = torch.zeros(1, 1, m, n, dtype=torch.bool)
+    elif kind == "slope":  # a steep linear bias, no hidden keys
+        return (-(rows - cols).abs().float() * 3.0).view(1, 1, m, n).to(dt).to(dev)
+    if dt is torch.bool:
+        return keep.contiguous().to(dev)
+    low = -float("inf") if kind == "holes" else torch.finfo(dt).min
+    return torch.zeros(keep.shape, dtype=dt).masked_fill_(~keep, low).to(dev)
+
+
+def _both(q8, qs, k8, ks, v, mask, hnd, out_dt=torch.float32):
+    """(o, lse) with the scan, (o, lse) of the launch that visits every tile."""
+    lib, res = _lib.load(), []
+    b, h = (q8.shape[0], q8.shape[1]) if hnd else (q8.shape[0], q8.shape[2])
+    m = q8.shape[2] if hnd else q8.shape[1]
+    stream = torch.cuda.current_stream().cuda_stream
+    for scan in (True, False):
+        o, lse = torch.empty(q8.shape, dtype=out_dt, device=q8.device), torch.empty(b, h, m, device=q8.device)
+        p = _params(q8, qs, k8, ks, v, mask, o, lse, KIND[mask.dtype], hnd)
+        if scan:
+            nbytes = lib.sage_attn_fwd_workspace_bytes(ctypes.byref(p))
+            assert nbytes > 0
+            ws = torch.full((nbytes,), 0x7f, dtype=torch.uint8, device=q8.device)
+            _lib.check(lib.sage_attn_fwd_ws(ctypes.byref(p), ws.data_ptr(), nbytes, stream), "ws")
+        else:
+            _lib.check(lib.sage_attn_fwd(ctypes.byref(p), stream), "fwd")
+        torch.cuda.synchronize()
+        res.append((o, lse))
+    return res
+
+
+def _check(res, dt):
+    (o, lse), (o_all, lse_all) = res
+    # NaN, infinities and empty rows in the same places
+    assert torch.equal(torch.isnan(o), torch.isnan(o_all)) and torch.equal(torch.isnan(lse), torch.isnan(lse_all))
+    assert torch.equal(torch.isinf(lse), torch.isinf(lse_all))
+    fin = torch.isfinite(o_all)
+    # The same scores and the same P up to the reference point of a row (which rounds P to 16 bits at another place): one
+    # unit of the 16-bit type per term at most
+    eps = 2.0 ** -8 if dt is torch.bfloat16 else 2.0 ** -11
+    assert (o - o_all)[fin].abs().max().item() <= 4 * eps * o_all[fin].abs().max().item() if fin.any() else True
+    lf = torch.isfinite(lse_all)
+    if lf.any():  # (fully hidden rows: lse near the type's lowest value)
+        assert ((lse - lse_all)[lf].abs() <= 2 * eps + 1e-6 * lse_all[lf].abs()).all()
+
+
+SHAPES = [  # b, h, hkv, m, n, d, hnd: whole tiles; a ragged last tile; more than 64 tiles (two per bit); more q-blocks than compute units
+    (2, 4, 2, 1280, 1280, 64, True), (2, 2, 2, 600, 1288, 128, False), (1, 4, 1, 512, 4304, 64, True), (3, 48, 2, 520, 776, 64, True)]
+
+
+@gpu
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("mask_dt", [torch.bool, torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["padding", "causal_padding", "left", "window", "holes", "none", "slope"])
+def test_scan_changes_nothing(shape, mask_dt, kind):
+    b, h, hkv, m, n, d, hnd = shape
+    if mask_dt is torch.bool and (kind == "slope" or n % 16):
+        pytest.skip("not a bool mask the kernel stages as it is")
+    dt = torch.bfloat16 if d == 128 else torch.float16
+    x = _inputs(b, h, hkv, m, n, d, dt, hnd)
+    _check(_both(*x, _mask(kind, mask_dt, b, m, n), hnd), dt)
+
+
+@gpu
+@pytest.mark.parametrize("mask_dt", [torch.bool, torch.bfloat16, torch.float16])
+def test_scan_nonfinite(mask_dt):
+    """Inf / NaN in V under hidden keys, in a block scale, in a mask entry; scales so large that no entry hides a key."""
+    b, h, hkv, m, n, d = 2, 2, 2, 512, 1280, 64
+    mask = _mask("causal_padding", mask_dt, b, m, n)
+    for what in ("v_inf", "v_nan", "ks_nan", "ks_inf", "qs_nan", "large", "entry"):
+        q8, qs, k8, ks, v = _inputs(b, h, hkv, m, n, d, torch.float16, True, scale=1e4 if what == "large" else 1.0)
+        mk = mask.clone()
+        if what == "v_inf":
+            v[0, 1, n - 2, 5] = float("inf")
+        elif what == "v_nan":
+            v[1, 0, n - 70, 9] = float("nan")
+        elif what == "ks_nan":
+            ks[0, 1, -1] = float("nan")
+        elif what == "ks_inf":
+            ks[1, 1, -2] = float("inf")
+        elif what == "qs_nan":
+            qs[0, 0, 1] = float("nan")
+        elif what == "entry":
+            if mask_dt is torch.bool:
+                continue
+            mk[0, 0, 300, 100] = float("nan")
+            mk[1, 0, 30, 1200] = float("inf")
+        res = _both(q8, qs, k8, ks, v, mk, True)
+        if what == "large":  # (exponents of thousands: P is 0 or 1, the rounding of the exponent shows)
+            assert torch.equal(torch.isnan(res[0][0]), torch.isnan(res[1][0]))
+            continue
+        _check(res, torch.float16)
+
+
+@gpu
+def test_scan_through_the_public_call_and_a_graph():
+    from flag_attn import sage_attention as sa
+
+    b, h, m, n, d = 2, 4, 768, 1280, 64
+    q8, qs, k8, ks, v = _inputs(b, h, h, m, n, d, torch.bfloat16, True)
+    for dt in (torch.bool, torch.bfloat16, torch.float32):
+        mask = _mask("causal_padding", dt, b, m, n)
+        want = _both(q8, qs, k8, ks, v, mask, True, torch.bfloat16)[1][0]
+        for _ in range(2):  # the second call takes the plan of the first
+            o, _l = sa.sage_attention(q8, k8, v, qs, ks, attn_mask=mask, output_dtype=torch.bfloat16)
+            torch.testing.assert_close(o, want, rtol=2e-2, atol=2e-2)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            og, _l = sa.sage_attention(q8, k8, v, qs, ks, attn_mask=mask, output_dtype=torch.bfloat16)
+        other = _mask("padding", dt, b, m, n).expand(b, 1, m, n).contiguous()
+        for i in range(3):  # the scan is part of the graph: it sees what the mask holds when the graph runs
+            if i == 2:
+                mask.copy_(other)
+                want = _both(q8, qs, k8, ks, v, mask, True, torch.bfloat16)[1][0]
+            og.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            torch.testing.assert_close(og, want, rtol=2e-2, atol=2e-2)
+
+
+@gpu
+def test_scan_follows_the_reference_for_bool_masks():
+    """A row without any visible key in the 128 x 64 tiles its block visits; blocks of 128 rows of one workgroup that visit
+    different tiles (attn_qk_int8_per_block.py:33-36)."""
+    from oracle import c_oracle as C
+
+    b, h, m, n, d = 1, 2, 768, 1280, 64
+    q8, qs, k8, ks, v = _inputs(b, h, h, m, n, d, torch.float16, True)
+    mask = torch.zeros(1, 1, m, n, dtype=torch.bool)
+    mask[..., :128, 64:256] = True
+    mask[..., 40:50, :] = False     # rows without a visible key in a visited tile
+    mask[..., 128:256, 512:576] = True
+    mask[..., 300:, 100:700] = torch.rand(m - 300, 600, generator=torch.Generator().manual_seed(1)) < 0.5
+    o, lse = A.forward(q8, k8, v, qs, ks, attn_mask=mask.cuda(), output_dtype=torch.float32, return_lse=True)
+    want, want_lse = C.attention_blockwise(q8.cpu(), k8.cpu(), v.cpu(), qs.cpu(), ks.cpu(), "HND", attn_mask=mask)
+    torch.testing.assert_close(o.cpu(), want.float(), rtol=2e-2, atol=2e-2)
+    torch.testing.assert_close(lse.cpu(), want_lse, rtol=1e-4, atol=2e-3)
