@@ -166,11 +166,11 @@ int launch_fast(const AttnArgs& a, int head_dim, int v_dtype, bool causal, hipSt
 // How a launch is laid out (split_combine.hip).  Whole: a workgroup per item (256 queries of a head), or under the causal
 // flag per pair of a short and a long one; longest_first: per item under the causal flag too, the longest first.  With a
 // workspace, where that leaves compute units idle: nsplit > 1 workgroups share the keys of each item (pair), or cut_wgs > 0
-// workgroups take equal shares of all steps of the launch.  apply_* turn the arguments of the whole launch into those of
+// workgroups take equal shares of all steps of the launch.  row_tiles: short calls, on attn_decode_kernel (launch_decode).  apply_* turn the arguments of the whole launch into those of
 // the other (partial results in `workspace`, plan_workspace_bytes large); launch_*_combine then write what the whole launch would have.
-struct LaunchPlan { int nsplit, cut_wgs; bool longest_first; };
+struct LaunchPlan { int nsplit, cut_wgs; bool longest_first, row_tiles; };
 LaunchPlan plan_launch(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal,
-                       bool with_workspace);
+                       int64_t head_dim, bool int8, bool with_workspace);
 int64_t plan_workspace_bytes(const LaunchPlan& plan, int64_t batch, int64_t heads_q, int64_t qo_len, int64_t head_dim);
 void apply_cut(AttnArgs& a, int cut_wgs, int64_t batch, int head_dim, void* workspace);
 int launch_cut_combine(const AttnArgs& a, int head_dim, hipStream_t stream);
@@ -178,7 +178,7 @@ void apply_key_split(AttnArgs& a, int nsplit, int64_t batch, int head_dim, void*
 int launch_split_combine(const AttnArgs& split, const AttnArgs& whole, int head_dim, int64_t batch, hipStream_t stream);
 
 // The kernel for few query rows (attn_decode.hip): no mask tensor, qo_len rows of each query head that shares a K/V
-// head, kDecodeRows of them at most; any kv_len, causal with any qo_len.  Splits its keys like the pipelined kernel.
+// head, up to kDecodeRows in a workgroup (decode_serves), more in tiles of 32 (row_tiles); any kv_len, causal with any qo_len.  Splits its keys like the pipelined kernel.
 constexpr int kDecodeRows = 64;
 bool decode_serves(int64_t heads_q, int64_t heads_kv, int64_t qo_len);
 int launch_decode(const AttnArgs& a, int64_t batch, int head_dim, int v_dtype, bool int8, hipStream_t stream);

@@ -16,6 +16,9 @@
 //   Measured (bf16, head_dim 128, with the combine launch; before: the 256-row tiles of the pipelined kernel): dense
 //   B8 H32/8 M1 N8192 197 -> 46 us = 5.8 TB/s of K and V (a 1 GiB copy moves 5.2 TB/s here), SageAttention on the same
 //   shape 144 -> 37 us = 5.4 TB/s, dense B64 H32/8 M1 N1024 229 -> 42 us = 6.4 TB/s.
+// * Short calls with more rows (plan_row_tiles) come here too, a workgroup per 32 packed rows: what counts there is the time of
+//   one workgroup.  The waves' results meet in LDS in one go where eight waves share it (32 channels at a time before: B1 H8
+//   N256 D128 int8 9.0 -> 8.2 us, N64 6.7 -> 5.9).
 // * The keys of a (batch, K/V head) are cut into runs (plan_decode_split) so that every CU holds eight waves; the
 //   waves of a workgroup are combined through LDS, the runs by split_combine_kernel.
 #include "attn_common.h"
@@ -48,20 +51,26 @@ __global__ __launch_bounds__(64 * kDecodeWaves, RT == 1 ? 8 / kDecodeWaves : 1) 
     constexpr int VCPR = V_RS / 16;       // 16-byte chunks per V row
     constexpr int VLOADS = kTileKeys * VCPR / 64;
     constexpr int V_TILE = kTileKeys * V_RS;
-    constexpr int SL_RS = 36;             // floats per row of the combine buffer (32 channels + padding)
+    constexpr int CH = kDecodeWaves == 8 ? D : 32;  // channels of the waves' results that meet in LDS at a time
+    constexpr int SL_RS = CH + 4;         // floats per row of the combine buffer
     constexpr int SLICE = kDecodeWaves * 32 * SL_RS * 4;
     __shared__ __attribute__((aligned(16))) unsigned char smem[kDecodeWaves * V_TILE > SLICE ? kDecodeWaves * V_TILE : SLICE];
     __shared__ float row_m[kDecodeWaves][32 * RT], row_l[kDecodeWaves][32 * RT];
 
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // the runs of one (batch, K/V head) are neighbours in the grid
+    // the runs, then the row tiles, of one (batch, K/V head) are neighbours in the grid
+    const int rows = a.groups * a.M, row_tiles = (rows + 32 * RT - 1) / (32 * RT);
     const int split = blockIdx.x % a.nsplit;
-    const int item = blockIdx.x / a.nsplit;
+    const int row0 = blockIdx.x / a.nsplit % row_tiles * (32 * RT);  // first row of the workgroup
+    const int item = blockIdx.x / a.nsplit / row_tiles;
     const int hk = item % a.Hkv, b = item / a.Hkv;
-    const int rows = a.groups * a.M;
+    // queries of the workgroup's rows: from q_lo to q_hi, all of a head's where the rows belong to several heads
+    const int q_first = row0 % a.M, in_head = min(a.M - q_first, rows - row0);
+    const bool one_head = in_head >= min(32 * RT, rows - row0);
+    const int q_lo = one_head ? q_first : 0, q_hi = one_head ? min(q_first + 32 * RT, a.M) - 1 : a.M - 1;
     const int kbeg = split * a.split_steps * BN;
-    const int kend = min(kbeg + a.split_steps * BN, a.N);
+    const int kend = min(kbeg + a.split_steps * BN, a.causal ? min(q_hi + a.N - a.M + 1, a.N) : a.N);  // (0 or less: no row sees a key)
 
     // this lane's query rows
     v4i qf[RT][KSTEPS];
@@ -69,7 +78,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, RT == 1 ? 8 / kDecodeWaves : 1) 
     float qs[RT];      // scale of the row's scores (int8: still to be multiplied by the K block's)
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
-        const int r = 32 * rt + l32;
+        const int r = row0 + 32 * rt + l32;
         const bool ok = r < rows;  // (rows past the last one multiply a copy of the group's first: nothing of theirs is stored)
         const int g = ok ? r / a.M : 0, mi = ok ? r - g * a.M : 0, h = hk * a.groups + g;
         const int8_t* qp = a.q + ((int64_t)b * a.qs_b + (int64_t)h * a.qs_h + (int64_t)mi * a.qs_n) * QB + 16 * half;
@@ -79,7 +88,7 @@ __global__ __launch_bounds__(64 * kDecodeWaves, RT == 1 ? 8 / kDecodeWaves : 1) 
         qs[rt] = INT8 ? a.q_scale[((int64_t)b * a.Hq + h) * a.nq + mi / BM] : a.qk_scale;
     }
     // keys below this one are visible to every row of the workgroup
-    const int all_see = a.causal ? min(a.N - a.M + 1, a.N) : a.N;
+    const int all_see = a.causal ? min(q_lo + a.N - a.M + 1, a.N) : a.N;
     // (constant address space: scalar loads, which the waits for K and V do not count)
     typedef __attribute__((address_space(4))) const float* const_f32_ptr;
     const const_f32_ptr ksp = (const_f32_ptr)(uintptr_t)(INT8 ? a.k_scale + ((int64_t)b * a.Hkv + hk) * a.nk : nullptr);
@@ -219,8 +228,8 @@ __global__ __launch_bounds__(64 * kDecodeWaves, RT == 1 ? 8 / kDecodeWaves : 1) 
     __syncthreads();
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
-        if (32 * rt >= rows) break;
-        const int r = 32 * rt + l32;
+        if (row0 + 32 * rt >= rows) break;
+        const int r = 32 * rt + l32;  // (within the workgroup)
         float m = -INFINITY, l = 0.0f;
 #pragma unroll
         for (int w = 0; w < kDecodeWaves; w++) m = fmaxf(m, row_m[w][r]);
@@ -229,31 +238,40 @@ __global__ __launch_bounds__(64 * kDecodeWaves, RT == 1 ? 8 / kDecodeWaves : 1) 
         for (int w = 0; w < kDecodeWaves; w++) l += row_l[w][r] * __builtin_amdgcn_exp2f(row_m[w][r] - m_use);
         // l = 0: a row that saw no key; its output is 0, its log-sum-exp -inf
         const float f = l > 0.0f ? __builtin_amdgcn_exp2f(m_i[rt] - m_use) / l : 0.0f;
-        if (a.lse && wave == 0 && half == 0 && r < rows) {
-            const int g = r / a.M, mi = r - g * a.M;
+        if (a.lse && wave == 0 && half == 0 && row0 + r < rows) {
+            const int g = (row0 + r) / a.M, mi = row0 + r - g * a.M;
             a.lse[((int64_t)b * a.Hq + hk * a.groups + g) * a.M + mi + split * a.lse_split_stride] = (__builtin_log2f(l) + m) * a.lse_mul;
         }
+        // CH channels of every wave's rows at a time through LDS: all of them where a wave slice fits, else 32
         float* slice = reinterpret_cast<float*>(smem);
 #pragma unroll
-        for (int dt = 0; dt < DT; dt++) {
-            __syncthreads();  // the V tiles / the previous 32 channels have been read
+        for (int d0 = 0; d0 < D; d0 += CH) {
+            __syncthreads();  // the V tiles / the previous channels have been read
 #pragma unroll
-            for (int g = 0; g < 4; g++)
-                *reinterpret_cast<v4f*>(slice + (wave * 32 + l32) * SL_RS + 8 * g + 4 * half) =
-                    v4f{o[rt][dt][4 * g] * f, o[rt][dt][4 * g + 1] * f, o[rt][dt][4 * g + 2] * f, o[rt][dt][4 * g + 3] * f};
+            for (int dt = 0; dt < CH / 32; dt++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const v16f& x = o[rt][d0 / 32 + dt];
+                    *reinterpret_cast<v4f*>(slice + (wave * 32 + l32) * SL_RS + 32 * dt + 8 * g + 4 * half) =
+                        v4f{x[4 * g] * f, x[4 * g + 1] * f, x[4 * g + 2] * f, x[4 * g + 3] * f};
+                }
             __syncthreads();
-            const int orow = 32 * rt + tid / 8, c = 4 * (tid % 8);  // 32 rows x 8 groups of four channels
-            if (tid < 256 && orow < rows) {
+            constexpr int GROUPS = CH / 4;  // groups of four channels per row
+#pragma unroll
+            for (int e = 0; e < (32 * GROUPS + 64 * kDecodeWaves - 1) / (64 * kDecodeWaves); e++) {
+                const int piece = tid + 64 * kDecodeWaves * e;
+                const int orow = row0 + 32 * rt + piece / GROUPS, c = 4 * (piece % GROUPS);
+                if (piece >= 32 * GROUPS || orow >= rows) continue;
                 v4f sum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int w = 0; w < kDecodeWaves; w++) {
-                    const v4f x = *reinterpret_cast<const v4f*>(slice + (w * 32 + tid / 8) * SL_RS + c);
+                    const v4f x = *reinterpret_cast<const v4f*>(slice + (w * 32 + piece / GROUPS) * SL_RS + c);
 #pragma unroll
                     for (int i = 0; i < 4; i++) sum[i] += x[i];
                 }
                 const int g = orow / a.M, mi = orow - g * a.M;
                 const int64_t off = (int64_t)b * a.os_b + (int64_t)(hk * a.groups + g) * a.os_h + (int64_t)mi * a.os_n +
-                                    split * a.out_split_stride + 32 * dt + c;
+                                    split * a.out_split_stride + d0 + c;
                 if (a.out_dt == SAGE_BF16) {
                     typedef __bf16 b4 __attribute__((ext_vector_type(4)));
                     *reinterpret_cast<b4*>(static_cast<__bf16*>(a.out) + off) = b4{(__bf16)sum[0], (__bf16)sum[1], (__bf16)sum[2], (__bf16)sum[3]};
@@ -270,10 +288,12 @@ __global__ __launch_bounds__(64 * kDecodeWaves, RT == 1 ? 8 / kDecodeWaves : 1) 
 
 template <int D, typename VT, int QB>
 int launch_rt(const AttnArgs& a, int64_t batch, hipStream_t stream) {
-    const int64_t wgs = batch * a.Hkv * a.nsplit;
+    const int64_t rows = (int64_t)a.groups * a.M;
+    const bool two = rows > 32 && rows <= kDecodeRows && a.groups > 1;  // two row tiles per workgroup
+    const int64_t wgs = batch * a.Hkv * a.nsplit * (two ? 1 : (rows + 31) / 32);
     if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "attention over few query rows: too many workgroups for one launch");
     dim3 grid((unsigned)wgs);
-    if (a.groups * a.M > 32) hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 2, 4>), grid, dim3(256), 0, stream, a);
+    if (two) hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 2, 4>), grid, dim3(256), 0, stream, a);
     else if (a.nsplit == 1 && wgs > 256) hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 1, 4>), grid, dim3(256), 0, stream, a);
     else hipLaunchKernelGGL((attn_decode_kernel<D, VT, QB, 1, 8>), grid, dim3(512), 0, stream, a);
     return check_launch("attn_decode_kernel");

@@ -525,7 +525,7 @@ int64_t attn_split_workspace_bytes(const sage_attn_params& p) {
         return fast_masked(p, a) ? attn::mask_scan_bytes(a, p.batch) : 0;
     }
     if (p.causal && p.qo_len > p.kv_len) return 0;  // (not a launch that can be split)
-    const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, true);
+    const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, p.head_dim, true, true);
     return attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim);
 }
 
@@ -544,14 +544,15 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
     else if (p.causal) mode = MODE_CAUSAL;
     const bool fast = p.mask_kind == SAGE_MASK_NONE && (!p.causal || p.qo_len <= p.kv_len);
     if (fast) {
-        const bool decode = attn::decode_serves(p.heads_q, p.heads_kv, p.qo_len);
+        bool decode = attn::decode_serves(p.heads_q, p.heads_kv, p.qo_len);
         auto launch = [&](const AttnArgs& x) {
             return decode ? attn::launch_decode(x, p.batch, (int)p.head_dim, p.v_dtype, true, stream)
                           : attn::launch_fast(x, (int)p.head_dim, p.v_dtype, p.causal != 0, stream);
         };
-        attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, workspace != nullptr);
+        attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, p.head_dim, true, workspace != nullptr);
         if (attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim) > workspace_bytes)  // (the whole launch then)
-            plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, false);
+            plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, p.head_dim, true, false);
+        decode |= plan.row_tiles;
         AttnArgs s = a;
         if (plan.cut_wgs > 0) {
             attn::apply_cut(s, plan.cut_wgs, p.batch, (int)p.head_dim, workspace);

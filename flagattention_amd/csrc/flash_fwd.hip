@@ -42,7 +42,7 @@ int launch_flash(const AttnArgs& a, int head_dim, int dtype, bool causal, hipStr
 }  // namespace attn
 
 int64_t flash_split_workspace_bytes(const sage_flash_params& p) {
-    const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, true);
+    const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, p.head_dim, false, true);
     return attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim);
 }
 
@@ -69,14 +69,15 @@ int launch_flash_attn(const sage_flash_params& p, void* workspace, int64_t works
         return fail(SAGE_E_UNSUPPORTED, "sage_flash_attn_fwd: k/v sequence stride out of range for 32-bit tile offsets");
     a.total_wg = (int)total;
     a.nsplit = 1; a.split_steps = a.nk;
-    const bool decode = decode_serves(p.heads_q, p.heads_kv, p.qo_len);
+    bool decode = decode_serves(p.heads_q, p.heads_kv, p.qo_len);
     auto launch = [&](const AttnArgs& x) {
         return decode ? launch_decode(x, p.batch, (int)p.head_dim, p.dtype, false, stream)
                       : launch_flash(x, (int)p.head_dim, p.dtype, p.causal != 0, stream);
     };
-    LaunchPlan plan = plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, workspace != nullptr);
+    LaunchPlan plan = plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, p.head_dim, false, workspace != nullptr);
     if (plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim) > workspace_bytes)  // (the whole launch then)
-        plan = plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, false);
+        plan = plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, p.head_dim, false, false);
+    decode |= plan.row_tiles;
     AttnArgs s = a;
     if (plan.cut_wgs > 0) {
         apply_cut(s, plan.cut_wgs, p.batch, (int)p.head_dim, workspace);

@@ -216,6 +216,39 @@ static int plan_decode_split(int64_t items, int64_t rows, int64_t nk) {
     return best_s;
 }
 
+// Short calls on attn_decode_kernel, a workgroup per 32-row tile of a K/V head's packed query rows (and run of its keys), instead
+// of one per 256 rows: they end in the time one workgroup takes, in which eight waves walk over the keys side by side instead of
+// one after the other, and a kernel that runs only a few steps spends less on its start.  Returns the runs of the keys, 0: not here.
+// Every workgroup has a compute unit of its own (under the causal flag half of them are short: two rounds), and the K/V rows
+// that all of them read, once per row tile, stay below 100 MB.  Times in us fitted to 350 launches within 12 %.
+// Measured, pipelined kernel -> here (us, in a graph):
+//   int8  D64  B1 H2 M256 N256 8.0 -> 5.4, H8 N512 causal 22 -> 6.6, H8 N1024 18 -> 9.2, H2 N2048 causal 25 -> 12; D128 H8 N512 17 -> 10.4
+//   dense D128 H2 N200 13.2 -> 9.4, H8 N512 causal 35 -> 12.6, H8 N128 causal 10.3 -> 7.5, H2 N2048 28 -> 23
+//   not here: int8 D128 H32 M64 N16384 52 (65 here), dense D128 H32/32 M128 N128 9.1 (11.5), H32 M64 N1024 15.0 (16.1)
+static int plan_row_tiles(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal,
+                          int64_t head_dim, bool int8, bool with_workspace) {
+    const int64_t rows = heads_q / heads_kv * qo_len, wgs = batch * heads_kv * ((rows + 31) / 32), nk = (kv_len + BN - 1) / BN;
+    if (wgs > (causal ? 2 : 1) * kComputeUnits || kv_len >= (1 << 22)) return 0;
+    const float mb = (float)wgs * (float)(kv_len * head_dim * (int8 ? 3 : 4)) * 1e-6f;
+    if (mb > 100.0f || (rows <= 64 && !int8 && kv_len >= 1024)) return 0;  // (two row tiles of a head: no gain in 16 bits)
+    if (qo_len > kv_len && kv_len >= 512) return 0;  // (cross attention over keys that can be split keeps the key split of 256-row blocks)
+    // a workgroup: its start and end, and each turn of its waves over 32 keys each; the K/V bytes; the second launch
+    const float start = int8 ? (head_dim == 64 ? 4.5f : 7.1f) : (head_dim == 64 ? 5.7f : 8.4f);
+    const float turn = int8 ? (head_dim == 64 ? 0.9f : 1.4f) : (head_dim == 64 ? 1.0f : 2.2f);
+    const float combine = head_dim == 64 ? 2.2f : 3.6f;
+    const int64_t smax = with_workspace ? (nk / kMinStepsPerSplit < kMaxSplits ? nk / kMinStepsPerSplit : kMaxSplits) : 1;
+    float best = 0.0f;
+    int best_s = 1;
+    for (int64_t s = 1; s <= smax; s++) {
+        const int64_t steps = (nk + s - 1) / s;
+        if ((nk + steps - 1) / steps != s || (s > 1 && wgs * s > kComputeUnits)) continue;  // (a run without a key; a second round)
+        const float cost = start + turn * (float)((2 * steps + 7) / 8) +
+                           (s > 1 ? combine + (head_dim == 64 ? 4.8f : 0.7f) * (float)(s * batch * heads_q * qo_len * head_dim) * 1e-6f : 0.0f);
+        if (s == 1 || cost < best) { best = cost; best_s = (int)s; }
+    }
+    return best_s;
+}
+
 // Plans of the pipelined kernel, in steps.  Fitted to 38 shapes (1 to 96 heads, 512 to 16384 keys, both flags, both
 // head_dims, int8 and 16-bit Q and K) within 5 % for the cut launch and 10 % for the others: a workgroup spends kFixed on
 // the prologue and epilogue of each item or piece of one, a launch kLaunch, a second one kCombine, a piece that leaves a
@@ -232,11 +265,16 @@ constexpr float kCombineRows = 4.0f, kPartialRows = 4.0f;  // the key split stor
 //                  short items lose (B6 H16 N1000 causal 46 -> 62)
 //   key split      B1 H30 M512 N4096 70 -> 44 / 76 -> 48; not B2 H16 N512 (25 against 14), B1 H20 N1024 (31 against 23)
 LaunchPlan plan_launch(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal,
-                       bool with_workspace) {
-    LaunchPlan plan{1, 0, false};
+                       int64_t head_dim, bool int8, bool with_workspace) {
+    LaunchPlan plan{1, 0, false, false};
     const int64_t nk = (kv_len + BN - 1) / BN;
     if (decode_serves(heads_q, heads_kv, qo_len)) {
         if (with_workspace) plan.nsplit = plan_decode_split(batch * heads_kv, heads_q / heads_kv * qo_len, nk);
+        return plan;
+    }
+    if (const int runs = plan_row_tiles(batch, heads_q, heads_kv, qo_len, kv_len, causal, head_dim, int8, with_workspace)) {
+        plan.nsplit = runs;
+        plan.row_tiles = true;
         return plan;
     }
     const int64_t nq = (qo_len + kFastRows - 1) / kFastRows, heads = batch * heads_q;
@@ -289,7 +327,7 @@ LaunchPlan plan_launch(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t
         const int64_t wgs = total / kMinStepsPerShare < kComputeUnits ? total / kMinStepsPerShare : kComputeUnits;
         const float cost = kLaunch + kCombine + (float)total / (float)wgs + kFixed * (1.0f + (float)items / (float)wgs) + 2.0f * kPartial +
                            0.25f * (float)nk * (float)wgs / (float)total;  // (the parts of an item)
-        if (cost < 0.93f * best) plan = LaunchPlan{1, (int)wgs, false};
+        if (cost < 0.93f * best) plan = LaunchPlan{1, (int)wgs, false, false};
     }
     return plan;
 }
