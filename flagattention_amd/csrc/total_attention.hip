@@ -14,7 +14,7 @@
 // (with only 32 keys per wave) asked the L1 for twice the bytes it delivers.  The tiles are loaded three ahead, straight
 // into LDS.  Workgroups are handed out longest first over all heads: with the key blocks of one head side by side, the
 // last heads' long blocks started late (B4 H32 M4096 N4096 D128 fp16 causal 425 us, longest first 280 us; without the
-// causal flag 523 us).  Where key blocks alone do not fill the chip the queries are cut into runs (total_runs), whose
+// causal flag 523 us).  Where key blocks alone do not fill the chip the queries are cut into runs (total_chunk), whose
 // sums go to a workspace and are added in order.  Before, with a wave per 32 keys loading queries into registers:
 // B1 H16 M4096 N4096 D128 causal 212 -> 41 us, B4 H32 M4096 N4096 1739 -> 275 us, B8 H16 M2048 N2048 D64 210 -> 50 us.
 // Issuing the matrix instructions of the next tile between the exponentials of the current one (two score sets, two
@@ -32,7 +32,7 @@ struct TotalArgs {
     const float* log_normalizer;  // [B, Hq, M], natural log
     float* total;                 // [B, Hq, N]; of run r at total + r * run_stride
     int64_t run_stride;
-    int32_t runs, run_tiles;      // runs of the queries, query tiles per run
+    int32_t chunk;                // query tiles of a run at most (TotalRuns)
     int32_t BH;                   // batch * heads
     int64_t qs_b, qs_h, qs_n;
     int64_t ks_b, ks_h, ks_n;
@@ -45,6 +45,17 @@ constexpr int kTotalThreads = 64 * kTotalWaves;
 constexpr int kWaveKeys = 64;
 constexpr int kWgKeys = kWaveKeys * kTotalWaves;
 constexpr int kTileQ = 32;
+// The queries that see a key block, cut into runs of about equal length, one workgroup each.
+struct TotalRuns {
+    int tiles, chunk, shift;  // query tiles in all; of a run at most; kv_len - qo_len
+    bool causal;
+    __host__ __device__ int first(int kb) const {  // first query tile that sees a key of block kb: m + shift >= its first key
+        const int m = causal ? kb * kWgKeys - shift : 0;
+        return m > 0 ? m / kTileQ : 0;
+    }
+    __host__ __device__ int count(int kb) const { return (tiles - first(kb) + chunk - 1) / chunk; }
+    __host__ __device__ int len(int kb) const { const int c = count(kb); return (tiles - first(kb) + c - 1) / c; }
+};
 constexpr int kRing = 4;  // query tiles resident in LDS: the one in work and three on their way
 
 // WIDE: the rows of a query tile lie further apart than 32-bit byte offsets reach, or in descending order (64-bit addresses
@@ -65,7 +76,11 @@ __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(Total
     // flag the last queries see every key and the first keys are seen by every query.
     const int nkb = (a.N + kWgKeys - 1) / kWgKeys;
     const int bh = blockIdx.x % a.BH, rest = blockIdx.x / a.BH;
-    const int kb = rest % nkb, run = a.runs - 1 - rest / nkb;
+    const TotalRuns runs{(a.M + kTileQ - 1) / kTileQ, a.chunk, a.N - a.M, a.causal != 0};
+    int kb = 0, run = rest;
+    if (a.chunk >= runs.tiles) kb = rest, run = 0;  // (one run per block)
+    else
+        for (int c; kb < nkb - 1 && run >= (c = runs.count(kb)); kb++) run -= c;
     const int h = bh % a.Hq, b = bh / a.Hq, hk = h / a.groups;
     const int n0 = kb * kWgKeys + wave * kWaveKeys;  // (may lie past the last key: such a wave multiplies copies of it)
     const int shift = a.N - a.M;
@@ -83,10 +98,9 @@ __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(Total
     const VT* qbase = static_cast<const VT*>(a.q) + (int64_t)b * a.qs_b + (int64_t)h * a.qs_h;
     const float* lbase = a.log_normalizer + ((int64_t)b * a.Hq + h) * a.M;
 
-    // the run's queries that can see any key of the workgroup: m + shift >= first key
-    int m_lo = run * a.run_tiles * kTileQ;
-    const int m_hi = min(m_lo + a.run_tiles * kTileQ, a.M);
-    if (a.causal) m_lo = max(m_lo, max(kb * kWgKeys - shift, 0) / kTileQ * kTileQ);
+    // the run's queries
+    const int m_lo = (runs.first(kb) + run * runs.len(kb)) * kTileQ;
+    const int m_hi = min(m_lo + runs.len(kb) * kTileQ, a.M);
 
     const int ntiles = max(m_hi - m_lo + kTileQ - 1, 0) / kTileQ;
 
@@ -209,30 +223,58 @@ __global__ __launch_bounds__(kTotalThreads, 3) void total_attention_kernel(Total
 }
 
 // total[i] = sum of the runs' sums, in order
-__global__ __launch_bounds__(256) void total_runs_kernel(const float* part, float* total, int64_t count, int runs) {
+__global__ __launch_bounds__(256) void total_runs_kernel(const float* part, float* total, int64_t count, int N, TotalRuns runs) {
     const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= count) return;
+    const int n = runs.count((int)(i % N) / kWgKeys);
     float x = 0.0f;
 #pragma unroll 8
-    for (int r = 0; r < runs; r++) x += part[(int64_t)r * count + i];
+    for (int r = 0; r < n; r++) x += part[(int64_t)r * count + i];
     total[i] = x;
 }
 
-// Runs of the queries: four workgroups per CU (under the causal flag half of them have little or nothing to do), at
-// least eight query tiles each.  (B1 H16 M4096 N4096 causal with two / three / four / six per CU: 68 / 63 / 55 / 61 us.)
-int total_runs(int64_t B, int64_t H, int64_t M, int64_t N) {
-    const int64_t items = B * H * ((N + kWgKeys - 1) / kWgKeys), tiles = (M + kTileQ - 1) / kTileQ;
-    int64_t runs = (4 * 256 + items - 1) / items;
-    if (runs > tiles / 8) runs = tiles / 8;
-    if (runs > 64) runs = 64;
-    if (runs <= 1) return 1;
-    const int64_t per = (tiles + runs - 1) / runs;
-    return (int)((tiles + per - 1) / per);  // (no run without a query)
+// Longest run of queries (in tiles): where the key blocks alone do not fill the chip the queries of each are cut into equal
+// runs of at least eight tiles, as many as make three workgroups per CU, all of them resident at once.  (With the same four
+// ranges of queries for every block some CUs held 84 tiles and others 40: B1 H16 M4096 N4096 D128 causal, whole call, 142 -> 135
+// us; B1 H16/2 M4032 136 -> 128, B3 H8/1 M2048 86.5 -> 83.)  Runs that would be long: three times as many, handed out as others
+// end (B6 H2 M9728 D64 causal 285 -> 280 us, 300 with what is resident at once).
+int total_chunk(int64_t BH, int64_t M, int64_t N, bool causal) {
+    constexpr int64_t kResident = 3 * 256, kLongRun = 32;
+    const int64_t nkb = (N + kWgKeys - 1) / kWgKeys, tiles = (M + kTileQ - 1) / kTileQ;
+    if (BH * nkb >= kResident || tiles < 16 || tiles > (1 << 24) || N > (1 << 29)) return (int)tiles;
+    TotalRuns runs{(int)tiles, 1, (int)(N - M), causal};
+    int64_t all = 0;
+    for (int kb = 0; kb < nkb; kb++) all += runs.count(kb);
+    int64_t slots = kResident, chunk = (BH * all + slots - 1) / slots;
+    if (chunk > kLongRun) {
+        slots = 3 * kResident;
+        chunk = (BH * all + slots - 1) / slots;
+        if (chunk < kLongRun) chunk = kLongRun;
+    }
+    if (chunk < (tiles + 63) / 64) chunk = (tiles + 63) / 64;  // (64 runs at most)
+    const int64_t most = tiles / 8;  // (at least eight tiles each)
+    if (chunk < (tiles + most - 1) / most) chunk = (tiles + most - 1) / most;
+    for (; chunk < tiles; chunk++) {
+        runs.chunk = (int)chunk;
+        int64_t wgs = 0;
+        for (int kb = 0; kb < nkb; kb++) wgs += BH * runs.count(kb);
+        if (wgs <= slots) break;
+    }
+    return (int)(chunk < tiles ? chunk : tiles);
 }
 
+int64_t total_run_count(int64_t M, int chunk) { return ((M + kTileQ - 1) / kTileQ + chunk - 1) / chunk; }  // (of the first key block, which has the most)
+
 template <int D, typename VT>
-int launch_total(const TotalArgs& a, int64_t B, int runs, hipStream_t stream) {
-    const int64_t wgs = (int64_t)((a.N + kWgKeys - 1) / kWgKeys) * runs * B * a.Hq;
+int launch_total(const TotalArgs& a, hipStream_t stream) {
+    const int64_t nkb = (a.N + kWgKeys - 1) / kWgKeys;
+    const TotalRuns runs{(a.M + kTileQ - 1) / kTileQ, a.chunk, a.N - a.M, a.causal != 0};
+    int64_t wgs = nkb;
+    if (a.chunk < runs.tiles) {
+        wgs = 0;
+        for (int kb = 0; kb < nkb; kb++) wgs += runs.count(kb);
+    }
+    wgs *= a.BH;
     if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_total_attention: too many key blocks for one launch");
     dim3 grid((unsigned)wgs), block(kTotalThreads);
     const bool wide = a.qs_n < 0 || a.qs_n >= (1LL << 25);  // 31 rows of 2-byte elements pass 2^31 bytes
@@ -244,8 +286,8 @@ int launch_total(const TotalArgs& a, int64_t B, int runs, hipStream_t stream) {
 }  // namespace
 
 int64_t total_workspace_bytes(const sage_flash_params& p) {
-    const int runs = total_runs(p.batch, p.heads_q, p.qo_len, p.kv_len);
-    return runs > 1 ? (int64_t)runs * p.batch * p.heads_q * p.kv_len * (int64_t)sizeof(float) : 0;
+    const int64_t runs = total_run_count(p.qo_len, total_chunk(p.batch * p.heads_q, p.qo_len, p.kv_len, p.causal != 0));
+    return runs > 1 ? runs * p.batch * p.heads_q * p.kv_len * (int64_t)sizeof(float) : 0;
 }
 
 int launch_flash_total_attention(const sage_flash_params& p, const float* log_normalizer, float* total, void* workspace,
@@ -257,11 +299,10 @@ int launch_flash_total_attention(const sage_flash_params& p, const float* log_no
     a.Hq = (int)p.heads_q; a.M = (int)p.qo_len; a.N = (int)p.kv_len; a.groups = (int)(p.heads_q / p.heads_kv);
     a.causal = p.causal ? 1 : 0;
     a.qk_scale = p.sm_scale * 1.44269504089f;
-    int runs = workspace ? total_runs(p.batch, p.heads_q, p.qo_len, p.kv_len) : 1;
-    if (runs > 1 && workspace_bytes < total_workspace_bytes(p)) runs = 1;
-    a.runs = runs;
     a.BH = (int)(p.batch * p.heads_q);
-    a.run_tiles = (int)(((p.qo_len + kTileQ - 1) / kTileQ + runs - 1) / runs);
+    const int tiles = (int)((p.qo_len + kTileQ - 1) / kTileQ);
+    a.chunk = workspace && workspace_bytes >= total_workspace_bytes(p) ? total_chunk(a.BH, p.qo_len, p.kv_len, p.causal != 0) : tiles;
+    const int64_t runs = total_run_count(p.qo_len, a.chunk);
     const int64_t count = p.batch * p.heads_q * p.kv_len;
     if (runs > 1) {
         a.total = static_cast<float*>(workspace);
@@ -269,13 +310,14 @@ int launch_flash_total_attention(const sage_flash_params& p, const float* log_no
     }
     int rc;
     if (p.head_dim == 128)
-        rc = p.dtype == SAGE_BF16 ? launch_total<128, __bf16>(a, p.batch, runs, stream) : launch_total<128, _Float16>(a, p.batch, runs, stream);
+        rc = p.dtype == SAGE_BF16 ? launch_total<128, __bf16>(a, stream) : launch_total<128, _Float16>(a, stream);
     else
-        rc = p.dtype == SAGE_BF16 ? launch_total<64, __bf16>(a, p.batch, runs, stream) : launch_total<64, _Float16>(a, p.batch, runs, stream);
+        rc = p.dtype == SAGE_BF16 ? launch_total<64, __bf16>(a, stream) : launch_total<64, _Float16>(a, stream);
     if (rc || runs == 1) return rc;
     const int64_t wgs = (count + 255) / 256;
     if (wgs > 0x7fffffffLL) return fail(SAGE_E_UNSUPPORTED, "sage_flash_total_attention: too many keys for one launch");
-    hipLaunchKernelGGL(total_runs_kernel, dim3((unsigned)wgs), dim3(256), 0, stream, (const float*)workspace, total, count, runs);
+    hipLaunchKernelGGL(total_runs_kernel, dim3((unsigned)wgs), dim3(256), 0, stream, (const float*)workspace, total, count, a.N,
+                       TotalRuns{tiles, a.chunk, a.N - a.M, a.causal != 0});
     return check_launch("total_runs_kernel");
 }
 

@@ -83,3 +83,33 @@ def test_total_attention_keeps_nan(M, N, causal, where, gpu_device):
     torch.cuda.synchronize()
     for got in (one, runs) if where == "normalizer_nan" else (tot, one, runs):
         assert torch.equal(torch.isnan(got), want) and bool(torch.isfinite(got[~want]).all())
+
+
+@pytest.mark.parametrize("B,H,Hk,M,N,D,causal", [
+    (1, 2, 2, 1024, 1024, 64, True),     # runs of the fewest tiles, a different number for every key block
+    (1, 3, 1, 700, 2300, 128, True),     # fewer queries than keys: every block is seen by the last queries
+    (1, 2, 2, 2300, 700, 64, True),      # more: the first queries see no key
+    (2, 4, 4, 3000, 2900, 64, False),    # long runs
+])
+def test_total_attention_runs(B, H, Hk, M, N, D, causal, gpu_device):
+    """Runs of different numbers per key block against one run per block (no workspace)."""
+    import flag_attn
+    from flagattention_amd import _lib
+    from flagattention_amd.sage_attention._common import tensor_desc
+
+    g = torch.Generator().manual_seed(M)
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(torch.float16).to(gpu_device) for h, n in ((H, M), (Hk, N), (Hk, N)))
+    o, L, tot, *_ = flag_attn.flash_attention(q, k, v, causal, return_log_normalizer=True, return_total_attention=True)
+    p = _lib.FlashParams()
+    p.q, p.k, p.v, p.out = (tensor_desc(t, True) for t in (q, k, v, o))
+    p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.head_dim = B, H, Hk, M, N, D
+    p.dtype = p.out_dtype = _lib.SAGE_F16
+    p.causal, p.sm_scale = int(causal), D ** -0.5
+    lib = _lib.load()
+    assert lib.sage_flash_total_attention_workspace_bytes(p) > 0
+    one = torch.empty_like(tot)
+    _lib.check(lib.sage_flash_total_attention(p, L.data_ptr(), one.data_ptr(), torch.cuda.current_stream().cuda_stream), "total")
+    torch.cuda.synchronize()
+    torch.testing.assert_close(tot, one, rtol=1e-5, atol=1e-5)  # (fp32 sums of the same terms in another order)
+    seen = int((~torch.isinf(L)).sum())
+    assert abs(tot.sum().item() - seen) <= 2e-3 * seen
