@@ -70,6 +70,7 @@ EXPORTS = (
     "sage_attn_fwd",
     "sage_attn_fwd_workspace_bytes",
     "sage_attn_fwd_ws",
+    "sage_attn_fwd_natural",
     "sage_lse_natural",
     "sage_flash_attn_fwd",
     "sage_flash_attn_fwd_workspace_bytes",
@@ -117,6 +118,9 @@ def load():
     lib.sage_attn_fwd_workspace_bytes.restype = c_i64
     lib.sage_attn_fwd_ws.argtypes = [ctypes.POINTER(AttnParams), ctypes.c_void_p, c_i64, ctypes.c_void_p]
     lib.sage_attn_fwd_ws.restype = ctypes.c_int
+    lib.sage_attn_fwd_natural.argtypes = [ctypes.POINTER(AttnParams), ctypes.c_void_p, ctypes.c_float, ctypes.c_void_p, c_i64,
+                                          ctypes.c_void_p]
+    lib.sage_attn_fwd_natural.restype = ctypes.c_int
     lib.sage_lse_natural.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, c_i64, ctypes.c_void_p]
     lib.sage_lse_natural.restype = ctypes.c_int
     lib.sage_flash_attn_fwd_workspace_bytes.argtypes = [ctypes.POINTER(FlashParams)]

@@ -69,6 +69,8 @@ struct AttnArgs {
     float* part_o;     // [2 * cut_wgs slots][256 rows x D, in the order of the accumulator registers]
     float* part_lse;   // [2 * cut_wgs][256]
     float lse_mul;     // factor on the base-2 log-sum-exp on its way out (1: as is; ln 2: natural log)
+    const float* lse_shift;  // (null: none) [B, Hq, M], added to it with the factor lse_shift_mul: what K smoothing took off the logits
+    float lse_shift_mul;
     // (mask tensors, pipelined kernel) what mask_scan_kernel found (null: every tile is visited): per strip of kScanRows mask
     // rows and 64-key tile the largest entry, per strip the smallest of its rows' largest entries, per 64-key tile of V
     // whether it holds an Inf or NaN.  scan_strips: strips of a mask batch.  visit_group: tiles per bit of the visit word.
@@ -119,6 +121,12 @@ struct CutLine {
         return r - (p == 0 ? 0 : first_pair + (p - 1) * pair) < len(longer) || 2 * p == live - 1 ? longer : dead + p;
     }
 };
+// the log-sum-exp of a row as the caller gets it, from its base-2 one
+__device__ __forceinline__ float lse_out(float lse2, float mul, const float* shift, float shift_mul, int64_t row) {
+    const float x = lse2 * mul;
+    return shift ? __builtin_fmaf(shift[row], shift_mul, x) : x;
+}
+
 // first step of share w of W (total steps < 2^23, W <= 256), and the share that holds step pos
 __host__ __device__ inline int cut_begin(int w, int W, int total) { return (int)((unsigned)w * (unsigned)total / (unsigned)W); }
 __host__ __device__ inline int cut_owner(int pos, int W, int total) {

@@ -240,7 +240,8 @@ __global__ __launch_bounds__(64 * kDecodeWaves, RT == 1 ? 8 / kDecodeWaves : 1) 
         const float f = l > 0.0f ? __builtin_amdgcn_exp2f(m_i[rt] - m_use) / l : 0.0f;
         if (a.lse && wave == 0 && half == 0 && row0 + r < rows) {
             const int g = (row0 + r) / a.M, mi = row0 + r - g * a.M;
-            a.lse[((int64_t)b * a.Hq + hk * a.groups + g) * a.M + mi + split * a.lse_split_stride] = (__builtin_log2f(l) + m) * a.lse_mul;
+            const int64_t row = ((int64_t)b * a.Hq + hk * a.groups + g) * a.M + mi;
+            a.lse[row + split * a.lse_split_stride] = lse_out(__builtin_log2f(l) + m, a.lse_mul, a.lse_shift, a.lse_shift_mul, row);
         }
         // CH channels of every wave's rows at a time through LDS: all of them where a wave slice fits, else 32
         float* slice = reinterpret_cast<float*>(smem);

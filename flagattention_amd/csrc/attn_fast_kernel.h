@@ -1129,7 +1129,10 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             }
     }
     if (row_ok && !to_part) {
-        if (a.lse && half == 0) a.lse[((int64_t)b * a.Hq + h) * a.M + my_m + split * a.lse_split_stride] = (__builtin_log2f(l_tot) + m_i) * a.lse_mul;
+        if (a.lse && half == 0) {
+            const int64_t row = ((int64_t)b * a.Hq + h) * a.M + my_m;
+            a.lse[row + split * a.lse_split_stride] = lse_out(__builtin_log2f(l_tot) + m_i, a.lse_mul, a.lse_shift, a.lse_shift_mul, row);
+        }
     }
     // The output staging in LDS has been read: the next q-block may fill the tile buffers.  (Not __syncthreads, which
     // would wait for the output to arrive in memory as well.)

@@ -529,8 +529,13 @@ int64_t attn_split_workspace_bytes(const sage_attn_params& p) {
     return attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim);
 }
 
-int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream) {
+int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream, bool natural,
+                const float* shift, float shift_mul) {
     AttnArgs a = attn_args(p);
+    if (natural) {
+        a.lse_mul = 0.693147180559945309f;
+        a.lse_shift = shift; a.lse_shift_mul = shift_mul;
+    }
     const int64_t total = p.batch * p.heads_q * a.nq;
     if (total > 0x7fffffffLL || p.qo_len > 0x7fffffffLL - BM || p.kv_len > 0x7fffffffLL - BN)
         return fail(SAGE_E_UNSUPPORTED, "sage_attn_fwd: problem too large for 32-bit tile indices");
@@ -574,12 +579,11 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
             if (int rc = attn::launch_mask_scan(a, p.batch, (int)p.head_dim, p.v_dtype, workspace, stream)) return rc;
         return attn::launch_fast_masked(a, (int)p.head_dim, p.v_dtype, stream);
     }
-    if (p.head_dim == 128) {
-        return p.v_dtype == SAGE_BF16 ? launch_mode<128, __bf16>(a, mode, stream)
-                                      : launch_mode<128, _Float16>(a, mode, stream);
-    }
-    return p.v_dtype == SAGE_BF16 ? launch_mode<64, __bf16>(a, mode, stream)
-                                  : launch_mode<64, _Float16>(a, mode, stream);
+    int rc;
+    if (p.head_dim == 128) rc = p.v_dtype == SAGE_BF16 ? launch_mode<128, __bf16>(a, mode, stream) : launch_mode<128, _Float16>(a, mode, stream);
+    else rc = p.v_dtype == SAGE_BF16 ? launch_mode<64, __bf16>(a, mode, stream) : launch_mode<64, _Float16>(a, mode, stream);
+    if (rc || !natural || !p.lse) return rc;
+    return attn::launch_lse_natural(p.lse, shift, shift_mul, p.batch * p.heads_q * p.qo_len, stream);  // (the general kernel writes base 2)
 }
 
 }  // namespace sage

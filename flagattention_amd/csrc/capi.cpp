@@ -167,6 +167,13 @@ extern "C" int sage_attn_fwd_ws(const sage_attn_params* p, void* workspace, int6
     return launch_attn(*p, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
+extern "C" int sage_attn_fwd_natural(const sage_attn_params* p, const float* shift, float shift_mul, void* workspace,
+                                     int64_t workspace_bytes, void* stream) {
+    if (int rc = check_attn_params(p)) return rc;
+    if (int rc = check_workspace("sage_attn_fwd_natural", workspace, workspace_bytes)) return rc;
+    return launch_attn(*p, workspace, workspace_bytes, (hipStream_t)stream, true, shift, shift_mul);
+}
+
 extern "C" int sage_lse_natural(float* lse, const float* shift, float shift_mul, int64_t n, void* stream) {
     if (!lse || n < 0) return fail(SAGE_E_INVALID, "sage_lse_natural: null pointer or negative size");
     if (n == 0) return SAGE_OK;

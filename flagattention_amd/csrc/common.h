@@ -27,7 +27,9 @@ int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_k
 int static_scratch(void** out);
 // workspace: device memory for the partial results of a key split, or null (then the keys are never split);
 // *_split_workspace_bytes: what the launch would use of it (0: it would not split)
-int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream);
+// natural: the log-sum-exp leaves as sage_lse_natural would make it
+int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream, bool natural = false,
+                const float* shift = nullptr, float shift_mul = 0.0f);
 int launch_flash_attn(const sage_flash_params& p, void* workspace, int64_t workspace_bytes, hipStream_t stream);
 int64_t attn_split_workspace_bytes(const sage_attn_params& p);
 int64_t flash_split_workspace_bytes(const sage_flash_params& p);

@@ -235,14 +235,15 @@ PyObject* put_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {  // + (params
     });
 }
 
-// ---- SageAttention forward: (q, k, v, q_scale, k_scale, layout, mask, out_dtype, return_lse, causal)
+// ---- SageAttention forward: (q, k, v, q_scale, k_scale, layout, mask, out_dtype, return_lse, causal, lse_mul, lse_shift)
 struct AttnCall {
-    const at::Tensor *q, *k, *v, *qs, *ks, *mask = nullptr;
-    bool hnd, want_lse, causal;
+    const at::Tensor *q, *k, *v, *qs, *ks, *mask = nullptr, *shift = nullptr;
+    bool hnd, want_lse, causal, natural = false;
+    double lse_mul = 0.0;
     at::ScalarType out;
     Key key;
     bool parse(PyObject* const* a, Py_ssize_t n) {
-        if (n < 10) return false;
+        if (n < 12) return false;
         for (int i = 0; i < 5; i++)
             if (!plain(a[i])) return false;
         q = &THPVariable_Unpack(a[0]); k = &THPVariable_Unpack(a[1]); v = &THPVariable_Unpack(a[2]);
@@ -253,6 +254,15 @@ struct AttnCall {
         }
         if (!is_hnd(a[5], hnd) || !THPDtype_Check(a[7]) || !is_bool(a[8], want_lse) || !is_bool(a[9], causal)) return false;
         out = reinterpret_cast<THPDtype*>(a[7])->scalar_type;
+        if (a[10] != Py_None) {
+            if (!PyFloat_CheckExact(a[10])) return false;
+            natural = true;
+            lse_mul = PyFloat_AS_DOUBLE(a[10]);
+            if (a[11] != Py_None) {
+                if (!plain(a[11])) return false;
+                shift = &THPVariable_Unpack(a[11]);
+            }
+        }
         key.add((int64_t)2);
         key.add(*q);
         key.add(*k);
@@ -262,7 +272,8 @@ struct AttnCall {
         key.add((int64_t)(mask != nullptr));
         if (mask) key.add(*mask);
         key.add((int64_t)out);
-        key.add((int64_t)(hnd | causal << 1));
+        key.add((int64_t)(hnd | causal << 1 | natural << 2 | (shift != nullptr) << 3));
+        if (shift) key.add(*shift);
         key.add((int64_t)q->device().index());
         return true;
     }
@@ -276,7 +287,8 @@ PyObject* attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
         if (!plan) return none();
         const at::Device dev = c.q->device();
         if (!dev.is_cuda() || c10::hip::current_device() != dev.index() || !ready(*c.q, dev) || !ready(*c.k, dev) || !ready(*c.v, dev) ||
-            c.qs->device() != dev || c.ks->device() != dev || (c.mask && !ready(*c.mask, dev)))
+            c.qs->device() != dev || c.ks->device() != dev || (c.mask && !ready(*c.mask, dev)) ||
+            (c.shift && c.shift->device() != dev))
             return none();
         auto& p = *reinterpret_cast<sage_attn_params*>(&plan->params[0]);
         const at::Tensor o = at::empty(c.q->sizes(), options(dev, c.out));
@@ -287,8 +299,11 @@ PyObject* attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
         p.lse = c.want_lse ? (float*)lse.data_ptr() : nullptr;
         p.mask = c.mask ? c.mask->data_ptr() : nullptr;
         void* stream = c10::hip::getCurrentHIPStream(dev.index()).stream();
-        const int rc = plan->workspace > 0 ? sage_attn_fwd_ws(&p, workspace(dev, plan->workspace).data_ptr(), plan->workspace, stream)
-                                           : sage_attn_fwd(&p, stream);
+        at::Tensor ws;
+        if (plan->workspace > 0) ws = workspace(dev, plan->workspace);
+        void* wp = plan->workspace > 0 ? ws.data_ptr() : nullptr;
+        const int rc = c.natural ? sage_attn_fwd_natural(&p, c.shift ? (const float*)c.shift->data_ptr() : nullptr, (float)c.lse_mul, wp, plan->workspace, stream)
+                                 : sage_attn_fwd_ws(&p, wp, plan->workspace, stream);
         if (rc) return PyLong_FromLong(rc);
         return pack({&o, &lse});
     });
@@ -297,8 +312,8 @@ PyObject* attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* put_attn(PyObject*, PyObject* const* a, Py_ssize_t n) {  // + (params, workspace bytes)
     return guarded([&]() -> PyObject* {
         AttnCall c;
-        if (n != 12 || !c.parse(a, n)) return none();
-        return put(c.key, a[10], a[11], false);
+        if (n != 14 || !c.parse(a, n)) return none();
+        return put(c.key, a[12], a[13], false);
     });
 }
 

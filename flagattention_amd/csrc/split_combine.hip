@@ -26,7 +26,8 @@ struct CombineArgs {
     int64_t os_b, os_h, os_n;
     int64_t rows;           // batch * heads_q * qo_len
     int32_t Hq, M, nsplit, out_dt;
-    float lse_mul;
+    float lse_mul, lse_shift_mul;
+    const float* lse_shift;
 };
 
 constexpr int kCombineThreads = 256;
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineA
     const int64_t b = row / ((int64_t)a.M * a.Hq);
     const int64_t o = b * a.os_b + (int64_t)h * a.os_h + (int64_t)mi * a.os_n + 4 * c;
     store4(a.out, a.out_dt, o, r);
-    if (a.lse && c == 0) a.lse[row] = (__builtin_log2f(den) + m) * a.lse_mul;  // den = 0: log2(0) + (-inf) = -inf
+    if (a.lse && c == 0) a.lse[row] = lse_out(__builtin_log2f(den) + m, a.lse_mul, a.lse_shift, a.lse_shift_mul, row);  // den = 0: log2(0) + (-inf) = -inf
 }
 
 // One wave tile (32 rows) of one item of a cut launch: the parts lie in the order of the accumulator registers, so a
@@ -151,7 +152,10 @@ __global__ __launch_bounds__(kCombineThreads) void cut_combine_kernel(AttnArgs a
     }
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;
     const int b = bh / a.Hq, h = bh % a.Hq;
-    if (a.lse && t < 32 && m0 + row < a.M) a.lse[(int64_t)bh * a.M + m0 + row] = (__builtin_log2f(den) + m) * a.lse_mul;
+    if (a.lse && t < 32 && m0 + row < a.M) {
+        const int64_t r = (int64_t)bh * a.M + m0 + row;
+        a.lse[r] = lse_out(__builtin_log2f(den) + m, a.lse_mul, a.lse_shift, a.lse_shift_mul, r);
+    }
 #pragma unroll
     for (int e = 0; e < kPieces; e++) {
         const int piece = t / 64 + 4 * e;  // 4 * (32-channel tile) + register group
@@ -364,6 +368,7 @@ void apply_key_split(AttnArgs& a, int nsplit, int64_t batch, int head_dim, void*
     a.lse = static_cast<float*>(workspace) + (int64_t)nsplit * rows * head_dim;
     a.lse_split_stride = rows;
     a.lse_mul = 1.0f;
+    a.lse_shift = nullptr;
 }
 
 int launch_split_combine(const AttnArgs& split, const AttnArgs& whole, int head_dim, int64_t batch, hipStream_t stream) {
@@ -374,7 +379,7 @@ int launch_split_combine(const AttnArgs& split, const AttnArgs& whole, int head_
     c.os_b = whole.os_b; c.os_h = whole.os_h; c.os_n = whole.os_n;
     c.rows = batch * whole.Hq * whole.M;
     c.Hq = whole.Hq; c.M = whole.M; c.nsplit = split.nsplit; c.out_dt = whole.out_dt;
-    c.lse_mul = whole.lse_mul;
+    c.lse_mul = whole.lse_mul; c.lse_shift = whole.lse_shift; c.lse_shift_mul = whole.lse_shift_mul;
     // eight groups per row while rows alone would leave compute units idle
     const int sg = c.rows * (head_dim / 4) < kComputeUnits * kCombineThreads && c.nsplit >= 8 ? 8 : 1;
     const int rows_per_wg = kCombineThreads / (head_dim / 4 * sg);

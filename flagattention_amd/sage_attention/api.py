@@ -1,9 +1,7 @@
 """One-call SageAttention: K mean -> fused smoothing + quantization -> INT8 attention."""
 from __future__ import annotations
 
-from .. import _lib
-from ._common import current_stream_ptr, device_guard
-from .attention import forward
+from .attention import _attend
 from .quant import per_block_int8, per_block_int8_smooth_k
 
 
@@ -26,16 +24,7 @@ def sageattn(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, smoot
                                                              with_q_dot_km=return_lse)
     else:
         q8, qs, k8, ks = per_block_int8(q, k, sm_scale=sm_scale, tensor_layout=tensor_layout)
-    o, lse2 = forward(q8, k8, v, qs, ks, tensor_layout=tensor_layout, output_dtype=output_dtype,
-                      return_lse=return_lse, causal=is_causal)
-    if not return_lse:
-        return o
-    # one pass over the fresh lse (three torch calls with the scale copied to the device cost 14 us of GPU time and
-    # a host wait of 30 us at B1 H32 M3001)
-    if lse2.numel():
-        shift = None if q_dot_km is None else q_dot_km.contiguous()
-        with device_guard(lse2.device):
-            _lib.check(_lib.load().sage_lse_natural(lse2.data_ptr(), None if shift is None else shift.data_ptr(),
-                                                    float(sm_scale), lse2.numel(), current_stream_ptr(lse2.device)),
-                       "sage_lse_natural")
-    return o, lse2
+    # (the attention launch itself writes the natural log-sum-exp: a launch of its own for it took 4.8 us of B1 H32/8 N3001's 94)
+    o, lse = _attend(q8, k8, v, qs, ks, tensor_layout, None, output_dtype, return_lse, None, is_causal, float(sm_scale),
+                     None if q_dot_km is None else q_dot_km.contiguous())
+    return (o, lse) if return_lse else o

@@ -168,7 +168,13 @@ def forward(q, k, v, q_scale, k_scale, tensor_layout="HND", attn_mask=None,
     ``causal=True`` (keyword only, not in the reference) applies the bottom-right aligned causal
     mask ``n <= m + (N - M)`` with whole-tile skipping.
     """
-    call = (q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, causal)
+    return _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg, causal)
+
+
+def _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg, causal, lse_mul=None, lse_shift=None):
+    """``forward``; with a number ``lse_mul`` the log-sum-exp is the natural one plus ``lse_mul * lse_shift`` (``[B, Hq, M]``
+    fp32 contiguous, or None), what ``sageattn`` returns."""
+    call = (q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, causal, lse_mul, lse_shift)
     if maxnreg is None:
         out = (_lib._host_module or _lib.host()).attn(*call)  # a call shape seen before: outputs, or a status
         if out is not None:
@@ -205,8 +211,8 @@ def forward(q, k, v, q_scale, k_scale, tensor_layout="HND", attn_mask=None,
         # copies (the reference takes whatever its compiler's dot takes, attn_qk_int8_per_block.py:161,185).
         pad = (0, 64 - head_dim)
         qp, kp, vp = (torch.nn.functional.pad(t, pad) for t in (q, k, v))
-        o, lse = forward(qp, kp, vp, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg,
-                         causal=causal)
+        o, lse = _attend(qp, kp, vp, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg, causal, lse_mul,
+                         lse_shift)
         return o[..., :head_dim].contiguous(), lse
     if head_dim not in (64, 128):
         raise ValueError(f"head_dim {head_dim} not supported (16, 32, 64 or 128)")
@@ -242,6 +248,8 @@ def forward(q, k, v, q_scale, k_scale, tensor_layout="HND", attn_mask=None,
             o.zero_()
             if return_lse:
                 lse.fill_(float("-inf"))
+                if lse_shift is not None:
+                    lse += lse_mul * lse_shift
             return o, lse
 
         stream = current_stream_ptr(dev)
@@ -333,7 +341,12 @@ def forward(q, k, v, q_scale, k_scale, tensor_layout="HND", attn_mask=None,
         p.mask = None if m is None else m.data_ptr()
         if ws_bytes > 0:
             ws = split_workspace(dev, ws_bytes)
-            _lib.check(lib.sage_attn_fwd_ws(p_ref, ws.data_ptr(), ws.numel(), stream), "sage_attn_fwd_ws")
+            ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
         else:
-            _lib.check(lib.sage_attn_fwd(p_ref, stream), "sage_attn_fwd")
+            ws_ptr, ws_bytes = None, 0
+        if lse_mul is None:
+            _lib.check(lib.sage_attn_fwd_ws(p_ref, ws_ptr, ws_bytes, stream), "sage_attn_fwd_ws")
+        else:
+            _lib.check(lib.sage_attn_fwd_natural(p_ref, None if lse_shift is None else lse_shift.data_ptr(), lse_mul, ws_ptr, ws_bytes,
+                                                 stream), "sage_attn_fwd_natural")
     return o, lse

@@ -132,6 +132,9 @@ int sage_attn_fwd_ws(const sage_attn_params* p, void* workspace, int64_t workspa
  * lse[i] = ln 2 * lse[i] + shift_mul * shift[i] for n contiguous values.  shift: what smoothing took off the logits of a
  * row before scaling (q_dot_km of sage_per_block_int8_smooth_k, shift_mul = sm_scale), or NULL.
  */
+/* sage_attn_fwd_ws whose log-sum-exp leaves as sage_lse_natural would make it (shift: [B, Hq, M] contiguous, or NULL). */
+int sage_attn_fwd_natural(const sage_attn_params* p, const float* shift, float shift_mul, void* workspace, int64_t workspace_bytes,
+                          void* stream);
 int sage_lse_natural(float* lse, const float* shift, float shift_mul, int64_t n, void* stream);
 
 /*
