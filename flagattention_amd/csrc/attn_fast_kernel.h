@@ -791,10 +791,14 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         v4f sum4 = {0.0f, 0.0f, 0.0f, 0.0f};
         unsigned long long large = 0;
         auto redo_if_large = [&]() {
+            // (In the padding step the sums of a NaN row are NaN too.  Redone, it would add the tile to the other rows of the wave
+            // once more; the sums are dropped instead: a row sum of the matrix core is NaN beside a NaN row as well.)
             if constexpr (MADD) {
                 // a ragged last tile always comes here: its keys past kv_len score -1e6 (the reference reads their
                 // mask entries as -1e6 and their K as zeros), which only this path accounts for
-                if (large != 0 || (ragged && live && vt0 == nk - 1)) {
+                if (large != 0 && !live) {
+                    lsum = 0.0f;
+                } else if (large != 0 || (ragged && live && vt0 == nk - 1)) {
                     float raw = -INFINITY;
                     float past_end = 0.0f;  // number of the lane's keys of this step that lie past kv_len
                     sfor<4>([&](auto tc) {
@@ -850,7 +854,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                 return;
             }
             if constexpr (MASK) {
-                if (large != 0 && !tile_has_visible_key(mslot)) {
+                if (large != 0 && (!live || !tile_has_visible_key(mslot))) {
                     // no visible key for this 128-row block in this tile: the reference skips it.  (Rows without a
                     // reference point get here every step until they see a key: their P came out inf or NaN.)
 #pragma unroll
@@ -907,7 +911,9 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                 }
                 return;
             }
-            if (large != 0) {
+            if (large != 0 && !live) {
+                lsum = 0.0f;
+            } else if (large != 0) {
                 float raw = -INFINITY;
 #pragma unroll
                 for (int kt = 0; kt < 2; kt++)

@@ -149,3 +149,44 @@ def test_additive_mask_rows_that_meet_hidden_tiles_first(mask_dtype, d, gpu_devi
     want = torch.softmax(s * math.log(2.0), -1) @ v.double()
     torch.testing.assert_close(o.double().cpu(), want, rtol=2e-2, atol=2e-2)
     torch.testing.assert_close(lse.double().cpu(), torch.logsumexp(s * math.log(2.0), -1) / math.log(2.0), rtol=1e-4, atol=2e-3)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("n", [2112, 2112 + 40])  # 33 steps of 64 keys, an odd number; a ragged last one
+def test_a_nan_query_leaves_its_neighbours_alone(n, causal, d, gpu_device):
+    """A NaN query row makes every step of its wave look too large, the padding step after an odd number included: the other
+    rows of the wave have to come out as without it."""
+    import flag_attn
+    from oracle import flash_oracle as FO
+
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(1, 16, x, d, generator=g).to(torch.float16) for x in (n, n, n))
+    bad = [3, 70, n - 5]
+    q_nan = q.clone()
+    q_nan[:, :, bad] = float("nan")
+    o, lse, *_ = flag_attn.flash_attention(q_nan.to(gpu_device), k.to(gpu_device), v.to(gpu_device), causal, return_log_normalizer=True)
+    want, want_lse = FO.attention(q[:, :2], k[:, :2], v[:, :2], causal, return_log_normalizer=True)
+    keep = [i for i in range(n) if i not in bad]
+    torch.testing.assert_close(lse.cpu()[:, :2, keep], want_lse[:, :, keep], atol=2e-3, rtol=1e-4)
+    torch.testing.assert_close(o.cpu()[:, :2, keep].float(), want[:, :, keep].float(), atol=4e-3, rtol=1e-2)
+    assert torch.isnan(o[:, :, bad]).all() and torch.isnan(lse[:, :, bad]).all()
+
+
+@pytest.mark.parametrize("mask_dtype", [torch.float16, torch.float32])
+def test_a_nan_mask_entry_leaves_its_neighbours_alone(mask_dtype, gpu_device):
+    from flag_attn import sage_attention as sa
+    from oracle import sage_oracle as O
+
+    g = torch.Generator().manual_seed(2)
+    n = 320
+    q, k, v = (torch.randn(1, 2, n, 64, generator=g).to(torch.float16) for _ in range(3))
+    args = [t.to(gpu_device) for t in O.per_block_int8(q, k)]
+    mask = torch.randn(1, 2, n, n, generator=g).to(mask_dtype).to(gpu_device)
+    o, lse = sa.sage_attention(args[0], args[2], v.to(gpu_device), args[1], args[3], attn_mask=mask, return_lse=True)
+    mask[0, :, 100, 7] = float("nan")
+    o_nan, lse_nan = sa.sage_attention(args[0], args[2], v.to(gpu_device), args[1], args[3], attn_mask=mask, return_lse=True)
+    rows = [i for i in range(n) if i != 100]
+    torch.testing.assert_close(lse_nan[:, :, rows], lse[:, :, rows], atol=2e-3, rtol=1e-4)
+    torch.testing.assert_close(o_nan[:, :, rows].float(), o[:, :, rows].float(), atol=4e-3, rtol=1e-2)
+    assert torch.isnan(o_nan[:, :, 100]).all() and torch.isnan(lse_nan[:, :, 100]).all()
