@@ -196,6 +196,7 @@ int launch_decode(const AttnArgs& a, int64_t batch, int head_dim, int v_dtype, b
 bool fast_serves_mask(const AttnArgs& a, int esz);
 int launch_fast_masked(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
 int launch_fast_additive(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
+int launch_fast_additive_causal(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
 
 // The scan of a mask that the heads share, ahead of the pipelined kernel (mask_scan.hip): bytes of workspace it takes (0: the
 // rule on sizes says no), and its launch, which fills the scan fields of `a`.

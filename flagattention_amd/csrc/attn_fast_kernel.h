@@ -116,7 +116,8 @@ __device__ __forceinline__ typename PV<VT>::vec tr_pair(const unsigned char* p0,
 // follows).  The entry is added to the exponent of its score: fma(score, scale, entry - m).  Rows start from the
 // reference point -inf like those of the bool instance, so the first step of every row runs the path that redoes a
 // step, which takes the row maximum of score * scale + entry; so does a ragged last tile, whose keys past kv_len
-// score -1e6 there as in the reference (mask entries read as -1e6, K as zeros).
+// score -1e6 there as in the reference (mask entries read as -1e6, K as zeros), and so do the tiles of the diagonal under the causal
+// flag (c_first below).
 // fp32 entries: 8 KB per wave and step, ONE step resident (two would not fit beside the K/V tiles): the entries of
 // step j + 1 are requested at the end of the vector phase of step j, once its last entry has been read, and waited for
 // at the end of the matrix phase that follows; the path that redoes a step reads its entries from memory again.
@@ -137,7 +138,9 @@ template <> __device__ __forceinline__ float mask_entry<_Float16>(unsigned word,
 // CUT: a workgroup takes share blockIdx of the launch's steps (CutLine) instead of whole q-blocks: the end of one item,
 // whole ones, the beginning of another.  Without a mask tensor.  The step loop is that of the whole launch (B2 H32/8 N4096
 // causal, where no item is cut: 214 us against 210 us for pairs); a piece costs about five steps, a partial result 2.5.
-template <int D, typename VT, bool CAUSAL, int QB, typename MT = void, bool CUT = false>
+// MC: an additive mask tensor with the causal flag, instances of their own (in the same ones B4 H8 M320 N320 D128 fp16 19.6 -> 21.0 us
+// without the flag).
+template <int D, typename VT, bool CAUSAL, int QB, typename MT = void, bool CUT = false, bool MC = false>
 __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast_kernel(AttnArgs args, int nq2) {
     const AttnArgs& a = args;
     using F = FT<D, QB>;
@@ -149,6 +152,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     constexpr int kMaskWaveBytes = 32 * BN * MaskT<MT>::BYTES;   // 32 rows x 64 keys
     constexpr int kMaskInstr = kMaskWaveBytes / 1024;            // loads per wave and step
     constexpr int kMaskBytes = kMaskSlots * kFastWaves * kMaskWaveBytes;
+    static_assert(!MC || MADD, "the causal flag on top of an additive mask");
     static_assert(!MASK || (CAUSAL && INT8), "the mask instances build on the key-hiding int8 instance");
     constexpr float BIAS = INT8 ? kBias : 0.0f;  // what the bits of a fresh score accumulator read as a float
     using PVT = PV<VT>;
@@ -342,6 +346,17 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     //      Additive 16-bit entries: 128 bytes per row, eight lanes per row, instruction e carries rows 8 e .. 8 e + 7;
     //      the eight chunks of a row are XOR-swizzled in pairs with bits 0-1 of the row number (a lane reads the two
     //      chunks of a 16-key slice with one instruction: they stay neighbours).
+    // (MC) Additive mask with the causal flag: the reference adds -1e6 where the causal mask hides a key, on top of the
+    // entry, and skips the 128 x 64 tiles that hide every key.  Steps whose tile reaches past the limit of the wave's first
+    // row (c_first) therefore take the path that redoes a step, which adds it; past the limit of the last row of the wave's
+    // 128-row block (c_block) their P is 0.
+    const int c_first = MC ? m0 + 32 * wave_u + shift : 0, c_block = MC ? min(m0 + BM * (wave_u / 4) + BM - 1, a.M - 1) + shift : 0;
+    // what the causal mask adds to the entry of score register i of tile kt, for the lane's row (derived again where it is used)
+    auto causal_entry = [&](int n_first, int kt, int i) {
+        const int ln = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+        const int n = n_first + 32 * kt + 8 * (i >> 2) + 4 * (ln >> 5) + (i & 3);
+        return n > c_first + (ln & 31) ? kMaskedScore : 0.0f;
+    };
     const unsigned char* mask_row0 = nullptr;  // uniform: this wave's first mask row
     constexpr int MB = MaskT<MT>::BYTES;       // bytes per mask entry
     constexpr int kMaskLPR = BN * MB / 16;     // lanes (16-byte chunks) per staged row: 4 | 8
@@ -418,7 +433,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     // ---- (MASK) the tiles this workgroup visits.  Bit g of `visits` stands for tiles g * visit_group .. of the walk
     //      over the keys (visit_group = 1 up to 4096 keys); clear where mask_scan_kernel found that a visit changes nothing:
     //      an additive entry so far below the largest one of every row that its P is exactly 0 whatever the scores
-    //      (|q.k| <= 2^14 D and the scales bound them), a bool tile without a visible key (the reference skips it), and no
+    //      (|q.k| <= 128 sum |q|, and the scales bound them), a bool tile without a visible key (the reference skips it), and no
     //      Inf or NaN in V (0 times those is NaN).  Comparisons with a NaN scale or entry are false: such a tile is visited.
     unsigned long long visits = ~0ull;
     int visit_group = 1, visit_g = 0, visit_rest = 0;  // tiles per bit; the bit of the youngest tile below, the tile within it
@@ -459,10 +474,27 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             }
 #pragma unroll
             for (int x = 1; x < 64; x <<= 1) ks_max = fmaxf(ks_max, __shfl_xor(ks_max, x));
-            const float* qsp = a.q_scale + ((int64_t)b * a.Hq + h) * a.nq;
-            const float bound = MADD ? 2.0f * 16384.0f * D * ks_max : 0.0f;  // 2 max |q.k| over the Q scale
-            const float q0 = qsp[min((kFastRows / BM) * iq, a.nq - 1)], q1 = qsp[min((kFastRows / BM) * iq + 1, a.nq - 1)];
-            const bool skip = top < low - 150.0f - bound * q0 && top < low - 150.0f - bound * q1 && !odd;
+            float bound = 0.0f;  // largest difference of two scores of a row
+            if constexpr (MADD) {
+                unsigned sum = 0;  // of the row's |q|, byte by byte
+#pragma unroll
+                for (int t = 0; t < F::KSTEPS; t++)
+#pragma unroll
+                    for (int i = 0; i < 4; i++) sum = __builtin_amdgcn_sad_u8((unsigned)qf[t][i] ^ 0x80808080u, 0x80808080u, sum);
+                sum += __shfl_xor(sum, 32);
+                float q_sum = (float)sum * qs;
+#pragma unroll
+                for (int x = 1; x < 32; x <<= 1) q_sum = fmaxf(q_sum, __shfl_xor(q_sum, x));
+                if (!(qs < 3.0e38f)) q_sum = INFINITY;
+                float* sums = reinterpret_cast<float*>(smem);  // (nothing is on its way into the tile buffers yet)
+                if (lane == 0) sums[wave] = q_sum;
+                __syncthreads();
+#pragma unroll
+                for (int w = 0; w < kFastWaves; w++) bound = fmaxf(bound, sums[w]);
+                bound *= 256.0f * ks_max;
+                __syncthreads();
+            }
+            const bool skip = top < low - 150.0f - bound && !odd;  // (bound NaN: 0 times infinity)
             visits = ~__builtin_amdgcn_ballot_w64(skip);
             asm volatile("" : "+s"(visits));
         }
@@ -642,13 +674,20 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
 #pragma unroll
                     for (int c = 0; c < 8; c++) e8[c] = mask_entry<MT>(w4[c >> 1], c & 1);
                 }
+                if (MC && BN * (vt0 + 1) - 1 > c_first) {
+#pragma unroll
+                    for (int c = 0; c < 8; c++) e8[c] += causal_entry(vt0 * BN, kt, 8 * (tp & 1) + c);
+                }
 #pragma unroll
                 for (int c = 0; c < 8; c++) {
                     const int bits = sbuf[0][kt][8 * (tp & 1) + c];
                     mx = fmaxf(mx, __builtin_fmaf(as_f(bits) - BIAS, sc, e8[c]));
                 }
             });
-            m_i = fmaxf(row_pair_max(mx), -1.0e30f);
+            // (under the causal flag without the bound: a row of the type's lowest entries alone weighs its keys evenly, one of
+            // -inf alone is NaN, as in the general kernel)
+            m_i = row_pair_max(mx);
+            if (!MC) m_i = fmaxf(m_i, -1.0e30f);
         }
     }
     int mslot = 0;  // slot of the current step's mask bytes (step % 3)
@@ -796,9 +835,16 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             if constexpr (MADD) {
                 // a ragged last tile always comes here: its keys past kv_len score -1e6 (the reference reads their
                 // mask entries as -1e6 and their K as zeros), which only this path accounts for
+                const bool diagonal = MC && live && n0 + BN - 1 > c_first;
                 if (large != 0 && !live) {
                     lsum = 0.0f;
-                } else if (large != 0 || (ragged && live && vt0 == nk - 1)) {
+                } else if (diagonal && n0 > c_block) {
+#pragma unroll
+                    for (int tp = 0; tp < 4; tp++)
+#pragma unroll
+                        for (int c = 0; c < 8; c++) pf[tp][c] = (VT)0.0f;
+                    lsum = 0.0f;
+                } else if (large != 0 || diagonal || (ragged && live && vt0 == nk - 1)) {
                     float raw = -INFINITY;
                     float past_end = 0.0f;  // number of the lane's keys of this step that lie past kv_len
                     sfor<4>([&](auto tc) {
@@ -815,6 +861,10 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                             mask_entries(mslot, tp, w4);
 #pragma unroll
                             for (int c = 0; c < 8; c++) e8[c] = mask_entry<MT>(w4[c >> 1], c & 1);
+                        }
+                        if (diagonal) {
+#pragma unroll
+                            for (int c = 0; c < 8; c++) e8[c] += causal_entry(n0, kt, 8 * (tp & 1) + c);
                         }
 #pragma unroll
                         for (int c = 0; c < 8; c++) {

@@ -27,6 +27,7 @@ int launch_additive_mt(const AttnArgs& a, hipStream_t stream) {
 }  // namespace
 
 int launch_fast_additive(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream) {
+    if (a.causal) return launch_fast_additive_causal(a, head_dim, v_dtype, stream);
     if (head_dim == 128)
         return v_dtype == SAGE_BF16 ? launch_additive_mt<128, __bf16>(a, stream) : launch_additive_mt<128, _Float16>(a, stream);
     return v_dtype == SAGE_BF16 ? launch_additive_mt<64, __bf16>(a, stream) : launch_additive_mt<64, _Float16>(a, stream);

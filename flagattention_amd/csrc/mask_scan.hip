@@ -176,11 +176,14 @@ namespace attn {
 // Worth its launch where the heads share the mask (one read of it serves all of them; a mask per head is a position bias as a
 // rule, and read once either way) and enough steps can go.  Where every q-block has a compute unit of its own only the longest
 // one counts, which padding shortens and a causal mask does not: 20 tiles (B3 H16 M640 N640 D128 causal and padded, bool: 39 us
-// without, 43 with; B2 H8 M1286 fp16 62, 53); with more q-blocks 12 (B3 H32 M858 N858 D128 padded fp32: 99.8, 98.4).  V is read
-// once more, so the queries per K/V head have to be many as well.
+// without, 43 with; B2 H8 M1286 fp16 62, 53), and for masks of rows only (a batch whose longest sequence fills the keys has
+// nothing to leave out there: B2 H16/2 M1792 padded fp32 79.5, 84.5); with more q-blocks 12 (B3 H32 M858 N858 D128 padded fp32:
+// 99.8, 98.4).  V is read once more, so the queries per K/V head have to be many as well.
 int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch) {
     const int64_t q_blocks = batch * a.Hq * ((a.M + kFastRows - 1) / kFastRows);
+    if (a.causal) return 0;  // (the largest entry of a row may lie where the causal mask adds -1e6 to it)
     if (a.ms_h != 0 || a.Hq < 2 || a.nk < (q_blocks > 256 ? 12 : 20) || (int64_t)a.groups * a.M < 512) return 0;
+    if (q_blocks <= 256 && a.ms_m == 0) return 0;
     const int64_t mask_wgs = mask_batches(a, batch) * scan_strips(a), v_tiles = batch * a.Hkv * a.nk;
     if (mask_wgs + v_tiles > 0x7fffffffLL) return 0;
     const int64_t bytes = 4 * (mask_wgs * (a.nk + 1) + v_tiles);

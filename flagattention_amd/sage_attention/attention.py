@@ -294,9 +294,9 @@ def _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, r
                                           torch.bfloat16: (_lib.MASK_BF16, _lib.MASK_BF16_PADDED),
                                           torch.float32: (_lib.MASK_F32, _lib.MASK_F32_PADDED)}[m.dtype]
                     mask_kind = plain
-                    # additive masks run on the pipelined kernel (no causal flag on top); one whose rows it cannot load
-                    # 16 bytes at a time goes there through a padded copy
-                    if not causal and not _additive_mask_is_direct(m.expand(b, h_qo, qo_len, kv_len), kv_len):
+                    # additive masks run on the pipelined kernel; one whose rows it cannot load 16 bytes at a time goes there
+                    # through a padded copy
+                    if (not causal or nk > 2) and not _additive_mask_is_direct(m.expand(b, h_qo, qo_len, kv_len), kv_len):
                         if torch.cuda.is_current_stream_capturing():
                             padded, _ = _stage_additive_mask(m, b, h_qo, qo_len, kv_len)
                         else:
