@@ -200,7 +200,8 @@ int launch_fast_additive_causal(const AttnArgs& a, int head_dim, int v_dtype, hi
 
 // The scan of a mask that the heads share, ahead of the pipelined kernel (mask_scan.hip): bytes of workspace it takes (0: the
 // rule on sizes says no), and its launch, which fills the scan fields of `a`.
-int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch);
+int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch, int head_dim);
+int mask_splits(const AttnArgs& a, int64_t batch, int head_dim);  // runs of the tiles to visit, where the mask is scanned
 int launch_mask_scan(AttnArgs& a, int64_t batch, int head_dim, int v_dtype, void* workspace, hipStream_t stream);
 
 // The pipelined kernel on 16-bit Q and K (dense attention); causal with any qo_len / kv_len.

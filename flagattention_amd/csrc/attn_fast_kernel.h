@@ -172,10 +172,10 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     if ((a.total_wg & 7) == 0) wg = (wg & 7) * (a.total_wg >> 3) + (wg >> 3);
     const bool paired = CAUSAL && !CUT && !MASK && a.causal && !a.longest_first;
     const int per_head = paired ? (nq2 + 1) / 2 : nq2;  // workgroups per (batch, head)
-    // The keys of one (batch, head, q-block) may be split over `nsplit` workgroups (never under a mask tensor).  A
-    // workgroup then sees the problem that starts at its first key: kv_len, the number of tiles and the causal
+    // The keys of one (batch, head, q-block) may be split over `nsplit` workgroups (under a mask tensor the tiles it leaves to
+    // visit: see `visits`).  A workgroup then sees the problem that starts at its first key: kv_len, the number of tiles and the causal
     // limits below all count from there, and its steps end where the next workgroup's begin.
-    const int nsplit = MASK || CUT ? 1 : a.nsplit;
+    const int nsplit = MC || CUT ? 1 : a.nsplit;
     const int split = wg % nsplit;
     const int item0 = wg / nsplit;
     // heads that alternate within a q-block: measured to pay only under a mask with the causal mask folded in
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     const_ptr args_again = (const_ptr)__builtin_amdgcn_kernarg_segment_ptr();
     if constexpr (CUT) asm volatile("" : "+s"(args_again));
     const AttnArgs& a = CUT ? *(const AttnArgs*)args_again : args;
-    int b = b0, h = h0, step0 = split * a.split_steps, cut_steps = 0;  // step0: first step of this workgroup's share of the keys
+    int b = b0, h = h0, step0 = MASK ? 0 : split * a.split_steps, cut_steps = 0;  // step0: first step of this workgroup's share of the keys
     int iq = (paired && pass == 1) || (MASK && a.mask_causal && !a.longest_first) ? nq2 - 1 - jq : jq;  // (a mask with the causal mask folded in: no pairs, the q-blocks with the most tiles are handed out first)
     bool partial = false;  // (CUT) the item has steps in other workgroups too
     if constexpr (CUT) {
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     const int lim = !CAUSAL ? 0 : a.causal ? min(my_m + shift, kv_len - 1) : kv_len - 1;                  // this lane's row
     const int wlim = !CAUSAL ? 0 : a.causal ? min(m0 + 32 * wave + shift, kv_len - 1) : kv_len - 1;      // first row of the wave
 
-    int nsteps = CUT ? cut_steps : min(a.split_steps, nk);
+    int nsteps = CUT ? cut_steps : MASK ? nk : min(a.split_steps, nk);
     if (CAUSAL && !CUT && (a.causal || (MASK && a.mask_causal))) {  // (a mask with the causal mask folded in: same bound)
         const int last_row = min(m0 + kFastRows, a.M) - 1;
         nsteps = max(min(nsteps, (last_row + shift + BN) / BN), 0);  // 0: no row of the workgroup sees a key (qo_len > kv_len)
@@ -451,6 +451,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     if constexpr (MASK) {
         visit_group = a.visit_group;
         const int groups = (nsteps + visit_group - 1) / visit_group;
+        bool hidden_row = false;
         if (a.scan_top) {
             const int mb = a.ms_b ? b : 0;
             const int s0 = a.ms_m ? (kFastRows / kScanRows) * iq : 0, s1 = min(s0 + kFastRows / kScanRows, a.scan_strips);
@@ -458,6 +459,8 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             float low = a.scan_low[(int64_t)mb * a.scan_strips + min(s0 + (lane & (kFastRows / kScanRows - 1)), s1 - 1)];
 #pragma unroll
             for (int x = 1; x < kFastRows / kScanRows; x <<= 1) low = fminf(low, __shfl_xor(low, x));
+            hidden_row = __builtin_amdgcn_readfirstlane((int)!(low >= -1.0e4f));
+            if (!MADD) low = 0.0f;  // (a bool tile goes by whether it holds a visible key)
             const int64_t kv_row = ((int64_t)b * a.Hkv + hk) * a.nk;
             float top = -INFINITY, ks_max = 0.0f;
             bool odd = false;
@@ -499,6 +502,16 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             asm volatile("" : "+s"(visits));
         }
         if (groups < 64) visits &= (1ull << groups) - 1;
+        if (nsplit > 1) {
+            // Run `split` of the tiles to visit.  All of them are one run's where a row of the q-block sees no key, or keys of
+            // entries far below 0 alone: its parts would be weighed by log-sum-exps too large for it.
+            const int n = __builtin_popcountll(visits), first = hidden_row ? (split ? n : 0) : n * split / nsplit;
+            const int mine = (hidden_row ? n : n * (split + 1) / nsplit) - first;
+            for (int i = 0; i < first; i++) visits &= visits - 1;
+            unsigned long long rest = visits;
+            for (int i = 0; i < mine; i++) rest &= rest - 1;
+            visits ^= rest;
+        }
         if (nsteps > 0) {
             const bool last_group = (visits >> (groups - 1)) & 1;
             nsteps = __builtin_popcountll(visits) * visit_group - (last_group ? groups * visit_group - nsteps : 0);

@@ -517,12 +517,19 @@ bool fast_masked(const sage_attn_params& p, const AttnArgs& a) {
     return p.mask_kind != SAGE_MASK_NONE && attn::fast_serves_mask(a, a.mask_additive ? dtype_bytes(a.mask_dt) : 1);
 }
 
+// workspace of the partial results under a scanned mask, behind the scan's
+int64_t masked_split_bytes(const sage_attn_params& p, const AttnArgs& a) {
+    const LaunchPlan plan{attn::mask_splits(a, p.batch, (int)p.head_dim), 0, false, false};
+    return attn::plan_workspace_bytes(plan, p.batch, p.heads_q, p.qo_len, p.head_dim);
+}
+
 }  // namespace
 
 int64_t attn_split_workspace_bytes(const sage_attn_params& p) {
     if (p.mask_kind != SAGE_MASK_NONE) {
         const AttnArgs a = attn_args(p);
-        return fast_masked(p, a) ? attn::mask_scan_bytes(a, p.batch) : 0;
+        const int64_t scan = fast_masked(p, a) ? attn::mask_scan_bytes(a, p.batch, (int)p.head_dim) : 0;
+        return scan > 0 ? scan + masked_split_bytes(p, a) : 0;
     }
     if (p.causal && p.qo_len > p.kv_len) return 0;  // (not a launch that can be split)
     const attn::LaunchPlan plan = attn::plan_launch(p.batch, p.heads_q, p.heads_kv, p.qo_len, p.kv_len, p.causal != 0, p.head_dim, true, true);
@@ -574,9 +581,19 @@ int launch_attn(const sage_attn_params& p, void* workspace, int64_t workspace_by
         return launch(s);
     }
     if (fast_masked(p, a)) {
-        const int64_t scan = attn::mask_scan_bytes(a, p.batch);
-        if (scan > 0 && workspace && workspace_bytes >= scan)
-            if (int rc = attn::launch_mask_scan(a, p.batch, (int)p.head_dim, p.v_dtype, workspace, stream)) return rc;
+        const int64_t scan = attn::mask_scan_bytes(a, p.batch, (int)p.head_dim);
+        if (scan > 0 && workspace && workspace_bytes >= scan) {
+            const int runs = attn::mask_splits(a, p.batch, (int)p.head_dim);
+            if (runs == 1 || workspace_bytes >= scan + masked_split_bytes(p, a))
+                if (int rc = attn::launch_mask_scan(a, p.batch, (int)p.head_dim, p.v_dtype, workspace, stream)) return rc;
+            if (runs > 1 && a.scan_top) {
+                AttnArgs s = a;
+                s.longest_first = 0;
+                attn::apply_key_split(s, runs, p.batch, (int)p.head_dim, static_cast<unsigned char*>(workspace) + scan);
+                if (int rc = attn::launch_fast_masked(s, (int)p.head_dim, p.v_dtype, stream)) return rc;
+                return attn::launch_split_combine(s, a, (int)p.head_dim, p.batch, stream);
+            }
+        }
         return attn::launch_fast_masked(a, (int)p.head_dim, p.v_dtype, stream);
     }
     int rc;

@@ -12,7 +12,7 @@ template <int D, typename VT, typename MT>
 int launch_additive(const AttnArgs& a, hipStream_t stream) {
     AttnArgs b = a;
     const int nq2 = (a.M + kFastRows - 1) / kFastRows;
-    b.total_wg = (int)((int64_t)a.total_wg / a.nq * nq2);
+    b.total_wg = (int)((int64_t)a.total_wg / a.nq * nq2) * a.nsplit;
     dim3 grid((unsigned)b.total_wg), block(kFastThreads);
     hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1, MT>), grid, block, 0, stream, b, nq2);
     return check_launch("sage_attn_fwd_fast_kernel (additive mask)");

@@ -118,7 +118,7 @@ __device__ __forceinline__ void scan_strip(const ScanArgs& a, int wg) {
             for (int w = 1; w < kScanThreads / 64; w++) m = fmaxf(m, row_top[w][r]);
             low = fminf(low, m);
         }
-        a.low[wg] = sizeof(MT) == 1 ? 0.0f : low;  // (bool: a tile is visited if it holds a visible key)
+        a.low[wg] = low;
     }
 }
 
@@ -173,17 +173,45 @@ int launch_scan(const AttnArgs& a, const ScanArgs& s, int64_t wgs, hipStream_t s
 
 namespace attn {
 
+// us: of a step of the attention kernel under a mask, and of the scan
+static float step_us(int head_dim) { return head_dim == 128 ? 1.5f : 0.85f; }
+static float scan_us(const AttnArgs& a, int64_t batch, int head_dim) {
+    const float esz = a.mask_additive ? (float)dtype_bytes(a.mask_dt) : 1.0f;
+    return 5.0f + ((float)mask_batches(a, batch) * (a.ms_m ? (float)a.M : 1.0f) * (float)a.N * esz +
+                   (float)(batch * a.Hkv) * (float)a.N * (float)(2 * head_dim)) * (1e-6f / 4.5f);
+}
+
+// Few q-blocks: the tiles left to visit are split over several workgroups each, like the keys of a call without a mask, where the
+// steps that saves are worth the scan, the second launch and the partial results (B2 H2 M3072 N3072 D128 causal and padded, bool:
+// 96 us whole, 62 in five runs; but B1 H32 M732 45, 55 in two, B2 H8 M832 48, 54 in three).
+int mask_splits(const AttnArgs& a, int64_t batch, int head_dim) {
+    const int64_t q_blocks = batch * a.Hq * ((a.M + kFastRows - 1) / kFastRows);
+    const float whole = 7.0f + step_us(head_dim) * (float)a.nk, rows = (float)(batch * a.Hq) * (float)a.M;
+    float best = 0.9f * whole;
+    int runs = 1;
+    if (a.ms_h != 0 || a.Hq < 2 || a.causal) return 1;  // (not scanned)
+    for (int s = 2; s <= 16 && s <= a.nk / 4 && s * q_blocks <= 256; s++) {
+        const float cost = scan_us(a, batch, head_dim) + 7.0f + step_us(head_dim) * (float)((a.nk + s - 1) / s) + 4.0f +
+                           (float)s * rows * (float)head_dim * (8e-6f / 4.0f);
+        if (cost < best) { best = cost; runs = s; }
+    }
+    return runs;
+}
+
 // Worth its launch where the heads share the mask (one read of it serves all of them; a mask per head is a position bias as a
-// rule, and read once either way) and enough steps can go.  Where every q-block has a compute unit of its own only the longest
-// one counts, which padding shortens and a causal mask does not: 20 tiles (B3 H16 M640 N640 D128 causal and padded, bool: 39 us
-// without, 43 with; B2 H8 M1286 fp16 62, 53), and for masks of rows only (a batch whose longest sequence fills the keys has
-// nothing to leave out there: B2 H16/2 M1792 padded fp32 79.5, 84.5); with more q-blocks 12 (B3 H32 M858 N858 D128 padded fp32:
-// 99.8, 98.4).  V is read once more, so the queries per K/V head have to be many as well.
-int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch) {
+// rule, and read once either way) and enough steps can go: 12 tiles where there are more q-blocks than compute units (B3 H32
+// M858 N858 D128 padded fp32: 99.8 us without, 98.4 with).  With fewer only the longest q-block counts, which padding shortens
+// and a causal mask does not: about 48 us of steps (B3 H8 M640 D128 39 without, 43 with, B3 H8 M1760 D64 59.6, 63.3; B1 H16 M3392 D128
+// 119, 108), and not for masks of rows only (a batch whose longest sequence fills the keys has nothing to leave out: B2 H16/2
+// M1792 padded 79.5, 84.5).  V is read once more, so the queries per K/V head have to be many as well.
+int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch, int head_dim) {
     const int64_t q_blocks = batch * a.Hq * ((a.M + kFastRows - 1) / kFastRows);
     if (a.causal) return 0;  // (the largest entry of a row may lie where the causal mask adds -1e6 to it)
-    if (a.ms_h != 0 || a.Hq < 2 || a.nk < (q_blocks > 256 ? 12 : 20) || (int64_t)a.groups * a.M < 512) return 0;
-    if (q_blocks <= 256 && a.ms_m == 0) return 0;
+    if (a.ms_h != 0 || a.Hq < 2) return 0;
+    if (mask_splits(a, batch, head_dim) == 1) {
+        if (q_blocks > 256 ? a.nk < 12 : (a.ms_m == 0 || step_us(head_dim) * (float)a.nk < 48.0f)) return 0;
+        if ((int64_t)a.groups * a.M < 512) return 0;
+    }
     const int64_t mask_wgs = mask_batches(a, batch) * scan_strips(a), v_tiles = batch * a.Hkv * a.nk;
     if (mask_wgs + v_tiles > 0x7fffffffLL) return 0;
     const int64_t bytes = 4 * (mask_wgs * (a.nk + 1) + v_tiles);
