@@ -223,18 +223,24 @@ static int plan_decode_split(int64_t items, int64_t rows, int64_t nk) {
 // Short calls on attn_decode_kernel, a workgroup per 32-row tile of a K/V head's packed query rows (and run of its keys), instead
 // of one per 256 rows: they end in the time one workgroup takes, in which eight waves walk over the keys side by side instead of
 // one after the other, and a kernel that runs only a few steps spends less on its start.  Returns the runs of the keys, 0: not here.
-// Every workgroup has a compute unit of its own (under the causal flag half of them are short: two rounds), and the K/V rows
-// that all of them read, once per row tile, stay below 100 MB.  Times in us fitted to 350 launches within 12 %.
+// Every workgroup has a compute unit of its own; or there are two or three for each where half of them are short (causal), where two
+// fit a CU (head_dim 64) or where the pipelined kernel runs its instance that hides keys (a ragged last tile).  The K/V rows that
+// all of them read, once per row tile, stay below 100 MB (causal, half of them: 130).  Times in us fitted to 350 launches within 12 %.
 // Measured, pipelined kernel -> here (us, in a graph):
 //   int8  D64  B1 H2 M256 N256 8.0 -> 5.4, H8 N512 causal 22 -> 6.6, H8 N1024 18 -> 9.2, H2 N2048 causal 25 -> 12; D128 H8 N512 17 -> 10.4
 //   dense D128 H2 N200 13.2 -> 9.4, H8 N512 causal 35 -> 12.6, H8 N128 causal 10.3 -> 7.5, H2 N2048 28 -> 23
+//   more than one per CU: int8 D64 H32 M512 N512 11.6 -> 9.1, H96 N200 causal 10.7 -> 7.3, H64 N384 causal 12.1 -> 9.1, dense D64 H64 N200
+//   10.0 -> 8.0; beyond: int8 D64 H96 N256 8.6 (10.3 here), dense D64 H64 N256 8.3 (9.2), int8 D128 H64 N256 10.2 (14.7)
 //   not here: int8 D128 H32 M64 N16384 52 (65 here), dense D128 H32/32 M128 N128 9.1 (11.5), H32 M64 N1024 15.0 (16.1)
 static int plan_row_tiles(int64_t batch, int64_t heads_q, int64_t heads_kv, int64_t qo_len, int64_t kv_len, bool causal,
                           int64_t head_dim, bool int8, bool with_workspace) {
     const int64_t rows = heads_q / heads_kv * qo_len, wgs = batch * heads_kv * ((rows + 31) / 32), nk = (kv_len + BN - 1) / BN;
-    if (wgs > (causal ? 2 : 1) * kComputeUnits || kv_len >= (1 << 22)) return 0;
+    const bool ragged = kv_len % BN != 0;
+    const int64_t halves = causal ? (head_dim == 64 ? (int8 ? 6 : 5) : 4)  // workgroups per two CUs
+                         : (head_dim == 64 && int8) || (ragged && (head_dim == 64 || int8)) ? 4 : 2;
+    if (2 * wgs > halves * kComputeUnits || kv_len >= (1 << 22)) return 0;
     const float mb = (float)wgs * (float)(kv_len * head_dim * (int8 ? 3 : 4)) * 1e-6f;
-    if (mb > 100.0f || (rows <= 64 && !int8 && kv_len >= 1024)) return 0;  // (two row tiles of a head: no gain in 16 bits)
+    if (mb > (causal ? 130.0f : 100.0f) || (rows <= 64 && !int8 && kv_len >= 1024)) return 0;  // (two row tiles of a head: no gain in 16 bits)
     if (qo_len > kv_len && kv_len >= 512) return 0;  // (cross attention over keys that can be split keeps the key split of 256-row blocks)
     // a workgroup: its start and end, and each turn of its waves over 32 keys each; the K/V bytes; the second launch
     const float start = int8 ? (head_dim == 64 ? 4.5f : 7.1f) : (head_dim == 64 ? 5.7f : 8.4f);
