@@ -170,7 +170,13 @@ __device__ __forceinline__ void mean_from_partials(const float* part, int nchunk
 #pragma unroll
             for (int i = 0; i < 16; i++) tot = tot + v[i];
         }
-        for (; c < nchunk; c++) tot = tot + p[(int64_t)c * D];
+        if (c < nchunk) {  // the rest as one more batch, the last chunk again past the end (one by one each load waits for the one before)
+            float v[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) v[i] = p[(int64_t)min(c + i, nchunk - 1) * D];
+#pragma unroll
+            for (int i = 0; i < 16; i++) tot = c + i < nchunk ? tot + v[i] : tot;
+        }
         const float mean = round_to(tot / (float)rows, out_dt);
         km[d] = mean;
         if (out) {
@@ -569,11 +575,19 @@ __device__ __forceinline__ void k_mean_partial_item(const KMeanArgs& a, int64_t 
 #pragma unroll
             for (int e = 0; e < W; e++) acc[e] = acc[e] + v[i][e];
     }
-    for (; r < rows; r++) {
-        float v[W];
-        loadw<DT, W>(a.k, base + (int64_t)(n0 + r) * a.s_n, v);
+    // The rest in batches of eight, the last row again past the end: one by one each load waits for the one before, which at 700
+    // keys (60 rows in the last chunk, 11 chunks) took a quarter of the call (B1 H8 N700 D64 14.4 -> 11.0 us).  Sixteen at a
+    // time would take the registers of three waves per SIMD, which the Q blocks of the grid miss.
+    constexpr int kRest = DT == SAGE_F32 ? 4 : 8;
+#pragma unroll 1
+    for (; r < rows; r += kRest) {
+        float v[kRest][W];
 #pragma unroll
-        for (int e = 0; e < W; e++) acc[e] = acc[e] + v[e];
+        for (int i = 0; i < kRest; i++) loadw<DT, W>(a.k, base + (int64_t)(n0 + min(r + i, rows - 1)) * a.s_n, v[i]);
+#pragma unroll
+        for (int i = 0; i < kRest; i++)
+#pragma unroll
+            for (int e = 0; e < W; e++) acc[e] = r + i < rows ? acc[e] + v[i][e] : acc[e];
     }
     float* dst = a.part + (bh * a.nchunk + chunk) * a.D + cw * W;
 #pragma unroll
@@ -664,7 +678,18 @@ __global__ __launch_bounds__(THREADS) void smooth_head_kernel(QuantArgs kq, Quan
 #pragma unroll
                 for (int i = 0; i < 16; i++) add(w[i]);
             }
-            for (; r < n; r++) add(p[r * (D / 2)]);
+            if (r < n) {  // the rest: the reads together, rows past the end added to nothing
+                uint32_t w[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) w[i] = p[min(r + i, n - 1) * (D / 2)];
+#pragma unroll
+                for (int i = 0; i < 16; i++) {
+                    const float t0 = s0, t1 = s1;
+                    add(w[i]);
+                    s0 = r + i < n ? s0 : t0;
+                    s1 = r + i < n ? s1 : t1;
+                }
+            }
             float* dst = part + (first_row / 64 + chunk) * D + 2 * cp;
             dst[0] = s0;
             dst[1] = s1;
@@ -733,14 +758,13 @@ __global__ __launch_bounds__(kThreads) void k_mean_final_kernel(KMeanArgs a, int
 #pragma unroll
         for (int i = 0; i < 32; i++) tot = tot + v[i];
     }
-    for (; c + 8 <= a.nchunk; c += 8) {
-        float v[8];
+    for (; c < a.nchunk; c += 16) {  // the rest in batches of 16, the last chunk again past the end
+        float v[16];
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = p[(int64_t)(c + i) * a.D];
+        for (int i = 0; i < 16; i++) v[i] = p[(int64_t)min(c + i, a.nchunk - 1) * a.D];
 #pragma unroll
-        for (int i = 0; i < 8; i++) tot = tot + v[i];
+        for (int i = 0; i < 16; i++) tot = c + i < a.nchunk ? tot + v[i] : tot;
     }
-    for (; c < a.nchunk; c++) tot = tot + p[(int64_t)c * a.D];
     const float mean = tot / (float)a.N;
     if (a.out_dt == SAGE_F32) static_cast<float*>(a.out)[ch] = mean;
     else if (a.out_dt == SAGE_BF16) static_cast<__bf16*>(a.out)[ch] = (__bf16)mean;
