@@ -61,19 +61,39 @@ __global__ __launch_bounds__(kCombineThreads) void split_combine_kernel(CombineA
     const int64_t row = (int64_t)blockIdx.x * ROWS + threadIdx.x / (TPR * SG);
     const bool ok = row < a.rows;
     const float* pl = a.part_lse + (ok ? row : 0);
+    // The loads of kBatch runs are on their way together, the last run again past the end (one after the other a row of seven
+    // runs took ten trips to memory).
+    constexpr int kBatch = 8;
+    const int last = a.nsplit - 1;
     float m = -INFINITY;
-    for (int s = sg; s < a.nsplit; s += SG) m = max_or_nan(m, pl[(int64_t)s * a.rows]);
+    for (int s0 = sg; s0 <= last; s0 += SG * kBatch) {
+        float x[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) x[u] = pl[(int64_t)min(s0 + SG * u, last) * a.rows];
+#pragma unroll
+        for (int u = 0; u < kBatch; u++) m = max_or_nan(m, x[u]);
+    }
     v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
     float den = 0.0f;
     if (m != -INFINITY) {  // (a row that saw no key in any run: every partial is 0 and every lse_s -inf)
         const float* po = a.part_o + (ok ? row : 0) * D + 4 * c;
-#pragma unroll 4
-        for (int s = sg; s < a.nsplit; s += SG) {
-            const float w = __builtin_amdgcn_exp2f(pl[(int64_t)s * a.rows] - m);
-            const v4f o = *reinterpret_cast<const v4f*>(po + (int64_t)s * a.rows * D);
-            den += w;
+        for (int s0 = sg; s0 <= last; s0 += SG * kBatch) {
+            v4f o[kBatch];
+            float x[kBatch];
 #pragma unroll
-            for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(w, o[i], acc[i]);
+            for (int u = 0; u < kBatch; u++) {
+                const int64_t s = min(s0 + SG * u, last);
+                x[u] = pl[s * a.rows];
+                o[u] = *reinterpret_cast<const v4f*>(po + s * a.rows * D);
+            }
+#pragma unroll
+            for (int u = 0; u < kBatch; u++) {
+                if (s0 + SG * u > last) break;
+                const float w = __builtin_amdgcn_exp2f(x[u] - m);
+                den += w;
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(w, o[u][i], acc[i]);
+            }
         }
     }
     if constexpr (SG > 1) {

@@ -228,8 +228,13 @@ __global__ __launch_bounds__(256) void total_runs_kernel(const float* part, floa
     if (i >= count) return;
     const int n = runs.count((int)(i % N) / kWgKeys);
     float x = 0.0f;
-#pragma unroll 8
-    for (int r = 0; r < n; r++) x += part[(int64_t)r * count + i];
+    for (int r = 0; r < n; r += 8) {  // eight loads on their way together, the last run again past the end
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = part[(int64_t)min(r + u, n - 1) * count + i];
+#pragma unroll
+        for (int u = 0; u < 8; u++) x = r + u < n ? x + v[u] : x;
+    }
     total[i] = x;
 }
 
@@ -237,11 +242,11 @@ __global__ __launch_bounds__(256) void total_runs_kernel(const float* part, floa
 // runs of at least eight tiles, as many as make three workgroups per CU, all of them resident at once.  (With the same four
 // ranges of queries for every block some CUs held 84 tiles and others 40: B1 H16 M4096 N4096 D128 causal, whole call, 142 -> 135
 // us; B1 H16/2 M4032 136 -> 128, B3 H8/1 M2048 86.5 -> 83.)  Runs that would be long: three times as many, handed out as others
-// end (B6 H2 M9728 D64 causal 285 -> 280 us, 300 with what is resident at once).
+// end (B6 H2 M9728 D64 causal 285 -> 280 us, 300 with what is resident at once; B1 H32/4 M6995, 896 key blocks, 1204, 1249 uncut).
 int total_chunk(int64_t BH, int64_t M, int64_t N, bool causal) {
     constexpr int64_t kResident = 3 * 256, kLongRun = 32;
     const int64_t nkb = (N + kWgKeys - 1) / kWgKeys, tiles = (M + kTileQ - 1) / kTileQ;
-    if (BH * nkb >= kResident || tiles < 16 || tiles > (1 << 24) || N > (1 << 29)) return (int)tiles;
+    if (BH * nkb >= 4 * 256 || tiles < 16 || tiles > (1 << 24) || N > (1 << 29)) return (int)tiles;
     TotalRuns runs{(int)tiles, 1, (int)(N - M), causal};
     int64_t all = 0;
     for (int kb = 0; kb < nkb; kb++) all += runs.count(kb);
