@@ -942,11 +942,11 @@ int launch_kmean(const sage_tensor& k, int k_dtype, void* km_out, int out_dtype,
     return launch_k_mean_final(a, B * H * D, stream);
 }
 
-// Sequences of up to this many 64-row chunks, in calls of up to this many K blocks, have the partials of the K mean added by
-// every K block instead of by a launch of its own: GPU time B1 H32 N1024 D128 16.6 -> 14.0 us, B8 H16 N1024 D64 23.2 -> 20.4
-// us, B1 H32 N2000 D128 21.2 -> 20.0 us, B2 H16 N2048 D64 16.3 -> 15.0 us; longer ones (B1 H32/8 N3001 22.6 -> 22.7 us, B1 H16
-// N5000 fp32 32.7 -> 33.6 us) and larger calls (B16 H32 N512, 4096 blocks: 53.2 -> 54.7 us) gain nothing.
-constexpr int kOwnMeanChunks = 32, kOwnMeanBlocks = 2048;
+// Up to this many 64-row chunks, K blocks, and partials read by all blocks together, every K block adds the chunk partials of its
+// head itself instead of a launch for the mean.  Quantizer call, GPU time in a graph: B1 H32/8 N3001 D128 21.1 -> 19.5 us, B1 H8 N4096
+// D128 16.4 -> 15.5, B1 H8 N6000 D128 20.7 -> 19.8, B1 H32 N2500 D64 19.6 -> 18.0.  Beyond it loses: 1.03 to 1.05 times as long at
+// B2 H32 N4096 (262144 partials), 1.04 at B1 H32 N6000 D128 (282752), 1.07 to 1.13 at B1 H32 N8192, 1.03 to 1.24 at N16384.
+constexpr int kOwnMeanChunks = 128, kOwnMeanBlocks = 2048, kOwnMeanReads = 110000;
 
 // K mean -> k - km -> quantization of K, and quantization of Q.  Short sequences: smooth_head_kernel, one launch.  Others:
 //   1. Q blocks and the chunk partials of the K mean, side by side in one grid;
@@ -998,7 +998,7 @@ int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_k
         }
         const bool shared = have_q && q_dot_km && both_fit(kq, qq, B * H * kq.nblk, q_blocks);  // one grid with the Q blocks
         if (!shared && kq.blk == 64 && kq.d8_shift >= 0 && D <= kMaxFusedMeanDim && kq.blk * kq.D8 <= 1024 && kq.nblk <= kOwnMeanChunks &&
-            B * H * kq.nblk <= kOwnMeanBlocks) {
+            B * H * kq.nblk <= kOwnMeanBlocks && B * H * kq.nblk * kq.nblk <= kOwnMeanReads) {
             kq.km = nullptr; kq.part = ka.part; kq.km_write = km_out;  // every block adds the chunk partials itself
         } else {
             if (int rc = launch_k_mean_final(ka, B * H * D, stream)) return rc;

@@ -1,5 +1,5 @@
 """The quantizer's fused launches at their edges, bit for bit against the oracle: one workgroup per head (up to 256 keys at
-head_dim 128, 512 at 64), K blocks that add the chunk partials of the mean themselves (up to 32 chunks), K and Q blocks in one
+head_dim 128, 512 at 64), K blocks that add the chunk partials of the mean themselves (up to 128 chunks), K and Q blocks in one
 grid, and the sizes just beyond each."""
 import pytest
 import torch
@@ -45,6 +45,21 @@ def test_smoothing_launch_forms(d, n, dtype, gpu_device):
         # fp32 sums of d products: each addition rounds once, d roundings of the running sum's magnitude
         bound = d * 2.0 ** -24 * (qh.double().abs() * kmh.double().abs().repeat_interleave(hq // hkv, dim=1)).sum(-1)
         assert bool(((dot.cpu().double() - ref).abs() <= bound + 1e-12).all())
+
+
+@pytest.mark.parametrize("b,h,n,d", [(1, 2, 2500, 64), (1, 1, 4097, 128), (1, 3, 6001, 64), (1, 6, 8191, 128), (1, 6, 8193, 128),
+                                     (1, 33, 3700, 64), (64, 1, 2048, 64), (65, 1, 2048, 64)])
+def test_mean_added_by_the_k_blocks(b, h, n, d, gpu_device):
+    """Each line of the rule and the size beyond it; the same bits as the mean from a launch of its own."""
+    from flagattention_amd.sage_attention.quant import per_block_int8_smooth_k
+
+    g = torch.Generator().manual_seed(n)
+    k = (torch.randn(b, h, n, d, generator=g) + 2.0).to(torch.bfloat16)
+    q = torch.randn(b, h, 70, d, generator=g).to(torch.bfloat16)
+    km = C.k_mean_fixed_order(k, "HND")
+    *got, km_got, _ = per_block_int8_smooth_k(q.to(gpu_device), k.to(gpu_device), tensor_layout="HND", with_q_dot_km=False)
+    assert torch.equal(km_got.cpu().view(torch.int16), km.view(torch.int16))
+    _check(got, C.per_block_int8(q, k, km=km, tensor_layout="HND"))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
