@@ -44,10 +44,11 @@ struct QuantArgs {
     // the per-row shift K smoothing takes out of every logit of row n.  km is then NOT subtracted from x.
     float* dot;
     int32_t dot_groups;
-    // Optional (K blocks of the K-smoothing entry point, short sequences): km is not there yet; every block adds the chunk
-    // partials of its head in order (k_mean_final_kernel's arithmetic), the head's first block writes km as well.
-    const float* part;   // [B * H, nblk, D]
-    void* km_write;      // [B * H, D], km_dt
+    // Optional (K-smoothing entry point): km is not there yet; every block adds the chunk partials of its K head in order
+    // (k_mean_final_kernel's arithmetic), the first K block of a head writes km as well.
+    const float* part;   // [B * K heads, part_chunks, D]
+    void* km_write;      // [B * H, D], km_dt (K blocks)
+    int32_t part_chunks, part_rows;  // 64-row chunks and rows of a K head
     int32_t small_offsets;  // every byte offset inside one block of x and of out fits 31 bits (host-checked)
 };
 
@@ -158,6 +159,7 @@ __device__ __forceinline__ float block_amax(float amax, float* wave_max) {
 
 // The K mean of one head from its chunk partials: added in chunk order from 0.0f, one IEEE divide by the number of rows, one
 // rounding; a thread per channel.  km: the rounded means as fp32; out: where they are stored in their own type, or null.
+template <bool SHORT_REST = false>
 __device__ __forceinline__ void mean_from_partials(const float* part, int nchunk, int D, int rows, int out_dt, float* km, void* out, int64_t out_off) {
     for (int d = threadIdx.x; d < D; d += blockDim.x) {
         const float* p = part + d;
@@ -170,13 +172,17 @@ __device__ __forceinline__ void mean_from_partials(const float* part, int nchunk
 #pragma unroll
             for (int i = 0; i < 16; i++) tot = tot + v[i];
         }
-        if (c < nchunk) {  // the rest as one more batch, the last chunk again past the end (one by one each load waits for the one before)
-            float v[16];
+        // the rest as one more batch (of 8 where that is enough and the caller has the registers), the last chunk again past the
+        // end: one by one each load waits for the one before
+        auto rest = [&](auto n) {
+            float v[n.value];
 #pragma unroll
-            for (int i = 0; i < 16; i++) v[i] = p[(int64_t)min(c + i, nchunk - 1) * D];
+            for (int i = 0; i < n.value; i++) v[i] = p[(int64_t)min(c + i, nchunk - 1) * D];
 #pragma unroll
-            for (int i = 0; i < 16; i++) tot = c + i < nchunk ? tot + v[i] : tot;
-        }
+            for (int i = 0; i < n.value; i++) tot = c + i < nchunk ? tot + v[i] : tot;
+        };
+        if (c < nchunk && (!SHORT_REST || c + 8 < nchunk)) rest(std::integral_constant<int, 16>{});
+        else if (SHORT_REST && c < nchunk) rest(std::integral_constant<int, 8>{});
         const float mean = round_to(tot / (float)rows, out_dt);
         km[d] = mean;
         if (out) {
@@ -191,7 +197,9 @@ __device__ __forceinline__ void mean_from_partials(const float* part, int nchunk
 // wave_max: THREADS / 64 floats of LDS.
 constexpr int kMaxFusedMeanDim = 256;  // head_dim up to which a block adds its head's chunk partials on its own
 
-template <int DT, int UNITS, int THREADS>
+// LOADS_FIRST: the partials of the mean are added with the block's own loads on their way: 3 to 4 % of the quantizer's time
+// where K and Q blocks do it, for 12 more registers, which cost K blocks alone 3 to 6 % from 1300 blocks on.
+template <int DT, int UNITS, int THREADS, bool LOADS_FIRST = false>
 __device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* wave_max, float* km_lds = nullptr) {
     const int tid = threadIdx.x;
     const int ib = bid % a.nblk;
@@ -210,13 +218,15 @@ __device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* 
     const bool fixed_c8 = a.ks_n == 0 && a.d8_shift >= 0 && a.D8 <= THREADS;
     float m_fixed[8];
     const bool own_mean = km_lds != nullptr && a.part != nullptr;
-    if (own_mean) {
-        mean_from_partials(a.part + ((int64_t)b * a.H + h) * a.nblk * (a.D8 * 8), a.nblk, a.D8 * 8, a.L, a.km_dt, km_lds,
-                           ib == 0 ? a.km_write : nullptr, ((int64_t)b * a.H + h) * (a.D8 * 8));
+    auto add_partials = [&] {
+        const int64_t kh = a.dot ? (int64_t)b * (a.H / a.dot_groups) + hm : (int64_t)b * a.H + h;
+        mean_from_partials<LOADS_FIRST>(a.part + kh * a.part_chunks * (a.D8 * 8), a.part_chunks, a.D8 * 8, a.part_rows, a.km_dt, km_lds,
+                           ib == 0 ? a.km_write : nullptr, kh * (a.D8 * 8));
         __syncthreads();
 #pragma unroll
         for (int e = 0; e < 8; e++) m_fixed[e] = km_lds[(tid & (a.D8 - 1)) * 8 + e];
-    }
+    };
+    if (!LOADS_FIRST && own_mean) add_partials();
     if (a.km && fixed_c8) load8_rt(a.km, a.km_dt, k_base + (tid & (a.D8 - 1)) * 8, m_fixed);
 
     constexpr int ESZ = DT == SAGE_F32 ? 4 : 2;
@@ -244,6 +254,7 @@ __device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* 
                 raw16[j] = *reinterpret_cast<const uint4*>(p);
             }
         }
+        if (LOADS_FIRST && own_mean) add_partials();
         float v[UNITS][8];
         float amax = 0.0f;
 #pragma unroll
@@ -322,6 +333,7 @@ __device__ __forceinline__ void quant_block(const QuantArgs& a, int bid, float* 
         }
         koff[j] = k_base + nc * a.ks_n + c8 * 8;
     }
+    if (LOADS_FIRST && own_mean) add_partials();
 
     float v[UNITS][8];
     float amax = 0.0f;
@@ -421,6 +433,25 @@ __global__ __launch_bounds__(THREADS) void quant_both_kernel(QuantArgs kq, Quant
     else quant_block<DT, QU, THREADS>(qq, blockIdx.x - k_blocks, wave_max);
 }
 
+// The same where both take the mean from its chunk partials.
+template <int DT, int KU, int QU, int THREADS>
+__global__ __launch_bounds__(THREADS) void quant_both_own_mean_kernel(QuantArgs kq, QuantArgs qq, int k_blocks) {
+    __shared__ float wave_max[THREADS / 64];
+    __shared__ float km_lds[kMaxFusedMeanDim];
+    if ((int)blockIdx.x < k_blocks) quant_block<DT, KU, THREADS, true>(kq, blockIdx.x, wave_max, km_lds);
+    else quant_block<DT, QU, THREADS, true>(qq, blockIdx.x - k_blocks, wave_max, km_lds);
+}
+
+template <int DT>
+int launch_both_own_mean_dt(const QuantArgs& kq, const QuantArgs& qq, int64_t k_blocks, int64_t q_blocks, hipStream_t stream) {
+    dim3 grid((unsigned)(k_blocks + q_blocks));
+    if (kq.blk * kq.D8 <= 2 * kThreads && qq.blk * qq.D8 <= 4 * kThreads)
+        hipLaunchKernelGGL((quant_both_own_mean_kernel<DT, 2, 4, kThreads>), grid, dim3(kThreads), 0, stream, kq, qq, (int)k_blocks);
+    else
+        hipLaunchKernelGGL((quant_both_own_mean_kernel<DT, 2, 4, 2 * kThreads>), grid, dim3(2 * kThreads), 0, stream, kq, qq, (int)k_blocks);
+    return check_launch("quant_both_own_mean_kernel");
+}
+
 template <int DT>
 int launch_both_dt(const QuantArgs& kq, const QuantArgs& qq, int64_t k_blocks, int64_t q_blocks, hipStream_t stream) {
     dim3 grid((unsigned)(k_blocks + q_blocks));
@@ -448,11 +479,18 @@ bool wide_both(const QuantArgs& kq, const QuantArgs& qq, int64_t blocks) {
 
 bool both_fit(const QuantArgs& kq, const QuantArgs& qq, int64_t k_blocks, int64_t q_blocks) {
     const int64_t blocks = k_blocks + q_blocks;
-    return k_blocks > 0 && q_blocks > 0 && !kq.part && kq.blk * kq.D8 <= 4 * kThreads && qq.blk * qq.D8 <= 8 * kThreads &&
+    return k_blocks > 0 && q_blocks > 0 && kq.blk * kq.D8 <= 4 * kThreads && qq.blk * qq.D8 <= 8 * kThreads &&
            (blocks <= kBothBlocks || wide_both(kq, qq, blocks));
 }
 
 int launch_both(const QuantArgs& kq, const QuantArgs& qq, int in_dtype, int64_t k_blocks, int64_t q_blocks, hipStream_t stream) {
+    if (kq.part) {
+        switch (in_dtype) {
+            case SAGE_F16: return launch_both_own_mean_dt<SAGE_F16>(kq, qq, k_blocks, q_blocks, stream);
+            case SAGE_BF16: return launch_both_own_mean_dt<SAGE_BF16>(kq, qq, k_blocks, q_blocks, stream);
+            default: return launch_both_own_mean_dt<SAGE_F32>(kq, qq, k_blocks, q_blocks, stream);
+        }
+    }
     switch (in_dtype) {
         case SAGE_F16: return launch_both_dt<SAGE_F16>(kq, qq, k_blocks, q_blocks, stream);
         case SAGE_BF16: return launch_both_dt<SAGE_BF16>(kq, qq, k_blocks, q_blocks, stream);
@@ -947,6 +985,11 @@ int launch_kmean(const sage_tensor& k, int k_dtype, void* km_out, int out_dtype,
 // D128 16.4 -> 15.5, B1 H8 N6000 D128 20.7 -> 19.8, B1 H32 N2500 D64 19.6 -> 18.0.  Beyond it loses: 1.03 to 1.05 times as long at
 // B2 H32 N4096 (262144 partials), 1.04 at B1 H32 N6000 D128 (282752), 1.07 to 1.13 at B1 H32 N8192, 1.03 to 1.24 at N16384.
 constexpr int kOwnMeanChunks = 128, kOwnMeanBlocks = 2048, kOwnMeanReads = 110000;
+// The same where the Q blocks need the mean too (q . km) and share the grid, with lines of their own: B1 H2 N1024 D128 13.7 -> 10.0
+// us, B1 H8 N2000 D128 15.0 -> 12.3, B1 H32/8 N2500 D128 21.0 -> 19.4, B1 H32/8 N3001 D128 23.0 -> 22.4, B1 H32 N3001 D64 21.6 -> 20.6,
+// B4 H32 N1024 D128 (3072 blocks, 6.3M floats) 37.0 -> 35.0; beyond: B1 H32 N2500 D128 (9.8M) 27.2 -> 27.2, B1 H32 N3001 D128
+// (13.7M) 30.3 -> 31.0, B2 H32 N2100 D64 (3200 blocks, 6.8M) 24.8 -> 25.2, B4 H32 N1500 D64 (4608 blocks, 7.1M) 30.5 -> 30.8.
+constexpr int kOwnMeanBothBlocks = 3072, kOwnMeanBothReads = 7 << 20;  // K and Q blocks, floats they read
 
 // K mean -> k - km -> quantization of K, and quantization of Q.  Short sequences: smooth_head_kernel, one launch.  Others:
 //   1. Q blocks and the chunk partials of the K mean, side by side in one grid;
@@ -954,8 +997,7 @@ constexpr int kOwnMeanChunks = 128, kOwnMeanBlocks = 2048, kOwnMeanReads = 11000
 //      chunks inside 3;
 //   3. K blocks, subtracting the mean just written.
 // With q_dot_km the Q blocks need the mean as well and move behind it: partials, mean, K and Q blocks in one grid (where
-// both_fit, also for few chunks: K blocks that add the partials themselves and the Q blocks behind them took B1 H32/8 N600
-// D128 19.2 us, this 17.1, B1 H8 N700 D64 17.5 -> 14.0, B4 H32/8 N1024 D128 25.4 -> 23.7, B2 H32 N2000 D128 35.4 -> 35.2).
+// both_fit), the mean inside the third as above.
 int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_km, void* workspace, hipStream_t stream) {
     const int64_t B = p.batch, H = p.heads_kv, N = p.kv_len, D = p.head_dim;
     KMeanArgs ka;
@@ -997,14 +1039,19 @@ int launch_smooth_quant(const sage_quant_params& p, void* km_out, float* q_dot_k
             if (int rc = launch_k_mean_partial(ka, p.in_dtype, stream)) return rc;
         }
         const bool shared = have_q && q_dot_km && both_fit(kq, qq, B * H * kq.nblk, q_blocks);  // one grid with the Q blocks
-        if (!shared && kq.blk == 64 && kq.d8_shift >= 0 && D <= kMaxFusedMeanDim && kq.blk * kq.D8 <= 1024 && kq.nblk <= kOwnMeanChunks &&
-            B * H * kq.nblk <= kOwnMeanBlocks && B * H * kq.nblk * kq.nblk <= kOwnMeanReads) {
-            kq.km = nullptr; kq.part = ka.part; kq.km_write = km_out;  // every block adds the chunk partials itself
+        const int64_t blocks = B * H * kq.nblk + (shared ? q_blocks : 0);
+        const bool own = kq.blk == 64 && kq.d8_shift >= 0 && D <= kMaxFusedMeanDim && kq.blk * kq.D8 <= 1024 && kq.nblk <= kOwnMeanChunks &&
+                         (shared ? blocks <= kOwnMeanBothBlocks && blocks * kq.nblk * D <= kOwnMeanBothReads
+                                 : blocks <= kOwnMeanBlocks && blocks * kq.nblk <= kOwnMeanReads);
+        if (own) {  // every block adds the chunk partials itself
+            kq.km = nullptr; kq.part = ka.part; kq.km_write = km_out;
+            kq.part_chunks = (int)ka.nchunk; kq.part_rows = (int)N;
         } else {
             if (int rc = launch_k_mean_final(ka, B * H * D, stream)) return rc;
         }
         if (shared) {
             q_dot();
+            if (own) { qq.km = nullptr; qq.part = ka.part; qq.part_chunks = kq.part_chunks; qq.part_rows = kq.part_rows; }
             return launch_both(kq, qq, p.in_dtype, B * H * kq.nblk, q_blocks, stream);
         }
         if (int rc = launch_tensor(kq, p.in_dtype, B * H * kq.nblk, stream)) return rc;

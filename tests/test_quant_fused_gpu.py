@@ -48,7 +48,8 @@ def test_smoothing_launch_forms(d, n, dtype, gpu_device):
 
 
 @pytest.mark.parametrize("b,h,n,d", [(1, 2, 2500, 64), (1, 1, 4097, 128), (1, 3, 6001, 64), (1, 6, 8191, 128), (1, 6, 8193, 128),
-                                     (1, 33, 3700, 64), (64, 1, 2048, 64), (65, 1, 2048, 64)])
+                                     (1, 33, 3700, 64), (64, 1, 2048, 64), (65, 1, 2048, 64), (90, 1, 2048, 64), (96, 1, 2048, 64),
+                                     (1, 24, 2500, 128), (1, 26, 2560, 128), (3, 5, 650, 128)])
 def test_mean_added_by_the_k_blocks(b, h, n, d, gpu_device):
     """Each line of the rule and the size beyond it; the same bits as the mean from a launch of its own."""
     from flagattention_amd.sage_attention.quant import per_block_int8_smooth_k
@@ -57,9 +58,14 @@ def test_mean_added_by_the_k_blocks(b, h, n, d, gpu_device):
     k = (torch.randn(b, h, n, d, generator=g) + 2.0).to(torch.bfloat16)
     q = torch.randn(b, h, 70, d, generator=g).to(torch.bfloat16)
     km = C.k_mean_fixed_order(k, "HND")
-    *got, km_got, _ = per_block_int8_smooth_k(q.to(gpu_device), k.to(gpu_device), tensor_layout="HND", with_q_dot_km=False)
-    assert torch.equal(km_got.cpu().view(torch.int16), km.view(torch.int16))
-    _check(got, C.per_block_int8(q, k, km=km, tensor_layout="HND"))
+    want = C.per_block_int8(q, k, km=km, tensor_layout="HND")
+    for with_dot in (False, True):
+        *got, km_got, dot = per_block_int8_smooth_k(q.to(gpu_device), k.to(gpu_device), tensor_layout="HND", with_q_dot_km=with_dot)
+        assert torch.equal(km_got.cpu().view(torch.int16), km.view(torch.int16))
+        _check(got, want)
+    ref = (q.double() * km.double()).sum(-1)
+    bound = d * 2.0 ** -24 * (q.double().abs() * km.double().abs()).sum(-1)  # fp32 sums of d products, one rounding per addition
+    assert bool(((dot.cpu().double() - ref).abs() <= bound + 1e-12).all())
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
