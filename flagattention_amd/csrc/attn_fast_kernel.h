@@ -349,7 +349,8 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     // (MC) Additive mask with the causal flag: the reference adds -1e6 where the causal mask hides a key, on top of the
     // entry, and skips the 128 x 64 tiles that hide every key.  Steps whose tile reaches past the limit of the wave's first
     // row (c_first) therefore take the path that redoes a step, which adds it; past the limit of the last row of the wave's
-    // 128-row block (c_block) their P is 0.
+    // 128-row block (c_block) a step leaves out the products with V (with P = 0 instead an Inf or NaN in V would reach rows
+    // whose block does not visit its tile).
     const int c_first = MC ? m0 + 32 * wave_u + shift : 0, c_block = MC ? min(m0 + BM * (wave_u / 4) + BM - 1, a.M - 1) + shift : 0;
     // what the causal mask adds to the entry of score register i of tile kt, for the lane's row (derived again where it is used)
     auto causal_entry = [&](int n_first, int kt, int i) {
@@ -742,6 +743,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         };
         const int n0 = (MASK ? vt0 : step) * BN, n0_next = (MASK ? vt1 : step + 1) * BN;  // first keys of this step and the next
         const bool live = step < nsteps;  // false only for the padding step after an odd number of steps
+        const bool past_block = MC && n0 > c_block;  // (MC) wave-uniform: the reference's 128-row block does not visit this tile
 
         // ===== VALU phase: exponentials of this step (scores in sbuf[P]) =====
         // No row maximum is taken: the exponentials use the reference point m_i the row already has, which
@@ -849,13 +851,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                 // a ragged last tile always comes here: its keys past kv_len score -1e6 (the reference reads their
                 // mask entries as -1e6 and their K as zeros), which only this path accounts for
                 const bool diagonal = MC && live && n0 + BN - 1 > c_first;
-                if (large != 0 && !live) {
-                    lsum = 0.0f;
-                } else if (diagonal && n0 > c_block) {
-#pragma unroll
-                    for (int tp = 0; tp < 4; tp++)
-#pragma unroll
-                        for (int c = 0; c < 8; c++) pf[tp][c] = (VT)0.0f;
+                if (past_block || (large != 0 && !live)) {
                     lsum = 0.0f;
                 } else if (large != 0 || diagonal || (ragged && live && vt0 == nk - 1)) {
                     float raw = -INFINITY;
@@ -1062,7 +1058,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                     redo_if_large();
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                o[dt] = PVT::mfma(vfr[j], pf[tp], o[dt]);
+                if (!past_block) o[dt] = PVT::mfma(vfr[j], pf[tp], o[dt]);
                 if constexpr (j + VDIST < PV_SLOTS) read_v(IC<j + VDIST>{});
                 // hidden keys of the next step's scores (Q.K^T finished above) are set to -inf under the
                 // P.V instructions

@@ -102,3 +102,30 @@ def test_against_the_oracle(dt, m, n, layout, gpu_device):
         cos, _, max_abs = O.accuracy_metrics(o.cpu(), want)
         assert cos >= 0.9995 and max_abs <= 2e-2
         torch.testing.assert_close(lse.cpu(), want_lse, atol=2e-3, rtol=1e-4)
+
+
+@pytest.mark.parametrize("m,n,d", [(256, 256, 64), (256, 320, 128), (700, 712, 64)])  # even and odd numbers of steps, a ragged last tile
+@pytest.mark.parametrize("dt", [torch.float16, torch.float32])
+def test_v_past_the_limit_of_a_block(dt, m, n, d, gpu_device):
+    """Inf and NaN in V reach the 128-row blocks that visit their tile and no other: the reference skips tiles that the causal
+    mask hides from every row of a block."""
+    g = torch.Generator().manual_seed(m + n)
+    q8 = torch.randint(-127, 128, (1, 2, m, d), generator=g, dtype=torch.int8)
+    k8 = torch.randint(-127, 128, (1, 2, n, d), generator=g, dtype=torch.int8)
+    qs = torch.rand(1, 2, -(-m // 128), generator=g) * 2e-3 + 1e-4
+    ks = torch.rand(1, 2, -(-n // 64), generator=g) * 2e-2 + 1e-3
+    mask = torch.randn(1, 2, m, n, generator=g).to(dt).to(gpu_device)
+    wide = torch.zeros(1, 2, m, n + 1, dtype=dt, device=gpu_device)[..., :n]  # rows 16-byte loads cannot take
+    wide.copy_(mask)
+    for key, bad in ((n - 1, float("inf")), (n - 60, float("nan")), (n - m + 128, float("-inf"))):
+        v = torch.randn(1, 2, n, d, generator=g).to(torch.bfloat16 if d == 128 else torch.float16)
+        v[:, 0, key, 3] = bad
+        x = [t.to(gpu_device) for t in (q8, qs, k8, ks, v)]
+        o, lse = _launch(*x, mask)
+        o2, lse2 = _launch(*x, wide)
+        torch.testing.assert_close(lse, lse2, atol=2e-3, rtol=1e-4)
+        assert torch.equal(torch.isfinite(o), torch.isfinite(o2))
+        # the first row of the first 128-row block that visits the key's tile
+        first = max(0, (key // 64 * 64 - (n - m)) // 128 * 128)
+        assert torch.isfinite(o[:, :, :first]).all() and not torch.isfinite(o[:, 0, first:, 3]).any()
+        assert torch.isfinite(o[:, 1]).all() and torch.isfinite(o[..., :3]).all()
