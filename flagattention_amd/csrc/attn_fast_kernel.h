@@ -467,7 +467,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             bool odd = false;
             for (int r = 0; r < visit_group; r++) {
                 const int t = min(lane * visit_group + r, a.nk - 1);
-                const float ks = a.k_scale[kv_row + t];
+                const float ks = fabsf(a.k_scale[kv_row + t]);  // (a caller's own scales may be negative)
                 odd |= !(ks < 3.0e38f) || a.scan_v[kv_row + t] != 0;
                 ks_max = fmaxf(ks_max, ks);
                 float e[kFastRows / kScanRows];
@@ -486,10 +486,10 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
 #pragma unroll
                     for (int i = 0; i < 4; i++) sum = __builtin_amdgcn_sad_u8((unsigned)qf[t][i] ^ 0x80808080u, 0x80808080u, sum);
                 sum += __shfl_xor(sum, 32);
-                float q_sum = (float)sum * qs;
+                float q_sum = (float)sum * fabsf(qs);
 #pragma unroll
                 for (int x = 1; x < 32; x <<= 1) q_sum = fmaxf(q_sum, __shfl_xor(q_sum, x));
-                if (!(qs < 3.0e38f)) q_sum = INFINITY;
+                if (!(fabsf(qs) < 3.0e38f)) q_sum = INFINITY;
                 float* sums = reinterpret_cast<float*>(smem);  // (nothing is on its way into the tile buffers yet)
                 if (lane == 0) sums[wave] = q_sum;
                 __syncthreads();

@@ -1,6 +1,7 @@
 """Tiles left out under a mask tensor that the heads share (csrc/mask_scan.hip): the launch with the scan (workspace given) against
 the one that visits every tile (no workspace), and against the oracle's arithmetic through the latter's own tests."""
 import ctypes
+import math
 
 import pytest
 import torch
@@ -155,6 +156,41 @@ def test_scan_nonfinite(mask_dt):
             assert torch.equal(torch.isnan(res[0][0]), torch.isnan(res[1][0]))
             continue
         _check(res, torch.float16)
+
+
+@gpu
+@pytest.mark.parametrize("sign", [1, -1])
+@pytest.mark.parametrize("mask_dt", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("d", [64, 128])
+def test_scores_that_outweigh_their_entries(d, mask_dt, sign):
+    """Tiles of entries of -296 that a good part of a row's weight lies in all the same.  sign 1: scores of 150 there and -150
+    elsewhere, 0.99 of the difference that the bound on the scores allows.  sign -1: scores of 300 there by negative block
+    scales on negative products, -1.5 elsewhere."""
+    b, h, m, n = 1, 2, 256, 3072
+    dev, dt = "cuda:0", torch.bfloat16 if d == 128 else torch.float16
+    q8, qs, k8, ks, v = _inputs(b, h, h, m, n, d, dt, True)
+    q8.fill_(127)
+    k8.fill_(-127)
+    ks.fill_(1e-2 if sign > 0 else 1e-4)
+    qs.fill_(150.0 / (127 * 127 * d) / 1e-2)
+    mask = torch.zeros(1, 1, m, n, dtype=mask_dt, device=dev)
+    for tile in (5, 30, 31, 47):
+        keys = slice(64 * tile, 64 * tile + 64)
+        mask[..., keys] = -296.0
+        if sign > 0:
+            k8[:, :, keys] = 127
+        else:
+            ks[..., tile] = -2e-2
+    o, lse = _both(q8, qs, k8, ks, v, mask, True)[0]
+    sc = qs.double().repeat_interleave(128, -1)[..., None] * ks.double().repeat_interleave(64, -1)[..., None, :]
+    s = (q8.double() @ k8.double().transpose(-1, -2).contiguous()) * sc + mask.double()
+    p = torch.softmax(s * math.log(2.0), -1)
+    assert p[..., 320:384].sum(-1).min() > 0.1
+    # An exponent is off by 2e-4 at most (the scale times 1.5 * 2^23 is near 3700: half of its unit, 1.2e-4; scores near 300: 3e-5 for
+    # each of two roundings), P by 1.4e-4 of itself and half a unit of the 16-bit type; twice that for the ratio of two sums
+    unit = 2.0 ** -8 if dt is torch.bfloat16 else 2.0 ** -11
+    torch.testing.assert_close(o.double(), p @ v.double(), rtol=0, atol=(2.8e-4 + unit) * v.abs().max().item())
+    torch.testing.assert_close(lse.double(), torch.logsumexp(s * math.log(2.0), -1) / math.log(2.0), rtol=0, atol=2e-4 + unit)
 
 
 @gpu
