@@ -199,17 +199,36 @@ int mask_splits(const AttnArgs& a, int64_t batch, int head_dim) {
 }
 
 // Worth its launch where the heads share the mask (one read of it serves all of them; a mask per head is a position bias as a
-// rule, and read once either way) and enough steps can go: 12 tiles where there are more q-blocks than compute units (B3 H32
-// M858 N858 D128 padded fp32: 99.8 us without, 98.4 with).  With fewer only the longest q-block counts, which padding shortens
-// and a causal mask does not: about 48 us of steps (B3 H8 M640 D128 39 without, 43 with, B3 H8 M1760 D64 59.6, 63.3; B1 H16 M3392 D128
-// 119, 108), and not for masks of rows only (a batch whose longest sequence fills the keys has nothing to leave out: B2 H16/2
-// M1792 padded 79.5, 84.5).  V is read once more, so the queries per K/V head have to be many as well.
+// rule, and read once either way) and enough steps can go.  What it costs (a launch, the bytes of the mask and of V, 1 to 2 us in
+// every workgroup) a mask that hides no tile loses; what it gains lies in the entries, which the rule does not see.  The lines lie
+// where the masks that model code builds gain, a causal one or the padding of sequences between half as long and as long as the
+// keys.  Attention call with the scan over the one without (mean of 1060 shapes: 2 to 32 heads, 1 to 8 sequences, 512 to 8192 keys):
+//   more q-blocks than compute units       hides nothing  causal  causal and padding
+//     entries per row, 8 to 12 tiles         1.16 - 1.24    0.85    0.85
+//     14 to 20                               1.11 - 1.20    0.76    0.76
+//     24 to 32                               1.05 - 1.11    0.72    0.71
+//     from 36                                0.98 - 1.09    0.62    0.61
+//   more q-blocks than compute units       hides nothing  padding
+//     one row of entries, 8 to 24 tiles      1.08 - 1.23    1.04    (not scanned; 0.83 to 1.20)
+//     from 28                                1.02 - 1.11    0.92
+//     causal mask folded into a bool one, whose walk ends at the limit anyway: padding 1.02 up to 30 tiles (not scanned; 0.90 to
+//     1.11), 0.95 from 36
+//   fewer, unsplit, 48 us of steps and more: the longest q-block alone counts, which a causal mask does not shorten and padding
+//   seldom where there are several sequences, the longest of which is nearly full
+//                                          hides nothing  causal  causal and padding
+//     one sequence                           1.05 - 1.20    1.12    0.92
+//     two to eight                           1.08 - 1.20    1.12    1.05    (not scanned)
+// V is read once more, so the queries per K/V head have to be many as well.
 int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch, int head_dim) {
     const int64_t q_blocks = batch * a.Hq * ((a.M + kFastRows - 1) / kFastRows);
     if (a.causal) return 0;  // (the largest entry of a row may lie where the causal mask adds -1e6 to it)
     if (a.ms_h != 0 || a.Hq < 2) return 0;
     if (mask_splits(a, batch, head_dim) == 1) {
-        if (q_blocks > 256 ? a.nk < 12 : (a.ms_m == 0 || step_us(head_dim) * (float)a.nk < 48.0f)) return 0;
+        if (q_blocks > 256) {
+            if (a.nk < (a.mask_causal ? 36 : a.ms_m == 0 ? 28 : 12)) return 0;
+        } else if (a.ms_m == 0 || batch > 1 || step_us(head_dim) * (float)a.nk < 48.0f) {
+            return 0;
+        }
         if ((int64_t)a.groups * a.M < 512) return 0;
     }
     const int64_t mask_wgs = mask_batches(a, batch) * scan_strips(a), v_tiles = batch * a.Hkv * a.nk;

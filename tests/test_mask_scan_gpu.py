@@ -108,9 +108,9 @@ def _check(res, dt):
 
 
 # b, h, hkv, m, n, d, hnd: few q-blocks, whose tiles are split over runs (a ragged last tile; more than 64 tiles, two per bit; fewer
-# tiles than a run of each); more q-blocks than compute units, unsplit
+# tiles than a run of each); more q-blocks than compute units, unsplit (29 tiles: from 28 on every kind of mask is scanned)
 SHAPES = [(2, 4, 2, 300, 3072, 64, True), (2, 2, 2, 600, 1608, 128, False), (1, 4, 1, 300, 4304, 64, True), (1, 2, 1, 7, 2000, 64, True),
-          (3, 48, 2, 520, 776, 64, True)]
+          (3, 48, 2, 520, 1800, 64, True)]
 
 
 @gpu
