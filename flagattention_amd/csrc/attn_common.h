@@ -193,7 +193,7 @@ int launch_decode(const AttnArgs& a, int64_t batch, int head_dim, int v_dtype, b
 
 // The pipelined kernel under a bool mask tensor or an additive fp16 / bf16 one, where fast_serves_mask() says so (a.mask
 // set; esz: bytes per mask entry).
-bool fast_serves_mask(const AttnArgs& a, int esz);
+bool fast_serves_mask(const AttnArgs& a, int head_dim, int esz);
 int launch_fast_masked(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
 int launch_fast_additive(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);
 int launch_fast_additive_causal(const AttnArgs& a, int head_dim, int v_dtype, hipStream_t stream);

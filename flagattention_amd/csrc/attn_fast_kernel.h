@@ -453,7 +453,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         visit_group = a.visit_group;
         const int groups = (nsteps + visit_group - 1) / visit_group;
         bool hidden_row = false;
-        if (a.scan_top) {
+        if (!MC && a.scan_top) {  // (masks under the causal flag are not scanned)
             const int mb = a.ms_b ? b : 0;
             const int s0 = a.ms_m ? (kFastRows / kScanRows) * iq : 0, s1 = min(s0 + kFastRows / kScanRows, a.scan_strips);
             const float* tops = a.scan_top + (int64_t)mb * a.scan_strips * a.nk;

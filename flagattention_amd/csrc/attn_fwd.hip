@@ -514,7 +514,7 @@ AttnArgs attn_args(const sage_attn_params& p) {
 
 // a mask tensor that the pipelined kernel stages
 bool fast_masked(const sage_attn_params& p, const AttnArgs& a) {
-    return p.mask_kind != SAGE_MASK_NONE && attn::fast_serves_mask(a, a.mask_additive ? dtype_bytes(a.mask_dt) : 1);
+    return p.mask_kind != SAGE_MASK_NONE && attn::fast_serves_mask(a, (int)p.head_dim, a.mask_additive ? dtype_bytes(a.mask_dt) : 1);
 }
 
 // workspace of the partial results under a scanned mask, behind the scan's

@@ -42,10 +42,14 @@ int launch_masked(const AttnArgs& a, hipStream_t stream) {
 // 16-byte aligned, no load that reaches past the end of a row (kv_len a multiple of 16, or rows that the caller
 // padded with zeros to one), no causal flag on top of a bool mask.
 // (esz: bytes per mask entry, 1 for bool masks, 2 / 4 for additive ones)
-bool fast_serves_mask(const AttnArgs& a, int esz) {
+bool fast_serves_mask(const AttnArgs& a, int head_dim, int esz) {
     const int per16 = 16 / esz;  // entries per 16-byte load
-    // (additive and causal: every step of two tiles lies on the diagonal; B1 H16 M128 N128 D128 fp32 18.5 us on the general kernel, 21.2)
-    return a.mask != nullptr && (!a.causal || (a.mask_additive && a.nk > 2)) && a.ms_n == 1 && ((uintptr_t)a.mask % 16) == 0 &&
+    // (additive and causal: nearly every step of a few tiles lies on the diagonal and is redone.  General kernel -> here, us:
+    // 16-bit entries, three tiles, head_dim 128 B4 H8/1 M156 22.1 -> 26.9, M192 18.9 -> 19.5, head_dim 64 0.87 to 1.00 times as long; four
+    // tiles 0.70 to 1.03.  fp32 entries, three tiles B4 H32/8 M192 D128 19.3 -> 23.7, D64 17.3 -> 18.6; four whole ones B2 H24 M256 D128
+    // 19.2 -> 22.3, B4 H24 M256 D64 17.5 -> 19.0, four with a ragged last one 0.86 to 0.92 times)
+    const int few = esz == 4 ? (a.N % BN ? 3 : 4) : head_dim == 128 ? 3 : 2;
+    return a.mask != nullptr && (!a.causal || (a.mask_additive && a.nk > few)) && a.ms_n == 1 && ((uintptr_t)a.mask % 16) == 0 &&
            a.ms_b % per16 == 0 && a.ms_h % per16 == 0 && a.ms_m % per16 == 0 && a.ms_m >= 0 && a.ms_m < (1 << 24) &&
            (a.N % per16 == 0 || a.mask_padded);
 }

@@ -294,9 +294,10 @@ def _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, r
                                           torch.bfloat16: (_lib.MASK_BF16, _lib.MASK_BF16_PADDED),
                                           torch.float32: (_lib.MASK_F32, _lib.MASK_F32_PADDED)}[m.dtype]
                     mask_kind = plain
-                    # additive masks run on the pipelined kernel; one whose rows it cannot load 16 bytes at a time goes there
-                    # through a padded copy
-                    if (not causal or nk > 2) and not _additive_mask_is_direct(m.expand(b, h_qo, qo_len, kv_len), kv_len):
+                    # additive masks run on the pipelined kernel (with the causal flag from a few key tiles on); one whose rows it
+                    # cannot load 16 bytes at a time goes there through a padded copy
+                    few = (3 if kv_len % 64 else 4) if m.dtype is torch.float32 else (3 if head_dim == 128 else 2)
+                    if (not causal or nk > few) and not _additive_mask_is_direct(m.expand(b, h_qo, qo_len, kv_len), kv_len):
                         if torch.cuda.is_current_stream_capturing():
                             padded, _ = _stage_additive_mask(m, b, h_qo, qo_len, kv_len)
                         else:

@@ -86,7 +86,8 @@ int sage_per_block_int8(const sage_quant_params* p, void* stream);
  *                the key tiles beyond that limit, which the reference would skip one by one as all-False tiles;
  *                SAGE_MASK_F32 / SAGE_MASK_F16 / SAGE_MASK_BF16: additive, in that storage type (:38,50); masks with
  *                unit stride along the keys, 16-byte aligned rows and kv_len * entry size a multiple of 16 bytes (with
- *                the causal flag: more than two tiles of 64 keys) run on the pipelined kernel, others on the general one;
+ *                the causal flag: and more than two to four tiles of 64 keys) run on the pipelined kernel, others on the
+ *                general one;
  *                SAGE_MASK_F16_PADDED / SAGE_MASK_BF16_PADDED / SAGE_MASK_F32_PADDED: the same, and the caller
  *                guarantees that every mask row can be read up to the next multiple of 16 bytes past kv_len (any finite
  *                values there): such a mask runs on the pipelined kernel for any kv_len
