@@ -207,7 +207,7 @@ def test_row_maximum_that_moves_between_tiles(pattern, causal, d, vdtype, gpu_de
 @pytest.mark.parametrize("path", ["ragged", "ragged_causal", "bool_mask", "additive_mask", "causal_m_gt_n"])
 def test_row_maximum_that_moves_between_tiles_other_paths(pattern, path, gpu_device):
     """The same K-scale patterns through a ragged last tile, through both mask kinds and through
-    causal with qo_len > kv_len (the last three run the general kernel)."""
+    causal with qo_len > kv_len (the last one runs the general kernel)."""
     m, n = (320, 700) if path.startswith("ragged") else (448, 384) if path == "causal_m_gt_n" else (200, 640)
     q8, qs, k8, ks, v = _quantized(37, 1, 2, 2, m, n, 128, torch.bfloat16)
     ks2 = ks.clone()
@@ -422,8 +422,8 @@ def test_additive_masks_on_the_pipelined_kernel(kind, d, vdtype, mdtype, m, n, g
 @pytest.mark.parametrize("mdtype", [torch.bfloat16, torch.float32])
 def test_additive_mask_views_and_the_general_kernel_agree(mdtype, gpu_device):
     """The same additive mask as a contiguous tensor (pipelined kernel as it is), as a column slice of a wider
-    tensor (padded copy), and with a causal flag on top (general kernel: a causal flag is not folded into an additive
-    mask): the first two give the same bits, the third matches the oracle's mask + causal arithmetic."""
+    tensor (padded copy), and with a causal flag on top (instances of their own: a causal flag is not folded into an
+    additive mask): the first two give the same bits, the third matches the oracle's mask + causal arithmetic."""
     b, hq, hkv, m, n = 1, 2, 2, 260, 328
     q8, qs, k8, ks, v = _quantized(53, b, hq, hkv, m, n, 128, torch.bfloat16)
     g = torch.Generator().manual_seed(29)

@@ -55,7 +55,9 @@ def test_wrapper_with_mixed_dtypes(layout, gpu_device):
     (2, 8, 2, 3, 3000, 64, False, None),      # few query rows
     (1, 2, 2, 256, 256, 64, False, torch.bool),
     (1, 2, 2, 300, 304, 64, False, torch.float16),
-    (1, 2, 2, 300, 304, 64, True, torch.float32),   # the general kernel
+    (1, 2, 2, 300, 304, 64, True, torch.float32),   # an additive mask with the causal flag
+    (1, 2, 2, 100, 112, 64, True, torch.float16),   # ... over two key tiles: the general kernel, and a launch for the log-sum-exp
+    (1, 2, 2, 100, 64, 128, True, None),            # more queries than keys: the general kernel
 ])
 def test_attention_writes_what_the_kernel_of_its_own_does(b, h, hkv, m, n, d, causal, mask, gpu_device):
     """The log-sum-exp of every route of the attention launch, with and without a shift, bit for bit."""

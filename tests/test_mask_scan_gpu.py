@@ -46,7 +46,7 @@ def _inputs(b, h, hkv, m, n, d, dt, hnd, scale=1.0):
 
 
 def _mask(kind, dt, b, m, n):
-    """Masks shared by the heads, and how many of 256 x 64 tiles a scan may leave out at least (share of all)."""
+    """Masks shared by the heads."""
     dev = "cuda:0"
     g = torch.Generator().manual_seed(n)
     cols, rows = torch.arange(n), torch.arange(m).view(m, 1) + (n - m)
@@ -125,6 +125,50 @@ def test_scan_changes_nothing(shape, mask_dt, kind):
     x = _inputs(b, h, hkv, m, n, d, dt, hnd)
     mask = _mask(kind, mask_dt, b, m, n)
     _check(_both(*x, mask, hnd), dt)
+
+
+@gpu
+@pytest.mark.parametrize("shape", [(2, 4, 2, 300, 3072, 64, True), (3, 48, 2, 520, 1808, 64, True)])
+@pytest.mark.parametrize("mask_dt", [torch.bool, torch.float16, torch.float32])
+@pytest.mark.parametrize("kind", ["padding", "causal_padding", "slope"])
+def test_what_the_scan_finds(kind, mask_dt, shape):
+    """The scan's results as it leaves them in the workspace, and that the rule of the attention kernel, applied to them here,
+    leaves out every tile that padding or the causal mask hides from a whole q-block."""
+    if mask_dt is torch.bool and kind == "slope":
+        pytest.skip("not a bool mask")
+    b, h, hkv, m, n, d, hnd = shape
+    q8, qs, k8, ks, v = _inputs(b, h, hkv, m, n, d, torch.float16, hnd)
+    v[1, 0, n - 1, 3], v[0, 1, 70, 9] = float("inf"), float("nan")
+    mask = _mask(kind, mask_dt, b, m, n)
+    o, lse = torch.empty(q8.shape, device=q8.device), torch.empty(b, h, m, device=q8.device)
+    p = _params(q8, qs, k8, ks, v, mask, o, lse, KIND[mask_dt], hnd)
+    lib = _lib.load()
+    nbytes = lib.sage_attn_fwd_workspace_bytes(ctypes.byref(p))
+    ws = torch.full((nbytes,), 0x7f, dtype=torch.uint8, device=q8.device)
+    _lib.check(lib.sage_attn_fwd_ws(ctypes.byref(p), ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream), "ws")
+    torch.cuda.synchronize()
+    nk, mb, rows = -(-n // 64), mask.shape[0] if mask.stride(0) or mask.shape[0] == 1 else 1, m if p.mask_stride_m else 1
+    strips = -(-rows // 16)
+    f = ws[: nbytes // 4 * 4].view(torch.float32)
+    top, low = f[: mb * strips * nk].view(mb, strips, nk), f[mb * strips * nk: mb * strips * (nk + 1)].view(mb, strips)
+    odd = f[mb * strips * (nk + 1): mb * strips * (nk + 1) + b * hkv * nk].view(torch.int32).view(b, hkv, nk)
+    e = torch.zeros(mask.shape, device=mask.device).masked_fill_(~mask, float("-inf")) if mask_dt is torch.bool else mask.float()
+    e = torch.nn.functional.pad(e[:mb, 0, :rows], (0, nk * 64 - n), value=float("-inf"))
+    e = torch.nn.functional.pad(e, (0, 0, 0, strips * 16 - rows), mode="replicate") if strips * 16 > rows else e
+    tiles = e.view(mb, strips, 16, nk, 64).amax((2, 4))
+    if mask_dt is not torch.bool and n % 64:
+        tiles[..., -1].clamp_(min=-1.0e6)
+    assert torch.equal(top, tiles) and torch.equal(low, e.view(mb, strips, 16, -1).amax(-1).amin(-1))
+    bad = ~torch.isfinite(torch.nn.functional.pad(v, (0, 0, 0, nk * 64 - n)).view(b, hkv, nk, 64 * d)).all(-1)
+    assert torch.equal(odd != 0, bad)
+    # the rule: 256-row q-blocks, the largest scales and sums of |q| of the call (a bound above that of every block)
+    bound = 256 * ks.max() * (q8.float().abs().sum(-1).amax() * qs.max())
+    per = 16 if p.mask_stride_m else 1
+    blocks = [slice(i, i + per) for i in range(0, strips, per)]
+    left = torch.stack([top[:, s].amax(1) < (0.0 if mask_dt is torch.bool else low[:, s].amin(1, keepdim=True)) - 150.0 - bound for s in blocks], 1)
+    hidden = torch.stack([tiles[:, s].amax(1) < -1e4 for s in blocks], 1)
+    assert torch.equal(left, hidden) if kind != "slope" else not hidden.any()
+    assert left.float().mean() > {"padding": 0.3, "causal_padding": 0.3, "slope": 0.0}[kind]
 
 
 @gpu
