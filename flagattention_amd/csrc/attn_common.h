@@ -57,7 +57,7 @@ struct AttnArgs {
     // other).  Under a mask shared by the heads, head_tile heads x several q-blocks run side by side on an XCD, so
     // that both the mask tiles (shared by the heads) and the K/V tiles (shared by the q-blocks) are re-read from L2.
     int32_t head_tile;
-    // Split of the keys over several workgroups per (batch, head, q-block) (never under a mask tensor): workgroup s
+    // Split of the keys (under a mask tensor: of the tiles it leaves to visit) over several workgroups per (batch, head, q-block): workgroup s
     // of `nsplit` takes steps s * split_steps .. and writes an fp32 partial output and its base-2 log-sum-exp to
     // out + s * out_split_stride / lse + s * lse_split_stride, which a second kernel combines.  Unsplit: 1, nk, 0, 0.
     int32_t nsplit, split_steps;

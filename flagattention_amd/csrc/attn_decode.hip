@@ -36,7 +36,7 @@ constexpr int kTileKeys = 32;
 template <int D>
 __device__ __forceinline__ int v_swizzle(int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); }
 
-// RT: 32-row tiles of query rows (groups * qo_len <= 32 * RT)
+// RT: 32-row tiles of packed query rows (groups * qo_len) per workgroup
 // kDecodeWaves: eight (one workgroup per CU), or four: with one row tile where the items alone fill the chip (two
 // workgroups per CU, finer rounds: B11 H32/32 M1 N700 D128 26 us against 32 us), and with two row tiles, which leave
 // registers for one wave per SIMD only.

@@ -105,11 +105,12 @@ __device__ __forceinline__ typename PV<VT>::vec tr_pair(const unsigned char* p0,
 // attn_qk_int8_per_block.py:46-52) and its skipping of 128 x 64 tiles without a visible key (:33-36) are
 // served by the path that redoes a step: such rows start from the reference point -inf, which drives every
 // step into that path until the row has seen a key.  a.mask_causal: the caller folded the causal mask into the
-// tensor, so tiles beyond the causal limit of the workgroup's last row need no visit.  Additive masks and masks
-// with unaligned rows stay with the general kernel (attn_fwd.hip).
+// tensor, so tiles beyond the causal limit of the workgroup's last row need no visit.  Masks with unaligned rows stay
+// with the general kernel (attn_fwd.hip).
 //
 // MT (the type of a mask entry): void = no mask tensor, bool = the bool mask above, _Float16 / __bf16 = an additive
-// mask tensor in that storage type (attn_qk_int8_per_block.py:37-38,49-50: score + mask entry, no tile is skipped).
+// mask tensor in that storage type (attn_qk_int8_per_block.py:37-38,49-50: score + mask entry; a tile is left out
+// only where that changes nothing: `visits` below).
 // Staged like the bool mask, 32 x 64 entries of 2 bytes per wave and step, two steps resident (with the four K/V
 // tiles that fills the 160 KB of the CU at head_dim 128: the entries of step j + 1 are requested during the
 // vector phase of step j, ahead of that phase's K/V loads, and waited for at the end of the matrix phase that

@@ -235,11 +235,11 @@ PyObject* put_quant(PyObject*, PyObject* const* a, Py_ssize_t n) {  // + (params
     });
 }
 
-// ---- SageAttention forward: (q, k, v, q_scale, k_scale, layout, mask, out_dtype, return_lse, causal, lse_mul, lse_shift)
+// ---- SageAttention forward: (q, k, v, q_scale, k_scale, layout, mask, out_dtype, return_lse, causal, shift_mul, shift)
 struct AttnCall {
     const at::Tensor *q, *k, *v, *qs, *ks, *mask = nullptr, *shift = nullptr;
     bool hnd, want_lse, causal, natural = false;
-    double lse_mul = 0.0;
+    double shift_mul = 0.0;
     at::ScalarType out;
     Key key;
     bool parse(PyObject* const* a, Py_ssize_t n) {
@@ -257,7 +257,7 @@ struct AttnCall {
         if (a[10] != Py_None) {
             if (!PyFloat_CheckExact(a[10])) return false;
             natural = true;
-            lse_mul = PyFloat_AS_DOUBLE(a[10]);
+            shift_mul = PyFloat_AS_DOUBLE(a[10]);
             if (a[11] != Py_None) {
                 if (!plain(a[11])) return false;
                 shift = &THPVariable_Unpack(a[11]);
@@ -302,7 +302,7 @@ PyObject* attn(PyObject*, PyObject* const* a, Py_ssize_t n) {
         at::Tensor ws;
         if (plan->workspace > 0) ws = workspace(dev, plan->workspace);
         void* wp = plan->workspace > 0 ? ws.data_ptr() : nullptr;
-        const int rc = c.natural ? sage_attn_fwd_natural(&p, c.shift ? (const float*)c.shift->data_ptr() : nullptr, (float)c.lse_mul, wp, plan->workspace, stream)
+        const int rc = c.natural ? sage_attn_fwd_natural(&p, c.shift ? (const float*)c.shift->data_ptr() : nullptr, (float)c.shift_mul, wp, plan->workspace, stream)
                                  : sage_attn_fwd_ws(&p, wp, plan->workspace, stream);
         if (rc) return PyLong_FromLong(rc);
         return pack({&o, &lse});

@@ -245,7 +245,9 @@ static int plan_decode_split(int64_t items, int64_t rows, int64_t nk) {
 // one after the other, and a kernel that runs only a few steps spends less on its start.  Returns the runs of the keys, 0: not here.
 // Every workgroup has a compute unit of its own; or there are two or three for each where half of them are short (causal), where two
 // fit a CU (head_dim 64) or where the pipelined kernel runs its instance that hides keys (a ragged last tile).  The K/V rows that
-// all of them read, once per row tile, stay below 100 MB (causal, half of them: 130).  Times in us fitted to 350 launches within 12 %.
+// all of them read, once per row tile, stay below 100 MB (causal, half of them: 130).  Times in us fitted to 350 launches within
+// 12 %; over 1750 others of its range 0.72 (int8) and 0.79 (dense) of the time on the pipelined kernel on average, five and 25 of them more
+// than 2.5 % slower (worst: int8 B6 H2 M67 N13312 D64 21.0 -> 23.3, dense B1 H8 M82 N3584 D128 17.3 -> 20.1).
 // Measured, pipelined kernel -> here (us, in a graph):
 //   int8  D64  B1 H2 M256 N256 8.0 -> 5.4, H8 N512 causal 22 -> 6.6, H8 N1024 18 -> 9.2, H2 N2048 causal 25 -> 12; D128 H8 N512 17 -> 10.4
 //   dense D128 H2 N200 13.2 -> 9.4, H8 N512 causal 35 -> 12.6, H8 N128 causal 10.3 -> 7.5, H2 N2048 28 -> 23

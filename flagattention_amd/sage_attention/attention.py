@@ -171,10 +171,10 @@ def forward(q, k, v, q_scale, k_scale, tensor_layout="HND", attn_mask=None,
     return _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg, causal)
 
 
-def _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg, causal, lse_mul=None, lse_shift=None):
-    """``forward``; with a number ``lse_mul`` the log-sum-exp is the natural one plus ``lse_mul * lse_shift`` (``[B, Hq, M]``
+def _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg, causal, shift_mul=None, shift=None):
+    """``forward``; with a number ``shift_mul`` the log-sum-exp is the natural one plus ``shift_mul * shift`` (``[B, Hq, M]``
     fp32 contiguous, or None), what ``sageattn`` returns."""
-    call = (q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, causal, lse_mul, lse_shift)
+    call = (q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, causal, shift_mul, shift)
     if maxnreg is None:
         out = (_lib._host_module or _lib.host()).attn(*call)  # a call shape seen before: outputs, or a status
         if out is not None:
@@ -211,8 +211,8 @@ def _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, r
         # copies (the reference takes whatever its compiler's dot takes, attn_qk_int8_per_block.py:161,185).
         pad = (0, 64 - head_dim)
         qp, kp, vp = (torch.nn.functional.pad(t, pad) for t in (q, k, v))
-        o, lse = _attend(qp, kp, vp, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg, causal, lse_mul,
-                         lse_shift)
+        o, lse = _attend(qp, kp, vp, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, return_lse, maxnreg, causal, shift_mul,
+                         shift)
         return o[..., :head_dim].contiguous(), lse
     if head_dim not in (64, 128):
         raise ValueError(f"head_dim {head_dim} not supported (16, 32, 64 or 128)")
@@ -248,8 +248,8 @@ def _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, r
             o.zero_()
             if return_lse:
                 lse.fill_(float("-inf"))
-                if lse_shift is not None:
-                    lse += lse_mul * lse_shift
+                if shift is not None:
+                    lse += shift_mul * shift
             return o, lse
 
         stream = current_stream_ptr(dev)
@@ -345,9 +345,9 @@ def _attend(q, k, v, q_scale, k_scale, tensor_layout, attn_mask, output_dtype, r
             ws_ptr, ws_bytes = ws.data_ptr(), ws.numel()
         else:
             ws_ptr, ws_bytes = None, 0
-        if lse_mul is None:
+        if shift_mul is None:
             _lib.check(lib.sage_attn_fwd_ws(p_ref, ws_ptr, ws_bytes, stream), "sage_attn_fwd_ws")
         else:
-            _lib.check(lib.sage_attn_fwd_natural(p_ref, None if lse_shift is None else lse_shift.data_ptr(), lse_mul, ws_ptr, ws_bytes,
+            _lib.check(lib.sage_attn_fwd_natural(p_ref, None if shift is None else shift.data_ptr(), shift_mul, ws_ptr, ws_bytes,
                                                  stream), "sage_attn_fwd_natural")
     return o, lse

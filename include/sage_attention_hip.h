@@ -110,18 +110,21 @@ int sage_attn_fwd(const sage_attn_params* p, void* stream);
 
 /*
  * The same call with a workspace, for launches that would leave most of the chip idle: when
- * batch * heads_q * ceil(qo_len / 256) is well below the 256 compute units and no mask tensor is given, the keys
+ * batch * heads_q * ceil(qo_len / 256) is well below the 256 compute units, the keys
  * of every (batch, head, 256-query block) are cut into runs of whole 64-key steps, one workgroup each; the runs
  * write normalized fp32 partial outputs and their base-2 log-sum-exps to the workspace and a second kernel
  * combines them (out = sum_s 2^(lse_s - lse) o_s, lse = log2 sum_s 2^lse_s).  Calls with few query rows per K/V
  * head (decoding: heads_q / heads_kv * qo_len of at most 32, or of at most 64 for grouped heads) cut the keys of a
  * (batch, K/V head) in the same way, for the kernel that packs those rows.  Launches whose last round over the compute
  * units, or whose causal q-blocks, leave many of them idle are cut into up to 256 equal shares of all their 64-key steps
- * instead (at most two partial results of 256 rows per share, 68 MB at head_dim 128).  The reference's SageAttention launch has no such split (attn_qk_int8_per_block.py:176-190 is one grid over q-blocks); its dense forward does
- * (see sage_flash_attn_fwd_ws).  Results agree with sage_attn_fwd to fp32 rounding of the combination.
- *   sage_attn_fwd_workspace_bytes  bytes the split of this call would use; 0 = the call would not split;
+ * instead (at most two partial results of 256 rows per share, 68 MB at head_dim 128).  Under a mask tensor that the heads
+ * share, longer calls first scan the mask into the workspace (the largest entry of every 16 rows and 64 keys, tiles of V that
+ * hold an Inf or NaN); tiles of keys that change nothing are then not visited, and the others are what a split cuts.  The reference's SageAttention launch has no such split (attn_qk_int8_per_block.py:176-190 is one grid over q-blocks); its dense forward does
+ * (see sage_flash_attn_fwd_ws).  Results agree with sage_attn_fwd to fp32 rounding of the combination, and under a scanned mask to the rounding of P
+ * to 16 bits, which the first tile a row visits decides.
+ *   sage_attn_fwd_workspace_bytes  bytes the split or scan of this call would use; 0 = neither;
  *                                  -1 = invalid params (sage_hip_last_error says why)
- *   workspace                      device memory, 16-byte aligned, at least that large; NULL or smaller: no split,
+ *   workspace                      device memory, 16-byte aligned, at least that large; NULL or smaller: neither,
  *                                  the call is sage_attn_fwd.  Contents need not be initialised and are not
  *                                  meaningful afterwards; calls on one stream may share one workspace.
  */
@@ -133,10 +136,14 @@ int sage_attn_fwd_ws(const sage_attn_params* p, void* workspace, int64_t workspa
  * lse[i] = ln 2 * lse[i] + shift_mul * shift[i] for n contiguous values.  shift: what smoothing took off the logits of a
  * row before scaling (q_dot_km of sage_per_block_int8_smooth_k, shift_mul = sm_scale), or NULL.
  */
-/* sage_attn_fwd_ws whose log-sum-exp leaves as sage_lse_natural would make it (shift: [B, Hq, M] contiguous, or NULL). */
+int sage_lse_natural(float* lse, const float* shift, float shift_mul, int64_t n, void* stream);
+
+/*
+ * sage_attn_fwd_ws whose log-sum-exp leaves as sage_lse_natural would make it (shift: [B, Hq, M] contiguous, or NULL).  shift
+ * and shift_mul count only where p->lse is set.
+ */
 int sage_attn_fwd_natural(const sage_attn_params* p, const float* shift, float shift_mul, void* workspace, int64_t workspace_bytes,
                           void* stream);
-int sage_lse_natural(float* lse, const float* shift, float shift_mul, int64_t n, void* stream);
 
 /*
  * Mean of K over the sequence axis in a fixed fp32 order, for callers that want the library
