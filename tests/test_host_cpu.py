@@ -117,7 +117,7 @@ def test_key_split_plan_and_workspace_size():
     assert size(1, 24, 32768, 32768, 128) == 0
     assert size(1, 205, 256, 65536, 64) == 0
     assert size(1, 4, 128, 448, 128) == 0
-    # a mask tensor keeps the call on one workgroup per q-block
+    # a mask tensor of the general kernel (no unit stride along the keys) keeps the call on one workgroup per q-block
     assert size(1, 4, 128, 8192, 128, mask_kind=_lib.MASK_BOOL) == 0
     # short queries against many keys: runs x batch x heads x rows x (head_dim + 1) fp32
     for b, h, m, n, d in ((1, 4, 128, 8192, 128), (2, 8, 1, 4096, 64), (1, 32, 300, 32768, 128)):
@@ -137,6 +137,27 @@ def test_key_split_plan_and_workspace_size():
     assert b"head_dim 96" in lib.sage_hip_last_error()
     f = _lib.FlashParams()
     assert lib.sage_flash_attn_fwd_workspace_bytes(ctypes.byref(f)) == -1
+
+
+@pytest.mark.parametrize("scanned,batch,heads,n,d,rows,folded", [
+    # more q-blocks than compute units: entries per row from 12 tiles of 64 keys, one row from 28, a folded causal mask from 36
+    (False, 8, 32, 11 * 64, 128, True, False), (True, 8, 32, 12 * 64, 128, True, False),
+    (False, 8, 32, 27 * 64, 64, False, False), (True, 8, 32, 28 * 64, 64, False, False),
+    (False, 8, 32, 35 * 64, 128, True, True), (True, 8, 32, 36 * 64, 128, True, True),
+    # fewer, too many to split: one sequence alone, of 48 us of steps (32 tiles at head_dim 128, 57 at 64)
+    (False, 1, 16, 31 * 64, 128, True, False), (True, 1, 16, 33 * 64, 128, True, False),
+    (False, 2, 8, 40 * 64, 128, True, False), (False, 1, 16, 33 * 64, 128, False, False),
+])
+def test_which_masks_are_scanned(scanned, batch, heads, n, d, rows, folded):
+    """The rule on sizes that decides whether a shared mask is scanned for tiles to leave out."""
+    from flagattention_amd import _lib
+
+    p = _attn_desc(batch, heads, n, n, d, mask_kind=_lib.MASK_BOOL_PADDED_CAUSAL if folded else _lib.MASK_BOOL)
+    p.mask_stride_n, p.mask_stride_m, p.mask_stride_b = 1, n if rows else 0, n * (n if rows else 1)
+    nk, strips = n // 64, -(-n // 16) if rows else 1
+    want = 4 * (batch * strips * (nk + 1) + batch * heads * nk)
+    got = _lib.load().sage_attn_fwd_workspace_bytes(ctypes.byref(p))
+    assert got == (-(-want // 16) * 16 if scanned else 0)
 
 
 def test_bool_mask_staging_copy():
