@@ -13,14 +13,17 @@
 // products 5.5, three-input XOR 4.8, exponential 9, FMA and XOR 3; with two waves per SIMD everything takes 5.7 or more):
 // * the generator is unrolled by hand (philox6_from_product): 4 full products, 3 high and 1 low half and one 64-bit addition per
 //   score instead of 12 full products; what depends on the row only is computed once per row;
+// * exclusive ors of three operands are one instruction each (xor3), and so are the last exclusive or and the subtraction of the
+//   keep decision;
 // * the keep decision is an integer threshold and a sign, applied to two 16-bit P at a time (no compare, no select);
 // * the rest is kept small: K and V tiles of 32 keys go straight into LDS for the four waves of a workgroup (32 queries
 //   each, S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16, V^T by ds_read_b64_tr_b16), one barrier per tile, loads
 //   one tile ahead (a tile takes microseconds), registers for four (head_dim 128: two) waves per SIMD;
 // * workgroups are handed out longest first over all heads.
-// B4 H16 M2048 N2048 D64 fp16 causal 397 -> 143 us, without the causal flag 404 -> 273 us; B2 H32 M4096 N4096 D128 3475 -> 1223
-// us, causal 3445 -> 629 us (before: the generator rolled out by the compiler, V^T gathered from LDS entry by entry,
-// short rows first).  At head_dim 128 three waves per SIMD need 18 spilled registers and run 6 % slower than two.
+// B4 H16 M2048 N2048 D64 fp16 causal 397 -> 143 us, without the causal flag 404 -> 272 us; B2 H32 M4096 N4096 D128 3475 -> 1207
+// us, causal 3445 -> 619 us (before: the generator rolled out by the compiler, V^T gathered from LDS entry by entry,
+// short rows first).  With xor3 120, 226, 1114 and 573 us.  At head_dim 128 three waves per SIMD need 18 spilled registers and
+// run 6 % slower than two.
 #include "attn_common.h"
 
 namespace sage {
@@ -64,7 +67,7 @@ struct DropArgs {
     int32_t Hq, M, N, groups, causal, out_dt;
     int32_t BH, nmb;   // batch * heads, 128-query blocks
     int32_t snake;     // blocks of one round over the CUs, 0: plain order
-    int32_t keep_from; // smallest folded output word that is kept
+    uint32_t minus_keep_from; // minus the smallest folded output word that is kept
     float qk_scale;    // sm_scale * log2(e)
     float dropout_p, keep_scale;  // keep_scale = 1 / (1 - dropout_p)
     uint32_t seed_lo, seed_hi;
@@ -94,24 +97,29 @@ __device__ __forceinline__ PhiloxRow philox_row(uint32_t hi_word, uint32_t k0, u
     return {hi_word, (uint32_t)(u >> 32) ^ (k1 + kPhiloxKeyB), (uint32_t)u ^ (k1 + 2 * kPhiloxKeyB)};
 }
 
+// Three operands in one instruction.  As two XORs (what the compiler makes of a ^ b ^ c) the six rounds and the decision took
+// 110 instead of 89 cycles per score and SIMD at four waves, 113 instead of 93 at two.
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96); }
+
 // first: A * low word, all 64 bits
 __device__ __forceinline__ uint32_t philox6_from_product(uint64_t first, const PhiloxRow& r, uint32_t k0, uint32_t k1) {
     auto hi = [](uint64_t x) { return (uint32_t)(x >> 32); };
     const uint64_t b1 = (uint64_t)kPhiloxB * (hi(first) ^ k1);
     const uint64_t a2 = (uint64_t)kPhiloxA * (hi(b1) ^ (k0 + kPhiloxKeyA));
     const uint64_t b2 = (uint64_t)kPhiloxB * ((uint32_t)first ^ r.x2);
-    const uint64_t a3 = (uint64_t)kPhiloxA * (hi(b2) ^ (uint32_t)b1 ^ (k0 + 2 * kPhiloxKeyA));
+    const uint64_t a3 = (uint64_t)kPhiloxA * xor3(hi(b2), (uint32_t)b1, k0 + 2 * kPhiloxKeyA);
     const uint32_t c2 = hi(a2) ^ r.x3;
-    const uint32_t c0 = __umulhi(kPhiloxB, c2) ^ (uint32_t)b2 ^ (k0 + 3 * kPhiloxKeyA);
-    const uint32_t d2 = hi(a3) ^ (uint32_t)a2 ^ (k1 + 3 * kPhiloxKeyB);
-    const uint32_t e2 = __umulhi(kPhiloxA, c0) ^ (uint32_t)a3 ^ (k1 + 4 * kPhiloxKeyB);
-    return __umulhi(kPhiloxB, e2) ^ (kPhiloxB * d2) ^ (k0 + 5 * kPhiloxKeyA);
+    const uint32_t c0 = xor3(__umulhi(kPhiloxB, c2), (uint32_t)b2, k0 + 3 * kPhiloxKeyA);
+    const uint32_t d2 = xor3(hi(a3), (uint32_t)a2, k1 + 3 * kPhiloxKeyB);
+    const uint32_t e2 = xor3(__umulhi(kPhiloxA, c0), (uint32_t)a3, k1 + 4 * kPhiloxKeyB);
+    return xor3(__umulhi(kPhiloxB, e2), kPhiloxB * d2, k0 + 5 * kPhiloxKeyA);
 }
 
 // negative iff the element with this output word is dropped: the word folds to [0, 2^31) and is kept from keep_from on
-__device__ __forceinline__ int32_t drop_sign(uint32_t word, int32_t keep_from) {
+// (exclusive or and addition are one instruction)
+__device__ __forceinline__ int32_t drop_sign(uint32_t word, uint32_t minus_keep_from) {
     const int32_t x = (int32_t)word;
-    return (int32_t)((uint32_t)(x ^ (x >> 31)) - (uint32_t)keep_from);
+    return (int32_t)((uint32_t)(x ^ (x >> 31)) + minus_keep_from);
 }
 
 template <int D> __device__ __forceinline__ int drop_v_swizzle(int row) { return D == 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1); }
@@ -313,7 +321,7 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
 #pragma unroll
                 for (int e = 0; e < 2; e++) {
                     const int k = 8 * ((i + e) >> 2) + ((i + e) & 3);
-                    sign[e] = drop_sign(philox6_from_product(product + (uint64_t)kPhiloxA * k, prow, a.seed_lo, a.seed_hi), a.keep_from);
+                    sign[e] = drop_sign(philox6_from_product(product + (uint64_t)kPhiloxA * k, prow, a.seed_lo, a.seed_hi), a.minus_keep_from);
                 }
                 put(i, sign[0], sign[1]);
                 __builtin_amdgcn_sched_barrier(0);  // (two scores at a time: all sixteen side by side would not fit the registers)
@@ -470,7 +478,7 @@ int launch_flash_dropout(const sage_flash_params& p, float dropout_p, uint64_t s
             if ((float)(int32_t)mid * 4.6566127342e-10f > dropout_p) hi = mid;
             else lo = mid + 1;
         }
-        a.keep_from = (int32_t)(uint32_t)lo;
+        a.minus_keep_from = 0u - (uint32_t)lo;
     }
     a.BH = (int)(p.batch * p.heads_q);
     a.nmb = (a.M + 32 * kDropWaves - 1) / (32 * kDropWaves);
