@@ -22,7 +22,8 @@
 // * workgroups are handed out longest first over all heads.
 // B4 H16 M2048 N2048 D64 fp16 causal 397 -> 143 us, without the causal flag 404 -> 272 us; B2 H32 M4096 N4096 D128 3475 -> 1207
 // us, causal 3445 -> 619 us (before: the generator rolled out by the compiler, V^T gathered from LDS entry by entry,
-// short rows first).  With xor3 120, 226, 1114 and 573 us.  At head_dim 128 three waves per SIMD need 18 spilled registers and
+// short rows first).  With xor3 120, 226, 1114 and 573 us, with reference points that move only when they have to 114, 214, 1058 and
+// 547 us.  At head_dim 128 three waves per SIMD need 18 spilled registers and
 // run 6 % slower than two.
 #include "attn_common.h"
 
@@ -77,6 +78,7 @@ struct DropArgs {
 constexpr int kDropWaves = 4;  // 128 queries per workgroup
 constexpr int kDropThreads = 64 * kDropWaves;
 constexpr int kDropKeys = 32;  // keys per tile
+constexpr float kNoScore = -3.0e38f;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -248,7 +250,9 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[dt][i] = 0.0f;
-    float m_i = -INFINITY, l_i = 0.0f;  // running maximum (unscaled scores) and this half's part of the row sum
+    // the row's reference point (in units of the exponent; below every score until the row has seen a key) and this half's part of
+    // the row sum
+    float m_i = kNoScore, l_i = 0.0f;
 
     if (group < ntiles) fetch(group, 0);
     const int rounds = (ntiles + KG - 1) / KG;
@@ -280,12 +284,11 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
         float tile_max = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 16; i++) tile_max = fmaxf(tile_max, s[i]);
-        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
-        const float m_new = fmaxf(m_i, tile_max);
-        // (a query that has seen no key yet keeps m = -inf: every p below is then 0)
-        const float m_use = m_new == -INFINITY ? 0.0f : m_new * a.qk_scale;
-        if (__builtin_amdgcn_ballot_w64(m_new > m_i) != 0) {
-            const float alpha = m_i == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m_i, a.qk_scale, -m_use));
+        // The reference point of a row moves only when the larger half of a P would pass 2^kTau: most tiles end the matter here, without
+        // the exchange between the two lanes of a row.
+        if (__builtin_amdgcn_ballot_w64(__builtin_fmaf(tile_max, a.qk_scale, -m_i) > kTau) != 0) {
+            const float m_new = fmaxf(m_i, fmaxf(tile_max, __shfl_xor(tile_max, 32)) * a.qk_scale);
+            const float alpha = __builtin_amdgcn_exp2f(m_i - m_new);
             l_i *= alpha;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
@@ -304,8 +307,8 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
         uint32_t pbits[8];
         // two scores and the signs of their words (bit 31 set: dropped) -> two 16-bit P
         auto put = [&](int i, int32_t sign0, int32_t sign1) {
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.qk_scale, -m_use));  // hidden keys: exp2(-inf) = 0
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], a.qk_scale, -m_use));
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.qk_scale, -m_i));  // hidden keys: exp2(-inf) = 0
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], a.qk_scale, -m_i));
             psum += p0;
             psum += p1;
             typedef VT vt2 __attribute__((ext_vector_type(2)));
@@ -358,14 +361,13 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
             row_l[group * 32 * kDropWaves + slot] = l_tot;
         }
         __syncthreads();
-        float m = -INFINITY, l = 0.0f;
+        float m = kNoScore, l = 0.0f;
 #pragma unroll
         for (int g = 0; g < KG; g++) m = fmaxf(m, row_m[g * 32 * kDropWaves + slot]);
-        const float base = m == -INFINITY ? 0.0f : m * a.qk_scale;
 #pragma unroll
         for (int g = 0; g < KG; g++)
-            l += row_l[g * 32 * kDropWaves + slot] * __builtin_amdgcn_exp2f(__builtin_fmaf(row_m[g * 32 * kDropWaves + slot], a.qk_scale, -base));
-        const float mine = __builtin_amdgcn_exp2f(__builtin_fmaf(m_i, a.qk_scale, -base));
+            l += row_l[g * 32 * kDropWaves + slot] * __builtin_amdgcn_exp2f(row_m[g * 32 * kDropWaves + slot] - m);
+        const float mine = __builtin_amdgcn_exp2f(m_i - m);
         float* park = reinterpret_cast<float*>(&smem[0][0][0][0]) + wave * 32 * D + lane;  // entry e of a lane: 64 e further on
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
@@ -416,7 +418,7 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
         }
     if (a.log_normalizer && half == 0)
         a.log_normalizer[((int64_t)b * a.Hq + h) * a.M + my_m] =
-            l_tot != 0.0f ? (__builtin_log2f(l_tot) + m_i * a.qk_scale) * 0.693147180559945309f : -INFINITY;
+            l_tot != 0.0f ? (__builtin_log2f(l_tot) + m_i) * 0.693147180559945309f : -INFINITY;
 }
 
 __global__ void dropout_mask_kernel(uint8_t* mask, int64_t count, uint64_t offset, uint32_t seed_lo, uint32_t seed_hi,
