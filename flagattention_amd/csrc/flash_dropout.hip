@@ -18,13 +18,13 @@
 // * the keep decision is an integer threshold and a sign, applied to two 16-bit P at a time (no compare, no select);
 // * the rest is kept small: K and V tiles of 32 keys go straight into LDS for the four waves of a workgroup (32 queries
 //   each, S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16, V^T by ds_read_b64_tr_b16), one barrier per tile, loads
-//   one tile ahead (a tile takes microseconds), registers for four (head_dim 128: two) waves per SIMD;
+//   one tile ahead (a tile takes microseconds), registers for four (head_dim 128: three) waves per SIMD;
 // * workgroups are handed out longest first over all heads.
 // B4 H16 M2048 N2048 D64 fp16 causal 397 -> 143 us, without the causal flag 404 -> 272 us; B2 H32 M4096 N4096 D128 3475 -> 1207
 // us, causal 3445 -> 619 us (before: the generator rolled out by the compiler, V^T gathered from LDS entry by entry,
 // short rows first).  With xor3 120, 226, 1114 and 573 us, with reference points that move only when they have to 114, 214, 1058 and
-// 547 us.  At head_dim 128 three waves per SIMD need 18 spilled registers and
-// run 6 % slower than two.
+// 547 us, with three waves per SIMD at head_dim 128 (two before: the addends of the counters' products took 30 vector registers)
+// 111, 214, 994 and 519 us.
 #include "attn_common.h"
 
 namespace sage {
@@ -103,6 +103,14 @@ __device__ __forceinline__ PhiloxRow philox_row(uint32_t hi_word, uint32_t k0, u
 // 110 instead of 89 cycles per score and SIMD at four waves, 113 instead of 93 at two.
 __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) { return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96); }
 
+// a + b, b the same for all lanes: one instruction, b in scalar registers (as the addend of a product, where the compiler puts it, every
+// b of the tile would keep two vector registers)
+__device__ __forceinline__ uint64_t add_u64(uint64_t a, uint64_t b) {
+    uint64_t r;
+    asm("v_lshl_add_u64 %0, %1, 0, %2" : "=v"(r) : "v"(a), "s"(b));
+    return r;
+}
+
 // first: A * low word, all 64 bits
 __device__ __forceinline__ uint32_t philox6_from_product(uint64_t first, const PhiloxRow& r, uint32_t k0, uint32_t k1) {
     auto hi = [](uint64_t x) { return (uint32_t)(x >> 32); };
@@ -129,8 +137,8 @@ template <int D> __device__ __forceinline__ int drop_v_swizzle(int row) { return
 // KG: groups of four waves that share the queries of a workgroup and take its key tiles in turn (drop_groups).  The second
 // launch bound is waves per SIMD, whatever KG is: with fewer asked for, two groups at head_dim 64 took 132 registers and one
 // workgroup filled a CU (B1 H32 M2048 N2048 D64 153 -> 140 us, causal 107 -> 80 us, B4 H16 M1024 N1024 83 -> 77 and 58 -> 45
-// us; where a lone workgroup of the longest blocks decides, B2 H16 M1500 causal, two spilled registers cost 59 -> 60 us).
-constexpr int drop_waves_per_simd(int head_dim) { return head_dim == 128 ? 2 : 4; }
+// us; three at head_dim 128: B2 H32 M4096 N4096 1058 -> 994 us).
+constexpr int drop_waves_per_simd(int head_dim) { return head_dim == 128 ? 3 : 4; }
 
 // WIDE: the rows of a K or V tile lie further apart than 32-bit byte offsets reach, or in descending order (64-bit
 // addresses per lane; one group of waves only).
@@ -152,7 +160,7 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
     const int l32 = lane & 31, half = lane >> 5;
     // heads fastest (a head stays on one XCD); under the causal flag the last queries, which see the most keys, first
     // (snake: all workgroups are resident at once, so every second round of 256, one per CU, goes in the reverse order of
-    // blocks and a CU holds long and short ones: B4 H16 M2048 N2048 D64 causal 177 -> 166 us)
+    // blocks and a CU holds long and short ones: B4 H16 M2048 N2048 D64 causal 177 -> 166 us, B3 H16 M2048 N2048 D128 124 -> 112)
     const int bh = blockIdx.x % a.BH;
     int rank = blockIdx.x / a.BH;
     if (a.snake > 0 && a.snake < a.nmb && a.nmb < 2 * a.snake) {
@@ -324,7 +332,7 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
 #pragma unroll
                 for (int e = 0; e < 2; e++) {
                     const int k = 8 * ((i + e) >> 2) + ((i + e) & 3);
-                    sign[e] = drop_sign(philox6_from_product(product + (uint64_t)kPhiloxA * k, prow, a.seed_lo, a.seed_hi), a.minus_keep_from);
+                    sign[e] = drop_sign(philox6_from_product(add_u64(product, (uint64_t)kPhiloxA * k), prow, a.seed_lo, a.seed_hi), a.minus_keep_from);
                 }
                 put(i, sign[0], sign[1]);
                 __builtin_amdgcn_sched_barrier(0);  // (two scores at a time: all sixteen side by side would not fit the registers)
@@ -428,10 +436,11 @@ __global__ void dropout_mask_kernel(uint8_t* mask, int64_t count, uint64_t offse
 }
 
 // Groups of waves per workgroup: as many as the SIMDs hold waves for, where there are fewer workgroups than that takes (a
-// SIMD with one wave issues a vector instruction every 5.7 cycles, with four waves every 3).
+// SIMD with one wave issues a vector instruction every 5.7 cycles, with four waves every 3).  Two at most at head_dim 128, up to 256
+// workgroups (three groups: B1 H4 M4096 N4096 137 -> 128 us, but B1 H8 M512 N512 23.9 -> 24.8).
 int drop_groups(int64_t wgs, int head_dim) {
     int groups = 1;
-    while (groups < drop_waves_per_simd(head_dim) && wgs * groups * 2 <= 256 * drop_waves_per_simd(head_dim)) groups *= 2;
+    while (2 * groups <= drop_waves_per_simd(head_dim) && wgs * 2 * groups <= 256 * (drop_waves_per_simd(head_dim) & ~1)) groups *= 2;
     return groups;
 }
 

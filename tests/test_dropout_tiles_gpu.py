@@ -59,3 +59,31 @@ def test_dropout_forward_keeps_nan(B, H, M, N, D, causal, p, gpu_device):
     sees = torch.arange(M, device=gpu_device) + (N - M) >= 0 if causal else torch.ones(M, dtype=torch.bool, device=gpu_device)
     assert torch.equal(torch.isnan(L), want) and torch.equal(torch.isneginf(L), ~sees.expand(B, H, M))
     assert torch.equal(torch.isnan(o).all(-1), want) and bool(torch.isfinite(o[~want]).all())
+
+
+@pytest.mark.parametrize("B,H,M,N,D,causal", [(1, 2, 70, 200, 64, False), (2, 3, 129, 300, 128, True), (6, 16, 1000, 70, 128, True)])
+@pytest.mark.parametrize("rise", [0.0, 1.0, -1.0])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_dropout_forward_reference_point(B, H, M, N, D, causal, rise, dtype, gpu_device):
+    """Scores whose level rises (falls) by 12 log2 units from one 32-key tile to the next, so that the reference point of a row has to
+    move with every tile (stays at the first one); the last shape fills three rounds of 128-query blocks at head_dim 128."""
+    import math
+
+    import flag_attn
+
+    g = torch.Generator().manual_seed(43)
+    q, k, v = (torch.randn(B, H, n, D, generator=g) for n in (M, N, N))
+    q[..., 0] = 4.0
+    level = torch.arange(N).div(32, rounding_mode="floor").float() * 12.0 * math.log(2.0) * math.sqrt(D) / 4.0
+    k[..., 0] = rise * level
+    q, k, v = (t.to(dtype) for t in (q, k, v))
+    dq, dk, dv = (t.to(gpu_device) for t in (q, k, v))
+    o, L, _, seed, off = flag_attn.flash_attention(dq, dk, dv, causal, dropout_p=0.25, return_log_normalizer=True, return_seed_offset=True)
+    mask = flag_attn.testing.recompute_mask(B, H, M, N, 0.25, seed, off, gpu_device).cpu()
+    o_ref, L_ref = FO.attention(q, k, v, causal, dropout_p=0.25, dropout_mask=mask, return_log_normalizer=True, upcast=True)
+    yard = FO.max_diff(FO.attention(q, k, v, causal, dropout_p=0.25, dropout_mask=mask, upcast=False), o_ref)
+    got = FO.max_diff(o.cpu(), o_ref)
+    assert got <= 2 * yard + 1e-5, (got, yard)
+    inf = torch.isinf(L_ref)
+    assert torch.equal(torch.isinf(L.cpu()), inf)
+    torch.testing.assert_close(L.cpu()[~inf], L_ref[~inf], atol=2e-3, rtol=2e-4)
