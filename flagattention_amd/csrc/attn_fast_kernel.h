@@ -543,12 +543,12 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
 
     // The int32 accumulators start from the bit pattern of the float 1.5 * 2^23: since |dot| < 2^22,
     // accumulator bits reinterpreted as fp32 ARE kBias + dot, so no int -> float conversion is needed.
-    // (16-bit Q and K: fp32 accumulators that start from zero, kept in the same registers as bits.)
+    // (16-bit Q and K: fp32 accumulators that start from zero, a constant operand of the instruction, kept as bits as well.)
     v16i bias16;
 #pragma unroll
     for (int i = 0; i < 16; i++) {
-        int b;  // materialised once through an opaque move, so the block stays in VGPRs for the whole kernel
-        asm volatile("v_mov_b32 %0, %1" : "=v"(b) : "s"(INT8 ? kBiasBits : 0));
+        int b = 0;  // int8: materialised once through an opaque move, so the block stays in VGPRs for the whole kernel
+        if constexpr (INT8) asm volatile("v_mov_b32 %0, %1" : "=v"(b) : "s"(kBiasBits));
         bias16[i] = b;
     }
     // Row sums of P by the matrix core: one 16x16x32 instruction per 16-key slice multiplies a 0/1 pattern
@@ -599,7 +599,15 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     constexpr int NSLOTS = QK_SLOTS + PV_SLOTS;
     constexpr int DEFER = (D == 64 && INT8 && !MF32) ? 4 : 0;  // exponential units moved into the MFMA phase (measured per instance;
                                                                // fp32 mask entries: every unit reads them before the slot is refilled)
-    constexpr bool kWholeRowSums = QB == 2 && !CAUSAL;      // row sums by the matrix core: every lane holds its whole row's sum
+    // Row sums by the matrix core (sum_pattern), every lane then holding its whole row's sum: the 16-bit instances, whose port the 32
+    // matrix instructions of a step already load.  v_dot2 also waits for the matrix instructions of the SIMD's other wave: 16 of them
+    // in the vector phase of the key-hiding instance cost 7 % (B2 H32 N8192 D128 bf16 causal 1006 -> 939 us, B1 H32/8 N3001 164
+    // -> 149 us, D64 292 -> 283 us), without hidden keys 5 %; the int8 instances gain and lose up to 1.5 % by it and keep v_dot2.
+    constexpr bool kWholeRowSums = QB == 2;
+    // The LDS offsets of the fragments of a step from one base each, whose bits the swizzle only flips, instead of a register for each:
+    // where registers are short (1 %; elsewhere the exclusive or costs more than the addition, up to 1 %).
+    constexpr bool kOneBase = QB == 2 && D == 128 && CAUSAL;
+    static_assert((F::KSTEPS & (F::KSTEPS - 1)) == 0, "half and step are separate bits of the chunk index");
     constexpr int KDIST = 4 < QK_SLOTS ? 4 : QK_SLOTS;      // K fragments in flight
     constexpr int VDIST = 3 < QK_SLOTS ? 3 : QK_SLOTS - 1;  // V fragments in flight
     static_assert(KDIST <= QK_SLOTS && VDIST < QK_SLOTS && 16 % QK_SLOTS == 0, "slot plan");
@@ -723,12 +731,12 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         int kaddr[F::KSTEPS], vaddr[F::DTILES];
 #pragma unroll
         for (int t = 0; t < F::KSTEPS; t++) {
-            kaddr[t] = kf_off[t] + ((step + 1) & 3) * F::K_BYTES;
+            kaddr[t] = kOneBase ? (kf_off[0] + ((step + 1) & 3) * F::K_BYTES) ^ (16 * t) : kf_off[t] + ((step + 1) & 3) * F::K_BYTES;
             asm volatile("" : "+v"(kaddr[t]));  // computed once per step, here in the VALU phase
         }
 #pragma unroll
         for (int dt = 0; dt < F::DTILES; dt++) {
-            vaddr[dt] = vtr_off[dt] + F::V_BASE + (step & 3) * F::V_BYTES;
+            vaddr[dt] = kOneBase ? (vtr_off[0] + F::V_BASE + (step & 3) * F::V_BYTES) ^ (64 * dt) : vtr_off[dt] + F::V_BASE + (step & 3) * F::V_BYTES;
             asm volatile("" : "+v"(vaddr[dt]));
         }
         v4i kfr[QK_SLOTS];
@@ -815,20 +823,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         };
         // The last DEFER of the 16 units wait for the MFMA phase (head_dim 64: that phase has half the
         // matrix instructions, so it takes a share of the exponentials to keep the two phases even).
-        // Where the row sums are taken is a measured choice per instance: in the shadow of the Q.K^T
-        // instructions everywhere (head_dim 128, int8: 10 % faster than here; 16-bit without hidden keys:
-        // 4 %), except in the 16-bit instance that hides keys, whose MFMA phase is the longer one (32 matrix
-        // instructions and the masking of the diagonal tiles): there they follow their exponentials (-4.5 %).
-        constexpr bool kSumsEarly = QB == 2 && CAUSAL && DEFER == 0;
-        sfor<16 - DEFER>([&](auto uc) {
-            constexpr int u = decltype(uc)::value;
-            exp_unit(uc);
-            if constexpr (kSumsEarly && u >= 2) lsum = PVT::dot2_ones(pf[(u - 2) >> 2], (u - 2) & 3, lsum);
-        });
-        if constexpr (kSumsEarly) {
-            lsum = PVT::dot2_ones(pf[3], 2, lsum);
-            lsum = PVT::dot2_ones(pf[3], 3, lsum);
-        }
+        sfor<16 - DEFER>(exp_unit);
         // (fp32 mask entries: the last one of this step has been read; the one slot takes those of the next step)
         if constexpr (MF32) dma_mask(vt1, 0);
         // A lane's 32 P of a step sum to less than kSumLimit, or the step is redone: so no P overflows the
@@ -838,11 +833,9 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         // The sums are complete SUM_SLOTS matrix instructions into the phase; the wave vote on them is taken
         // there and only tested before the first P.V instruction, four matrix instructions later, so that
         // neither the last sum nor the compare is waited for (2-3 % on the causal and the 16-bit instances).
-        // ... and in the 16-bit instance without hidden keys the matrix core takes them (sum_pattern above): four
-        // cheap matrix instructions instead of 16 v_dot2 on an issue port that the 32 matrix instructions of
-        // its step already load (-5 %; neutral for the int8 instances, which keep v_dot2 and half-row sums).
-        constexpr bool kMfmaSums = kWholeRowSums;
-        constexpr int SUM_SLOTS = kSumsEarly ? -1 : (DEFER == 0 && QK_SLOTS >= 8) ? QK_SLOTS - 4 : QK_SLOTS;
+        // (The 16-bit instances: kWholeRowSums.  v_dot2 rides in the shadow of the Q.K^T instructions, 10 % faster than behind the
+        // exponentials at head_dim 128.)
+        constexpr int SUM_SLOTS = (DEFER == 0 && QK_SLOTS >= 8) ? QK_SLOTS - 4 : QK_SLOTS;
         v4f sum4 = {0.0f, 0.0f, 0.0f, 0.0f};
         unsigned long long large = 0;
         auto redo_if_large = [&]() {
@@ -998,10 +991,9 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                     exp_unit(uc);
                     lsum = PVT::dot2_ones(pf[u >> 2], u & 3, lsum);
                 });
-                if constexpr (kMfmaSums) lsum += __shfl_xor(lsum, 32);  // this instance keeps whole-row sums in every lane
+                if constexpr (kWholeRowSums) lsum += __shfl_xor(lsum, 32);  // these instances keep whole-row sums in every lane
             }
         };
-        if constexpr (kSumsEarly) large = __builtin_amdgcn_ballot_w64(!(lsum < kSumLimit));
         sc = step_scale(MASK ? vt1 : min(step + 1, nsteps - 1), HIDES);
         __builtin_amdgcn_sched_barrier(0);
         // The first K fragments of the coming MFMA phase are requested before the barrier (their tile
@@ -1029,7 +1021,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                 if constexpr (i + KDIST < QK_SLOTS) read_k(IC<i + KDIST>{});
                 if constexpr (i >= QK_SLOTS - VDIST) read_v(IC<i - (QK_SLOTS - VDIST)>{});
                 // row sums of P ride in the shadow of the Q.K^T instructions
-                if constexpr (kMfmaSums) {
+                if constexpr (kWholeRowSums) {
                     if constexpr (i < 4) {  // one per slot, behind the first four Q.K^T instructions
                         if constexpr (i == 0) sum4 = PVT::mfma16(sum_pattern, pf[0], v4f{0.0f, 0.0f, 0.0f, 0.0f});
                         else sum4 = PVT::mfma16(sum_pattern, pf[i], sum4);
@@ -1042,20 +1034,20 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                 } else {
                     sfor<16 - DEFER>([&](auto rc) {
                         constexpr int u = decltype(rc)::value;
-                        if constexpr (!kSumsEarly && u * SUM_SLOTS / (16 - DEFER) == i) {
+                        if constexpr (u * SUM_SLOTS / (16 - DEFER) == i) {
                             lsum = PVT::dot2_ones(pf[u >> 2], u & 3, lsum);
                             asm volatile("" ::"v"(lsum));
                         }
                     });
                 }
-                if constexpr (!kMfmaSums && i == SUM_SLOTS - 1 && SUM_SLOTS < QK_SLOTS) {
+                if constexpr (!kWholeRowSums && i == SUM_SLOTS - 1 && SUM_SLOTS < QK_SLOTS) {
                     large = __builtin_amdgcn_ballot_w64(!(lsum < kSumLimit));  // also set for inf and NaN
                     asm volatile("" ::"s"(large));
                 }
             } else {
                 constexpr int j = i - QK_SLOTS, tp = j / F::DTILES, dt = j % F::DTILES;
                 if constexpr (j == 0) {
-                    if constexpr (!kSumsEarly && SUM_SLOTS == QK_SLOTS) large = __builtin_amdgcn_ballot_w64(!(lsum < kSumLimit));
+                    if constexpr (!kWholeRowSums && SUM_SLOTS == QK_SLOTS) large = __builtin_amdgcn_ballot_w64(!(lsum < kSumLimit));
                     redo_if_large();
                     __builtin_amdgcn_sched_barrier(0);
                 }
