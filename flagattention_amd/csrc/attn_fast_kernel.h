@@ -713,6 +713,25 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             if (!MC) m_i = fmaxf(m_i, -1.0e30f);
         }
     }
+    // The bias taken from the scores of a step whose scale is too large for it to be folded into the exponent (kBiasFoldLimit).
+    // kEarlyBias: at the end of the matrix phase that made them.  The wave with the exponentials is the one the other waits for in
+    // the mask instances and at head_dim 64, so 32 vector instructions less there are time saved, B8 H16 N2048 D64 fp16 with outlier
+    // channels 172 -> 167 us, B1 H12 N4096 D64 81.2 -> 77.1, bool mask 97.7 -> 92.3 (the branch gone from that phase: N(0,1) data,
+    // B4 H16 N1536 D64 fp16 bias 93.7 -> 91.6, D128 fp32 bias 142.6 -> 137.4 us).  Not in the others: head_dim 128, whose phases are
+    // even, 441 -> 445 us (B2 H32 N4096), causal head_dim 64 121.4 -> 122.9 us.  Between the P.V instructions instead, in a second copy of
+    // them: 172 us and 79.8 of the first two.
+    auto take_bias = [&](auto pc) {
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int bits = sbuf[decltype(pc)::value][kt][i];
+                sbuf[decltype(pc)::value][kt][i] = __builtin_bit_cast(int, as_f(bits) - kBias);
+            }
+    };
+    constexpr bool kEarlyBias = INT8 && (MASK || (D == 64 && !CAUSAL));
+    bool bias_folded = !INT8 || kBias * sc < kBiasFoldLimit;  // (kEarlyBias) of the current step
+    if (kEarlyBias && !bias_folded) take_bias(IC<0>{});
     int mslot = 0;  // slot of the current step's mask bytes (step % 3)
 
     // ---- one step.  Each wave alternates a VALU phase (exponentials of its step) and an MFMA phase
@@ -760,16 +779,8 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         // Should it make a P too large, the row sums show it before the first P.V instruction, and the step
         // is redone against its true maximum: see redo_if_large below.
         float neg_m;
-        const bool folded = !INT8 || kBias * sc < kBiasFoldLimit;
-        if (!folded) {
-#pragma unroll
-            for (int kt = 0; kt < 2; kt++)
-#pragma unroll
-                for (int i = 0; i < 16; i++) {
-                    const int bits = sbuf[P][kt][i];
-                    sbuf[P][kt][i] = __builtin_bit_cast(int, as_f(bits) - kBias);
-                }
-        }
+        const bool folded = kEarlyBias ? bias_folded : !INT8 || kBias * sc < kBiasFoldLimit;
+        if (!kEarlyBias && !folded) take_bias(IC<P>{});
         neg_m = folded ? __builtin_fmaf(-BIAS, sc, -m_i) : -m_i;
         if (!live) neg_m = -INFINITY;  // padding step: every P is exp2(-inf) = 0
 
@@ -1074,6 +1085,11 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             }
             __builtin_amdgcn_sched_barrier(0);
         });
+        if constexpr (kEarlyBias) {  // (sc: already the next step's)
+            bias_folded = kBias * sc < kBiasFoldLimit;
+            if (!bias_folded) take_bias(IC<1 - P>{});
+            __builtin_amdgcn_sched_barrier(0);
+        }
         l_i += lsum;
         mslot = mslot_next;
         if constexpr (MASK) {

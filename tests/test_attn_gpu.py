@@ -233,6 +233,28 @@ def test_row_maximum_that_moves_between_tiles_other_paths(pattern, path, gpu_dev
     torch.testing.assert_close(lse.cpu()[rows], expected_lse[rows], atol=6e-3, rtol=1e-5)
 
 
+@pytest.mark.parametrize("factors", [(1.0, 20.0), (20.0, 1.0, 1.0), (20.0,)])
+@pytest.mark.parametrize("d,n,mask", [(64, 448, None), (64, 512, None), (64, 448, "bool"), (64, 448, "fp16"), (64, 448, "fp32"),
+                                      (128, 448, "bool"), (128, 512, "bf16"), (128, 448, "fp32")])
+def test_scales_on_both_sides_of_the_folded_bias(d, n, mask, factors, gpu_device):
+    """K scales of blocks in turn below and above the limit up to which the accumulators' bias is folded into the exponent: the
+    step before decides for the next one (odd and even step counts, each mask type; heads enough for the pipelined kernel)."""
+    h, m = (64, 512) if mask is None else (4, 700)
+    q8, qs, k8, ks, v = _quantized(43, 1, h, h // 2, m, n, d, torch.float16)
+    ks2 = ks.clone()
+    for j in range(ks2.shape[-1]):
+        ks2[..., j] *= factors[j % len(factors)]
+    kw, okw = {}, {}
+    if mask is not None:
+        t = torch.randn(1, h, m, n, generator=torch.Generator().manual_seed(8))
+        t = t > -1.0 if mask == "bool" else t.to({"fp16": torch.float16, "bf16": torch.bfloat16, "fp32": torch.float32}[mask])
+        kw, okw = {"attn_mask": t.to(gpu_device)}, {"attn_mask": t}
+    o, lse = _run(gpu_device, q8, qs, k8, ks2, v, return_lse=True, output_dtype=torch.float16, **kw)
+    expected, expected_lse = O.attention_dequant(q8, k8, v, qs, ks2, **okw)
+    _gate(o, expected, f"{mask} {factors}")
+    torch.testing.assert_close(lse.cpu(), expected_lse, atol=6e-3, rtol=1e-5)
+
+
 def _mask_case(kind, b, h, m, n, seed):
     g = torch.Generator().manual_seed(seed)
     if kind == "random":  # 70 % visible, per (batch, head)
