@@ -74,7 +74,7 @@ struct AttnArgs {
     // (mask tensors, pipelined kernel) what mask_scan_kernel found (null: every tile is visited): per strip of kScanRows mask
     // rows and 64-key tile the largest entry, per strip the smallest of its rows' largest entries, per 64-key tile of V
     // whether it holds an Inf or NaN.  scan_strips: strips of a mask batch.  visit_group: tiles per bit of the visit word.
-    const float* scan_top;  // [mask batches][scan_strips][nk]
+    const float* scan_top;  // [mask batches][scan_strips][nk]  (+0: every entry is 0, -0: the largest one is)
     const float* scan_low;  // [mask batches][scan_strips]
     const unsigned* scan_v; // [B][Hkv][nk]
     int32_t scan_strips, visit_group;

@@ -141,7 +141,7 @@ template <> __device__ __forceinline__ float mask_entry<_Float16>(unsigned word,
 // causal, where no item is cut: 214 us against 210 us for pairs); a piece costs about five steps, a partial result 2.5.
 // MC: an additive mask tensor with the causal flag, instances of their own (in the same ones B4 H8 M320 N320 D128 fp16 19.6 -> 21.0 us
 // without the flag).
-template <int D, typename VT, bool CAUSAL, int QB, typename MT = void, bool CUT = false, bool MC = false>
+template <int D, typename VT, bool CAUSAL, int QB, typename MT = void, bool CUT = false, bool MC = false, bool SCAN = false>
 __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast_kernel(AttnArgs args, int nq2) {
     const AttnArgs& a = args;
     using F = FT<D, QB>;
@@ -154,7 +154,9 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     constexpr int kMaskInstr = kMaskWaveBytes / 1024;            // loads per wave and step
     constexpr int kMaskBytes = kMaskSlots * kFastWaves * kMaskWaveBytes;
     static_assert(!MC || MADD, "the causal flag on top of an additive mask");
+    static_assert(!SCAN || (MASK && !MC), "the tiles of a mask tensor");
     static_assert(!MASK || (CAUSAL && INT8), "the mask instances build on the key-hiding int8 instance");
+    constexpr bool WALK_BITS = SCAN || (MC && D == 128);
     constexpr float BIAS = INT8 ? kBias : 0.0f;  // what the bits of a fresh score accumulator read as a float
     using PVT = PV<VT>;
     using vec16 = typename PVT::vec;
@@ -176,7 +178,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     // The keys of one (batch, head, q-block) may be split over `nsplit` workgroups (under a mask tensor the tiles it leaves to
     // visit: see `visits`).  A workgroup then sees the problem that starts at its first key: kv_len, the number of tiles and the causal
     // limits below all count from there, and its steps end where the next workgroup's begin.
-    const int nsplit = MC || CUT ? 1 : a.nsplit;
+    const int nsplit = MC || CUT || (MASK && !SCAN) ? 1 : a.nsplit;
     const int split = wg % nsplit;
     const int item0 = wg / nsplit;
     // heads that alternate within a q-block: measured to pay only under a mask with the causal mask folded in
@@ -437,12 +439,23 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     //      an additive entry so far below the largest one of every row that its P is exactly 0 whatever the scores
     //      (|q.k| <= 128 sum |q|, and the scales bound them), a bool tile without a visible key (the reference skips it), and no
     //      Inf or NaN in V (0 times those is NaN).  Comparisons with a NaN scale or entry are false: such a tile is visited.
-    unsigned long long visits = ~0ull;
+    //      SCAN: instances of their own for scanned masks; the others walk over every tile without any of this (B4 H16 N1536 D64
+    //      bool 88.5 -> 86.8 us, D64 fp16 bias 91.4 -> 88.8, D128 bf16 bias 116.5 -> 114.9).  WALK_BITS: in the causal instances at
+    //      head_dim 128 the words of bits cost nothing and dropping them three more spilled registers (85.1 -> 85.4 us).
+    //      Bit t of `plain` (visit_group = 1): tile t leaves the scores of this wave's rows as they are (scan: +0).  The steps the
+    //      walk begins with, as long as that holds (masks that hide keys past a limit: most of them), neither read nor stage entries,
+    //      half of the bytes a step brings into LDS, and have no mask arithmetic, a third of the vector phase: B4 H16 N1536 causal and
+    //      padded, whole step, D128 bf16 89.7 -> 87.9 us, D64 fp32 75.7 -> 71.5; B1 H32/8 N4096 D128 fp16 167 -> 152, bool 155 -> 147;
+    //      B4 H16 N2048 bf16 padding 155 -> 146.  (Chosen per step the two bodies cost 76 to 169 spilled registers, as a branch
+    //      around the exponentials alone 3 % wherever entries are needed.)
+    unsigned long long visits = ~0ull, plain = 0;
+    int plain_steps = 0;
     int visit_group = 1, visit_g = 0, visit_rest = 0;  // tiles per bit; the bit of the youngest tile below, the tile within it
     // (k_at / v_at below hide the tiles' addresses from the compiler: known as base + tile * bytes they end in vector registers,
     // 180 of which the instances at head_dim 128 then spill)
     int vt0 = 0, vt1 = 0, vt2 = 0, vt3 = 0;  // tiles of this step and the next three (the last one again past the end)
     auto next_tile = [&](int t, bool more) {  // the tile visited after t, t itself if there are no more (no branch: this runs in the step loop)
+        if constexpr (!WALK_BITS) return more ? t + 1 : t;
         const bool same = visit_rest + 1 < visit_group;
         const int g = visit_g + 1 + __builtin_ctzll((visits >> visit_g) >> 1 | 1ull << 63);
         const int next = same ? t + 1 : g * visit_group;
@@ -450,11 +463,15 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         visit_g = more && !same ? g : visit_g;
         return more ? next : t;
     };
-    if constexpr (MASK) {
+    if constexpr (MASK && !WALK_BITS) {
+        vt1 = next_tile(vt0, nsteps > 1);
+        vt2 = next_tile(vt1, nsteps > 2);
+        vt3 = next_tile(vt2, nsteps > 3);
+    } else if constexpr (MASK) {
         visit_group = a.visit_group;
         const int groups = (nsteps + visit_group - 1) / visit_group;
         bool hidden_row = false;
-        if (!MC && a.scan_top) {  // (masks under the causal flag are not scanned)
+        if constexpr (SCAN) {
             const int mb = a.ms_b ? b : 0;
             const int s0 = a.ms_m ? (kFastRows / kScanRows) * iq : 0, s1 = min(s0 + kFastRows / kScanRows, a.scan_strips);
             const float* tops = a.scan_top + (int64_t)mb * a.scan_strips * a.nk;
@@ -465,6 +482,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             if (!MADD) low = 0.0f;  // (a bool tile goes by whether it holds a visible key)
             const int64_t kv_row = ((int64_t)b * a.Hkv + hk) * a.nk;
             float top = -INFINITY, ks_max = 0.0f;
+            unsigned own = 0;  // of the wave's own strips, bit by bit
             bool odd = false;
             for (int r = 0; r < visit_group; r++) {
                 const int t = min(lane * visit_group + r, a.nk - 1);
@@ -475,8 +493,12 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
 #pragma unroll
                 for (int x = 0; x < kFastRows / kScanRows; x++) e[x] = tops[(int64_t)min(s0 + x, s1 - 1) * a.nk + t];
 #pragma unroll
-                for (int x = 0; x < kFastRows / kScanRows; x++) top = fmaxf(top, e[x]);
+                for (int x = 0; x < kFastRows / kScanRows; x++) {
+                    top = fmaxf(top, e[x]);
+                    own |= x / (32 / kScanRows) == wave_u ? __builtin_bit_cast(unsigned, e[x]) : 0u;
+                }
             }
+            if (visit_group == 1) plain = __builtin_amdgcn_ballot_w64(own == 0);
 #pragma unroll
             for (int x = 1; x < 64; x <<= 1) ks_max = fmaxf(ks_max, __shfl_xor(ks_max, x));
             float bound = 0.0f;  // largest difference of two scores of a row
@@ -518,6 +540,9 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             const bool last_group = (visits >> (groups - 1)) & 1;
             nsteps = __builtin_popcountll(visits) * visit_group - (last_group ? groups * visit_group - nsteps : 0);
         }
+        const unsigned long long entries = visits & ~plain;
+        plain_steps = __builtin_popcountll(visits & ((entries & -entries) - 1)) & ~1;  // before the first tile that is not plain
+        asm volatile("" : "+s"(plain_steps));
         if (nsteps > 0) {
             visit_g = __builtin_ctzll(visits);
             vt0 = visit_g * visit_group;
@@ -742,8 +767,11 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     // HIDES = false is the body for steps that hide no key of this step or the next and fetch no ragged tile:
     // the code of the instance that cannot hide keys at all.  Both bodies pass the same two barriers, so the
     // waves of a workgroup may be in different ones.
-    auto body = [&](auto pc, auto hc, int step) {
+    // plain_c: the mask leaves the scores of this wave in this step as they are.  An additive one's entries are then staged
+    // for the last of these steps' successor only; the waits allow for the K/V loads alone, whatever else was requested.
+    auto body = [&](auto pc, auto hc, auto plain_c, int step) {
         constexpr int P = decltype(pc)::value;  // == step & 1
+        constexpr bool ENTRIES = MASK && !decltype(plain_c)::value;
         constexpr bool HIDES = CAUSAL && decltype(hc)::value;
         // tile t of K (of V) lives in LDS buffer t % 4: this step reads K of step+1 and V of step, and
         // fetches K of step+3 and V of step+2 into the buffers that K of step-1 and V of step-2 left
@@ -789,7 +817,10 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         const int mslot_next = mslot == kMaskSlots - 1 ? 0 : mslot + 1;
         // (additive: the entries of step + 1, into the slot that step - 1 left; ahead of the K/V loads, because they
         // are the ones waited for first: at the end of the coming matrix phase)
-        if constexpr (MADD && !MF32) dma_mask(vt1, mslot_next);
+        const bool stage_next = ENTRIES || !MADD || (P == 1 && step + 1 >= plain_steps);  // the next step needs its entries
+        if constexpr (MADD && !MF32) {
+            if (stage_next) dma_mask(vt1, mslot_next);
+        }
         sfor<NDMA_KV>([&](auto ec) { dma_unit(ec, IC<HIDES>{}, (step + 3) & 3, k_fetch, k_tile, (step + 2) & 3, v_fetch, v_tile); });
         if constexpr (MASK && !MADD) dma_mask(vt2, mslot_next == kMaskSlots - 1 ? 0 : mslot_next + 1);  // the mask bytes of step + 2
         vec16 pf[4];
@@ -798,20 +829,20 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         unsigned mw[2][2] = {{0, 0}, {0, 0}};  // (bool mask) the lane's mask bytes of the 16-key slice in work and of the next one
         unsigned me[2][4] = {};                // (additive 16-bit mask) the lane's entries of the slice in work and of the next one
         v4f mf[2] = {};                        // (additive fp32 mask) the lane's entries of the half-slice in work and of the next one
-        if constexpr (MASK && !MADD) mask_words(mslot, 0, mw[0][0], mw[0][1]);
-        if constexpr (MADD && !MF32) mask_entries(mslot, 0, me[0]);
-        if constexpr (MF32) mask_half(0, mf[0]);
+        if constexpr (ENTRIES && !MADD) mask_words(mslot, 0, mw[0][0], mw[0][1]);
+        if constexpr (ENTRIES && MADD && !MF32) mask_entries(mslot, 0, me[0]);
+        if constexpr (ENTRIES && MF32) mask_half(0, mf[0]);
         auto exp_unit = [&](auto uc) {  // two scores -> two 16-bit P values
             constexpr int u = decltype(uc)::value;
             constexpr int tp = u >> 2, w = u & 3, kt = tp >> 1, i0 = 8 * (tp & 1) + 2 * w;
             const int b0 = sbuf[P][kt][i0], b1 = sbuf[P][kt][i0 + 1];
             float t0 = neg_m, t1 = neg_m;
-            if constexpr (MF32) {  // the mask entry joins the exponent: score * scale + entry - m
+            if constexpr (ENTRIES && MF32) {  // the mask entry joins the exponent: score * scale + entry - m
                 constexpr int hs = 2 * tp + (w >> 1);
                 if constexpr ((w & 1) == 0 && hs < 7) mask_half(hs + 1, mf[(hs + 1) & 1]);
                 t0 += mf[hs & 1][2 * (w & 1)];
                 t1 += mf[hs & 1][2 * (w & 1) + 1];
-            } else if constexpr (MADD) {
+            } else if constexpr (ENTRIES && MADD) {
                 if constexpr (w == 0 && tp < 3) mask_entries(mslot, tp + 1, me[(tp + 1) & 1]);
                 const unsigned word = me[tp & 1][w];
                 t0 += mask_entry<MT>(word, 0);
@@ -819,7 +850,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             }
             float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(as_f(b0), sc_e, t0));
             float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(as_f(b1), sc_e, t1));
-            if constexpr (MASK && !MADD) {
+            if constexpr (ENTRIES && !MADD) {
                 // P of a hidden key is 0.  An overflowed P times 0 is NaN: the row sum then
                 // sends the step into the path that redoes it.
                 if constexpr (w == 0 && tp < 3) mask_words(mslot, tp + 1, mw[(tp + 1) & 1][0], mw[(tp + 1) & 1][1]);
@@ -836,7 +867,9 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         // matrix instructions, so it takes a share of the exponentials to keep the two phases even).
         sfor<16 - DEFER>(exp_unit);
         // (fp32 mask entries: the last one of this step has been read; the one slot takes those of the next step)
-        if constexpr (MF32) dma_mask(vt1, 0);
+        if constexpr (MF32) {
+            if (stage_next) dma_mask(vt1, 0);
+        }
         // A lane's 32 P of a step sum to less than kSumLimit, or the step is redone: so no P overflows the
         // 16-bit type (nor does a sum or a product with V come near the fp32 range), and a row whose scores
         // rise keeps its reference point within log2(kSumLimit) of its maximum.  Wave-wide decision; rare
@@ -863,8 +896,9 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                     float past_end = 0.0f;  // number of the lane's keys of this step that lie past kv_len
                     sfor<4>([&](auto tc) {
                         constexpr int tp = decltype(tc)::value, kt = tp >> 1;
-                        float e8[8];
-                        if constexpr (MF32) {
+                        float e8[8] = {};
+                        if constexpr (!ENTRIES) {
+                        } else if constexpr (MF32) {
                             v4f lo, hi;
                             mask_half_global(n0, 2 * tp, lo);
                             mask_half_global(n0, 2 * tp + 1, hi);
@@ -1013,7 +1047,7 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         __builtin_amdgcn_sched_barrier(0);
         // The loads issued in the previous VALU phase have landed (all but the NDMA just issued): the
         // tiles they belong to are first read two barriers from here.
-        __builtin_amdgcn_s_waitcnt(0x0F70 | NDMA);
+        __builtin_amdgcn_s_waitcnt(0x0F70 | (MADD && !ENTRIES ? NDMA_KV : NDMA));
         __builtin_amdgcn_s_barrier();        // phase switch: this wave takes the matrix core
         __builtin_amdgcn_sched_barrier(0);
 
@@ -1104,8 +1138,11 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         }
         __builtin_amdgcn_s_setprio(0);
         // (additive mask: the entries of the next step, requested ahead of this step's K/V loads, have landed)
-        if constexpr (MF32) __builtin_amdgcn_s_waitcnt(0x0F70);
-        else if constexpr (MADD) __builtin_amdgcn_s_waitcnt(0x0F70 | NDMA_KV);
+        if constexpr (MF32) {
+            if (stage_next) __builtin_amdgcn_s_waitcnt(0x0F70);
+        } else if constexpr (MADD && ENTRIES) {
+            __builtin_amdgcn_s_waitcnt(0x0F70 | NDMA_KV);
+        }
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): every fragment read of this phase has returned
         __builtin_amdgcn_s_barrier();        // phase switch: this wave goes back to the VALU
         __builtin_amdgcn_sched_barrier(0);
@@ -1121,21 +1158,30 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     if (CAUSAL) {
         const int first_hidden_step = (__builtin_amdgcn_readfirstlane(wlim) + 1) / BN;  // tile that holds key wlim + 1 (may lie past the last step); wave-uniform
         hide_from = max(min(first_hidden_step - 1, ragged ? nk - 4 : nsteps), 0) & ~1;
-        if constexpr (MASK) {  // (no causal limit: only a ragged last tile hides keys, the last step if it is visited at all)
+        // (a mask tensor: no causal limit, only a ragged last tile hides keys, the last step if it is visited at all)
+        if constexpr (MASK && !WALK_BITS) hide_from = ragged && nsteps == nk ? max(nsteps - 4, 0) & ~1 : nsteps + 1;
+        if constexpr (WALK_BITS) {
             const int last_group = (nk - 1) / visit_group;
             hide_from = ragged && last_group < 64 && (visits >> last_group) & 1 ? max(nsteps - 4, 0) & ~1 : nsteps + 1;
         }
     }
     int step = 0;
+    if constexpr (SCAN) {  // the tiles the walk begins with that leave the scores of the wave's rows as they are
+        plain_steps = min(plain_steps, min(hide_from, nsteps));
+        for (; step < plain_steps; step += 2) {
+            body(IC<0>{}, IC<0>{}, IC<1>{}, step);
+            body(IC<1>{}, IC<0>{}, IC<1>{}, step + 1);
+        }
+    }
     if (CAUSAL) {
         for (; step < min(hide_from, nsteps); step += 2) {
-            body(IC<0>{}, IC<0>{}, step);
-            body(IC<1>{}, IC<0>{}, step + 1);
+            body(IC<0>{}, IC<0>{}, IC<0>{}, step);
+            body(IC<1>{}, IC<0>{}, IC<0>{}, step + 1);
         }
     }
     for (; step < nsteps; step += 2) {
-        body(IC<0>{}, IC<1>{}, step);
-        body(IC<1>{}, IC<1>{}, step + 1);
+        body(IC<0>{}, IC<1>{}, IC<0>{}, step);
+        body(IC<1>{}, IC<1>{}, IC<0>{}, step + 1);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // every direct-to-LDS load of this wave has landed
     if (wave < kFastWaves / 2) __syncthreads();

@@ -32,7 +32,8 @@ int launch_masked(const AttnArgs& a, hipStream_t stream) {
     const int nq2 = (a.M + kFastRows - 1) / kFastRows;
     b.total_wg = (int)((int64_t)a.total_wg / a.nq * nq2) * a.nsplit;
     dim3 grid((unsigned)b.total_wg), block(kFastThreads);
-    hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1, bool>), grid, block, 0, stream, b, nq2);
+    if (a.scan_top) hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1, bool, false, false, true>), grid, block, 0, stream, b, nq2);
+    else hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1, bool>), grid, block, 0, stream, b, nq2);
     return check_launch("sage_attn_fwd_fast_kernel (bool mask)");
 }
 

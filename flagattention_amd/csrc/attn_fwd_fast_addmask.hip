@@ -1,7 +1,7 @@
 // SageAttention forward for gfx950, pipelined kernel under an additive mask tensor stored as fp16, bf16 or fp32: the
 // instances of attn_fast_kernel.h that stage mask entries of those types (FlagAttention
 // src/flag_attn/sage_attention/attn_qk_int8_per_block.py:37-38,49-50: score + mask entry).  A translation unit of
-// its own: twelve more instances of the kernel.
+// its own: 24 more instances of the kernel.
 #include "attn_fast_kernel.h"
 
 namespace sage {
@@ -14,7 +14,8 @@ int launch_additive(const AttnArgs& a, hipStream_t stream) {
     const int nq2 = (a.M + kFastRows - 1) / kFastRows;
     b.total_wg = (int)((int64_t)a.total_wg / a.nq * nq2) * a.nsplit;
     dim3 grid((unsigned)b.total_wg), block(kFastThreads);
-    hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1, MT>), grid, block, 0, stream, b, nq2);
+    if (a.scan_top) hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1, MT, false, false, true>), grid, block, 0, stream, b, nq2);
+    else hipLaunchKernelGGL((sage_attn_fwd_fast_kernel<D, VT, true, 1, MT>), grid, block, 0, stream, b, nq2);
     return check_launch("sage_attn_fwd_fast_kernel (additive mask)");
 }
 

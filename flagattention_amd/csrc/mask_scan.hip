@@ -7,11 +7,13 @@
 // the block scales, which the attention kernel looks at: `visits` in attn_fast_kernel.h).  Padding and causal masks in additive
 // form, the ones model code builds, leave out their hidden half that way; a row that sees no key at all makes its q-block visit
 // every tile.  A tile of V with an Inf or NaN is visited by all (0 times those is NaN).
+// The scan also tells the tiles whose entries are all 0 (bool: all visible), whose steps need no mask arithmetic: +0 stands for them,
+// -0 for any other tile with 0 as its largest entry.
 //
 // Bound by the bytes of the mask and of V.  A workgroup takes a strip of 16 mask rows, a thread 16 bytes of each of them at a time
 // (16 loads on their way), so that the scan of one [M, N] mask fills the chip; or one 64-key tile of V.
 // B4 H16 M1536 N1536 D128, [B, 1, M, N] bf16 mask (19 MB, V 25 MB) with causal and padding in one: attention 102 us -> scan 12
-// and attention 56; quantization and attention 117.5 -> 90.7 us.  B1 H32/8 M2560 N2560, bool: 150 -> 77 us; B2 H24 M3840 N3840
+// and attention 53; quantization and attention 117.5 -> 87.9 us (89.7 with entries taken in every step).  B1 H32/8 M2560 N2560, bool: 150 -> 77 us; B2 H24 M3840 N3840
 // D64, fp32 entries (118 MB): 301 -> 200 us.
 #include <type_traits>
 
@@ -69,6 +71,19 @@ __device__ __forceinline__ float chunk_max(uint4 w, int live) {
     return m;
 }
 
+// do all entries of a 16-byte chunk leave their scores as they are?  (additive: zeros of either sign; bool: non-zero bytes)
+template <typename MT>
+__device__ __forceinline__ bool chunk_plain(uint4 w) {
+    const unsigned word[4] = {w.x, w.y, w.z, w.w};
+    unsigned changes = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if constexpr (sizeof(MT) == 1) changes |= (word[i] - 0x01010101u) & ~word[i] & 0x80808080u;  // a zero byte sets bits from its own up
+        else changes |= word[i] & (sizeof(MT) == 4 ? 0x7fffffffu : 0x7fff7fffu);
+    }
+    return changes == 0;
+}
+
 template <typename MT>
 __device__ __forceinline__ void scan_strip(const ScanArgs& a, int wg) {
     constexpr int E = 16 / sizeof(MT), LPT = BN / E;  // entries per chunk; chunks (lanes) per tile
@@ -83,6 +98,7 @@ __device__ __forceinline__ void scan_strip(const ScanArgs& a, int wg) {
     for (int c0 = 0; c0 < chunks; c0 += kScanThreads) {
         const int c = c0 + tid, live = a.N - c * E;  // entries of the chunk that are keys
         float t = -INFINITY;
+        bool plain = live >= E;
         if (live > 0) {
             uint4 w[kScanRows];
 #pragma unroll
@@ -93,10 +109,15 @@ __device__ __forceinline__ void scan_strip(const ScanArgs& a, int wg) {
                 const float m = chunk_max<MT>(w[r], live);
                 row[r] = fmaxf(row[r], m);
                 t = fmaxf(t, m);
+                plain &= chunk_plain<MT>(w[r]);
             }
         }
 #pragma unroll
-        for (int x = 1; x < LPT; x <<= 1) t = fmaxf(t, __shfl_xor(t, x));
+        for (int x = 1; x < LPT; x <<= 1) {
+            t = fmaxf(t, __shfl_xor(t, x));
+            plain &= __shfl_xor((int)plain, x) != 0;
+        }
+        if (t == 0.0f) t = plain ? 0.0f : -0.0f;
         const int tile = c / LPT;
         if (c < chunks && c % LPT == 0) {
             // (additive: the last tile of a kv_len that is not a multiple of 64 also holds keys that score -1e6)

@@ -172,6 +172,35 @@ def test_what_the_scan_finds(kind, mask_dt, shape):
 
 
 @gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("mask_dt", [torch.bool, torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n", [832, 896, 800])
+@pytest.mark.parametrize("rows", ["all", "one"])
+def test_tiles_that_the_mask_leaves_as_they_are(rows, n, mask_dt, d):
+    """No tile is hidden, one entry changes a score: in every tile it is found where it is (waves of other rows take the steps
+    without entries before it, that wave up to it: odd and even numbers of them), and the results are those of the full walk bit for
+    bit.  The first mask of each changes nothing at all (additive: zeros of both signs)."""
+    b, h, m = 2, 48, 768
+    dt = torch.float16 if mask_dt is torch.float16 else torch.bfloat16
+    x = _inputs(b, h, 2, m, n, d, dt, True)
+    zero = torch.ones(b, 1, m, n, dtype=torch.bool, device="cuda:0") if mask_dt is torch.bool else torch.zeros(b, 1, m, n, dtype=mask_dt, device="cuda:0")
+    if mask_dt is not torch.bool:
+        zero[:, :, ::3] = -0.0
+    plain = None
+    for t in [None, *range(n // 64), (n - 1) // 64]:
+        mask = zero.clone()
+        if t is not None:
+            where = (1, 0, slice(None) if rows == "all" else 300 + 7 * t, 64 * t + (5 * t + 3) % 32)
+            mask[where] = False if mask_dt is torch.bool else 9.0
+        (o, lse), (o_all, lse_all) = _both(*x, mask, True)
+        assert torch.equal(o, o_all) and torch.equal(lse, lse_all), t
+        if t is None:
+            plain = lse
+        elif mask_dt is not torch.bool:
+            assert (lse[1, :, where[2]] > plain[1, :, where[2]]).any() and torch.equal(lse[0], plain[0])
+
+
+@gpu
 @pytest.mark.parametrize("mask_dt", [torch.bool, torch.bfloat16, torch.float16])
 def test_scan_nonfinite(mask_dt):
     """Inf / NaN in V under hidden keys, in a block scale, in a mask entry; scales so large that no entry hides a key."""
