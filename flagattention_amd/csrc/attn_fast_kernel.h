@@ -463,6 +463,25 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
         visit_g = more && !same ? g : visit_g;
         return more ? next : t;
     };
+    static_assert(kFastRows / kScanRows == 16, "a row of lanes per q-block's strips");
+    auto row_min = [](float x) {  // the smallest of a row of 16 lanes
+        auto step = [&](auto cc) {
+            const int y = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(cc)::value, 0xf, 0xf, true);
+            x = fminf(x, __builtin_bit_cast(float, y));
+        };
+        step(IC<0x121>{}); step(IC<0x122>{}); step(IC<0x124>{}); step(IC<0x128>{});  // row_ror 1, 2, 4, 8
+        return x;
+    };
+    // the largest of the wave's values, none of them negative
+    auto wave_max = [](float x) {
+        auto step = [&](auto cc) {
+            const int y = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(cc)::value, 0xf, 0xf, true);
+            x = fmaxf(x, __builtin_bit_cast(float, y));
+        };
+        step(IC<0x111>{}); step(IC<0x112>{}); step(IC<0x114>{}); step(IC<0x118>{});  // row_shr 1, 2, 4, 8: lane 15 of a row of 16 holds its maximum
+        step(IC<0x142>{}); step(IC<0x143>{});                                      // row_bcast 15, 31: lane 63 all of them
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
+    };
     if constexpr (MASK && !WALK_BITS) {
         vt1 = next_tile(vt0, nsteps > 1);
         vt2 = next_tile(vt1, nsteps > 2);
@@ -475,32 +494,36 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
             const int mb = a.ms_b ? b : 0;
             const int s0 = a.ms_m ? (kFastRows / kScanRows) * iq : 0, s1 = min(s0 + kFastRows / kScanRows, a.scan_strips);
             const float* tops = a.scan_top + (int64_t)mb * a.scan_strips * a.nk;
-            float low = a.scan_low[(int64_t)mb * a.scan_strips + min(s0 + (lane & (kFastRows / kScanRows - 1)), s1 - 1)];
-#pragma unroll
-            for (int x = 1; x < kFastRows / kScanRows; x <<= 1) low = fminf(low, __shfl_xor(low, x));
-            hidden_row = __builtin_amdgcn_readfirstlane((int)!(low >= -1.0e4f));
-            if (!MADD) low = 0.0f;  // (a bool tile goes by whether it holds a visible key)
+            // (All of it in one round trip to memory, the maxima by lane moves inside the vector unit: with three round trips and exchanges
+            // through LDS a workgroup took 5 us to get here, without a scan 1.6.  B4 H16 N1536 causal and padded, whole step: D128 bf16
+            // 88.2 -> 86.1 us, fp32 94.4 -> 91.5, D64 bf16 68.5 -> 67.2; N2048 bf16 padding 142.8 -> 139.8.)
             const int64_t kv_row = ((int64_t)b * a.Hkv + hk) * a.nk;
+            float low = a.scan_low[(int64_t)mb * a.scan_strips + min(s0 + (lane & (kFastRows / kScanRows - 1)), s1 - 1)];
             float top = -INFINITY, ks_max = 0.0f;
             unsigned own = 0;  // of the wave's own strips, bit by bit
             bool odd = false;
-            for (int r = 0; r < visit_group; r++) {
+            auto look = [&](int r) {
                 const int t = min(lane * visit_group + r, a.nk - 1);
-                const float ks = fabsf(a.k_scale[kv_row + t]);  // (a caller's own scales may be negative)
-                odd |= !(ks < 3.0e38f) || a.scan_v[kv_row + t] != 0;
-                ks_max = fmaxf(ks_max, ks);
                 float e[kFastRows / kScanRows];
 #pragma unroll
                 for (int x = 0; x < kFastRows / kScanRows; x++) e[x] = tops[(int64_t)min(s0 + x, s1 - 1) * a.nk + t];
+                const float ks = fabsf(a.k_scale[kv_row + t]);  // (a caller's own scales may be negative)
+                const unsigned v_odd = a.scan_v[kv_row + t];  // (not behind a branch: that would be a second round trip)
+                asm volatile("" :: "v"(v_odd));
+                odd |= !(ks < 3.0e38f) || v_odd != 0;
+                ks_max = fmaxf(ks_max, ks);
 #pragma unroll
                 for (int x = 0; x < kFastRows / kScanRows; x++) {
                     top = fmaxf(top, e[x]);
                     own |= x / (32 / kScanRows) == wave_u ? __builtin_bit_cast(unsigned, e[x]) : 0u;
                 }
-            }
+            };
+            look(0);
+            for (int r = 1; r < visit_group; r++) look(r);
+            low = row_min(low);
+            hidden_row = __builtin_amdgcn_readfirstlane((int)!(low >= -1.0e4f));
+            if (!MADD) low = 0.0f;  // (a bool tile goes by whether it holds a visible key)
             if (visit_group == 1) plain = __builtin_amdgcn_ballot_w64(own == 0);
-#pragma unroll
-            for (int x = 1; x < 64; x <<= 1) ks_max = fmaxf(ks_max, __shfl_xor(ks_max, x));
             float bound = 0.0f;  // largest difference of two scores of a row
             if constexpr (MADD) {
                 unsigned sum = 0;  // of the row's |q|, byte by byte
@@ -508,18 +531,16 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
                 for (int t = 0; t < F::KSTEPS; t++)
 #pragma unroll
                     for (int i = 0; i < 4; i++) sum = __builtin_amdgcn_sad_u8((unsigned)qf[t][i] ^ 0x80808080u, 0x80808080u, sum);
-                sum += __shfl_xor(sum, 32);
-                float q_sum = (float)sum * fabsf(qs);
-#pragma unroll
-                for (int x = 1; x < 32; x <<= 1) q_sum = fmaxf(q_sum, __shfl_xor(q_sum, x));
+                const v2u halves = __builtin_amdgcn_permlane32_swap(sum, sum, false, false);
+                const unsigned lower = halves[0], upper = halves[1];
+                float q_sum = wave_max((float)(lower + upper)) * fabsf(qs);
                 if (!(fabsf(qs) < 3.0e38f)) q_sum = INFINITY;
-                float* sums = reinterpret_cast<float*>(smem);  // (nothing is on its way into the tile buffers yet)
+                float* sums = reinterpret_cast<float*>(smem + F::V_BASE + (F::NBUF - 1) * F::V_BYTES);  // (filled in step 1 for the first time)
                 if (lane == 0) sums[wave] = q_sum;
                 __syncthreads();
 #pragma unroll
                 for (int w = 0; w < kFastWaves; w++) bound = fmaxf(bound, sums[w]);
-                bound *= 256.0f * ks_max;
-                __syncthreads();
+                bound *= 256.0f * wave_max(ks_max);
             }
             const bool skip = top < low - 150.0f - bound && !odd;  // (bound NaN: 0 times infinity)
             visits = ~__builtin_amdgcn_ballot_w64(skip);
