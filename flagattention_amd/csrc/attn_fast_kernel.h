@@ -301,8 +301,8 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     // indexed by compile-time constants).  tests/test_host_cpu.py compiles this file to assembly and fails if
     // anything but these moves mentions m0.
     auto dma16 = [](const unsigned char* base, unsigned voff, unsigned lds_addr) {
-        if constexpr (SCAN && D == 128)  // (short of scalar registers: the second clobber keeps the address out of vcc, so that every
-                                         // move into m0 names an s register; at head_dim 64 it would cost 1 to 2 %)
+        if constexpr (QB == 2 && D == 128 && CAUSAL)  // (short of scalar registers: the second clobber keeps the address out of vcc, so
+                                                      // that every move into m0 names an s register)
             asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                          :: "v"(voff), "s"(base), "s"(lds_addr) : "memory", "vcc");
         else
