@@ -22,9 +22,10 @@
 // * workgroups are handed out longest first over all heads.
 // B4 H16 M2048 N2048 D64 fp16 causal 397 -> 143 us, without the causal flag 404 -> 272 us; B2 H32 M4096 N4096 D128 3475 -> 1207
 // us, causal 3445 -> 619 us (before: the generator rolled out by the compiler, V^T gathered from LDS entry by entry,
-// short rows first).  With xor3 120, 226, 1114 and 573 us, with reference points that move only when they have to 114, 214, 1058 and
-// 547 us, with three waves per SIMD at head_dim 128 (two before: the addends of the counters' products took 30 vector registers)
-// 111, 214, 994 and 519 us.
+// short rows first).  With xor3, the addends of the counters' products in scalar registers (30 vector registers less at head_dim
+// 128) and an exchange of row maxima only where a tile raises one 119, 224, 1031 and 536 us.  Reference points that lag behind
+// the maximum of their row by up to 2^8 would make it 112, 212, 977 and 505 us, but P is then rounded at another place than where its
+// row's largest is exactly 1, and the error of the output grows by 2 to 23 %.
 #include "attn_common.h"
 
 namespace sage {
@@ -78,7 +79,6 @@ struct DropArgs {
 constexpr int kDropWaves = 4;  // 128 queries per workgroup
 constexpr int kDropThreads = 64 * kDropWaves;
 constexpr int kDropKeys = 32;  // keys per tile
-constexpr float kNoScore = -3.0e38f;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -137,7 +137,8 @@ template <int D> __device__ __forceinline__ int drop_v_swizzle(int row) { return
 // KG: groups of four waves that share the queries of a workgroup and take its key tiles in turn (drop_groups).  The second
 // launch bound is waves per SIMD, whatever KG is: with fewer asked for, two groups at head_dim 64 took 132 registers and one
 // workgroup filled a CU (B1 H32 M2048 N2048 D64 153 -> 140 us, causal 107 -> 80 us, B4 H16 M1024 N1024 83 -> 77 and 58 -> 45
-// us; three at head_dim 128: B2 H32 M4096 N4096 1058 -> 994 us).
+// us; three instead of two at head_dim 128: 131 -> 120 us for B3 H16 M2048 N2048 causal, whose blocks are then resident at once, 85 ->
+// 80 us for M1500; nothing in longer launches, B2 H32 M4096 N4096 1028 and 1031 us).
 constexpr int drop_waves_per_simd(int head_dim) { return head_dim == 128 ? 3 : 4; }
 
 // WIDE: the rows of a K or V tile lie further apart than 32-bit byte offsets reach, or in descending order (64-bit
@@ -160,7 +161,8 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
     const int l32 = lane & 31, half = lane >> 5;
     // heads fastest (a head stays on one XCD); under the causal flag the last queries, which see the most keys, first
     // (snake: all workgroups are resident at once, so every second round of 256, one per CU, goes in the reverse order of
-    // blocks and a CU holds long and short ones: B4 H16 M2048 N2048 D64 causal 177 -> 166 us, B3 H16 M2048 N2048 D128 124 -> 112)
+    // blocks and a CU holds long and short ones: B4 H16 M2048 N2048 D64 causal 177 -> 166 us, B3 H16 M2048 N2048 D128
+    // 132 -> 120)
     const int bh = blockIdx.x % a.BH;
     int rank = blockIdx.x / a.BH;
     if (a.snake > 0 && a.snake < a.nmb && a.nmb < 2 * a.snake) {
@@ -258,9 +260,7 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
     for (int dt = 0; dt < DT; dt++)
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[dt][i] = 0.0f;
-    // the row's reference point (in units of the exponent; below every score until the row has seen a key) and this half's part of
-    // the row sum
-    float m_i = kNoScore, l_i = 0.0f;
+    float m_i = -INFINITY, l_i = 0.0f;  // running maximum (unscaled scores) and this half's part of the row sum
 
     if (group < ntiles) fetch(group, 0);
     const int rounds = (ntiles + KG - 1) / KG;
@@ -292,11 +292,12 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
         float tile_max = -INFINITY;
 #pragma unroll
         for (int i = 0; i < 16; i++) tile_max = fmaxf(tile_max, s[i]);
-        // The reference point of a row moves only when the larger half of a P would pass 2^kTau: most tiles end the matter here, without
-        // the exchange between the two lanes of a row.
-        if (__builtin_amdgcn_ballot_w64(__builtin_fmaf(tile_max, a.qk_scale, -m_i) > kTau) != 0) {
-            const float m_new = fmaxf(m_i, fmaxf(tile_max, __shfl_xor(tile_max, 32)) * a.qk_scale);
-            const float alpha = __builtin_amdgcn_exp2f(m_i - m_new);
+        // A row's exponentials are taken against its maximum so far, so that its largest P is exactly 1 in 16 bits: the row sum adds P
+        // before they are rounded.  A tile that raises no row of the wave needs no exchange between the two lanes of a row (1 %).
+        if (__builtin_amdgcn_ballot_w64(tile_max > m_i) != 0) {
+            const float m_new = fmaxf(m_i, fmaxf(tile_max, __shfl_xor(tile_max, 32)));
+            // (a query that has seen no key yet keeps m = -inf: every p below is then 0)
+            const float alpha = m_i == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(__builtin_fmaf(m_i, a.qk_scale, -(m_new * a.qk_scale)));
             l_i *= alpha;
 #pragma unroll
             for (int dt = 0; dt < DT; dt++)
@@ -304,6 +305,7 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
                 for (int i = 0; i < 16; i++) acc[dt][i] *= alpha;
             m_i = m_new;
         }
+        const float m_use = m_i == -INFINITY ? 0.0f : m_i * a.qk_scale;
         // ---- P, its row sum (which does not see the dropout mask), and the mask
         const uint64_t first = rng_row + (uint64_t)n0;
         const uint32_t lo = (uint32_t)first;
@@ -315,8 +317,8 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
         uint32_t pbits[8];
         // two scores and the signs of their words (bit 31 set: dropped) -> two 16-bit P
         auto put = [&](int i, int32_t sign0, int32_t sign1) {
-            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.qk_scale, -m_i));  // hidden keys: exp2(-inf) = 0
-            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], a.qk_scale, -m_i));
+            const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], a.qk_scale, -m_use));  // hidden keys: exp2(-inf) = 0
+            const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], a.qk_scale, -m_use));
             psum += p0;
             psum += p1;
             typedef VT vt2 __attribute__((ext_vector_type(2)));
@@ -369,13 +371,14 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
             row_l[group * 32 * kDropWaves + slot] = l_tot;
         }
         __syncthreads();
-        float m = kNoScore, l = 0.0f;
+        float m = -INFINITY, l = 0.0f;
 #pragma unroll
         for (int g = 0; g < KG; g++) m = fmaxf(m, row_m[g * 32 * kDropWaves + slot]);
+        const float base = m == -INFINITY ? 0.0f : m * a.qk_scale;
 #pragma unroll
         for (int g = 0; g < KG; g++)
-            l += row_l[g * 32 * kDropWaves + slot] * __builtin_amdgcn_exp2f(row_m[g * 32 * kDropWaves + slot] - m);
-        const float mine = __builtin_amdgcn_exp2f(m_i - m);
+            l += row_l[g * 32 * kDropWaves + slot] * __builtin_amdgcn_exp2f(__builtin_fmaf(row_m[g * 32 * kDropWaves + slot], a.qk_scale, -base));
+        const float mine = __builtin_amdgcn_exp2f(__builtin_fmaf(m_i, a.qk_scale, -base));
         float* park = reinterpret_cast<float*>(&smem[0][0][0][0]) + wave * 32 * D + lane;  // entry e of a lane: 64 e further on
 #pragma unroll
         for (int dt = 0; dt < DT; dt++)
@@ -426,7 +429,7 @@ __global__ __launch_bounds__(kDropThreads * KG, drop_waves_per_simd(D)) void fla
         }
     if (a.log_normalizer && half == 0)
         a.log_normalizer[((int64_t)b * a.Hq + h) * a.M + my_m] =
-            l_tot != 0.0f ? (__builtin_log2f(l_tot) + m_i) * 0.693147180559945309f : -INFINITY;
+            l_tot != 0.0f ? (__builtin_log2f(l_tot) + m_i * a.qk_scale) * 0.693147180559945309f : -INFINITY;
 }
 
 __global__ void dropout_mask_kernel(uint8_t* mask, int64_t count, uint64_t offset, uint32_t seed_lo, uint32_t seed_hi,
@@ -437,7 +440,7 @@ __global__ void dropout_mask_kernel(uint8_t* mask, int64_t count, uint64_t offse
 
 // Groups of waves per workgroup: as many as the SIMDs hold waves for, where there are fewer workgroups than that takes (a
 // SIMD with one wave issues a vector instruction every 5.7 cycles, with four waves every 3).  Two at most at head_dim 128, up to 256
-// workgroups (three groups: B1 H4 M4096 N4096 137 -> 128 us, but B1 H8 M512 N512 23.9 -> 24.8).
+// workgroups (three groups: B1 H4 M4096 N4096 148 -> 140 us, but B1 H8 M512 N512 25.0 -> 25.8).
 int drop_groups(int64_t wgs, int head_dim) {
     int groups = 1;
     while (2 * groups <= drop_waves_per_simd(head_dim) && wgs * 2 * groups <= 256 * (drop_waves_per_simd(head_dim) & ~1)) groups *= 2;
