@@ -332,13 +332,22 @@ def test_only_the_lds_load_sequence_touches_m0(tmp_path):
     only as the destination of the s_mov_b32 that precedes each direct-to-LDS load."""
     import re
     import subprocess
+    from concurrent.futures import ThreadPoolExecutor
 
     csrc = os.path.join(ROOT, "flagattention_amd", "csrc")
-    for unit in ("attn_fwd_fast.hip", "attn_fwd_fast_addmask.hip", "flash_fwd.hip", "flash_dropout.hip", "total_attention.hip"):
+    units = ("attn_fwd_fast.hip", "attn_fwd_fast_addmask.hip", "attn_fwd_fast_addcausal.hip", "flash_fwd.hip", "flash_dropout.hip",
+             "total_attention.hip")
+
+    def assembly(unit):
         out = tmp_path / (unit + ".s")
         subprocess.run(["/opt/rocm/bin/hipcc", "-O3", "-std=c++17", "--offload-arch=gfx950", "-ffp-contract=off", "-Xclang",
                         "-target-feature", "-Xclang", "-packed-fp32-ops", "-S", "--cuda-device-only", "-o", str(out),
                         os.path.join(csrc, unit)], check=True, capture_output=True, timeout=600)
+        return out
+
+    with ThreadPoolExecutor(4) as pool:
+        outs = list(pool.map(assembly, units))
+    for unit, out in zip(units, outs):
         mentions = [ln.strip() for ln in out.read_text().splitlines() if re.search(r"\bm0\b", ln.split(";")[0])]
         assert mentions, "expected the direct-to-LDS load sequence in " + unit
         other = [ln for ln in mentions if not re.fullmatch(r"s_mov_b32 m0, s\d+", ln)]
