@@ -63,6 +63,9 @@ def _mask(kind, dt, b, m, n):
         keep = (torch.rand(b, 1, m, n, generator=g) < 0.3) & ((cols // 64) % 3 != 1)
     elif kind == "none":
         keep = torch.zeros(1, 1, m, n, dtype=torch.bool)
+    elif kind == "all":  # nothing hidden; one row of all takes one key away in two tiles, the ragged last one is left whole
+        keep = torch.ones(1, 1, m, n, dtype=torch.bool)
+        keep[0, 0, m - 1, 70] = keep[0, 0, 5, 200] = False
     elif kind == "slope":  # a steep linear bias, no hidden keys
         return (-(rows - cols).abs().float() * 3.0).view(1, 1, m, n).to(dt).to(dev)
     if dt is torch.bool:
@@ -130,16 +133,19 @@ def test_scan_changes_nothing(shape, mask_dt, kind):
 @gpu
 @pytest.mark.parametrize("shape", [(2, 4, 2, 300, 3072, 64, True), (3, 48, 2, 520, 1808, 64, True)])
 @pytest.mark.parametrize("mask_dt", [torch.bool, torch.float16, torch.float32])
-@pytest.mark.parametrize("kind", ["padding", "causal_padding", "slope"])
+@pytest.mark.parametrize("kind", ["padding", "causal_padding", "slope", "all"])
 def test_what_the_scan_finds(kind, mask_dt, shape):
     """The scan's results as it leaves them in the workspace, and that the rule of the attention kernel, applied to them here,
-    leaves out every tile that padding or the causal mask hides from a whole q-block."""
+    leaves out every tile that padding or the causal mask hides from a whole q-block.  Where the largest entry of a tile is 0 its sign
+    tells whether the tile is whole and every entry a zero of either sign (bool: visible): +0 for those, -0 for the others."""
     if mask_dt is torch.bool and kind == "slope":
         pytest.skip("not a bool mask")
     b, h, hkv, m, n, d, hnd = shape
     q8, qs, k8, ks, v = _inputs(b, h, hkv, m, n, d, torch.float16, hnd)
     v[1, 0, n - 1, 3], v[0, 1, 70, 9] = float("inf"), float("nan")
     mask = _mask(kind, mask_dt, b, m, n)
+    if mask_dt is not torch.bool and kind != "slope":
+        mask = torch.where((mask == 0) & (torch.arange(n, device=mask.device) % 3 == 0), torch.full_like(mask, -0.0), mask)
     o, lse = torch.empty(q8.shape, device=q8.device), torch.empty(b, h, m, device=q8.device)
     p = _params(q8, qs, k8, ks, v, mask, o, lse, KIND[mask_dt], hnd)
     lib = _lib.load()
@@ -159,6 +165,9 @@ def test_what_the_scan_finds(kind, mask_dt, shape):
     if mask_dt is not torch.bool and n % 64:
         tiles[..., -1].clamp_(min=-1.0e6)
     assert torch.equal(top, tiles) and torch.equal(low, e.view(mb, strips, 16, -1).amax(-1).amin(-1))
+    unchanged, zero = (e == 0).view(mb, strips, 16, nk, 64).all(4).all(2), tiles == 0
+    assert torch.equal(torch.signbit(top)[zero], ~unchanged[zero])
+    assert bool(unchanged.any()) == (kind != "slope") and (bool((zero & ~unchanged).any()) or kind in ("padding", "slope"))
     bad = ~torch.isfinite(torch.nn.functional.pad(v, (0, 0, 0, nk * 64 - n)).view(b, hkv, nk, 64 * d)).all(-1)
     assert torch.equal(odd != 0, bad)
     # the rule: 256-row q-blocks, the largest scales and sums of |q| of the call (a bound above that of every block)
@@ -168,7 +177,7 @@ def test_what_the_scan_finds(kind, mask_dt, shape):
     left = torch.stack([top[:, s].amax(1) < (0.0 if mask_dt is torch.bool else low[:, s].amin(1, keepdim=True)) - 150.0 - bound for s in blocks], 1)
     hidden = torch.stack([tiles[:, s].amax(1) < -1e4 for s in blocks], 1)
     assert torch.equal(left, hidden) if kind != "slope" else not hidden.any()
-    assert left.float().mean() > {"padding": 0.3, "causal_padding": 0.3, "slope": 0.0}[kind]
+    assert left.float().mean() > {"padding": 0.3, "causal_padding": 0.3, "slope": 0.0, "all": -1.0}[kind]
 
 
 @gpu
