@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
     (3, 16, 16, 700, 97, 128, True),   # 288 blocks at head_dim 128: one
     (1, 16, 16, 130, 300, 128, False),
     (1, 24, 8, 1700, 97, 64, True), (1, 20, 20, 1700, 40, 128, True),  # a second round of blocks on some of the CUs
+    (3, 16, 16, 1300, 1300, 128, True),  # 528 blocks at head_dim 128, rounds of 5 per head, the third one partial; no row without a key
 ])
 def test_dropout_forward_tiles(B, H, Hk, M, N, D, causal, p, offset, gpu_device):
     import flag_attn
@@ -66,7 +67,7 @@ def test_dropout_forward_keeps_nan(B, H, M, N, D, causal, p, gpu_device):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_dropout_forward_reference_point(B, H, M, N, D, causal, rise, dtype, gpu_device):
     """Scores whose level rises (falls) by 12 log2 units from one 32-key tile to the next, so that the reference point of a row has to
-    move with every tile (stays at the first one); the last shape fills three rounds of 128-query blocks at head_dim 128."""
+    move with every tile (stays at the first one); the last shape takes one group of waves, four rounds of 128-query blocks."""
     import math
 
     import flag_attn
