@@ -447,9 +447,10 @@ __global__ __launch_bounds__(kFastThreads, kFastWgPerCu) void sage_attn_fwd_fast
     //      SCAN: instances of their own for scanned masks; the others walk over every tile without any of this (B4 H16 N1536 D64
     //      bool 88.5 -> 86.8 us, D64 fp16 bias 91.4 -> 88.8, D128 bf16 bias 116.5 -> 114.9).  WALK_BITS: in the causal instances at
     //      head_dim 128 the words of bits cost nothing and dropping them three more spilled registers (85.1 -> 85.4 us).
-    //      Bit t of `plain` (visit_group = 1): tile t leaves the scores of this wave's rows as they are (scan: +0).  The steps the
-    //      walk begins with, as long as that holds (masks that hide keys past a limit: most of them), neither read nor stage entries,
-    //      half of the bytes a step brings into LDS, and have no mask arithmetic, a third of the vector phase: B4 H16 N1536 causal and
+    //      Bit t of `plain` (visit_group = 1; with several tiles to a bit every step takes its entries): tile t leaves the scores of
+    //      this wave's rows as they are (scan: +0).  The steps the walk begins with, as long as that holds (masks that hide keys past a
+    //      limit: most of them), read no entries and have no mask arithmetic, a third of the vector phase, and additive entries are not
+    //      staged for them, half of the bytes a step brings into LDS (bool ones are, in every step): B4 H16 N1536 causal and
     //      padded, whole step, D128 bf16 89.7 -> 87.9 us, D64 fp32 75.7 -> 71.5; B1 H32/8 N4096 D128 fp16 167 -> 152, bool 155 -> 147;
     //      B4 H16 N2048 bf16 padding 155 -> 146.  (Chosen per step the two bodies cost 76 to 169 spilled registers, as a branch
     //      around the exponentials alone 3 % wherever entries are needed.)

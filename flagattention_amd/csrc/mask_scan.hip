@@ -12,9 +12,11 @@
 //
 // Bound by the bytes of the mask and of V.  A workgroup takes a strip of 16 mask rows, a thread 16 bytes of each of them at a time
 // (16 loads on their way), so that the scan of one [M, N] mask fills the chip; or one 64-key tile of V.
-// B4 H16 M1536 N1536 D128, [B, 1, M, N] bf16 mask (19 MB, V 25 MB) with causal and padding in one: attention 102 us -> scan 12
-// and attention 53; quantization and attention 117.5 -> 87.9 us (89.7 with entries taken in every step).  B1 H32/8 M2560 N2560, bool: 150 -> 77 us; B2 H24 M3840 N3840
-// D64, fp32 entries (118 MB): 301 -> 200 us.
+// 10 to 25 us at 4 TB/s (4.7 is a copy's); taking note of the zeros costs it nothing that shows (bool B4 N1536 10.1 -> 10.3 us, B1
+// N4096 12.4 -> 11.6, at 125 registers and four waves per SIMD; bf16 12.4 -> 12.5 and 15.0 -> 15.4).
+// Attention call without the scan -> with it, launch and all: B4 H16 M1536 N1536 D128, [B, 1, M, N] bf16 mask (19 MB, V 25 MB) with
+// causal and padding in one 96 -> 66 us; B1 H32/8 M2560 N2560 D128, causal, bool 135 -> 76; B2 H24 M3840 N3840 D64, causal and
+// padding, fp32 entries (118 MB) 270 -> 134 us.
 #include <type_traits>
 
 #include "attn_common.h"
@@ -223,22 +225,26 @@ int mask_splits(const AttnArgs& a, int64_t batch, int head_dim) {
 // rule, and read once either way) and enough steps can go.  What it costs (a launch, the bytes of the mask and of V, 1 to 2 us in
 // every workgroup) a mask that hides no tile loses; what it gains lies in the entries, which the rule does not see.  The lines lie
 // where the masks that model code builds gain, a causal one or the padding of sequences between half as long and as long as the
-// keys.  Attention call with the scan over the one without (mean of 1060 shapes: 2 to 32 heads, 1 to 8 sequences, 512 to 8192 keys):
-//   more q-blocks than compute units       hides nothing  causal  causal and padding
-//     entries per row, 8 to 12 tiles         1.16 - 1.24    0.85    0.85
-//     14 to 20                               1.11 - 1.20    0.76    0.76
-//     24 to 32                               1.05 - 1.11    0.72    0.71
-//     from 36                                0.98 - 1.09    0.62    0.61
-//   more q-blocks than compute units       hides nothing  padding
-//     one row of entries, 8 to 24 tiles      1.08 - 1.23    1.04    (not scanned; 0.83 to 1.20)
-//     from 28                                1.02 - 1.11    0.92
-//     causal mask folded into a bool one, whose walk ends at the limit anyway: padding 1.02 up to 30 tiles (not scanned; 0.90 to
-//     1.11), 0.95 from 36
+// keys.  Attention call with the scan over the one without, every shape run both ways (means of 2500 shapes, in brackets the
+// tenths of them at either end: 2 to 32 heads, 1 to 8 sequences, 512 to 8192 keys; "entries" change a score in every tile,
+// "zeros" in none):
+//   more q-blocks than compute units   entries             zeros               causal              causal and padding
+//     rows of entries, 8 to 11 tiles   1.29 (1.24 - 1.34)  1.22 (1.17 - 1.27)  0.92 (0.81 - 1.05)  0.91 (0.80 - 1.03)  (not scanned)
+//     12 to 20                         1.22 (1.17 - 1.28)  1.12 (1.06 - 1.18)  0.81 (0.69 - 0.93)  0.79 (0.68 - 0.92)
+//     21 to 35                         1.16 (1.11 - 1.21)  1.04 (0.98 - 1.09)  0.68 (0.59 - 0.76)  0.66 (0.54 - 0.74)
+//     36 to 64                         1.13 (1.08 - 1.21)  0.99 (0.92 - 1.06)  0.59 (0.52 - 0.67)  0.55 (0.45 - 0.65)
+//     65 to 128                        1.17 (1.08 - 1.31)  1.17 (1.08 - 1.32)  0.67 (0.59 - 0.81)  0.61 (0.48 - 0.78)
+//   more q-blocks than compute units   entries             zeros               padding
+//     one row of entries, 8 to 27      1.19 (1.13 - 1.27)  1.09 (1.00 - 1.20)  0.99 (0.84 - 1.16)  (not scanned)
+//     28 to 64                         1.11 (1.08 - 1.14)  0.96 (0.89 - 1.02)  0.82 (0.67 - 0.94)
+//     65 to 128                        1.08 (1.06 - 1.10)  1.08 (1.06 - 1.10)  0.91 (0.69 - 1.05)
+//     causal mask folded into a bool one, whose walk ends at the limit anyway, 8 to 35 tiles 1.13 (0.98 - 1.33) with padding (not
+//     scanned), 0.80 (0.59 - 1.13) from 36
 //   fewer, unsplit, 48 us of steps and more: the longest q-block alone counts, which a causal mask does not shorten and padding
 //   seldom where there are several sequences, the longest of which is nearly full
-//                                          hides nothing  causal  causal and padding
-//     one sequence                           1.05 - 1.20    1.12    0.92
-//     two to eight                           1.08 - 1.20    1.12    1.05    (not scanned)
+//                                      entries             causal              causal and padding
+//     one sequence                     1.18 (1.13 - 1.25)  1.09 (0.95 - 1.19)  0.87 (0.71 - 1.06)
+//     two to eight                     1.30 (1.18 - 1.43)  1.19 (1.04 - 1.36)  1.07 (0.86 - 1.27)  (not scanned)
 // V is read once more, so the queries per K/V head have to be many as well.
 int64_t mask_scan_bytes(const AttnArgs& a, int64_t batch, int head_dim) {
     const int64_t q_blocks = batch * a.Hq * ((a.M + kFastRows - 1) / kFastRows);
